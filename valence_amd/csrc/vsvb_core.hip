@@ -187,6 +187,24 @@ __global__ void k_prim_screen(Pair* __restrict__ pairs, int np, const Shell* __r
   pairs[t].npp = k;
 }
 
+// Segments of the shell pairs: consecutive parts of a pair's screened primitive
+// list, each a work pair of its own (the contracted integral is the sum over
+// bra segments x ket segments, and the contraction with the densities is linear
+// in it).  The parent's Schwarz bound comes along, so a quartet of segments is
+// screened exactly as the quartet of its parents.
+__global__ void k_split(const Pair* __restrict__ pairs, const SegSrc* __restrict__ src, int n,
+                        Pair* __restrict__ out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const SegSrc s = src[t];
+  Pair P = pairs[s.pair];
+  const int b = s.seg * P.npp / s.nseg, e = (s.seg + 1) * P.npp / s.nseg;
+  P.pp0 += b;
+  P.npp = e - b;
+  P.seg = s.seg;
+  out[t] = P;
+}
+
 // ---------------------------------------------------------------------------
 // device: one-electron integrals (Obara-Saika), one wavefront per shell pair
 // ---------------------------------------------------------------------------
@@ -970,6 +988,17 @@ static int class_bra(int q) {
   return kNPairClass - 1;
 }
 
+// Algorithmic FP64 operations of the density contraction per contracted quartet.
+static double digestion_flops(int q, int nspin, bool jk) {
+  int bc = 0, kc = 0;
+  for (int b = 0; b < kNPairClass; ++b)
+    for (int k = 0; k <= b; ++k)
+      if (quartet_class_index(b, k) == q) { bc = b; kc = k; }
+  const double nab = ncart(kPairLs[bc][0]) * ncart(kPairLs[bc][1]);
+  const double ncd = ncart(kPairLs[kc][0]) * ncart(kPairLs[kc][1]);
+  return jk ? nab * ncd * (4.0 + 8.0 * nspin) : nab * ncd * (2.0 + 4.0 * nspin) + 2.0 * nab;
+}
+
 // Straight-line kernel: energy units are 64-pair bra tiles x chunks of ket
 // pairs (one wavefront each, four per workgroup); J/K units are 256-pair bra
 // strips x chunks of ket pairs (one workgroup each), with the exchange rows of
@@ -983,9 +1012,49 @@ constexpr double kEnergyUnitsPerWave = 32.0;
 constexpr long long kMaxUnits = (long long)INT32_MAX - (1LL << 24);
 constexpr double kJkUnitsPerBlock = 16.0;
 
+// Work lists of a quartet class.  A lane evaluates its quartet's primitive
+// quartets one after another, about 0.25 us each when few wavefronts share a
+// SIMD (a (ss|ss) quartet of six-fold contracted shells: 1296 of them, 330 us),
+// so a class with few quartets takes segments of its pairs instead: more lanes,
+// each with a shorter chain, for one more density contraction per segment
+// quartet.  Of the nine pairs of levels the one with the least estimated time is
+// taken: the chain of the longest entries, plus the wavefronts per SIMD times
+// the average chain, in units of a primitive quartet, where what a quartet costs
+// beside its primitives is `tail` of them.  The tails are fitted to the class
+// times of all nine pairs of levels on water, C2H6, C3H8, C5H12, C8H18 and the
+// H8 and H12 chains: the pairs chosen sum to 5.43 ms where the best sum to 5.26
+// (energy), 14.2 to 13.5 ms (J/K); whole pairs alone 16.5 and 18.1 ms.
+constexpr double kTailEnergy = 6.0, kTailJk = 45.0, kTailDensity = 25.0;
+static void choose_levels(const vsvb_context* c, int bc, int kc, bool jk, bool tr, int* lb, int* lk) {
+  *lb = *lk = 0;
+  if (c->nlevels < 2 || c->pair_chunk > 0) return;  // a forced chunk width: whole pairs
+  const int q = bc * (bc + 1) / 2 + kc;
+  const int nd = jk ? c->ndens : 1;
+  const double digest = digestion_flops(q, c->nunpd > 0 ? 2 : 1, jk) * nd;
+  const double tail = (jk ? kTailJk + kTailDensity * (nd - 1) : kTailEnergy) +
+                      (kFlopsHrr[q] + digest) / kFlopsPerPrimQuartet[q];
+  double best = 0.0;
+  for (int b = 0; b < c->nlevels; ++b)
+    for (int k = 0; k < c->nlevels; ++k) {
+      if (bc == kc && b != k) continue;
+      const WorkList &B = c->work[bc][b], &K = c->work[kc][k];
+      const WorkList &lane = tr ? K : B, &uni = tr ? B : K;
+      const double tiles = jk ? 4.0 * ((lane.n + kStripB - 1) / kStripB) : (double)((lane.n + kTileB - 1) / kTileB);
+      const double waves = tiles * uni.n * (bc == kc ? 0.5 : 1.0);
+      const double t = B.longest * (double)K.longest + tail + waves / (4.0 * c->ncu) * (B.mean * K.mean + tail);
+      if ((b == 0 && k == 0) || t < best) {
+        best = t;
+        *lb = b;
+        *lk = k;
+      }
+    }
+}
+
 static ClassLaunch straight_launch(vsvb_context* c, int bc, int kc, bool jk, int per_cu, bool lds_on, bool tr) {
   ClassLaunch L;
-  const int nb = c->pair_off[bc + 1] - c->pair_off[bc], nk = c->pair_off[kc + 1] - c->pair_off[kc];
+  L.tr = jk && tr && bc != kc;
+  choose_levels(c, bc, kc, jk, L.tr, &L.lb, &L.lk);
+  const int nb = c->work[bc][L.lb].n, nk = c->work[kc][L.lk].n;
   L.per_cu = per_cu;
   if (nb <= 0 || nk <= 0) return L;
   if (!jk) {
@@ -1000,7 +1069,9 @@ static ClassLaunch straight_launch(vsvb_context* c, int bc, int kc, bool jk, int
            (double)nbt * ((nk + 2 * kch - 1) / (2 * kch)) >= kEnergyUnitsPerWave * 4.0 * cap)
       kch *= 2;
     L.kchunk = kch;
-    const long long units = (long long)nbt * ((nk + kch - 1) / kch);
+    // one-ket units of one class stop at the diagonal: tile t has 64 (t + 1) kets
+    const long long units = kch == 1 && bc == kc ? (long long)kTileB / 2 * nbt * (nbt + 1)
+                                                 : (long long)nbt * ((nk + kch - 1) / kch);
     L.overflow = units > kMaxUnits;
     L.units = L.overflow ? 0 : (int)units;
     // several counter segments once claims are chunked (large systems: many
@@ -1008,9 +1079,15 @@ static ClassLaunch straight_launch(vsvb_context* c, int bc, int kc, bool jk, int
     L.seg_tiles = kch > 1 ? kSegTiles : nbt;
     L.strips = (nbt + L.seg_tiles - 1) / L.seg_tiles;
     L.blocks = std::min((L.units + 3) / 4, cap);
+    if (kch == 1 && bc != kc && nbt > 2) {
+      // a step over the tiles of about 0.38 of their number, coprime to it
+      const int nw = 4 * L.blocks;
+      int step = std::max(1, (int)std::lround(0.382 * nbt));
+      while (std::gcd(step, nbt) != 1) ++step;
+      L.shift = ((step - nw) % nbt + nbt) % nbt % nw;
+    }
     return L;
   }
-  L.tr = tr && bc != kc;
   const int rows = L.tr ? ncart(kPairLs[bc][0]) + ncart(kPairLs[bc][1]) : ncart(kPairLs[kc][0]) + ncart(kPairLs[kc][1]);
   L.strips = L.tr ? (nk + kStripK - 1) / kStripK : (nb + kStripB - 1) / kStripB;
   const int side = L.tr ? nb : nk;  // pairs claimed from each strip's counter
@@ -1088,6 +1165,77 @@ static ClassLaunch coop_launch(vsvb_context* c, int q, bool jk, int per_cu, int 
   return L;
 }
 
+static ClassLaunch policy_launch(vsvb_context* c, int q, const Policy& p) {
+  const int bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
+  if (p.coop && c->coop_idx[q] >= 0) return coop_launch(c, q, true, p.per_cu, p.claim);
+  return straight_launch(c, bc, kc, true, p.per_cu, p.lds_on, p.tr);
+}
+
+// Most primitive pairs per segment, by level and pair class (ss, ps, pp, ds,
+// dp, dd): a quarter and a twelfth of the pairs of six-fold, three-fold and
+// uncontracted shells.
+constexpr int kSegLen[kLevels][kNPairClass] = {{0, 0, 0, 0, 0, 0}, {9, 6, 3, 3, 1, 1}, {3, 2, 1, 1, 1, 1}};
+// Shell pairs up to which a context holds segment lists: above, every class
+// that matters fills the chip with whole pairs.
+constexpr int kSplitMaxPairs = 20000;
+
+// Work lists and class launches for the screened primitive counts kept[pair]
+// (scheduled order; null: unscreened, before the first geometry).
+static int plan_work(vsvb_context* c, const int* kept) {
+  c->h_seg.clear();
+  for (int pc = 0; pc < kNPairClass; ++pc) {
+    const int b = c->pair_off[pc], e = c->pair_off[pc + 1];
+    auto count = [&](int i) { return kept ? kept[i] : c->h_pairs[i].npp; };
+    double sum = 0.0;
+    int most = 0;
+    for (int i = b; i < e; ++i) {
+      sum += count(i);
+      most = std::max(most, count(i));
+    }
+    for (int l = 0; l < c->nlevels; ++l) {
+      WorkList& W = c->work[pc][l];
+      if (l > 0 && !kept) W.n = W.cap;
+      if (l > 0 && kept) {
+        // segment by segment over the pairs, so that neighbouring lanes hold
+        // different pairs (their accumulators' rows differ)
+        W.off = (int)c->h_seg.size();
+        for (int s = 0, any = 1; any; ++s) {
+          any = 0;
+          for (int i = b; i < e; ++i) {
+            const int ns = std::max(1, (count(i) + kSegLen[l][pc] - 1) / kSegLen[l][pc]);
+            if (s < ns) {
+              c->h_seg.push_back(SegSrc{i, s, ns});
+              any = 1;
+            }
+          }
+        }
+        W.n = (int)c->h_seg.size() - W.off;
+      }
+      W.longest = l > 0 ? std::min(most, kSegLen[l][pc]) : most;
+      W.mean = W.n > 0 ? sum / W.n : 0.0;
+    }
+  }
+  c->partial_total = 0;
+  for (int q = 0; q < kNQuartetClass; ++q) {
+    const int bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
+    const bool coop = coop_default(c->coop_idx[q]);
+    const bool tr = transposed_default(c, bc, kc);
+    const bool coop_e = coop || !straight_allowed(c, q, false, false);
+    const bool coop_jk = coop || !straight_allowed(c, q, true, tr);
+    c->le[q] = coop_e ? coop_launch(c, q, false, 0, 0) : straight_launch(c, bc, kc, false, 0, false, false);
+    c->ljk[q] = coop_jk ? coop_launch(c, q, true, 0, 0) : straight_launch(c, bc, kc, true, kDefaultJkPerCu, true, tr);
+    if (c->le[q].overflow || c->ljk[q].overflow)
+      return fail(VSVB_ERR_UNSUPPORTED, "shell-pair classes too large for 32-bit work-unit indices");
+    if (c->has_pol[q]) {
+      const ClassLaunch cl = policy_launch(c, q, c->pol[q]);
+      if (!cl.overflow && (cl.units > 0 || c->ljk[q].units <= 0)) c->ljk[q] = cl;
+    }
+    c->partial_per_class[q] = (size_t)c->le[q].blocks * 4;  // energy kernels write four slots per block
+    c->partial_total += c->partial_per_class[q];
+  }
+  return VSVB_OK;
+}
+
 // A device buffer of the context: allocated, or carved from the context's
 // arena (the allocation-free entry point); an arena too small is reported with
 // the size the system needs.
@@ -1130,6 +1278,7 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
       return fail(VSVB_ERR_UNSUPPORTED, "beta_only_last needs nunpd >= 1 and ndocc >= 1");
     c->nalpha_rows = c->nsp - 1;
   }
+  if (c->npair > 0) c->ndens = c->nsp * (c->nsp + 1) / 2;  // one Coulomb pass over the orbital-pair densities
   c->first_ndf = s->norbs - s->ndf;
   c->dtol = std::pow(10.0, -(double)s->ntol_d);
   if (c->nsp < 1) return fail(VSVB_ERR_ARG, "no electrons");
@@ -1293,45 +1442,73 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   HIP_OK(device_buffer(c, c->d_Z, (size_t)c->nsp * c->nbf));
   HIP_OK(device_buffer(c, c->d_grad, std::max(1, s->totlen)));
   HIP_OK(device_buffer(c, c->d_scal, 16));
-  HIP_OK(device_buffer(c, c->d_counters, kCounterWords));  // 4 counters, then 2 stamps, per class
+  HIP_OK(device_buffer(c, c->d_counters, kCounterWords));
   HIP_OK(device_buffer(c, c->d_stamps, (size_t)2 * kStampSlots * kNQuartetClass));
   // quartet launch geometry (grids sized to the occupancy of each class kernel) and partial buffer
   int ncu = 0;
   HIP_OK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
+  c->ncu = ncu;
+  // work lists: the shell pairs, and for systems of up to kSplitMaxPairs pairs
+  // their segments (counts here for unscreened primitive lists, the most a
+  // geometry can give)
+  size_t seg_cap = 0;
+  for (int pc = 0; pc < kNPairClass; ++pc) {
+    WorkList& W0 = c->work[pc][0];
+    W0.off = c->pair_off[pc];
+    W0.n = W0.cap = c->pair_off[pc + 1] - c->pair_off[pc];
+    for (int l = 1; l < kLevels; ++l) {
+      WorkList& W = c->work[pc][l];
+      W.cap = 0;
+      for (int i = c->pair_off[pc]; i < c->pair_off[pc + 1]; ++i)
+        W.cap += std::max(1, (pairs[i].npp + kSegLen[l][pc] - 1) / kSegLen[l][pc]);
+      seg_cap += W.cap;
+    }
+  }
   // work counters: one per energy segment of kSegTiles bra tiles, one per J/K
   // strip (bra strips, or ket strips transposed), one for the cooperative kernel
   static_assert(kSegTiles * kTileB == kStripB, "an energy segment covers one bra strip");
+  const bool split = c->npairs <= kSplitMaxPairs;
   c->ctr_total = 0;
   for (int bc = 0, q = 0; bc < kNPairClass; ++bc)
     for (int kc = 0; kc <= bc; ++kc, ++q) {
-      const int nb = c->pair_off[bc + 1] - c->pair_off[bc], nk = c->pair_off[kc + 1] - c->pair_off[kc];
+      int most = 1;
+      for (int l = 0; l < (split ? kLevels : 1); ++l)
+        most = std::max({most, (c->work[bc][l].cap + kStripB - 1) / kStripB, (c->work[kc][l].cap + kStripK - 1) / kStripK});
       c->ctr_off[q] = c->ctr_total;
-      c->ctr_len[q] = std::max({1, (nb + kStripB - 1) / kStripB, (nk + kStripK - 1) / kStripK});
-      c->ctr_total += c->ctr_len[q];
+      c->ctr_len[q] = most;
+      c->ctr_total += most;
     }
   HIP_OK(device_buffer(c, c->d_tilectr, c->ctr_total));
   HIP_OK(coop_prepare(c->device));
-  c->ncu = ncu;
-  c->partial_total = 0;
-  for (int bc = 0; bc < kNPairClass; ++bc)
-    for (int kc = 0; kc <= bc; ++kc) {
-      const int q = quartet_class_index(bc, kc);
+  // energy partial sums: four slots per workgroup of the largest grid of each class
+  size_t partial_cap = 0;
+  for (int bc = 0, q = 0; bc < kNPairClass; ++bc)
+    for (int kc = 0; kc <= bc; ++kc, ++q) {
       c->coop_idx[q] = coop_class(kPairLs[bc][0], kPairLs[bc][1], kPairLs[kc][0], kPairLs[kc][1]);
-      const bool coop = coop_default(c->coop_idx[q]);
-      const bool tr = transposed_default(c, bc, kc);
-      const bool coop_e = coop || !straight_allowed(c, q, false, false);
-      const bool coop_jk = coop || !straight_allowed(c, q, true, tr);
-      c->le[q] = coop_e ? coop_launch(c, q, false, 0, 0) : straight_launch(c, bc, kc, false, 0, false, false);
-      c->ljk[q] = coop_jk ? coop_launch(c, q, true, 0, 0)
-                          : straight_launch(c, bc, kc, true, kDefaultJkPerCu, true, tr);
-      if (c->le[q].overflow || c->ljk[q].overflow)
-        return fail(VSVB_ERR_UNSUPPORTED, "shell-pair classes too large for 32-bit work-unit indices");
-      c->partial_per_class[q] = (size_t)c->le[q].blocks * 4;  // energy kernels write four slots per block
-      c->partial_total += c->partial_per_class[q];
+      const int nb = c->work[bc][0].n, nk = c->work[kc][0].n;
+      if (nb <= 0 || nk <= 0) continue;
+      size_t blocks = 0;
+      if (coop_default(c->coop_idx[q]) || !straight_allowed(c, q, false, false))
+        blocks = coop_launch(c, q, false, 0, 0).blocks;
+      else
+        blocks = std::min<size_t>(2048, (size_t)class_occupancy(bc, kc, false, false, 0) * ncu);
+      partial_cap += 4 * blocks;
     }
-  HIP_OK(device_buffer(c, c->d_partial, std::max<size_t>(c->partial_total, 1) * 2));
+  HIP_OK(device_buffer(c, c->d_partial, std::max<size_t>(partial_cap, 1) * 2));
+  // segment lists last: in the allocation-free entry they are left out where
+  // the static array has no room for them
+  const size_t seg_bytes = seg_cap * (sizeof(Pair) + sizeof(SegSrc)) + 1024;
+  if (split && (!c->arena || c->arena->used + seg_bytes <= c->arena->cap)) {
+    HIP_OK(device_buffer(c, c->d_split, seg_cap));
+    HIP_OK(device_buffer(c, c->d_segsrc, seg_cap));
+    c->nlevels = kLevels;
+  }
+  {
+    const int rc = plan_work(c, nullptr);
+    if (rc) return rc;
+  }
   // uploads
-  auto boys = make_boys_table();
+  static const std::vector<double> boys = make_boys_table();  // the same in every context
   HIP_OK(hipMemcpy(c->d_shells.p, shells.data(), shells.size() * sizeof(Shell), hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(c->d_pairs.p, pairs.data(), pairs.size() * sizeof(Pair), hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(c->d_ppsrc.p, ppsrc.data(), ppsrc.size() * sizeof(PPSrc), hipMemcpyHostToDevice));
@@ -1389,9 +1566,18 @@ static int schedule_pairs(vsvb_context* c) {
       return r2[x] < r2[y];
     });
   }
-  for (int i = 0; i < np; ++i) sorted[i] = c->h_pairs[idx[i]];
+  std::vector<int> skept(np);
+  for (int i = 0; i < np; ++i) {
+    sorted[i] = c->h_pairs[idx[i]];
+    skept[i] = kept[idx[i]];
+  }
   c->h_pairs.swap(sorted);
+  const int rc = plan_work(c, skept.data());
+  if (rc) return rc;
   HIP_OK(hipMemcpyAsync(c->d_pairs.p, c->h_pairs.data(), np * sizeof(Pair), hipMemcpyHostToDevice, c->stream));
+  if (!c->h_seg.empty())
+    HIP_OK(hipMemcpyAsync(c->d_segsrc.p, c->h_seg.data(), c->h_seg.size() * sizeof(SegSrc), hipMemcpyHostToDevice,
+                          c->stream));
   c->sched_coords = c->coords;
   return VSVB_OK;
 }
@@ -1420,6 +1606,11 @@ int vsvb::prepare_geometry(vsvb_context* c, const double* coords) {
     HIP_OK(launch_one_e(pc, c->d_pairs.p, p0, np, c->d_shells.p, c->d_pexp.p, c->d_pcoef.p, c->d_xyz.p,
                         c->d_charge.p, c->natom, c->d_boys.p, c->d_S.p, c->d_H.p, c->nbf, st));
     HIP_OK(launch_schwarz(pc, c->d_pairs.p, c->d_pp.p, c->d_boys.p, p0, np, st));
+  }
+  if (!c->h_seg.empty()) {
+    const int ns = (int)c->h_seg.size();
+    hipLaunchKernelGGL(k_split, dim3((ns + 255) / 256), dim3(256), 0, st, c->d_pairs.p, c->d_segsrc.p, ns, c->d_split.p);
+    HIP_OK(hipGetLastError());
   }
   c->geom_ready = true;
   return VSVB_OK;
@@ -1495,14 +1686,15 @@ static QuartetArgs class_args(vsvb_context* c, int bc, int kc, const ClassLaunch
                               const double* dens, double* jacc, double* kacc, double* partial) {
   const int q = quartet_class_index(bc, kc);
   QuartetArgs a{};
-  a.pairs = c->d_pairs.p;
+  const int lb = cl.coop ? 0 : cl.lb, lk = cl.coop ? 0 : cl.lk;
+  const WorkList &B = c->work[bc][lb], &K = c->work[kc][lk];
+  a.bra = (lb ? c->d_split.p : c->d_pairs.p) + B.off;
+  a.ket = (lk ? c->d_split.p : c->d_pairs.p) + K.off;
+  a.nbra = B.n;
+  a.nket = K.n;
   a.pp = c->d_pp.p;
   a.shells = c->d_shells.p;
   a.boys = c->d_boys.p;
-  a.bra0 = c->pair_off[bc];
-  a.nbra = c->pair_off[bc + 1] - a.bra0;
-  a.ket0 = c->pair_off[kc];
-  a.nket = c->pair_off[kc + 1] - a.ket0;
   a.same = bc == kc;
   a.ntk = cl.claim;
   a.ntiles = cl.units;
@@ -1522,6 +1714,7 @@ static QuartetArgs class_args(vsvb_context* c, int bc, int kc, const ClassLaunch
   a.tile_ctr = c->d_tilectr.p + c->ctr_off[q];
   a.nstrip = cl.coop ? 1 : cl.strips;
   a.seg_tiles = cl.seg_tiles;
+  a.shift = cl.shift;
   return a;
 }
 
@@ -1562,7 +1755,7 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, double* e2_dev, int nwfn, const
   if (!dens) dens = c->d_R.p;
   if (!jacc) jacc = c->d_J.p;
   if (!kacc) kacc = c->d_K.p;
-  HIP_OK(quartet_pass_clear(c, jk, nwfn, nspin, jacc, kacc, 4 * kNQuartetClass));
+  HIP_OK(quartet_pass_clear(c, jk, nwfn, nspin, jacc, kacc, kCtrSlots * kCtrStride));
   // Stage timing: HIP events on direct runs (under stream capture a record is
   // only a dependency, so replays take the per-class wall-clock stamps the
   // kernels write when profiling is on).
@@ -1580,7 +1773,7 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, double* e2_dev, int nwfn, const
     const int q = c->class_rev ? kNQuartetClass - 1 - t : t;
     const int bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
     const ClassLaunch& cl = jk ? c->ljk[q] : c->le[q];
-    const int nb = c->pair_off[bc + 1] - c->pair_off[bc], nk = c->pair_off[kc + 1] - c->pair_off[kc];
+    const int nb = c->work[bc][0].n, nk = c->work[kc][0].n;
     // a class with pairs on both sides always has work units: a launch
     // configuration without any would drop its quartets silently
     if (nb > 0 && nk > 0 && cl.units <= 0)
@@ -1594,23 +1787,12 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, double* e2_dev, int nwfn, const
   }
   if (c->profile)
     hipLaunchKernelGGL(k_stamp_reduce, dim3(kNQuartetClass), dim3(kStampSlots), 0, st, c->d_stamps.p,
-                       c->d_counters.p + 4 * kNQuartetClass);
+                       c->d_counters.p + kCtrSlots * kCtrStride);
   if (!jk) {
     hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, st, c->d_partial.p, (long)poff, 1, e2_dev);
     HIP_OK(hipGetLastError());
   }
   return VSVB_OK;
-}
-
-// Algorithmic FP64 operations of the density contraction per contracted quartet.
-static double digestion_flops(int q, int nspin, bool jk) {
-  int bc = 0, kc = 0;
-  for (int b = 0; b < kNPairClass; ++b)
-    for (int k = 0; k <= b; ++k)
-      if (quartet_class_index(b, k) == q) { bc = b; kc = k; }
-  const double nab = ncart(kPairLs[bc][0]) * ncart(kPairLs[bc][1]);
-  const double ncd = ncart(kPairLs[kc][0]) * ncart(kPairLs[kc][1]);
-  return jk ? nab * ncd * (4.0 + 8.0 * nspin) : nab * ncd * (2.0 + 4.0 * nspin) + 2.0 * nab;
 }
 
 // Counters of the last quartet stage.  hcnt: the stage's counters and stamps
@@ -1630,7 +1812,9 @@ int vsvb::finish_counters(vsvb_context* c, const unsigned long long* hcnt) {
     std::memcpy(h, hcnt, sizeof(h));
   else
     HIP_OK(hipMemcpy(h, c->d_counters.p, sizeof(h), hipMemcpyDeviceToHost));
-  const unsigned long long* stamp = h + 4 * kNQuartetClass;
+  for (int s = 1; s < kCtrSlots; ++s)
+    for (int k = 0; k < kCtrStride; ++k) h[k] += h[s * kCtrStride + k];
+  const unsigned long long* stamp = h + kCtrSlots * kCtrStride;
   const double tick_ms = c->wall_khz > 0 ? 1.0 / c->wall_khz : 0.0;
   const int nspin = c->last_nspin;
   double tot[3] = {0, 0, 0};
@@ -1970,6 +2154,10 @@ static int batch_plan(vsvb_batch* b) {
   b->glaunch.clear();
   b->h_qargs.clear();
   if (b->chunks <= 0) return VSVB_OK;
+  for (auto& g : b->groups) {  // the argument records hold the work lists of the geometry to be run
+    const int rc = schedule_pairs(b->ctx[g.members[0]]);
+    if (rc) return rc;
+  }
   for (int l = 0; l < (int)b->lanes.size(); ++l) {
     std::vector<int> gl;
     double tot = 0.0;
@@ -2201,20 +2389,6 @@ static int batch_gather(vsvb_batch* b) {
 // candidate already 1.5x slower than the best after one launch gets no
 // second).  The launches accumulate into the leader's J/K arrays,
 // which the first run clears again.
-struct Policy {
-  bool coop = false;
-  int per_cu = 0;
-  bool lds_on = true;
-  int claim = 0;
-  bool tr = false;
-};
-
-static ClassLaunch policy_launch(vsvb_context* c, int q, const Policy& p) {
-  const int bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
-  if (p.coop && c->coop_idx[q] >= 0) return coop_launch(c, q, true, p.per_cu, p.claim);
-  return straight_launch(c, bc, kc, true, p.per_cu, p.lds_on, p.tr);
-}
-
 static int tune_leader(vsvb_batch* b, BatchGroup* gs, double (*tuning)[kTuneCols], std::vector<Policy>& best) {
   vsvb_context* L = b->ctx[gs->members[0]];
   int rc;
@@ -2371,6 +2545,8 @@ static int tune_batch(vsvb_batch* b) {
         // the representative's best launch may not fit a larger molecule of the
         // bucket (too many work units for 32-bit indices): that group keeps its
         // own default launch, which its context was created with
+        c->pol[q] = best[k][q];
+        c->has_pol[q] = true;
         const ClassLaunch cl = policy_launch(c, q, best[k][q]);
         if (!cl.overflow && (cl.units > 0 || c->ljk[q].units <= 0)) c->ljk[q] = cl;
       }
@@ -2901,6 +3077,7 @@ int vsvb_batch_create(int32_t nwfn, const vsvb_system* const* systems, const vsv
   for (auto& g : bt->groups) {
     vsvb_context* lead = bt->ctx[g.members[0]];
     if (g.members.size() < 2) continue;
+    lead->ndens = (int)g.members.size();  // its work lists are planned with the first geometry
     const size_t nn = (size_t)lead->nbf * lead->nbf;
     const int nspin = lead->nunpd > 0 ? 2 : 1;
     const size_t G = g.members.size();

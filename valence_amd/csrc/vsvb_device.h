@@ -75,7 +75,7 @@ struct Pair {
   int A, B;        // shells; l(A) >= l(B)
   int pp0, npp;    // primitive pairs
   int offdiag;     // 1 if A != B
-  int pad;
+  int seg;         // segment of the pair's primitive list (0 for a whole pair)
   double ABx, ABy, ABz;
   double Q;        // sqrt(max |(ab|ab)|)
 };

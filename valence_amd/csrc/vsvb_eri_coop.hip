@@ -97,7 +97,7 @@ __device__ __forceinline__ void coop_body(const QuartetArgs& a, const CoopDesc& 
       if (c0 + lane < claim && um < a.ntiles) {
         const int b0 = um / a.nket, k0 = um - b0 * a.nket;
         if (!a.same || k0 <= b0) {
-          keep = a.pairs[a.bra0 + b0].Q * a.pairs[a.ket0 + k0].Q >= a.tau;
+          keep = a.bra[b0].Q * a.ket[k0].Q >= a.tau;
           if (!keep) ++nskip;
         }
       }
@@ -108,8 +108,8 @@ __device__ __forceinline__ void coop_body(const QuartetArgs& a, const CoopDesc& 
       const int u = (int)((long long)uc + (long long)(c0 + bit) * stride);
       const int ib = u / a.nket;
       const int ik = u - ib * a.nket;
-      const Pair P = a.pairs[a.bra0 + ib];
-      const Pair K = a.pairs[a.ket0 + ik];
+      const Pair P = a.bra[ib];
+      const Pair K = a.ket[ik];
       __syncthreads();  // the previous unit is done with the LDS
       for (int s = lane; s < d.nT; s += 64) S[s] = 0.0;
       const UniformPrimPairs bp = as_uniform(a.pp + P.pp0);
@@ -303,15 +303,8 @@ __device__ __forceinline__ void coop_body(const QuartetArgs& a, const CoopDesc& 
     }
   }
   stamp_wave(a.stamp, true);
-  if (a.counters) {
-    unsigned long long sk = nskip;  // per lane; nq and nprimq are wave-uniform
-    for (int o = 32; o > 0; o >>= 1) sk += __shfl_xor(sk, o, 64);
-    if (lane == 0) {
-      atomicAdd(&a.counters[0], nq);
-      atomicAdd(&a.counters[1], nprimq);
-      atomicAdd(&a.counters[2], sk);
-    }
-  }
+  // nq and nprimq are wave-uniform, nskip is per lane
+  add_counters(a.counters, lane == 0 ? nq : 0, lane == 0 ? nprimq : 0, nskip);
 }
 
 template <bool kJK>

@@ -29,18 +29,19 @@ namespace vsvb {
 #include "eri_gen.inc"
 
 struct QuartetArgs {
-  const Pair* pairs;
+  const Pair* bra;      // work pairs of the bra class: shell pairs, or segments of them (Pair::seg)
+  const Pair* ket;      // work pairs of the ket class
   const PrimPair* pp;
   const Shell* shells;
   const double* boys;
-  int bra0, nbra;       // pair index range of the bra class
-  int ket0, nket;       // pair index range of the ket class
-  int same;             // bra class == ket class: only ket <= bra
+  int nbra, nket;       // work pairs of the bra and of the ket class
+  int same;             // bra class == ket class (one list): only ket <= bra
   int ntk;              // cooperative kernel: units claimed per wavefront (1..1024)
   int ntiles;           // work units: energy: bra tiles (64 pairs) x ket chunks; J/K: strips x claims
   int kchunk;           // pairs of the wave-uniform side per claim (1..64): kets; bras in transposed J/K units
   int nkc;              // energy: ket chunks, ceil(nket / kchunk)
   int seg_tiles;        // energy: bra tiles per counter segment (nstrip segments)
+  int shift;            // energy, one-ket units: change of a wavefront's place from round to round (below the grid)
   double tau;           // skip quartet if Q_bra * Q_ket < tau
   int nbf;
   int nwfn;             // wave functions sharing this geometry
@@ -50,7 +51,7 @@ struct QuartetArgs {
   double* partial;      // energy: [gridDim.x * 4][nwfn] per-wave partial sums
   double* jacc;         // J/K mode: Coulomb accumulators [nwfn][nbf][nbf]
   double* kacc;         // J/K mode: exchange accumulators [nwfn][nspin][nbf][nbf]
-  unsigned long long* counters;  // [0] quartets evaluated, [1] primitive quartets, [2] skipped
+  unsigned long long* counters;  // the class's {quartets evaluated, primitive quartets, skipped} in slot 0
   int* tile_ctr;        // dynamic tile counter(s), zero before the launch: one, or one per strip (J/K)
   int nstrip;           // straight-line units: energy segments of kSegTiles bra tiles, J/K strips (bra, or ket
                         // when transposed), each with its own work counter
@@ -73,6 +74,35 @@ __device__ __forceinline__ void stamp_wave(unsigned long long* st, bool end) {
       atomicMax(st + 2 * slot + 1, t);
     else
       atomicMin(st + 2 * slot, t);
+  }
+}
+
+// Work counters of a launch: the lanes' counts are summed over the workgroup and
+// added to one of kCtrSlots copies (the host adds the copies up).  Three atomics
+// per wavefront on one address cost 7 ns each: 86 us at the end of every launch
+// of 4096 wavefronts.
+constexpr int kCtrSlots = 16;
+constexpr int kCtrStride = 4 * kNQuartetClass;  // words per copy
+__device__ __forceinline__ void add_counters(unsigned long long* counters, unsigned long long q, unsigned long long pq,
+                                             unsigned long long sk) {
+  __shared__ unsigned long long red[4][3];
+  if (!counters) return;
+  for (int o = 32; o > 0; o >>= 1) {
+    q += __shfl_xor(q, o, 64);
+    pq += __shfl_xor(pq, o, 64);
+    sk += __shfl_xor(sk, o, 64);
+  }
+  const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    red[wave][0] = q;
+    red[wave][1] = pq;
+    red[wave][2] = sk;
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    unsigned long long s = 0;
+    for (int w = 0; w < nw; ++w) s += red[w][threadIdx.x];
+    if (s) atomicAdd(counters + (blockIdx.x % kCtrSlots) * kCtrStride + threadIdx.x, s);
   }
 }
 
@@ -143,56 +173,86 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
   unsigned long long nq = 0, nprimq = 0, nskip = 0;
   stamp_wave(a.stamp, false);
 
-  // Work units (64 bra pairs x a chunk of kchunk ket pairs) are handed to
-  // wavefronts one at a time from atomic counters, with no barrier, so
-  // wavefronts never wait for each other.  The unit indices form nstrip
-  // segments of seg_tiles * nkc units, each with its own counter: a wavefront
-  // starts on segment (global wave index) mod nstrip and moves to the next one
-  // only when its segment is exhausted, leaving after it has found every
-  // segment exhausted once (counters only grow, so every wavefront ends);
-  // spreading the claims over several counters keeps them from queueing on
-  // one address.  Pairs sort heaviest first (most primitive pairs), so low
-  // unit indices hold the heaviest quartets and the tail is short.  With
-  // chunks of several kets, one lane per ket tests it
-  // against the largest bra bound of the tile, and the wavefront visits only
-  // the kets that can pass the Schwarz test for some lane: sparse systems,
-  // where most (tile, ket) slots are screened out, then cost one counter claim
+  // Work units are 64 bra pairs x a chunk of kchunk ket pairs; pairs sort
+  // heaviest first (most primitive pairs), so low unit indices hold the
+  // heaviest quartets and the tail is short.
+  //
+  // One-ket units go to the wavefronts by a fixed rule, one per wavefront and
+  // round: claims from one counter cost 6-8 ns each, all wavefronts queueing on
+  // its address, which was the whole time of C8H18's (ss|ss), (ps|ss) and
+  // (ps|ps) launches (151000, 129000 and 111000 claims in 0.97, 0.96 and 0.89
+  // ms).  Units of different bra and ket classes go ket-major, so that the
+  // wavefronts in flight share few kets and their primitive data stay in the
+  // scalar caches; `shift` moves every wavefront over the tiles by about 0.38 of
+  // their number from round to round, so that none keeps to the heavy ones
+  // (without it (ps|ss) took 1.72 ms: its stride left a wavefront on every
+  // second tile).  Units of one class go tile by tile up to the tile's last ket,
+  // with none above the diagonal.
+  //
+  // Chunked units (sparse systems, where the work of a unit varies widely) are
+  // claimed one at a time from atomic counters, with no barrier.  The unit
+  // indices form nstrip segments of seg_tiles * nkc units, each with its own
+  // counter: a wavefront starts on segment (global wave index) mod nstrip and
+  // moves to the next one only when its segment is exhausted, leaving after it
+  // has found every segment exhausted once (counters only grow, so every
+  // wavefront ends).  One lane per ket tests it against the largest bra bound
+  // of the tile, and the wavefront visits only the kets that can pass the
+  // Schwarz test for some lane, so screened (tile, ket) slots cost one claim
   // per chunk instead of one per ket.
   const int nbt = (a.nbra + kTileB - 1) / kTileB;
-  int sg = (int)((blockIdx.x * 4u + (unsigned)wave) % (unsigned)a.nstrip), left = a.nstrip;
+  const bool fixed = a.kchunk == 1;
+  const unsigned gw = blockIdx.x * 4u + (unsigned)wave, nw = gridDim.x * 4u;
+  unsigned slot = gw, round0 = 0;
+  int sg = (int)(gw % (unsigned)a.nstrip), left = a.nstrip;
   for (;;) {
-    int ul = 0;
-    if (lane == 0) ul = atomicAdd(a.tile_ctr + sg, 1);
-    ul = __builtin_amdgcn_readfirstlane(__shfl(ul, 0, 64));
-    const int t0 = sg * a.seg_tiles;
-    if (ul >= min(a.seg_tiles, nbt - t0) * a.nkc) {  // this segment is exhausted
-      if (--left == 0) break;
-      sg = sg + 1 == a.nstrip ? 0 : sg + 1;
-      continue;
+    int tb, k0;
+    if (fixed) {
+      const unsigned un = round0 + slot;
+      if (round0 >= (unsigned)a.ntiles) break;
+      round0 += nw;
+      slot += (unsigned)a.shift;
+      if (slot >= nw) slot -= nw;
+      if (un >= (unsigned)a.ntiles) continue;
+      if (a.same) {
+        // tile tb owns units [32 tb (tb + 1), 32 (tb + 1)(tb + 2)): kets 0 .. 64 tb + 63
+        tb = (int)((sqrt(1.0 + 0.125 * (double)un) - 1.0) * 0.5);
+        while (32u * (unsigned)(tb + 1) * (unsigned)(tb + 2) <= un) ++tb;
+        while (32u * (unsigned)tb * (unsigned)(tb + 1) > un) --tb;
+        k0 = (int)(un - 32u * (unsigned)tb * (unsigned)(tb + 1));
+      } else {
+        k0 = (int)(un / (unsigned)nbt);
+        tb = (int)(un - (unsigned)k0 * (unsigned)nbt);
+      }
+      tb = __builtin_amdgcn_readfirstlane(tb);
+      k0 = __builtin_amdgcn_readfirstlane(k0);
+      if (k0 >= a.nket) continue;  // one class: the last tile is not full
+    } else {
+      int ul = 0;
+      if (lane == 0) ul = atomicAdd(a.tile_ctr + sg, 1);
+      ul = __builtin_amdgcn_readfirstlane(__shfl(ul, 0, 64));
+      const int t0 = sg * a.seg_tiles;
+      if (ul >= min(a.seg_tiles, nbt - t0) * a.nkc) {  // this segment is exhausted
+        if (--left == 0) break;
+        sg = sg + 1 == a.nstrip ? 0 : sg + 1;
+        continue;
+      }
+      const int u = t0 * a.nkc + ul;
+      tb = u / a.nkc;
+      k0 = __builtin_amdgcn_readfirstlane((u - tb * a.nkc) * a.kchunk);
     }
-    // Bra-tile-major order, except for one-ket units of different bra and ket
-    // classes: ket-major there, so that the wavefronts in flight share few
-    // kets and their primitive data stay in the scalar caches (2% faster on
-    // C8H18's off-diagonal classes; slower for LiF128's 64-ket chunks, and a
-    // same-class tile's kets end at its diagonal).
-    const int u = t0 * a.nkc + ul;
-    const bool km = !a.same && a.kchunk == 1;
-    const int kci = km ? u / nbt : 0;
-    const int tb = km ? u - kci * nbt : u / a.nkc;
-    const int k0 = __builtin_amdgcn_readfirstlane((km ? kci : u - tb * a.nkc) * a.kchunk);
     const int klast = tb * kTileB + kTileB - 1;  // same class: last ket any lane of the tile takes
     if (a.same && k0 > klast) continue;  // whole wave above the diagonal
     const int ib = tb * kTileB + lane;
     const bool bra_ok = ib < a.nbra;
     Pair P{};
-    if (bra_ok) P = a.pairs[a.bra0 + ib];
+    if (bra_ok) P = a.bra[ib];
     unsigned long long live = 1;
     if (a.kchunk > 1) {
       const double qmax = wave_max(bra_ok ? P.Q : 0.0);
       const int ikl = k0 + lane;
       bool lv = false;
       if (lane < a.kchunk && ikl < a.nket && (!a.same || ikl <= klast)) {
-        lv = a.pairs[a.ket0 + ikl].Q * qmax >= a.tau;
+        lv = a.ket[ikl].Q * qmax >= a.tau;
         if (!lv) {  // every bra lane that takes this ket is screened out
           const int lo = a.same ? max(ikl, tb * kTileB) : tb * kTileB;
           const int hi = min(a.nbra, tb * kTileB + kTileB);
@@ -204,17 +264,18 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
     while (live) {
       const int ik = __builtin_amdgcn_readfirstlane(k0 + __builtin_ctzll(live));
       live &= live - 1;
-      const Pair K = a.pairs[a.ket0 + ik];
+      const Pair K = a.ket[ik];
       bool act = bra_ok && (!a.same || ik <= ib);
+      const bool first = (P.seg | K.seg) == 0;  // a quartet of segments is counted once
       if (act && P.Q * K.Q < a.tau) {
         act = false;
-        ++nskip;
+        nskip += first;
       }
       double v[NAB * NCD];
       if (act) {
         eri_block<LA, LB, LC, LD>(a.pp + P.pp0, P.npp, a.pp + K.pp0, K.npp, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy,
                                   K.ABz, btab, v);
-        ++nq;
+        nq += first;
         nprimq += (unsigned long long)P.npp * K.npp;
       } else {
 #pragma unroll
@@ -288,19 +349,7 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
     }
   }
   stamp_wave(a.stamp, true);
-  if (a.counters) {
-    unsigned long long q = nq, pq = nprimq, sk = nskip;
-    for (int o = 32; o > 0; o >>= 1) {
-      q += __shfl_xor(q, o, 64);
-      pq += __shfl_xor(pq, o, 64);
-      sk += __shfl_xor(sk, o, 64);
-    }
-    if (lane == 0) {
-      atomicAdd(&a.counters[0], q);
-      atomicAdd(&a.counters[1], pq);
-      atomicAdd(&a.counters[2], sk);
-    }
-  }
+  add_counters(a.counters, nq, nprimq, nskip);
 }
 
 
@@ -351,7 +400,7 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
   auto flush_j = [&](int s_) {
     const int ibf = s_ * kStripB + wave * kTileB + lane;
     if (s_ < 0 || ibf >= a.nbra) return;
-    const Pair Pf = a.pairs[a.bra0 + ibf];
+    const Pair Pf = a.bra[ibf];
     const int fa = a.shells[Pf.A].ao, fb = a.shells[Pf.B].ao;
 #pragma unroll
     for (int ij = 0; ij < (kRegJ ? NAB : 1); ++ij) {
@@ -384,7 +433,7 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
     const int ib = tile0 + lane;
     // every lane holds a pair of the bra class (the last one past the end), so
     // that the density blocks read below stay inside the matrix
-    const Pair P = a.pairs[a.bra0 + (ib < a.nbra ? ib : a.nbra - 1)];
+    const Pair P = a.bra[(ib < a.nbra ? ib : a.nbra - 1)];
     unsigned long long live = 1;
     if (a.kchunk > 1) {
       const double qw = wave_max(ib < a.nbra ? P.Q : 0.0);
@@ -394,7 +443,7 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
       const int ikl = k0 + lane;
       bool lv = false;
       if (lane < a.kchunk && ikl < a.nket && (!a.same || ikl <= klast)) {
-        lv = a.pairs[a.ket0 + ikl].Q * qmax >= a.tau;
+        lv = a.ket[ikl].Q * qmax >= a.tau;
         if (!lv) {  // every bra lane of this wavefront that takes the ket is screened out
           const int lo = a.same ? max(ikl, tile0) : tile0, hi = min(a.nbra, tile0 + kTileB);
           nskip += hi > lo ? hi - lo : 0;
@@ -405,17 +454,18 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
     while (live) {
       const int ik = __builtin_amdgcn_readfirstlane(k0 + __builtin_ctzll(live));
       live &= live - 1;
-      const Pair K = a.pairs[a.ket0 + ik];
+      const Pair K = a.ket[ik];
       bool act = ib < a.nbra && (!a.same || ik <= ib);
+      const bool first = (P.seg | K.seg) == 0;  // a quartet of segments is counted once
       if (act && P.Q * K.Q < a.tau) {
         act = false;
-        ++nskip;
+        nskip += first;
       }
       double v[NAB * NCD];
       if (act) {
         eri_block<LA, LB, LC, LD>(a.pp + P.pp0, P.npp, a.pp + K.pp0, K.npp, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy,
                                   K.ABz, btab, v);
-        ++nq;
+        nq += first;
         nprimq += (unsigned long long)P.npp * K.npp;
       } else {
 #pragma unroll
@@ -548,19 +598,7 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
   }
   if (racc) flush_j(jst);
   stamp_wave(a.stamp, true);
-  if (a.counters) {
-    unsigned long long q = nq, pq = nprimq, sk = nskip;
-    for (int o = 32; o > 0; o >>= 1) {
-      q += __shfl_xor(q, o, 64);
-      pq += __shfl_xor(pq, o, 64);
-      sk += __shfl_xor(sk, o, 64);
-    }
-    if (lane == 0) {
-      atomicAdd(&a.counters[0], q);
-      atomicAdd(&a.counters[1], pq);
-      atomicAdd(&a.counters[2], sk);
-    }
-  }
+  add_counters(a.counters, nq, nprimq, nskip);
 }
 
 // Transposed J/K unit, for classes whose bra and ket pair classes differ: one
@@ -605,7 +643,7 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const dou
   auto flush_j = [&](int s_) {
     const int ikf = s_ * kStripK + wave * kTileB + lane;
     if (s_ < 0 || ikf >= a.nket) return;
-    const Pair Kf = a.pairs[a.ket0 + ikf];
+    const Pair Kf = a.ket[ikf];
     const int fc = a.shells[Kf.A].ao, fd = a.shells[Kf.B].ao;
 #pragma unroll
     for (int kl = 0; kl < (kRegJ ? NCD : 1); ++kl) {
@@ -635,7 +673,7 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const dou
     const int ik = tile0 + lane;
     const bool kin = ik < a.nket;
     // every lane holds a pair of the ket class (the last one past the end)
-    const Pair K = a.pairs[a.ket0 + (kin ? ik : a.nket - 1)];
+    const Pair K = a.ket[(kin ? ik : a.nket - 1)];
     unsigned long long live = 1;
     if (a.kchunk > 1) {
       const double qw = wave_max(kin ? K.Q : 0.0);
@@ -645,7 +683,7 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const dou
       const int ibl = b0 + lane;
       bool lv = false;
       if (lane < a.kchunk && ibl < a.nbra) {
-        lv = a.pairs[a.bra0 + ibl].Q * qmax >= a.tau;
+        lv = a.bra[ibl].Q * qmax >= a.tau;
         if (!lv) {  // every ket lane of this wavefront is screened out
           const int hi = min(a.nket, tile0 + kTileB);
           nskip += hi > tile0 ? hi - tile0 : 0;
@@ -656,17 +694,18 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const dou
     while (live) {
       const int ib = __builtin_amdgcn_readfirstlane(b0 + __builtin_ctzll(live));
       live &= live - 1;
-      const Pair P = a.pairs[a.bra0 + ib];
+      const Pair P = a.bra[ib];
       bool act = kin;
+      const bool first = (P.seg | K.seg) == 0;  // a quartet of segments is counted once
       if (act && P.Q * K.Q < a.tau) {
         act = false;
-        ++nskip;
+        nskip += first;
       }
       double v[NAB * NCD];
       if (act) {
         eri_block_ub<LA, LB, LC, LD>(a.pp + P.pp0, P.npp, a.pp + K.pp0, K.npp, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy,
                                      K.ABz, btab, v);
-        ++nq;
+        nq += first;
         nprimq += (unsigned long long)P.npp * K.npp;
       } else {
 #pragma unroll
@@ -798,19 +837,7 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const dou
   }
   if (racc) flush_j(jst);
   stamp_wave(a.stamp, true);
-  if (a.counters) {
-    unsigned long long q = nq, pq = nprimq, sk = nskip;
-    for (int o = 32; o > 0; o >>= 1) {
-      q += __shfl_xor(q, o, 64);
-      pq += __shfl_xor(pq, o, 64);
-      sk += __shfl_xor(sk, o, 64);
-    }
-    if (lane == 0) {
-      atomicAdd(&a.counters[0], q);
-      atomicAdd(&a.counters[1], pq);
-      atomicAdd(&a.counters[2], sk);
-    }
-  }
+  add_counters(a.counters, nq, nprimq, nskip);
 }
 
 template <int LA, int LB, int LC, int LD>

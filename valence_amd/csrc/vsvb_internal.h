@@ -17,9 +17,10 @@ namespace vsvb {
 
 // Largest exchange LDS block of a J/K workgroup (nbf x ket columns doubles).
 constexpr size_t kMaxLdsK = 60 * 1024;
-// Device counter words of a quartet stage: per class {evaluated, primitive
-// quartets, skipped, spare}, then per class {earliest start, latest end} stamps.
-constexpr int kCounterWords = 6 * kNQuartetClass;
+// Device counter words of a quartet stage: kCtrSlots copies of, per class,
+// {evaluated, primitive quartets, skipped, spare}, then per class {earliest
+// start, latest end} stamps.
+constexpr int kCounterWords = kCtrSlots * kCtrStride + 2 * kNQuartetClass;
 
 extern thread_local std::string g_last_error;
 int fail(int code, const std::string& msg);
@@ -33,6 +34,11 @@ int fail(int code, const std::string& msg);
 
 struct PPSrc {
   int sA, sB, ia, ib;  // shell indices of A and B, global primitive indices of A and B
+};
+
+// Segment seg of nseg of shell pair `pair` (index into d_pairs).
+struct SegSrc {
+  int pair, seg, nseg;
 };
 
 struct OrbEntry {
@@ -114,8 +120,27 @@ struct SpinCoupled {
   DevBuf<double> d_q4;                            // [npairs][2][4] sign, P_R, d1, d2
 };
 
+// How one quartet class is launched in J/K mode (the batch tuner's choice).
+struct Policy {
+  bool coop = false;
+  int per_cu = 0;
+  bool lds_on = true;
+  int claim = 0;
+  bool tr = false;
+};
+
+// Work lists of a pair class: level 0 holds its shell pairs, levels 1 and 2
+// hold segments of at most kSegLen[level][class] primitive pairs (k_split).
+constexpr int kLevels = 3;
+struct WorkList {
+  int off = 0, n = 0, cap = 0;  // offset (d_pairs, or d_split above level 0), entries, largest count at any geometry
+  int longest = 0;              // primitive pairs of the longest entry
+  double mean = 0.0;            // primitive pairs per entry
+};
+
 // Launch configuration of one quartet class in one mode (energy or J/K).
 struct ClassLaunch {
+  int lb = 0, lk = 0;  // work-list levels of the bra and of the ket class
   bool coop = false;  // cooperative kernel (one wavefront per contracted quartet)
   int units = 0;      // work units handed out by the class counter
   int blocks = 0;     // workgroups
@@ -126,6 +151,7 @@ struct ClassLaunch {
   int strips = 1;     // straight-line: energy segments, J/K bra strips (ket strips transposed), one work counter each
   int kchunk = 1;     // straight-line: pairs of the uniform side (ket; bra when transposed) per claim
   int seg_tiles = 1;  // straight-line energy: bra tiles per counter segment
+  int shift = 0;      // straight-line energy, one-ket units: QuartetArgs::shift
   bool overflow = false;  // the class has more work units than 32-bit indices allow in this shape
 };
 
@@ -158,15 +184,24 @@ struct vsvb_context {
                         // nsp - 1 when the last doubly occupied orbital holds only a beta electron)
   double dtol = 0.0;
   int pair_off[vsvb::kNPairClass + 1] = {0};
+  // work lists of the pair classes; levels above 0 only when nlevels > 1
+  vsvb::WorkList work[vsvb::kNPairClass][vsvb::kLevels];
+  int nlevels = 1;
+  int ndens = 1;  // densities of the context's quartet pass (J/K mode)
+  vsvb::Policy pol[vsvb::kNQuartetClass];
+  bool has_pol[vsvb::kNQuartetClass] = {false};
   // host copies
   std::vector<double> coords, charges, coeff;
   // host copies for the per-geometry pair schedule
   std::vector<Shell> h_shells;
   std::vector<Pair> h_pairs;
   std::vector<double> h_pexp, h_pcoef, sched_coords;
+  std::vector<vsvb::SegSrc> h_seg;
   std::vector<OrbEntry> ent;
   std::vector<int> orb_start;
   // device
+  DevBuf<Pair> d_split;            // segments of the shell pairs (levels 1 and 2)
+  DevBuf<vsvb::SegSrc> d_segsrc;   // which pair and which part of it each segment is
   DevBuf<Shell> d_shells;
   DevBuf<Pair> d_pairs;
   DevBuf<PPSrc> d_ppsrc;
