@@ -84,11 +84,12 @@ class Emitter:
         self.lines.append(s)
 
 
-def vrr_plan(la, lb, lc, ld):
-    """Intermediates [e0|f0]^(m) needed for the class, in dependency order, with
-    the recurrence used for each (greedy choice of the decrement direction)."""
-    targets = [(e, f) for le in range(la, la + lb + 1) for e in cart(le)
-               for lf in range(lc, lc + ld + 1) for f in cart(lf)]
+def vrr_plan(la, lb, lc, ld, es=None):
+    """Intermediates [e0|f0]^(m) needed for the class (for the bra functions es
+    only, where given), in dependency order, with the recurrence used for each
+    (greedy choice of the decrement direction)."""
+    es = es or [e for le in range(la, la + lb + 1) for e in cart(le)]
+    targets = [(e, f) for e in es for lf in range(lc, lc + ld + 1) for f in cart(lf)]
     order: List[Tuple] = []
     recipe: Dict[Tuple, Tuple] = {}
     seen = set()
@@ -151,9 +152,9 @@ def vrr_plan(la, lb, lc, ld):
     return order, recipe, targets
 
 
-def gen_vrr(la, lb, lc, ld, em: Emitter):
+def gen_vrr(la, lb, lc, ld, em: Emitter, es=None):
     """Emit VRR for one primitive quartet; returns dict target->(var name)."""
-    order, recipe, targets = vrr_plan(la, lb, lc, ld)
+    order, recipe, targets = vrr_plan(la, lb, lc, ld, es)
 
     def var(k):
         e, f, m = k
@@ -193,8 +194,10 @@ def gen_vrr(la, lb, lc, ld, em: Emitter):
     return {(e, f): var((e, f, 0)) for (e, f) in targets}, len(order), targets
 
 
-def gen_hrr(la, lb, lc, ld, accname, em: Emitter):
-    """Emit bra then ket HRR on contracted accumulators; returns out index map."""
+def gen_hrr(la, lb, lc, ld, accname, em: Emitter, avec=None):
+    """Emit bra then ket HRR on contracted accumulators; returns out index map.
+    avec: the functions wanted of the bra's first shell (all by default)."""
+    avec = avec or cart(la)
     fs = [f for lf in range(lc, lc + ld + 1) for f in cart(lf)]
     # bra: (a,b|f) for |a|=la, |b|=lb
     seen = {}
@@ -213,7 +216,7 @@ def gen_hrr(la, lb, lc, ld, accname, em: Emitter):
         order.append(key)
         return key
 
-    finals_ab = [(a, b) for a in cart(la) for b in cart(lb)]
+    finals_ab = [(a, b) for a in avec for b in cart(lb)]
     for a, b in finals_ab:
         bra(a, b)
 
@@ -260,7 +263,7 @@ def gen_hrr(la, lb, lc, ld, accname, em: Emitter):
 
     out_map = {}
     nB, nC, nD = len(cart(lb)), len(cart(lc)), len(cart(ld))
-    for ia, a in enumerate(cart(la)):
+    for ia, a in enumerate(avec):
         for ib, b in enumerate(cart(lb)):
             ab = (a, b)
             for key in korder:
@@ -294,20 +297,45 @@ def _suffix_block(lines, suf):
     return [pat.sub(lambda m: m.group(1) + suf, ln) for ln in lines]
 
 
-def gen_class(la, lb, lc, ld, uniform_bra=False):
-    """One class's contracted-quartet routine.  By default the ket primitive pairs
+# Classes evaluated in parts: each part computes the quartets' integrals for one
+# Cartesian function of the bra's first shell, so that its accumulators and the
+# VRR terms they need fit the register file (whole, these classes spill 0.6 to
+# 2.9 KB per lane).  The parts repeat some VRR terms: summed over the parts, 1.7
+# ((dp|pp)), 1.9 ((dp|dp)), 2.3 ((dd|pp)) and 2.4 ((dd|ds)) times the whole
+# class's VRR operations; restricting the ket instead would cost 2.4 and more for
+# the last three, since the recurrence raises the bra first.  In J/K mode (dp|pp)
+# stays whole: there its parts' contractions cost more than its spills (C8H18:
+# 0.18 ms whole, 0.30 ms in parts; energy 0.30 and 0.13).
+PARTS_ENERGY = {(2, 1, 1, 1), (2, 1, 2, 1), (2, 2, 1, 1), (2, 2, 2, 0)}
+PARTS_JK = {(2, 1, 2, 1), (2, 2, 1, 1), (2, 2, 2, 0)}
+
+
+def part_functions(la, lb, part):
+    """The bra function of a part (index into cart(la)) and the [e0| its HRR starts from."""
+    a = cart(la)[part]
+    es = {(a[0] + x, a[1] + y, a[2] + z) for b in cart(lb) for x in range(b[0] + 1) for y in range(b[1] + 1)
+          for z in range(b[2] + 1)}
+    return [a], sorted(es, key=lambda e: (sum(e), e))
+
+
+def gen_class(la, lb, lc, ld, uniform_bra=False, part=None):
+    """One class's contracted-quartet routine, or one part of it (PARTS_ENERGY, PARTS_JK).  By default the ket primitive pairs
     are wave-uniform (scalar loads) and the bra's are per lane; uniform_bra swaps
     the two (the transposed J/K kernel: one bra pair per wavefront, ket pairs per
     lane).  The arithmetic is the same."""
     L = la + lb + lc + ld
     em = Emitter()
     name = f"eri_{la}{lb}{lc}{ld}" + ("_ub" if uniform_bra else "")
+    avec = es = None
+    if part is not None:
+        avec, es = part_functions(la, lb, part)
+        name += f"_p{part}"
     em.emit(f"// class ({'spd'[la]}{'spd'[lb]}|{'spd'[lc]}{'spd'[ld]}), L = {L}")
     em.emit(f"__device__ __forceinline__ void {name}(const PrimPair* __restrict__ bp, int nbp,")
     em.emit(f"        const PrimPair* __restrict__ kp, int nkp, double ABx, double ABy, double ABz,")
     em.emit(f"        double CDx, double CDy, double CDz, const double* __restrict__ btab, double* __restrict__ out) {{")
     body = Emitter()
-    accmap, nvrr, targets = gen_vrr(la, lb, lc, ld, body)
+    accmap, nvrr, targets = gen_vrr(la, lb, lc, ld, body, es)
     acc = {t: f"acc{n}" for n, t in enumerate(targets)}
     em.emit("    " + " ".join(f"double {acc[t]} = 0.0;" for t in targets))
     if uniform_bra:
@@ -365,7 +393,7 @@ def gen_class(la, lb, lc, ld, uniform_bra=False):
     em.flops += blk.flops
     em.emit("    }")
     hr = Emitter()
-    gen_hrr(la, lb, lc, ld, acc, hr)
+    gen_hrr(la, lb, lc, ld, acc, hr, avec)
     em.lines += hr.lines
     em.emit("}")
     # per primitive quartet: setup ~ 25 flops + boys (approx 2*8 + 3*L + exp~20) + VRR + accumulate
@@ -376,15 +404,14 @@ def gen_class(la, lb, lc, ld, uniform_bra=False):
 
 
 # Classes evaluated by the cooperative kernel (one wavefront per contracted
-# quartet, intermediates in LDS): the (dd| classes with p or d kets, whose
-# one-lane-per-quartet code spills thousands of registers and whose quartets are
-# few.  Classes with many smaller quartets ((dp|pp), (dp|dp), (dd|ds)) measured
-# faster on the straight-line kernels despite their spills.
-COOP_DEFAULT = [(2, 2, 1, 1), (2, 2, 2, 1), (2, 2, 2, 2)]
-# Tables exist for every class whose straight-line code spills; the batch
-# tuner may move the others onto the cooperative kernel.
-COOP_CLASSES = [(2, 1, 1, 1), (2, 1, 2, 0), (2, 1, 2, 1), (2, 2, 1, 0), (2, 2, 1, 1), (2, 2, 2, 0),
-                (2, 2, 2, 1), (2, 2, 2, 2)]
+# quartet, intermediates in LDS).  Their quartets are few, and one lane per
+# quartet would need 36 parts (one per pair of bra functions, 5.2 times the VRR
+# operations and 0.5 to 1.3 MB of code per kernel) or spill 6 to 13 KB per lane.
+# C8H18, in 36 parts against this kernel: (dd|dp) 0.075 and 0.17 ms in energy
+# mode but 0.18 and 0.18 ms in J/K mode, (dd|dd) 0.05 and 0.08, 0.11 and 0.08 ms,
+# for ten minutes of compilation.
+COOP_DEFAULT = [(2, 2, 2, 1), (2, 2, 2, 2)]
+COOP_CLASSES = [(2, 2, 2, 1), (2, 2, 2, 2)]
 
 
 def coop_plan(la, lb, lc, ld):
@@ -598,36 +625,49 @@ def write_coop(path: str) -> None:
 
 
 def main(out_path: str) -> Dict:
+    sig = ["    const PrimPair* __restrict__ bp, int nbp, const PrimPair* __restrict__ kp, int nkp,",
+           "    double ABx, double ABy, double ABz, double CDx, double CDy, double CDz,",
+           "    const double* __restrict__ btab, double* __restrict__ out)"]
     chunks = ["// Generated by gen_eri.py -- do not edit.", "",
-              "template <int LA, int LB, int LC, int LD>",
-              "__device__ void eri_block(const PrimPair* __restrict__ bp, int nbp, const PrimPair* __restrict__ kp,",
-              "    int nkp, double ABx, double ABy, double ABz, double CDx, double CDy, double CDz,",
-              "    const double* __restrict__ btab, double* __restrict__ out);",
-              "template <int LA, int LB, int LC, int LD>",
-              "__device__ void eri_block_ub(const PrimPair* __restrict__ bp, int nbp, const PrimPair* __restrict__ kp,",
-              "    int nkp, double ABx, double ABy, double ABz, double CDx, double CDy, double CDz,",
-              "    const double* __restrict__ btab, double* __restrict__ out);", ""]
+              "// AP: the part of the class (Cartesian function of the bra's first shell; -1: all of them)"]
+    for fn in ("eri_block", "eri_block_ub"):
+        chunks += ["template <int LA, int LB, int LC, int LD, int AP>", f"__device__ void {fn}("] + sig[:2]
+        chunks += [sig[2] + ";"]
     infos = []
-    for (la, lb, lc, ld) in quartet_classes():
-        code, info = gen_class(la, lb, lc, ld)
+
+    def emit(cls, uniform_bra, part):
+        code, _ = gen_class(*cls, uniform_bra=uniform_bra, part=part)
+        name = "eri_" + "".join(str(x) for x in cls) + ("_ub" if uniform_bra else "")
+        if part is not None:
+            name += f"_p{part}"
         chunks.append(code)
-        if (la, lb) != (lc, ld):
-            code_ub, _ = gen_class(la, lb, lc, ld, uniform_bra=True)
-            chunks.append(code_ub)
-            chunks.append(f"template <> __device__ __forceinline__ void eri_block_ub<{la}, {lb}, {lc}, {ld}>(")
-            chunks.append("    const PrimPair* __restrict__ bp, int nbp, const PrimPair* __restrict__ kp, int nkp,")
-            chunks.append("    double ABx, double ABy, double ABz, double CDx, double CDy, double CDz,")
-            chunks.append("    const double* __restrict__ btab, double* __restrict__ out) {")
-            chunks.append(f"  eri_{la}{lb}{lc}{ld}_ub(bp, nbp, kp, nkp, ABx, ABy, ABz, CDx, CDy, CDz, btab, out);")
-            chunks.append("}")
-        chunks.append(f"template <> __device__ __forceinline__ void eri_block<{la}, {lb}, {lc}, {ld}>(")
-        chunks.append("    const PrimPair* __restrict__ bp, int nbp, const PrimPair* __restrict__ kp, int nkp,")
-        chunks.append("    double ABx, double ABy, double ABz, double CDx, double CDy, double CDz,")
-        chunks.append("    const double* __restrict__ btab, double* __restrict__ out) {")
-        chunks.append(f"  eri_{la}{lb}{lc}{ld}(bp, nbp, kp, nkp, ABx, ABy, ABz, CDx, CDy, CDz, btab, out);")
+        chunks.append(f"template <> __device__ __forceinline__ void eri_block{'_ub' if uniform_bra else ''}<"
+                      f"{', '.join(str(x) for x in cls)}, {-1 if part is None else part}>(")
+        chunks.extend(sig[:2])
+        chunks.append(sig[2] + " {")
+        chunks.append(f"  {name}(bp, nbp, kp, nkp, ABx, ABy, ABz, CDx, CDy, CDz, btab, out);")
         chunks.append("}")
         chunks.append("")
+
+    for cls in quartet_classes():
+        la, lb, lc, ld = cls
+        _, info = gen_class(*cls)
         infos.append(info)
+        parts = list(range(len(cart(la))))
+        same = (la, lb) == (lc, ld)
+        # whole class: also for the Schwarz kernels, which take the diagonal classes whole
+        if cls not in PARTS_ENERGY or cls not in PARTS_JK or same:
+            emit(cls, False, None)
+        if cls in PARTS_ENERGY or cls in PARTS_JK:
+            for p in parts:
+                emit(cls, False, p)
+        if not same:
+            for p in parts if cls in PARTS_JK else [None]:
+                emit(cls, True, p)
+    # number of parts by class, in launch order: energy, J/K
+    for nm, st in (("kPartsEnergy", PARTS_ENERGY), ("kPartsJk", PARTS_JK)):
+        chunks.append(f"constexpr int {nm}[21] = {{" + ", ".join(str(len(cart(c[0])) if c in st else 1)
+                                                                for c in quartet_classes()) + "};")
     text = "\n".join(chunks) + "\n"
     # algorithmic FP64 operation counts per class, in launch order (bra class major)
     flops = ["// Generated by gen_eri.py -- do not edit.",

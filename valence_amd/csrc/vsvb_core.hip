@@ -982,6 +982,8 @@ static hipError_t launch_schwarz(int pc, Pair* pairs, const PrimPair* pp, const 
 
 static int quartet_class_index(int bc, int kc) { return bc * (bc + 1) / 2 + kc; }
 
+static int class_parts(int q, bool jk) { return jk ? kPartsJk[q] : kPartsEnergy[q]; }
+
 static int class_bra(int q) {
   for (int b = 0; b < kNPairClass; ++b)
     if (q < quartet_class_index(b, b) + 1) return b;
@@ -1028,6 +1030,11 @@ constexpr double kTailEnergy = 6.0, kTailJk = 45.0, kTailDensity = 25.0;
 static void choose_levels(const vsvb_context* c, int bc, int kc, bool jk, bool tr, int* lb, int* lk) {
   *lb = *lk = 0;
   if (c->nlevels < 2 || c->pair_chunk > 0) return;  // a forced chunk width: whole pairs
+  if (const char* ev = getenv("VSVB_LV")) {
+    *lb = ev[0] - '0'; *lk = ev[2] - '0';
+    if (bc == kc) *lk = *lb;
+    return;
+  }
   const int q = bc * (bc + 1) / 2 + kc;
   const int nd = jk ? c->ndens : 1;
   const double digest = digestion_flops(q, c->nunpd > 0 ? 2 : 1, jk) * nd;
@@ -1152,7 +1159,11 @@ static ClassLaunch coop_launch(vsvb_context* c, int q, bool jk, int per_cu, int 
   L.coop = true;
   L.per_cu = per_cu;
   const int bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
-  const int nb = c->pair_off[bc + 1] - c->pair_off[bc], nk = c->pair_off[kc + 1] - c->pair_off[kc];
+  // few quartets: one wavefront per primitive quartet ((dd|dp) of water, nine
+  // contracted quartets of three primitive ones each: 41 -> 17 us)
+  if (c->nlevels > 1 && c->pair_chunk == 0 && c->ndens == 1 && c->work[bc][1].n * (double)c->work[kc][1].n <= 8.0 * c->ncu)
+    L.lb = L.lk = 1;
+  const int nb = c->work[bc][L.lb].n, nk = c->work[kc][L.lk].n;
   if (nb <= 0 || nk <= 0 || c->coop_idx[q] < 0) return L;  // an empty class launches nothing
   L.overflow = (long long)nb * nk > kMaxUnits;
   if (L.overflow) return L;
@@ -1230,7 +1241,8 @@ static int plan_work(vsvb_context* c, const int* kept) {
       const ClassLaunch cl = policy_launch(c, q, c->pol[q]);
       if (!cl.overflow && (cl.units > 0 || c->ljk[q].units <= 0)) c->ljk[q] = cl;
     }
-    c->partial_per_class[q] = (size_t)c->le[q].blocks * 4;  // energy kernels write four slots per block
+    // energy kernels write four slots per block and part
+    c->partial_per_class[q] = (size_t)c->le[q].blocks * 4 * (c->le[q].coop ? 1 : class_parts(q, false));
     c->partial_total += c->partial_per_class[q];
   }
   return VSVB_OK;
@@ -1475,8 +1487,8 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
       for (int l = 0; l < (split ? kLevels : 1); ++l)
         most = std::max({most, (c->work[bc][l].cap + kStripB - 1) / kStripB, (c->work[kc][l].cap + kStripK - 1) / kStripK});
       c->ctr_off[q] = c->ctr_total;
-      c->ctr_len[q] = most;
-      c->ctr_total += most;
+      c->ctr_len[q] = most * std::max(kPartsEnergy[q], kPartsJk[q]);
+      c->ctr_total += c->ctr_len[q];
     }
   HIP_OK(device_buffer(c, c->d_tilectr, c->ctr_total));
   HIP_OK(coop_prepare(c->device));
@@ -1487,12 +1499,8 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
       c->coop_idx[q] = coop_class(kPairLs[bc][0], kPairLs[bc][1], kPairLs[kc][0], kPairLs[kc][1]);
       const int nb = c->work[bc][0].n, nk = c->work[kc][0].n;
       if (nb <= 0 || nk <= 0) continue;
-      size_t blocks = 0;
-      if (coop_default(c->coop_idx[q]) || !straight_allowed(c, q, false, false))
-        blocks = coop_launch(c, q, false, 0, 0).blocks;
-      else
-        blocks = std::min<size_t>(2048, (size_t)class_occupancy(bc, kc, false, false, 0) * ncu);
-      partial_cap += 4 * blocks;
+      const size_t blocks = std::min<size_t>(2048, (size_t)class_occupancy(bc, kc, false, false, 0) * ncu);
+      partial_cap += 4 * blocks * class_parts(q, false);
     }
   HIP_OK(device_buffer(c, c->d_partial, std::max<size_t>(partial_cap, 1) * 2));
   // segment lists last: in the allocation-free entry they are left out where
@@ -1686,10 +1694,9 @@ static QuartetArgs class_args(vsvb_context* c, int bc, int kc, const ClassLaunch
                               const double* dens, double* jacc, double* kacc, double* partial) {
   const int q = quartet_class_index(bc, kc);
   QuartetArgs a{};
-  const int lb = cl.coop ? 0 : cl.lb, lk = cl.coop ? 0 : cl.lk;
-  const WorkList &B = c->work[bc][lb], &K = c->work[kc][lk];
-  a.bra = (lb ? c->d_split.p : c->d_pairs.p) + B.off;
-  a.ket = (lk ? c->d_split.p : c->d_pairs.p) + K.off;
+  const WorkList &B = c->work[bc][cl.lb], &K = c->work[kc][cl.lk];
+  a.bra = (cl.lb ? c->d_split.p : c->d_pairs.p) + B.off;
+  a.ket = (cl.lk ? c->d_split.p : c->d_pairs.p) + K.off;
   a.nbra = B.n;
   a.nket = K.n;
   a.pp = c->d_pp.p;

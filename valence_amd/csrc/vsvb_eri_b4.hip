@@ -1,6 +1,4 @@
 // Instantiates the quartet kernels whose bra pair class is (dp|; one translation unit per bra class so they compile in parallel.
-// (dp|dp) has no straight-line kernel: it would spill 2.5 to 13.5 KB per lane, and the
-// cooperative kernel takes it (scratch reported as SIZE_MAX).
 #include "vsvb_eri_kernels.h"
 
 namespace vsvb {
@@ -11,6 +9,7 @@ hipError_t launch_quartet_b4(int kc, const QuartetArgs& a, bool jk, bool tr, int
     case 1: return launch_q<2, 1, 1, 0>(a, jk, tr, nblocks, lds, st);
     case 2: return launch_q<2, 1, 1, 1>(a, jk, tr, nblocks, lds, st);
     case 3: return launch_q<2, 1, 2, 0>(a, jk, tr, nblocks, lds, st);
+    case 4: return launch_q<2, 1, 2, 1>(a, jk, tr, nblocks, lds, st);
     default: return hipErrorInvalidValue;
   }
 }
@@ -22,6 +21,7 @@ hipError_t launch_groups_b4(int kc, const QuartetArgs* gs, int ng, bool tr, int 
     case 1: return launch_q_groups<2, 1, 1, 0>(gs, ng, tr, nblocks, lds, stamp, st);
     case 2: return launch_q_groups<2, 1, 1, 1>(gs, ng, tr, nblocks, lds, stamp, st);
     case 3: return launch_q_groups<2, 1, 2, 0>(gs, ng, tr, nblocks, lds, stamp, st);
+    case 4: return launch_q_groups<2, 1, 2, 1>(gs, ng, tr, nblocks, lds, stamp, st);
     default: return hipErrorInvalidValue;
   }
 }
@@ -32,6 +32,7 @@ int occupancy_b4(int kc, bool jk, bool tr, size_t lds) {
     case 1: return occupancy_q<2, 1, 1, 0>(jk, tr, lds);
     case 2: return occupancy_q<2, 1, 1, 1>(jk, tr, lds);
     case 3: return occupancy_q<2, 1, 2, 0>(jk, tr, lds);
+    case 4: return occupancy_q<2, 1, 2, 1>(jk, tr, lds);
     default: return 1;
   }
 }
@@ -42,7 +43,7 @@ size_t scratch_b4(int kc, bool jk, bool tr) {
     case 1: return scratch_q<2, 1, 1, 0>(jk, tr);
     case 2: return scratch_q<2, 1, 1, 1>(jk, tr);
     case 3: return scratch_q<2, 1, 2, 0>(jk, tr);
-    case 4: return SIZE_MAX;
+    case 4: return scratch_q<2, 1, 2, 1>(jk, tr);
     default: return 0;
   }
 }

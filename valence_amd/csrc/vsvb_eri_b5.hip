@@ -1,6 +1,4 @@
 // Instantiates the quartet kernels whose bra pair class is (dd|; one translation unit per bra class so they compile in parallel.
-// (dd|pp), (dd|dp) and (dd|dd) have no straight-line kernel: they would spill 2.5 to 13.5 KB per lane, and the
-// cooperative kernel takes them (scratch reported as SIZE_MAX).
 #include "vsvb_eri_kernels.h"
 
 namespace vsvb {
@@ -9,6 +7,7 @@ hipError_t launch_quartet_b5(int kc, const QuartetArgs& a, bool jk, bool tr, int
   switch (kc) {
     case 0: return launch_q<2, 2, 0, 0>(a, jk, tr, nblocks, lds, st);
     case 1: return launch_q<2, 2, 1, 0>(a, jk, tr, nblocks, lds, st);
+    case 2: return launch_q<2, 2, 1, 1>(a, jk, tr, nblocks, lds, st);
     case 3: return launch_q<2, 2, 2, 0>(a, jk, tr, nblocks, lds, st);
     default: return hipErrorInvalidValue;
   }
@@ -19,6 +18,7 @@ hipError_t launch_groups_b5(int kc, const QuartetArgs* gs, int ng, bool tr, int 
   switch (kc) {
     case 0: return launch_q_groups<2, 2, 0, 0>(gs, ng, tr, nblocks, lds, stamp, st);
     case 1: return launch_q_groups<2, 2, 1, 0>(gs, ng, tr, nblocks, lds, stamp, st);
+    case 2: return launch_q_groups<2, 2, 1, 1>(gs, ng, tr, nblocks, lds, stamp, st);
     case 3: return launch_q_groups<2, 2, 2, 0>(gs, ng, tr, nblocks, lds, stamp, st);
     default: return hipErrorInvalidValue;
   }
@@ -28,6 +28,7 @@ int occupancy_b5(int kc, bool jk, bool tr, size_t lds) {
   switch (kc) {
     case 0: return occupancy_q<2, 2, 0, 0>(jk, tr, lds);
     case 1: return occupancy_q<2, 2, 1, 0>(jk, tr, lds);
+    case 2: return occupancy_q<2, 2, 1, 1>(jk, tr, lds);
     case 3: return occupancy_q<2, 2, 2, 0>(jk, tr, lds);
     default: return 1;
   }
@@ -37,7 +38,7 @@ size_t scratch_b5(int kc, bool jk, bool tr) {
   switch (kc) {
     case 0: return scratch_q<2, 2, 0, 0>(jk, tr);
     case 1: return scratch_q<2, 2, 1, 0>(jk, tr);
-    case 2: return SIZE_MAX;
+    case 2: return scratch_q<2, 2, 1, 1>(jk, tr);
     case 3: return scratch_q<2, 2, 2, 0>(jk, tr);
     case 4: return SIZE_MAX;
     case 5: return SIZE_MAX;

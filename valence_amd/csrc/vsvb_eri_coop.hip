@@ -97,8 +97,9 @@ __device__ __forceinline__ void coop_body(const QuartetArgs& a, const CoopDesc& 
       if (c0 + lane < claim && um < a.ntiles) {
         const int b0 = um / a.nket, k0 = um - b0 * a.nket;
         if (!a.same || k0 <= b0) {
-          keep = a.bra[b0].Q * a.ket[k0].Q >= a.tau;
-          if (!keep) ++nskip;
+          const Pair &B = a.bra[b0], &K = a.ket[k0];
+          keep = B.Q * K.Q >= a.tau;
+          if (!keep && (B.seg | K.seg) == 0) ++nskip;
         }
       }
       unsigned long long live = __ballot(keep);
@@ -162,7 +163,7 @@ __device__ __forceinline__ void coop_body(const QuartetArgs& a, const CoopDesc& 
         }
         __syncthreads();
       }
-      ++nq;
+      nq += (P.seg | K.seg) == 0;  // a quartet of segments is counted once
       nprimq += (unsigned long long)P.npp * K.npp;
       const double deg = (P.offdiag ? 2.0 : 1.0) * (K.offdiag ? 2.0 : 1.0) * ((ib != ik || !a.same) ? 2.0 : 1.0);
       const int ma = a.shells[P.A].ao, mb = a.shells[P.B].ao;

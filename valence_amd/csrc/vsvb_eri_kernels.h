@@ -28,6 +28,19 @@ namespace vsvb {
 
 #include "eri_gen.inc"
 
+// Pair class of two angular momenta and quartet class of four (launch order).
+__host__ __device__ constexpr int pair_class(int la, int lb) { return la * (la + 1) / 2 + lb; }
+__host__ __device__ constexpr int quartet_class(int la, int lb, int lc, int ld) {
+  return pair_class(la, lb) * (pair_class(la, lb) + 1) / 2 + pair_class(lc, ld);
+}
+// Parts of a quartet class in one mode: part p has the A function p; a class
+// that is not split is one part, -1 (see PARTS_ENERGY in gen_eri.py).
+template <int LA, int LB, int LC, int LD, bool kJK>
+struct Parts {
+  static constexpr int n = kJK ? kPartsJk[quartet_class(LA, LB, LC, LD)] : kPartsEnergy[quartet_class(LA, LB, LC, LD)];
+  static constexpr int a(int p) { return n > 1 ? p : -1; }
+};
+
 struct QuartetArgs {
   const Pair* bra;      // work pairs of the bra class: shell pairs, or segments of them (Pair::seg)
   const Pair* ket;      // work pairs of the ket class
@@ -48,11 +61,11 @@ struct QuartetArgs {
   int nspin;            // 1 = closed shell (D = R, RT = 2R, x = 2); 2 = open (alpha, beta);
                         // 0 = Coulomb only (J/K mode): J of each of nwfn general symmetric densities
   const double* dens;   // [nwfn][nspin][nbf][nbf]
-  double* partial;      // energy: [gridDim.x * 4][nwfn] per-wave partial sums
+  double* partial;      // energy: [parts][gridDim.x * 4][nwfn] per-wave partial sums
   double* jacc;         // J/K mode: Coulomb accumulators [nwfn][nbf][nbf]
   double* kacc;         // J/K mode: exchange accumulators [nwfn][nspin][nbf][nbf]
   unsigned long long* counters;  // the class's {quartets evaluated, primitive quartets, skipped} in slot 0
-  int* tile_ctr;        // dynamic tile counter(s), zero before the launch: one, or one per strip (J/K)
+  int* tile_ctr;        // dynamic tile counters, zero before the launch: nstrip per part
   int nstrip;           // straight-line units: energy segments of kSegTiles bra tiles, J/K strips (bra, or ket
                         // when transposed), each with its own work counter
   int lds_k;            // J/K mode: accumulate exchange rows in LDS (nbf * (NC + ND) doubles of dynamic LDS)
@@ -156,9 +169,11 @@ __device__ __forceinline__ void stage_boys(const double* __restrict__ boys, doub
   __syncthreads();
 }
 
-template <int LA, int LB, int LC, int LD>
+template <int LA, int LB, int LC, int LD, int AP>
 __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const double* __restrict__ btab) {
-  constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
+  constexpr int NA = AP < 0 ? ncart(LA) : 1, NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
+  constexpr int A0 = AP < 0 ? 0 : AP;  // the part's first A function
+  constexpr bool kFirst = A0 == 0;     // the part that counts the quartets
   constexpr int NAB = NA * NB, NCD = NC * ND;
   const int n = a.nbf;
   const size_t nn = (size_t)n * n;
@@ -228,7 +243,7 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
       if (k0 >= a.nket) continue;  // one class: the last tile is not full
     } else {
       int ul = 0;
-      if (lane == 0) ul = atomicAdd(a.tile_ctr + sg, 1);
+      if (lane == 0) ul = atomicAdd(a.tile_ctr + blockIdx.y * a.nstrip + sg, 1);
       ul = __builtin_amdgcn_readfirstlane(__shfl(ul, 0, 64));
       const int t0 = sg * a.seg_tiles;
       if (ul >= min(a.seg_tiles, nbt - t0) * a.nkc) {  // this segment is exhausted
@@ -273,7 +288,7 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
       }
       double v[NAB * NCD];
       if (act) {
-        eri_block<LA, LB, LC, LD>(a.pp + P.pp0, P.npp, a.pp + K.pp0, K.npp, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy,
+        eri_block<LA, LB, LC, LD, AP>(a.pp + P.pp0, P.npp, a.pp + K.pp0, K.npp, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy,
                                   K.ABz, btab, v);
         nq += first;
         nprimq += (unsigned long long)P.npp * K.npp;
@@ -285,7 +300,7 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
       const double deg =
           act ? (P.offdiag ? 2.0 : 1.0) * (K.offdiag ? 2.0 : 1.0) * ((ib != ik || !a.same) ? 2.0 : 1.0) : 0.0;
       // inactive lanes read valid blocks and contribute zero
-      const int ma = a.shells[P.A].ao, mb = a.shells[P.B].ao;
+      const int ma = a.shells[P.A].ao + A0, mb = a.shells[P.B].ao;
       const int mc = a.shells[K.A].ao, md = a.shells[K.B].ao;
       for (int w = 0; w < a.nwfn; ++w) {
         const double* D0 = a.dens + (size_t)w * (a.nspin > 0 ? a.nspin : 1) * nn;
@@ -345,11 +360,11 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
       for (int ww = 0; ww < kMaxW; ++ww)
         if (ww == w) s = esum[ww];
       s = wave_sum(s);
-      if (lane == 0) a.partial[((size_t)blockIdx.x * 4 + wave) * a.nwfn + w] = s;
+      if (lane == 0) a.partial[(((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 4 + wave) * a.nwfn + w] = s;
     }
   }
   stamp_wave(a.stamp, true);
-  add_counters(a.counters, nq, nprimq, nskip);
+  add_counters(kFirst ? a.counters : nullptr, nq, nprimq, nskip);
 }
 
 
@@ -365,9 +380,11 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
 // to the global accumulators.
 constexpr int kStripB = 4 * kTileB;
 
-template <int LA, int LB, int LC, int LD>
+template <int LA, int LB, int LC, int LD, int AP>
 __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const double* __restrict__ btab) {
-  constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
+  constexpr int NA = AP < 0 ? ncart(LA) : 1, NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
+  constexpr int A0 = AP < 0 ? 0 : AP;  // the part's first A function
+  constexpr bool kFirst = A0 == 0;     // the part that counts the quartets
   constexpr int NAB = NA * NB, NCD = NC * ND, NK = NC + ND;
   extern __shared__ double kbuf[];
   __shared__ int s_unit;
@@ -401,7 +418,7 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
     const int ibf = s_ * kStripB + wave * kTileB + lane;
     if (s_ < 0 || ibf >= a.nbra) return;
     const Pair Pf = a.bra[ibf];
-    const int fa = a.shells[Pf.A].ao, fb = a.shells[Pf.B].ao;
+    const int fa = a.shells[Pf.A].ao + A0, fb = a.shells[Pf.B].ao;
 #pragma unroll
     for (int ij = 0; ij < (kRegJ ? NAB : 1); ++ij) {
       if (jreg[ij] != 0.0) unsafeAtomicAdd(&a.jacc[(size_t)(fa + ij / NB) * n + fb + ij % NB], jreg[ij]);
@@ -415,7 +432,7 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
   int st = (int)(blockIdx.x % (unsigned)a.nstrip), left = a.nstrip;
   for (;;) {
     __syncthreads();  // the previous unit is flushed and s_unit, s_qmax are free
-    if (threadIdx.x == 0) s_unit = atomicAdd(a.tile_ctr + st, a.kchunk);
+    if (threadIdx.x == 0) s_unit = atomicAdd(a.tile_ctr + blockIdx.y * a.nstrip + st, a.kchunk);
     __syncthreads();
     const int k0 = __builtin_amdgcn_readfirstlane(s_unit);
     if (k0 >= a.nket) {  // this strip is exhausted
@@ -463,7 +480,7 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
       }
       double v[NAB * NCD];
       if (act) {
-        eri_block<LA, LB, LC, LD>(a.pp + P.pp0, P.npp, a.pp + K.pp0, K.npp, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy,
+        eri_block<LA, LB, LC, LD, AP>(a.pp + P.pp0, P.npp, a.pp + K.pp0, K.npp, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy,
                                   K.ABz, btab, v);
         nq += first;
         nprimq += (unsigned long long)P.npp * K.npp;
@@ -474,8 +491,8 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
       const bool wact = __any(act);  // wave-uniform
       const double deg = act ? (P.offdiag ? 2.0 : 1.0) * (K.offdiag ? 2.0 : 1.0) * ((ib != ik || !a.same) ? 2.0 : 1.0)
                              : 0.0;
-      // inactive lanes read a valid (ket) block and contribute zero
-      const int ma = act ? a.shells[P.A].ao : a.shells[K.A].ao, mb = act ? a.shells[P.B].ao : a.shells[K.B].ao;
+      // inactive lanes read the block of their (valid) bra pair and contribute zero
+      const int ma = a.shells[P.A].ao + A0, mb = a.shells[P.B].ao;
       const int mc = a.shells[K.A].ao, md = a.shells[K.B].ao;
       const double fj = 0.25 * deg, fk = 0.125 * deg * xfac;
       for (int w = 0; w < a.nwfn; ++w) {
@@ -598,7 +615,7 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
   }
   if (racc) flush_j(jst);
   stamp_wave(a.stamp, true);
-  add_counters(a.counters, nq, nprimq, nskip);
+  add_counters(kFirst ? a.counters : nullptr, nq, nprimq, nskip);
 }
 
 // Transposed J/K unit, for classes whose bra and ket pair classes differ: one
@@ -611,9 +628,11 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
 // idle) or large bra blocks (fewer global atomics per quartet).
 constexpr int kStripK = 256;
 
-template <int LA, int LB, int LC, int LD>
+template <int LA, int LB, int LC, int LD, int AP>
 __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const double* __restrict__ btab) {
-  constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
+  constexpr int NA = AP < 0 ? ncart(LA) : 1, NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
+  constexpr int A0 = AP < 0 ? 0 : AP;  // the part's first A function
+  constexpr bool kFirst = A0 == 0;     // the part that counts the quartets
   constexpr int NAB = NA * NB, NCD = NC * ND, NR = NA + NB;
   extern __shared__ double kbuf[];
   __shared__ int s_unit;
@@ -657,7 +676,7 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const dou
   int st = (int)(blockIdx.x % (unsigned)a.nstrip), left = a.nstrip;
   for (;;) {
     __syncthreads();  // the previous unit is flushed and s_unit, s_qmax are free
-    if (threadIdx.x == 0) s_unit = atomicAdd(a.tile_ctr + st, a.kchunk);
+    if (threadIdx.x == 0) s_unit = atomicAdd(a.tile_ctr + blockIdx.y * a.nstrip + st, a.kchunk);
     __syncthreads();
     const int b0 = __builtin_amdgcn_readfirstlane(s_unit);
     if (b0 >= a.nbra) {  // this ket strip is exhausted
@@ -703,7 +722,7 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const dou
       }
       double v[NAB * NCD];
       if (act) {
-        eri_block_ub<LA, LB, LC, LD>(a.pp + P.pp0, P.npp, a.pp + K.pp0, K.npp, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy,
+        eri_block_ub<LA, LB, LC, LD, AP>(a.pp + P.pp0, P.npp, a.pp + K.pp0, K.npp, P.ABx, P.ABy, P.ABz, K.ABx, K.ABy,
                                      K.ABz, btab, v);
         nq += first;
         nprimq += (unsigned long long)P.npp * K.npp;
@@ -714,7 +733,7 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const dou
       const bool wact = __any(act);  // wave-uniform
       // bra and ket classes differ, so every quartet stands for its (cd|ab) image too
       const double deg = act ? (P.offdiag ? 2.0 : 1.0) * (K.offdiag ? 2.0 : 1.0) * 2.0 : 0.0;
-      const int ma = a.shells[P.A].ao, mb = a.shells[P.B].ao;
+      const int ma = a.shells[P.A].ao + A0, mb = a.shells[P.B].ao;
       const int mc = a.shells[K.A].ao, md = a.shells[K.B].ao;
       const double fj = 0.25 * deg, fk = 0.125 * deg * xfac;
       for (int w = 0; w < a.nwfn; ++w) {
@@ -837,24 +856,40 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const dou
   }
   if (racc) flush_j(jst);
   stamp_wave(a.stamp, true);
-  add_counters(a.counters, nq, nprimq, nskip);
+  add_counters(kFirst ? a.counters : nullptr, nq, nprimq, nskip);
+}
+
+// The body of one mode for the part this workgroup was launched for
+// (blockIdx.y): kMode 0 energy, 1 J/K, 2 J/K transposed.
+template <int LA, int LB, int LC, int LD, int kMode, int kPart = 0>
+__device__ __forceinline__ void quartet_part(const QuartetArgs& a, const double* __restrict__ btab) {
+  using P = Parts<LA, LB, LC, LD, kMode != 0>;
+  if constexpr (kPart + 1 < P::n) {
+    if (blockIdx.y != (unsigned)kPart) {
+      quartet_part<LA, LB, LC, LD, kMode, kPart + 1>(a, btab);
+      return;
+    }
+  }
+  if constexpr (kMode == 0)
+    quartet_energy_body<LA, LB, LC, LD, P::a(kPart)>(a, btab);
+  else if constexpr (kMode == 1)
+    quartet_jk_body<LA, LB, LC, LD, P::a(kPart)>(a, btab);
+  else
+    quartet_jkt_body<LA, LB, LC, LD, P::a(kPart)>(a, btab);
 }
 
 template <int LA, int LB, int LC, int LD>
 __global__ void __launch_bounds__(256) quartet_jkt_kernel(QuartetArgs a) {
   __shared__ __attribute__((aligned(16))) double btab[kBoysCLen];  // this class's compact Boys table
   stage_boys<LA + LB + LC + LD>(a.boys, btab);
-  quartet_jkt_body<LA, LB, LC, LD>(a, btab);
+  quartet_part<LA, LB, LC, LD, 2>(a, btab);
 }
 
 template <int LA, int LB, int LC, int LD, bool kJK>
 __global__ void __launch_bounds__(256) quartet_kernel(QuartetArgs a) {
   __shared__ __attribute__((aligned(16))) double btab[kBoysCLen];  // this class's compact Boys table
   stage_boys<LA + LB + LC + LD>(a.boys, btab);
-  if constexpr (kJK)
-    quartet_jk_body<LA, LB, LC, LD>(a, btab);
-  else
-    quartet_energy_body<LA, LB, LC, LD>(a, btab);
+  quartet_part<LA, LB, LC, LD, kJK ? 1 : 0>(a, btab);
 }
 
 // One J/K launch of a class over several groups (molecules) of a batch, with
@@ -874,10 +909,7 @@ __global__ void __launch_bounds__(256) quartet_jk_groups_kernel(const QuartetArg
   for (int g = 0; g < ng; ++g) {
     const QuartetArgs a = gs[g];
     if (a.ntiles > 0) {
-      if constexpr (kTr)
-        quartet_jkt_body<LA, LB, LC, LD>(a, btab);
-      else
-        quartet_jk_body<LA, LB, LC, LD>(a, btab);
+      quartet_part<LA, LB, LC, LD, kTr ? 2 : 1>(a, btab);
     }
     __syncthreads();  // the group's LDS blocks are flushed before the next group's zeroing
   }
@@ -900,7 +932,7 @@ __global__ void __launch_bounds__(256) schwarz_kernel(Pair* pairs, const PrimPai
   for (int k = 0; k < NAB; ++k) dsum[k] = 0.0;
   for (int b = lane; b < P.npp; b += 64) {
     double v[NAB * NAB];
-    eri_block<LA, LB, LA, LB>(pp + P.pp0 + b, 1, pp + P.pp0, P.npp, P.ABx, P.ABy, P.ABz, P.ABx, P.ABy, P.ABz,
+    eri_block<LA, LB, LA, LB, -1>(pp + P.pp0 + b, 1, pp + P.pp0, P.npp, P.ABx, P.ABy, P.ABz, P.ABx, P.ABy, P.ABz,
                               boys + kBoysCOff + (size_t)(2 * (LA + LB)) * kBoysCLen, v);
 #pragma unroll
     for (int k = 0; k < NAB; ++k) dsum[k] += v[k * NAB + k];
@@ -950,16 +982,16 @@ static hipError_t launch_q(const QuartetArgs& a, bool jk, bool tr, int nblocks, 
   if (nblocks <= 0 || a.ntiles <= 0) return hipSuccess;
   if constexpr (LA != LC || LB != LD) {
     if (jk && tr) {
-      hipLaunchKernelGGL((quartet_jkt_kernel<LA, LB, LC, LD>), dim3(nblocks), dim3(256), lds_bytes, st, a);
+      hipLaunchKernelGGL((quartet_jkt_kernel<LA, LB, LC, LD>), dim3(nblocks, Parts<LA, LB, LC, LD, true>::n), dim3(256), lds_bytes, st, a);
       return hipGetLastError();
     }
   } else {
     if (tr) return hipErrorInvalidValue;  // no transposed kernel for a class paired with itself
   }
   if (jk)
-    hipLaunchKernelGGL((quartet_kernel<LA, LB, LC, LD, true>), dim3(nblocks), dim3(256), lds_bytes, st, a);
+    hipLaunchKernelGGL((quartet_kernel<LA, LB, LC, LD, true>), dim3(nblocks, Parts<LA, LB, LC, LD, true>::n), dim3(256), lds_bytes, st, a);
   else
-    hipLaunchKernelGGL((quartet_kernel<LA, LB, LC, LD, false>), dim3(nblocks), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((quartet_kernel<LA, LB, LC, LD, false>), dim3(nblocks, Parts<LA, LB, LC, LD, false>::n), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
@@ -969,14 +1001,14 @@ static hipError_t launch_q_groups(const QuartetArgs* gs, int ng, bool tr, int nb
   if (nblocks <= 0 || ng <= 0) return hipSuccess;
   if constexpr (LA != LC || LB != LD) {
     if (tr) {
-      hipLaunchKernelGGL((quartet_jk_groups_kernel<LA, LB, LC, LD, true>), dim3(nblocks), dim3(256), lds_bytes, st, gs,
+      hipLaunchKernelGGL((quartet_jk_groups_kernel<LA, LB, LC, LD, true>), dim3(nblocks, Parts<LA, LB, LC, LD, true>::n), dim3(256), lds_bytes, st, gs,
                          ng, stamp);
       return hipGetLastError();
     }
   } else {
     if (tr) return hipErrorInvalidValue;  // no transposed kernel for a class paired with itself
   }
-  hipLaunchKernelGGL((quartet_jk_groups_kernel<LA, LB, LC, LD, false>), dim3(nblocks), dim3(256), lds_bytes, st, gs, ng,
+  hipLaunchKernelGGL((quartet_jk_groups_kernel<LA, LB, LC, LD, false>), dim3(nblocks, Parts<LA, LB, LC, LD, true>::n), dim3(256), lds_bytes, st, gs, ng,
                      stamp);
   return hipGetLastError();
 }
