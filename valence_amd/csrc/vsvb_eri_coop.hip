@@ -356,13 +356,15 @@ size_t coop_lds_bytes(int idx, bool jk) {
 bool coop_default(int idx) { return idx >= 0 && kCoopDesc[idx].dflt != 0; }
 
 int coop_occupancy(int idx, bool jk) {
-  int nb = 0;
-  const size_t lds = coop_lds_bytes(idx, jk);
-  if (jk)
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, coop_kernel<true>, 64, lds);
-  else
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, coop_kernel<false>, 64, lds);
-  return nb > 0 ? nb : 1;
+  struct Table {
+    hipFuncAttributes at[2] = {};
+    Table() {
+      (void)hipFuncGetAttributes(&at[0], reinterpret_cast<const void*>(coop_kernel<false>));
+      (void)hipFuncGetAttributes(&at[1], reinterpret_cast<const void*>(coop_kernel<true>));
+    }
+  };
+  static const Table t;
+  return blocks_per_cu(t.at[jk ? 1 : 0], 64, coop_lds_bytes(idx, jk));
 }
 
 // The step tables on a device: a device array initialized in the code object,

@@ -22,6 +22,8 @@
 // written in closed form, D = C S^-1 C^T (Jacobi's complementary-minor
 // identity applied to the strikes of det, src/valence.F90:1895-2056).
 #pragma once
+#include <algorithm>
+
 #include "vsvb_device.h"
 
 namespace vsvb {
@@ -943,38 +945,48 @@ __global__ void __launch_bounds__(256) schwarz_kernel(Pair* pairs, const PrimPai
   if (lane == 0) pairs[p0 + i].Q = sqrt(m);
 }
 
+// Workgroups of `threads` threads that fit a CU at once: 512 registers per lane
+// of a SIMD in blocks of 8, at most 8 wavefronts per SIMD, 160 KB of LDS.  Not
+// hipOccupancyMaxActiveBlocksPerMultiprocessor: the HIP runtime of ROCm 7.2
+// counts 256 registers for these kernels and halves most grids ((ss|ss) 2
+// instead of 4 workgroups per CU: C8H18 energies 1.07 ms instead of 0.41 ms in
+// that class), while the one in torch's wheel counts 512.
+inline int blocks_per_cu(const hipFuncAttributes& at, int threads, size_t dynamic_lds) {
+  const int regs = (std::max(at.numRegs, 1) + 7) / 8 * 8;
+  const int waves = std::min(8, 512 / regs) * 4;
+  const size_t lds = at.sharedSizeBytes + dynamic_lds;
+  const int by_lds = lds > 0 ? (int)((size_t)163840 / lds) : waves;
+  return std::max(1, std::min(waves / ((threads + 63) / 64), by_lds));
+}
+
+// Attributes of the straight-line kernel of a class in one mode and orientation.
+template <int LA, int LB, int LC, int LD>
+static const hipFuncAttributes& attributes_q(bool jk, bool tr) {
+  struct Table {
+    hipFuncAttributes at[3] = {};  // energy, J/K, J/K transposed
+    Table() {
+      (void)hipFuncGetAttributes(&at[0], reinterpret_cast<const void*>(quartet_kernel<LA, LB, LC, LD, false>));
+      (void)hipFuncGetAttributes(&at[1], reinterpret_cast<const void*>(quartet_kernel<LA, LB, LC, LD, true>));
+      if constexpr (LA != LC || LB != LD)
+        (void)hipFuncGetAttributes(&at[2], reinterpret_cast<const void*>(quartet_jkt_kernel<LA, LB, LC, LD>));
+      else
+        at[2] = at[1];
+    }
+  };
+  static const Table t;
+  return t.at[jk ? (tr ? 2 : 1) : 0];
+}
+
 template <int LA, int LB, int LC, int LD>
 static int occupancy_q(bool jk, bool tr, size_t lds_bytes) {
-  int n = 0;
-  if constexpr (LA != LC || LB != LD) {
-    if (jk && tr) {
-      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, quartet_jkt_kernel<LA, LB, LC, LD>, 256, lds_bytes);
-      return n > 0 ? n : 1;
-    }
-  }
-  if (jk)
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, quartet_kernel<LA, LB, LC, LD, true>, 256, lds_bytes);
-  else
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, quartet_kernel<LA, LB, LC, LD, false>, 256, 0);
-  return n > 0 ? n : 1;
+  return blocks_per_cu(attributes_q<LA, LB, LC, LD>(jk, tr), 256, jk ? lds_bytes : 0);
 }
 
 // Private (scratch) bytes per lane of the straight-line kernel of a class in
 // one mode and orientation: the register spills of its generated code.
 template <int LA, int LB, int LC, int LD>
 static size_t scratch_q(bool jk, bool tr) {
-  hipFuncAttributes at{};
-  if constexpr (LA != LC || LB != LD) {
-    if (jk && tr) {
-      (void)hipFuncGetAttributes(&at, reinterpret_cast<const void*>(quartet_jkt_kernel<LA, LB, LC, LD>));
-      return at.localSizeBytes;
-    }
-  }
-  if (jk)
-    (void)hipFuncGetAttributes(&at, reinterpret_cast<const void*>(quartet_kernel<LA, LB, LC, LD, true>));
-  else
-    (void)hipFuncGetAttributes(&at, reinterpret_cast<const void*>(quartet_kernel<LA, LB, LC, LD, false>));
-  return at.localSizeBytes;
+  return attributes_q<LA, LB, LC, LD>(jk, tr).localSizeBytes;
 }
 
 template <int LA, int LB, int LC, int LD>
