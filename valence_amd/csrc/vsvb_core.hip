@@ -1081,17 +1081,15 @@ static ClassLaunch straight_launch(vsvb_context* c, int bc, int kc, bool jk, int
                                                  : (long long)nbt * ((nk + kch - 1) / kch);
     L.overflow = units > kMaxUnits;
     L.units = L.overflow ? 0 : (int)units;
-    // several counter segments once claims are chunked (large systems: many
-    // short claims); one counter, heaviest tiles first, otherwise
-    L.seg_tiles = kch > 1 ? kSegTiles : nbt;
-    L.strips = (nbt + L.seg_tiles - 1) / L.seg_tiles;
     L.blocks = std::min((L.units + 3) / 4, cap);
-    if (kch == 1 && bc != kc && nbt > 2) {
-      // a step over the tiles of about 0.38 of their number, coprime to it
-      const int nw = 4 * L.blocks;
-      int step = std::max(1, (int)std::lround(0.382 * nbt));
-      while (std::gcd(step, nbt) != 1) ++step;
-      L.shift = ((step - nw) % nbt + nbt) % nbt % nw;
+    L.strips = (nbt + kSegTiles - 1) / kSegTiles;
+    // a wavefront's step over the tiles (one-ket units) or chunks (chunked ones)
+    // from round to round: about 0.38 of their number, coprime to it
+    const int nw = 4 * L.blocks, period = kch > 1 ? (nk + kch - 1) / kch : (bc != kc ? nbt : 0);
+    if (period > 2 && period < nw) {
+      int step = std::max(1, (int)std::lround(0.382 * period));
+      while (std::gcd(step, period) != 1) ++step;
+      L.shift = ((step - nw) % period + period) % period;
     }
     return L;
   }
@@ -1476,8 +1474,8 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
       seg_cap += W.cap;
     }
   }
-  // work counters: one per energy segment of kSegTiles bra tiles, one per J/K
-  // strip (bra strips, or ket strips transposed), one for the cooperative kernel
+  // work counters: per part one per energy segment of kSegTiles bra tiles and one
+  // per J/K strip (bra strips, or ket strips transposed); one for the cooperative kernel
   static_assert(kSegTiles * kTileB == kStripB, "an energy segment covers one bra strip");
   const bool split = c->npairs <= kSplitMaxPairs;
   c->ctr_total = 0;
@@ -1720,7 +1718,6 @@ static QuartetArgs class_args(vsvb_context* c, int bc, int kc, const ClassLaunch
   a.stamp = c->profile ? c->d_stamps.p + (size_t)q * 2 * kStampSlots : nullptr;
   a.tile_ctr = c->d_tilectr.p + c->ctr_off[q];
   a.nstrip = cl.coop ? 1 : cl.strips;
-  a.seg_tiles = cl.seg_tiles;
   a.shift = cl.shift;
   return a;
 }

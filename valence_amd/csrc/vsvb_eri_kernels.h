@@ -43,6 +43,11 @@ struct Parts {
   static constexpr int a(int p) { return n > 1 ? p : -1; }
 };
 
+// Place of a workgroup in its class's launch: block of blocks, in part `part`.
+struct Place {
+  unsigned block, blocks, part;
+};
+
 struct QuartetArgs {
   const Pair* bra;      // work pairs of the bra class: shell pairs, or segments of them (Pair::seg)
   const Pair* ket;      // work pairs of the ket class
@@ -55,8 +60,7 @@ struct QuartetArgs {
   int ntiles;           // work units: energy: bra tiles (64 pairs) x ket chunks; J/K: strips x claims
   int kchunk;           // pairs of the wave-uniform side per claim (1..64): kets; bras in transposed J/K units
   int nkc;              // energy: ket chunks, ceil(nket / kchunk)
-  int seg_tiles;        // energy: bra tiles per counter segment (nstrip segments)
-  int shift;            // energy, one-ket units: change of a wavefront's place from round to round (below the grid)
+  int shift;            // energy: change of a wavefront's place from round to round (below the grid)
   double tau;           // skip quartet if Q_bra * Q_ket < tau
   int nbf;
   int nwfn;             // wave functions sharing this geometry
@@ -67,9 +71,9 @@ struct QuartetArgs {
   double* jacc;         // J/K mode: Coulomb accumulators [nwfn][nbf][nbf]
   double* kacc;         // J/K mode: exchange accumulators [nwfn][nspin][nbf][nbf]
   unsigned long long* counters;  // the class's {quartets evaluated, primitive quartets, skipped} in slot 0
-  int* tile_ctr;        // dynamic tile counters, zero before the launch: nstrip per part
-  int nstrip;           // straight-line units: energy segments of kSegTiles bra tiles, J/K strips (bra, or ket
-                        // when transposed), each with its own work counter
+  int* tile_ctr;        // J/K and cooperative kernels: work counters, zero before the launch: nstrip per part
+  int nstrip;           // J/K strips (bra, or ket when transposed), energy segments of kSegTiles bra tiles: one work
+                        // counter each
   int lds_k;            // J/K mode: accumulate exchange rows in LDS (nbf * (NC + ND) doubles of dynamic LDS)
   unsigned long long* stamp;  // per-class timing (null when off): kStampSlots pairs {earliest wavefront
                               // start, latest wavefront end} in wall-clock ticks, ~0 and 0 before the launch
@@ -121,9 +125,10 @@ __device__ __forceinline__ void add_counters(unsigned long long* counters, unsig
   }
 }
 
-// Bra pairs of an energy unit (one per lane of a wavefront), and bra tiles of
-// an energy counter segment when the class has several.
+// Bra pairs of an energy unit (one per lane of a wavefront), ket chunk widths
+// from which energy units are claimed, and bra tiles per counter then.
 constexpr int kTileB = 64;
+constexpr int kClaimChunk = 16;
 constexpr int kSegTiles = 4;
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -172,7 +177,7 @@ __device__ __forceinline__ void stage_boys(const double* __restrict__ boys, doub
 }
 
 template <int LA, int LB, int LC, int LD, int AP>
-__device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const double* __restrict__ btab) {
+__device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const Place& at, const double* __restrict__ btab) {
   constexpr int NA = AP < 0 ? ncart(LA) : 1, NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
   constexpr int A0 = AP < 0 ? 0 : AP;  // the part's first A function
   constexpr bool kFirst = A0 == 0;     // the part that counts the quartets
@@ -194,43 +199,47 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
   // heaviest first (most primitive pairs), so low unit indices hold the
   // heaviest quartets and the tail is short.
   //
-  // One-ket units go to the wavefronts by a fixed rule, one per wavefront and
-  // round: claims from one counter cost 6-8 ns each, all wavefronts queueing on
-  // its address, which was the whole time of C8H18's (ss|ss), (ps|ss) and
-  // (ps|ps) launches (151000, 129000 and 111000 claims in 0.97, 0.96 and 0.89
-  // ms).  Units of different bra and ket classes go ket-major, so that the
-  // wavefronts in flight share few kets and their primitive data stay in the
-  // scalar caches; `shift` moves every wavefront over the tiles by about 0.38 of
-  // their number from round to round, so that none keeps to the heavy ones
-  // (without it (ps|ss) took 1.72 ms: its stride left a wavefront on every
-  // second tile).  Units of one class go tile by tile up to the tile's last ket,
-  // with none above the diagonal.
+  // Units go to the wavefronts by a fixed rule, one per wavefront and round:
+  // claims from one counter cost 6-8 ns each, all wavefronts queueing on its
+  // address, which was the whole time of C8H18's (ss|ss), (ps|ss) and (ps|ps)
+  // launches (151000, 129000 and 111000 claims in 0.97, 0.96 and 0.89 ms), and
+  // a counter per segment of the tiles still cost C12H26's (ss|ss) 3.5 ms (1.1
+  // by the fixed rule).  One-ket units of different bra and ket classes go
+  // ket-major, so that the wavefronts in flight share few kets and their
+  // primitive data stay in the scalar caches; `shift` moves every wavefront over
+  // the tiles by about 0.38 of their number from round to round, so that none
+  // keeps to the heavy ones (without it (ps|ss) took 1.72 ms: its stride left a
+  // wavefront on every second tile).  One-ket units of one class go tile by tile
+  // up to the tile's last ket, with none above the diagonal; chunks go tile by
+  // tile, shifted over the chunks.
   //
-  // Chunked units (sparse systems, where the work of a unit varies widely) are
-  // claimed one at a time from atomic counters, with no barrier.  The unit
-  // indices form nstrip segments of seg_tiles * nkc units, each with its own
-  // counter: a wavefront starts on segment (global wave index) mod nstrip and
-  // moves to the next one only when its segment is exhausted, leaving after it
-  // has found every segment exhausted once (counters only grow, so every
-  // wavefront ends).  One lane per ket tests it against the largest bra bound
-  // of the tile, and the wavefront visits only the kets that can pass the
-  // Schwarz test for some lane, so screened (tile, ket) slots cost one claim
-  // per chunk instead of one per ket.
+  // With chunks of several kets (large, sparse systems) one lane per ket tests
+  // it against the largest bra bound of the tile, and the wavefront visits only
+  // the kets that can pass the Schwarz test for some lane.  The work of wide
+  // chunks varies too much for a fixed rule (LiF128, chunks of 64: 0.48 s by it,
+  // 0.36 s claimed), so they are claimed one at a time from the counters of
+  // nstrip segments of kSegTiles tiles: a wavefront starts on segment (global
+  // wave index) mod nstrip, moves to the next one when its segment is exhausted
+  // and leaves after it has found every segment exhausted once (counters only
+  // grow, so every wavefront ends).
   const int nbt = (a.nbra + kTileB - 1) / kTileB;
-  const bool fixed = a.kchunk == 1;
-  const unsigned gw = blockIdx.x * 4u + (unsigned)wave, nw = gridDim.x * 4u;
-  unsigned slot = gw, round0 = 0;
-  int sg = (int)(gw % (unsigned)a.nstrip), left = a.nstrip;
+  const bool fixed = a.kchunk < kClaimChunk;
+  const unsigned nw = at.blocks * 4u;
+  unsigned slot = at.block * 4u + (unsigned)wave, round0 = 0;
+  int sg = (int)(slot % (unsigned)a.nstrip), left = a.nstrip;
   for (;;) {
     int tb, k0;
     if (fixed) {
-      const unsigned un = round0 + slot;
       if (round0 >= (unsigned)a.ntiles) break;
+      const unsigned un = round0 + slot;
       round0 += nw;
       slot += (unsigned)a.shift;
       if (slot >= nw) slot -= nw;
       if (un >= (unsigned)a.ntiles) continue;
-      if (a.same) {
+      if (a.kchunk > 1) {
+        tb = (int)(un / (unsigned)a.nkc);
+        k0 = (int)(un - (unsigned)tb * (unsigned)a.nkc) * a.kchunk;
+      } else if (a.same) {
         // tile tb owns units [32 tb (tb + 1), 32 (tb + 1)(tb + 2)): kets 0 .. 64 tb + 63
         tb = (int)((sqrt(1.0 + 0.125 * (double)un) - 1.0) * 0.5);
         while (32u * (unsigned)(tb + 1) * (unsigned)(tb + 2) <= un) ++tb;
@@ -245,17 +254,16 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
       if (k0 >= a.nket) continue;  // one class: the last tile is not full
     } else {
       int ul = 0;
-      if (lane == 0) ul = atomicAdd(a.tile_ctr + blockIdx.y * a.nstrip + sg, 1);
+      if (lane == 0) ul = atomicAdd(a.tile_ctr + at.part * a.nstrip + sg, 1);
       ul = __builtin_amdgcn_readfirstlane(__shfl(ul, 0, 64));
-      const int t0 = sg * a.seg_tiles;
-      if (ul >= min(a.seg_tiles, nbt - t0) * a.nkc) {  // this segment is exhausted
+      const int t0 = sg * kSegTiles;
+      if (ul >= min(kSegTiles, nbt - t0) * a.nkc) {  // this segment is exhausted
         if (--left == 0) break;
         sg = sg + 1 == a.nstrip ? 0 : sg + 1;
         continue;
       }
-      const int u = t0 * a.nkc + ul;
-      tb = u / a.nkc;
-      k0 = __builtin_amdgcn_readfirstlane((u - tb * a.nkc) * a.kchunk);
+      tb = t0 + ul / a.nkc;
+      k0 = __builtin_amdgcn_readfirstlane((ul % a.nkc) * a.kchunk);
     }
     const int klast = tb * kTileB + kTileB - 1;  // same class: last ket any lane of the tile takes
     if (a.same && k0 > klast) continue;  // whole wave above the diagonal
@@ -362,7 +370,7 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
       for (int ww = 0; ww < kMaxW; ++ww)
         if (ww == w) s = esum[ww];
       s = wave_sum(s);
-      if (lane == 0) a.partial[(((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 4 + wave) * a.nwfn + w] = s;
+      if (lane == 0) a.partial[(((size_t)at.part * at.blocks + at.block) * 4 + wave) * a.nwfn + w] = s;
     }
   }
   stamp_wave(a.stamp, true);
@@ -383,7 +391,7 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
 constexpr int kStripB = 4 * kTileB;
 
 template <int LA, int LB, int LC, int LD, int AP>
-__device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const double* __restrict__ btab) {
+__device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const Place& at, const double* __restrict__ btab) {
   constexpr int NA = AP < 0 ? ncart(LA) : 1, NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
   constexpr int A0 = AP < 0 ? 0 : AP;  // the part's first A function
   constexpr bool kFirst = A0 == 0;     // the part that counts the quartets
@@ -431,10 +439,10 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
   // more than one, kets that fail the Schwarz test against the strip's largest
   // bra bound are skipped without a visit (one lane tests each), which spares
   // sparse systems a claim and an exchange flush per screened-out ket.
-  int st = (int)(blockIdx.x % (unsigned)a.nstrip), left = a.nstrip;
+  int st = (int)(at.block % (unsigned)a.nstrip), left = a.nstrip;
   for (;;) {
     __syncthreads();  // the previous unit is flushed and s_unit, s_qmax are free
-    if (threadIdx.x == 0) s_unit = atomicAdd(a.tile_ctr + blockIdx.y * a.nstrip + st, a.kchunk);
+    if (threadIdx.x == 0) s_unit = atomicAdd(a.tile_ctr + at.part * a.nstrip + st, a.kchunk);
     __syncthreads();
     const int k0 = __builtin_amdgcn_readfirstlane(s_unit);
     if (k0 >= a.nket) {  // this strip is exhausted
@@ -631,7 +639,7 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const doub
 constexpr int kStripK = 256;
 
 template <int LA, int LB, int LC, int LD, int AP>
-__device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const double* __restrict__ btab) {
+__device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const Place& at, const double* __restrict__ btab) {
   constexpr int NA = AP < 0 ? ncart(LA) : 1, NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
   constexpr int A0 = AP < 0 ? 0 : AP;  // the part's first A function
   constexpr bool kFirst = A0 == 0;     // the part that counts the quartets
@@ -675,10 +683,10 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const dou
   // A claim takes a chunk of kchunk consecutive bra pairs; with more than one,
   // bra pairs that fail the Schwarz test against the strip's largest ket bound
   // are skipped without a visit.
-  int st = (int)(blockIdx.x % (unsigned)a.nstrip), left = a.nstrip;
+  int st = (int)(at.block % (unsigned)a.nstrip), left = a.nstrip;
   for (;;) {
     __syncthreads();  // the previous unit is flushed and s_unit, s_qmax are free
-    if (threadIdx.x == 0) s_unit = atomicAdd(a.tile_ctr + blockIdx.y * a.nstrip + st, a.kchunk);
+    if (threadIdx.x == 0) s_unit = atomicAdd(a.tile_ctr + at.part * a.nstrip + st, a.kchunk);
     __syncthreads();
     const int b0 = __builtin_amdgcn_readfirstlane(s_unit);
     if (b0 >= a.nbra) {  // this ket strip is exhausted
@@ -861,37 +869,37 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const dou
   add_counters(kFirst ? a.counters : nullptr, nq, nprimq, nskip);
 }
 
-// The body of one mode for the part this workgroup was launched for
-// (blockIdx.y): kMode 0 energy, 1 J/K, 2 J/K transposed.
+// The body of one mode for the part of the workgroup's place: kMode 0 energy, 1
+// J/K, 2 J/K transposed.
 template <int LA, int LB, int LC, int LD, int kMode, int kPart = 0>
-__device__ __forceinline__ void quartet_part(const QuartetArgs& a, const double* __restrict__ btab) {
+__device__ __forceinline__ void quartet_part(const QuartetArgs& a, const Place& at, const double* __restrict__ btab) {
   using P = Parts<LA, LB, LC, LD, kMode != 0>;
   if constexpr (kPart + 1 < P::n) {
-    if (blockIdx.y != (unsigned)kPart) {
-      quartet_part<LA, LB, LC, LD, kMode, kPart + 1>(a, btab);
+    if (at.part != (unsigned)kPart) {
+      quartet_part<LA, LB, LC, LD, kMode, kPart + 1>(a, at, btab);
       return;
     }
   }
   if constexpr (kMode == 0)
-    quartet_energy_body<LA, LB, LC, LD, P::a(kPart)>(a, btab);
+    quartet_energy_body<LA, LB, LC, LD, P::a(kPart)>(a, at, btab);
   else if constexpr (kMode == 1)
-    quartet_jk_body<LA, LB, LC, LD, P::a(kPart)>(a, btab);
+    quartet_jk_body<LA, LB, LC, LD, P::a(kPart)>(a, at, btab);
   else
-    quartet_jkt_body<LA, LB, LC, LD, P::a(kPart)>(a, btab);
+    quartet_jkt_body<LA, LB, LC, LD, P::a(kPart)>(a, at, btab);
 }
 
 template <int LA, int LB, int LC, int LD>
 __global__ void __launch_bounds__(256) quartet_jkt_kernel(QuartetArgs a) {
   __shared__ __attribute__((aligned(16))) double btab[kBoysCLen];  // this class's compact Boys table
   stage_boys<LA + LB + LC + LD>(a.boys, btab);
-  quartet_part<LA, LB, LC, LD, 2>(a, btab);
+  quartet_part<LA, LB, LC, LD, 2>(a, Place{blockIdx.x, gridDim.x, blockIdx.y}, btab);
 }
 
 template <int LA, int LB, int LC, int LD, bool kJK>
 __global__ void __launch_bounds__(256) quartet_kernel(QuartetArgs a) {
   __shared__ __attribute__((aligned(16))) double btab[kBoysCLen];  // this class's compact Boys table
   stage_boys<LA + LB + LC + LD>(a.boys, btab);
-  quartet_part<LA, LB, LC, LD, kJK ? 1 : 0>(a, btab);
+  quartet_part<LA, LB, LC, LD, kJK ? 1 : 0>(a, Place{blockIdx.x, gridDim.x, blockIdx.y}, btab);
 }
 
 // One J/K launch of a class over several groups (molecules) of a batch, with
@@ -911,7 +919,7 @@ __global__ void __launch_bounds__(256) quartet_jk_groups_kernel(const QuartetArg
   for (int g = 0; g < ng; ++g) {
     const QuartetArgs a = gs[g];
     if (a.ntiles > 0) {
-      quartet_part<LA, LB, LC, LD, kTr ? 2 : 1>(a, btab);
+      quartet_part<LA, LB, LC, LD, kTr ? 2 : 1>(a, Place{blockIdx.x, gridDim.x, blockIdx.y}, btab);
     }
     __syncthreads();  // the group's LDS blocks are flushed before the next group's zeroing
   }

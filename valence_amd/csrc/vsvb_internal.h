@@ -148,11 +148,18 @@ struct ClassLaunch {
   int claim = 1;      // cooperative kernel: units per claim
   int per_cu = 0;     // workgroups per CU requested (0 = the kernel's occupancy)
   bool tr = false;    // straight-line J/K: transposed units (one bra pair x 256 ket pairs)
-  int strips = 1;     // straight-line: energy segments, J/K bra strips (ket strips transposed), one work counter each
+  int strips = 1;     // straight-line J/K: bra strips (ket strips transposed), one work counter each
   int kchunk = 1;     // straight-line: pairs of the uniform side (ket; bra when transposed) per claim
-  int seg_tiles = 1;  // straight-line energy: bra tiles per counter segment
-  int shift = 0;      // straight-line energy, one-ket units: QuartetArgs::shift
+  int shift = 0;      // straight-line energy: QuartetArgs::shift
   bool overflow = false;  // the class has more work units than 32-bit indices allow in this shape
+};
+
+// One launch over several classes (vsvb_eri_small.hip): class q[k] has the
+// workgroups [block0[k], block0[k] + blocks[k] * its parts).
+struct SmallLaunch {
+  int n = 0, total = 0;
+  int q[kNQuartetClass] = {}, block0[kNQuartetClass] = {}, blocks[kNQuartetClass] = {};
+  unsigned lds = 0;  // J/K: dynamic LDS, the largest of the classes' exchange staging
 };
 
 }  // namespace vsvb
@@ -255,6 +262,8 @@ int run_quartets(vsvb_context* c, bool jk, double* e2_dev, int nwfn = 1, const d
                  double* jacc = nullptr, double* kacc = nullptr, int nspin_override = -1);
 int finish_counters(vsvb_context* c, const unsigned long long* host_counters = nullptr);
 int check_status(vsvb_context* c, bool for_grad);
+
+hipError_t launch_small(const SmallLaunch& s, const QuartetArgs* gs, bool jk, hipStream_t st);
 
 // cooperative kernel for the register-heavy classes (vsvb_eri_coop.hip)
 int coop_class(int la, int lb, int lc, int ld);  // index of the class, or -1
