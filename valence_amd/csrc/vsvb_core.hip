@@ -1184,6 +1184,9 @@ static ClassLaunch policy_launch(vsvb_context* c, int q, const Policy& p) {
 // dp, dd): a quarter and a twelfth of the pairs of six-fold, three-fold and
 // uncontracted shells.
 constexpr int kSegLen[kLevels][kNPairClass] = {{0, 0, 0, 0, 0, 0}, {9, 6, 3, 3, 1, 1}, {3, 2, 1, 1, 1, 1}};
+// Workgroups up to which a class joins the shared launch of a small system: it
+// runs one workgroup per CU, so a class that fills the chip is faster alone.
+constexpr int kSmallBlocks = 320;
 // Shell pairs up to which a context holds segment lists: above, every class
 // that matters fills the chip with whole pairs.
 constexpr int kSplitMaxPairs = 20000;
@@ -1225,6 +1228,10 @@ static int plan_work(vsvb_context* c, const int* kept) {
     }
   }
   c->partial_total = 0;
+  for (int m = 0; m < 2; ++m) {
+    c->small[m] = SmallLaunch{};
+    std::fill(c->in_small[m], c->in_small[m] + kNQuartetClass, false);
+  }
   for (int q = 0; q < kNQuartetClass; ++q) {
     const int bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
     const bool coop = coop_default(c->coop_idx[q]);
@@ -1239,9 +1246,36 @@ static int plan_work(vsvb_context* c, const int* kept) {
       const ClassLaunch cl = policy_launch(c, q, c->pol[q]);
       if (!cl.overflow && (cl.units > 0 || c->ljk[q].units <= 0)) c->ljk[q] = cl;
     }
+    if (c->d_small.p && c->ndens == 1 && c->coop_idx[q] < 0) {
+      c->in_small[0][q] = c->le[q].units > 0 && c->le[q].kchunk == 1 && c->le[q].blocks * kPartsEnergy[q] <= kSmallBlocks;
+      // the shared J/K launch has the transposed units of classes of different bra and ket
+      const ClassLaunch cl = straight_launch(c, bc, kc, true, kDefaultJkPerCu, true, bc != kc);
+      if (cl.units > 0 && !cl.overflow && cl.kchunk == 1 && cl.blocks * kPartsJk[q] <= kSmallBlocks) {
+        c->in_small[1][q] = true;
+        c->ljk[q] = cl;
+      }
+    }
     // energy kernels write four slots per block and part
     c->partial_per_class[q] = (size_t)c->le[q].blocks * 4 * (c->le[q].coop ? 1 : class_parts(q, false));
     c->partial_total += c->partial_per_class[q];
+  }
+  // the shared launches: high angular momenta (the longest chains) first
+  for (int m = 0; m < 2; ++m) {
+    SmallLaunch& s = c->small[m];
+    for (int q = kNQuartetClass - 1; q >= 0; --q) {
+      if (!c->in_small[m][q]) continue;
+      const ClassLaunch& cl = m ? c->ljk[q] : c->le[q];
+      s.q[s.n] = q;
+      s.block0[s.n] = s.total;
+      s.blocks[s.n] = cl.blocks;
+      s.total += cl.blocks * class_parts(q, m != 0);
+      s.lds = std::max(s.lds, (unsigned)cl.lds);
+      ++s.n;
+    }
+    if (s.n < 2) {  // nothing to share
+      std::fill(c->in_small[m], c->in_small[m] + kNQuartetClass, false);
+      s = SmallLaunch{};
+    }
   }
   return VSVB_OK;
 }
@@ -1503,10 +1537,11 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   HIP_OK(device_buffer(c, c->d_partial, std::max<size_t>(partial_cap, 1) * 2));
   // segment lists last: in the allocation-free entry they are left out where
   // the static array has no room for them
-  const size_t seg_bytes = seg_cap * (sizeof(Pair) + sizeof(SegSrc)) + 1024;
+  const size_t seg_bytes = seg_cap * (sizeof(Pair) + sizeof(SegSrc)) + 2 * kNQuartetClass * sizeof(QuartetArgs) + 1024;
   if (split && (!c->arena || c->arena->used + seg_bytes <= c->arena->cap)) {
     HIP_OK(device_buffer(c, c->d_split, seg_cap));
     HIP_OK(device_buffer(c, c->d_segsrc, seg_cap));
+    HIP_OK(device_buffer(c, c->d_small, 2 * kNQuartetClass));
     c->nlevels = kLevels;
   }
   {
@@ -1773,8 +1808,34 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, double* e2_dev, int nwfn, const
     offs[q] = poff;
     poff += c->partial_per_class[q];
   }
+  // Small classes share one launch: their argument records go to the device when
+  // they differ from the last ones (under capture nothing is uploaded; records
+  // that differ then take separate launches).
+  const int m = jk ? 1 : 0;
+  bool shared = c->small[m].n > 0 && nwfn == 1;
+  if (shared) {
+    const SmallLaunch& s = c->small[m];
+    std::vector<QuartetArgs> rec(s.n);
+    for (int k = 0; k < s.n; ++k) {
+      const int q = s.q[k], bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
+      rec[k] = class_args(c, bc, kc, jk ? c->ljk[q] : c->le[q], jk, nwfn, nspin, dens, jacc, kacc,
+                          c->d_partial.p + offs[q]);
+    }
+    std::vector<QuartetArgs>& old = c->h_small[m];
+    QuartetArgs* dev = c->d_small.p + (size_t)m * kNQuartetClass;
+    if (old.size() != rec.size() || std::memcmp(old.data(), rec.data(), rec.size() * sizeof(QuartetArgs)) != 0) {
+      if (c->capturing) {
+        shared = false;
+      } else {
+        old.swap(rec);
+        HIP_OK(hipMemcpyAsync(dev, old.data(), old.size() * sizeof(QuartetArgs), hipMemcpyHostToDevice, st));
+      }
+    }
+    if (shared) HIP_OK(launch_small(s, dev, jk, st));
+  }
   for (int t = 0; t < kNQuartetClass; ++t) {
     const int q = c->class_rev ? kNQuartetClass - 1 - t : t;
+    if (shared && c->in_small[m][q]) continue;
     const int bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
     const ClassLaunch& cl = jk ? c->ljk[q] : c->le[q];
     const int nb = c->work[bc][0].n, nk = c->work[kc][0].n;
@@ -2418,7 +2479,7 @@ static int tune_leader(vsvb_batch* b, BatchGroup* gs, double (*tuning)[kTuneCols
   for (int bc = 0; bc < kNPairClass; ++bc)
     for (int kc = 0; kc <= bc; ++kc) {
       const int q = quartet_class_index(bc, kc);
-      if (L->ljk[q].units <= 0) continue;
+      if (L->ljk[q].units <= 0 || L->in_small[1][q]) continue;  // (small classes share one launch)
       std::vector<Policy> cand;
       Policy d0;  // the default
       d0.coop = L->ljk[q].coop;
@@ -2551,6 +2612,7 @@ static int tune_batch(vsvb_batch* b) {
         // own default launch, which its context was created with
         c->pol[q] = best[k][q];
         c->has_pol[q] = true;
+        if (c->in_small[1][q]) continue;  // runs in the shared launch
         const ClassLaunch cl = policy_launch(c, q, best[k][q]);
         if (!cl.overflow && (cl.units > 0 || c->ljk[q].units <= 0)) c->ljk[q] = cl;
       }

@@ -229,6 +229,11 @@ struct vsvb_context {
   size_t partial_per_class[vsvb::kNQuartetClass] = {0};
   // launch configuration per quartet class: energy mode and J/K mode
   vsvb::ClassLaunch le[vsvb::kNQuartetClass], ljk[vsvb::kNQuartetClass];
+  // classes that share one launch, in energy and in J/K mode, and their argument records
+  vsvb::SmallLaunch small[2];
+  bool in_small[2][vsvb::kNQuartetClass] = {};
+  std::vector<vsvb::QuartetArgs> h_small[2];
+  DevBuf<vsvb::QuartetArgs> d_small;
   int coop_idx[vsvb::kNQuartetClass] = {0};  // cooperative step tables of the class, or -1
   int ncu = 0;
   size_t partial_total = 0;
