@@ -1288,6 +1288,58 @@ static hipError_t device_buffer(vsvb_context* c, vsvb::DevBuf<T>& b, size_t coun
   return c->arena ? b.carve(*c->arena, count) : b.alloc(count);
 }
 
+// The orbital algebra of this wave function runs in one workgroup
+// (vsvb_orbital.hip): few enough orbitals for its LDS and no more than AOs (its
+// m x m results stand in nsp x nbf arrays), no NDFs, no spin-coupled pairs, and no
+// spin block that is to be inverted grid-wide.
+static bool one_block_orbitals(const vsvb_context* c) {
+  return c->ndf == 0 && c->npair == 0 && c->nsp <= std::min(kOrbMax, c->nbf) && c->nbf <= kOrbMaxBasis &&
+         std::max(c->nalpha_rows, c->ndocc) < c->grid_inverse_min;
+}
+
+static OrbArgs orb_args(const vsvb_context* c) {
+  OrbArgs a{};
+  a.ent = c->d_ent.p;
+  a.orb_start = c->d_orb_start.p;
+  a.ao_ptr = c->d_ao_ptr.p;
+  a.ao_orb = c->d_ao_orb.p;
+  a.shells = c->d_shells.p;
+  a.coeff = c->d_coeff.p;
+  a.angn = c->d_angn.p;
+  a.S = c->d_S.p;
+  a.H = c->d_H.p;
+  a.J = c->d_J.p;
+  a.K = c->d_K.p;
+  a.Ct = c->d_Ct.p;
+  a.Cs = c->d_Cs.p;
+  a.T = c->d_tmp.p;
+  a.TH = c->d_tmp2.p;
+  a.Y[0] = c->d_X.p;
+  a.Y[1] = c->d_Z.p;
+  a.V[0] = c->d_tmp2.p;  // C h is done with by then
+  a.V[1] = c->d_Rfull.p;
+  a.Sorb = c->d_Sorb.p;
+  a.Horb = c->d_Horb.p;
+  a.P = c->d_P.p;
+  a.R = c->d_R.p;
+  a.F = c->d_F.p;
+  a.G = c->d_gradC.p;
+  a.grad = c->d_grad.p;
+  a.partial = c->d_partial.p;
+  a.scal = c->d_scal.p;
+  a.status = c->d_status.p;
+  a.nbf = c->nbf;
+  a.nsp = c->nsp;
+  a.nsh = c->nsh;
+  a.totlen = c->totlen;
+  a.nspin = c->nunpd > 0 ? 2 : 1;
+  a.nalpha = c->nalpha_rows;
+  a.nunpd = c->nunpd;
+  a.ndocc = c->ndocc;
+  a.dtol = c->dtol;
+  return a;
+}
+
 static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_context* c) {
   if (!s) return fail(VSVB_ERR_ARG, "null system");
   if (s->natom < 1 || s->nshell_type < 1) return fail(VSVB_ERR_ARG, "empty molecule or basis");
@@ -1440,6 +1492,20 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
       c->ent[k] = e;
     }
   }
+  // the orbitals that hold each AO (each once), for the one-workgroup orbital algebra
+  c->ao_ptr.assign(c->nbf + 1, 0);
+  if (c->ndf == 0) {
+    std::vector<std::vector<int>> of(c->nbf);
+    for (int p = 0; p < c->nsp; ++p)
+      for (int k = s->orb_start[p]; k < s->orb_start[p + 1]; ++k) {
+        auto& v = of[c->ent[k].tgt];
+        if (v.empty() || v.back() != p) v.push_back(p);
+      }
+    for (int m = 0; m < c->nbf; ++m) {
+      c->ao_ptr[m + 1] = c->ao_ptr[m] + (int)of[m].size();
+      c->ao_orb.insert(c->ao_orb.end(), of[m].begin(), of[m].end());
+    }
+  }
   // host copies of inputs
   c->coords.assign(s->coords, s->coords + 3 * s->natom);
   c->charges.resize(s->natom);
@@ -1534,7 +1600,8 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
       const size_t blocks = std::min<size_t>(2048, (size_t)class_occupancy(bc, kc, false, false, 0) * ncu);
       partial_cap += 4 * blocks * class_parts(q, false);
     }
-  HIP_OK(device_buffer(c, c->d_partial, std::max<size_t>(partial_cap, 1) * 2));
+  // (also the Fock tiles' shares of E2: at most 20 x 20 per spin)
+  HIP_OK(device_buffer(c, c->d_partial, std::max<size_t>(partial_cap, 512) * 2));
   // segment lists last: in the allocation-free entry they are left out where
   // the static array has no room for them
   const size_t seg_bytes = seg_cap * (sizeof(Pair) + sizeof(SegSrc)) + 2 * kNQuartetClass * sizeof(QuartetArgs) + 1024;
@@ -1543,6 +1610,14 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
     HIP_OK(device_buffer(c, c->d_segsrc, seg_cap));
     HIP_OK(device_buffer(c, c->d_small, 2 * kNQuartetClass));
     c->nlevels = kLevels;
+  }
+  const size_t list_bytes = (c->ao_ptr.size() + c->ao_orb.size()) * sizeof(int) + 1024;
+  if (one_block_orbitals(c) && (!c->arena || c->arena->used + list_bytes <= c->arena->cap)) {
+    HIP_OK(device_buffer(c, c->d_ao_ptr, c->ao_ptr.size()));
+    HIP_OK(device_buffer(c, c->d_ao_orb, c->ao_orb.size()));
+    HIP_OK(hipMemcpy(c->d_ao_ptr.p, c->ao_ptr.data(), c->ao_ptr.size() * sizeof(int), hipMemcpyHostToDevice));
+    if (!c->ao_orb.empty())
+      HIP_OK(hipMemcpy(c->d_ao_orb.p, c->ao_orb.data(), c->ao_orb.size() * sizeof(int), hipMemcpyHostToDevice));
   }
   {
     const int rc = plan_work(c, nullptr);
@@ -1657,17 +1732,24 @@ int vsvb::prepare_geometry(vsvb_context* c, const double* coords) {
   return VSVB_OK;
 }
 
+// New weights (from the host or the device) into d_coeff.
+static int upload_coeff(vsvb_context* c, const double* coeff_host, const double* coeff_dev) {
+  if (coeff_host) {
+    c->coeff.assign(coeff_host, coeff_host + c->totlen);
+    HIP_OK(hipMemcpyAsync(c->d_coeff.p, c->coeff.data(), c->totlen * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  } else if (coeff_dev) {
+    HIP_OK(hipMemcpyAsync(c->d_coeff.p, coeff_dev, c->totlen * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+  }
+  return VSVB_OK;
+}
+
 // weights -> Ct, Cs, orbital S and h, P per spin block, R per spin block, E1.
 // Spin blocks (npair = 0): alpha = all spatial orbitals (unpaired then docc),
 // beta = the trailing ndocc (docc); closed shell when nunpd = 0.
 int vsvb::prepare_orbital_basis(vsvb_context* c, const double* coeff_host, const double* coeff_dev) {
   hipStream_t st = c->stream;
-  if (coeff_host) {
-    c->coeff.assign(coeff_host, coeff_host + c->totlen);
-    HIP_OK(hipMemcpyAsync(c->d_coeff.p, c->coeff.data(), c->totlen * sizeof(double), hipMemcpyHostToDevice, st));
-  } else if (coeff_dev) {
-    HIP_OK(hipMemcpyAsync(c->d_coeff.p, coeff_dev, c->totlen * sizeof(double), hipMemcpyDeviceToDevice, st));
-  }
+  const int rc = upload_coeff(c, coeff_host, coeff_dev);
+  if (rc) return rc;
   const int n = c->nbf, ns = c->nsp;
   hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, c->d_scal.p, (size_t)16, 0.0);
   HIP_OK(launch_zero(st, c->d_status.p, 4 * sizeof(int)));
@@ -1694,8 +1776,36 @@ int vsvb::prepare_orbital_basis(vsvb_context* c, const double* coeff_host, const
   return VSVB_OK;
 }
 
-static int prepare_orbitals(vsvb_context* c, const double* coeff_host, const double* coeff_dev) {
+// What the quartet pass (1: energy, 2: J/K into jacc, kacc) needs cleared.
+static ZeroArgs pass_zero(vsvb_context* c, int pass, int nwfn, double* jacc, double* kacc) {
+  ZeroArgs z;
+  if (pass <= 0) return z;
+  const size_t nn = (size_t)c->nbf * c->nbf, words = sizeof(double) / sizeof(uint32_t);
+  z.p[0] = reinterpret_cast<uint32_t*>(c->d_counters.p);
+  z.n[0] = kCtrSlots * kCtrStride * sizeof(unsigned long long) / sizeof(uint32_t);
+  z.p[1] = reinterpret_cast<uint32_t*>(c->d_tilectr.p);
+  z.n[1] = c->ctr_total;
+  if (pass == 2) {
+    z.p[2] = reinterpret_cast<uint32_t*>(jacc);
+    z.n[2] = nwfn * nn * words;
+    z.p[3] = reinterpret_cast<uint32_t*>(kacc);
+    z.n[3] = nwfn * (c->nunpd > 0 ? 2 : 1) * nn * words;
+  }
+  return z;
+}
+
+// Orbital stage of one wave function; pass: the quartet pass that follows (1
+// energy, 2 J/K of this wave function alone, 0 neither), cleared along where the
+// algebra runs in one workgroup.
+static int prepare_orbitals(vsvb_context* c, const double* coeff_host, const double* coeff_dev, int pass) {
   int rc;
+  c->cleared = 0;
+  if (c->d_ao_ptr.p) {
+    if ((rc = upload_coeff(c, coeff_host, coeff_dev))) return rc;
+    HIP_OK(launch_orbital_front(c->stream, orb_args(c), nullptr, 1, pass_zero(c, pass, 1, c->d_J.p, c->d_K.p)));
+    c->cleared = pass;
+    return VSVB_OK;
+  }
   if ((rc = prepare_orbital_basis(c, coeff_host, coeff_dev))) return rc;
   hipStream_t st = c->stream;
   const int n = c->nbf, ns = c->nsp;
@@ -1770,14 +1880,17 @@ static hipError_t quartet_pass_clear(vsvb_context* c, bool jk, int nwfn, int nsp
                                      int words) {
   hipStream_t st = c->stream;
   const size_t nn = (size_t)c->nbf * c->nbf;
-  hipError_t e;
-  if ((e = launch_zero(st, c->d_counters.p, words * sizeof(unsigned long long))) != hipSuccess) return e;
-  if ((e = launch_zero(st, c->d_tilectr.p, c->ctr_total * sizeof(int))) != hipSuccess) return e;
+  hipError_t e = hipSuccess;
+  const int cleared = c->cleared;
+  c->cleared = 0;
   c->last_jk = jk;
   c->last_nwfn = nwfn;
   c->last_nspin = nspin;
   c->ran_quartets = true;
   c->ev_valid = false;
+  if (cleared == (jk ? 2 : 1) && words == kCtrSlots * kCtrStride) return e;
+  if ((e = launch_zero(st, c->d_counters.p, words * sizeof(unsigned long long))) != hipSuccess) return e;
+  if ((e = launch_zero(st, c->d_tilectr.p, c->ctr_total * sizeof(int))) != hipSuccess) return e;
   if (jk) {
     hipLaunchKernelGGL(k_fill, dim3(1024), dim3(256), 0, st, jacc, nwfn * nn, 0.0);
     hipLaunchKernelGGL(k_fill, dim3(1024), dim3(256), 0, st, kacc, nwfn * nspin * nn, 0.0);
@@ -1787,7 +1900,7 @@ static hipError_t quartet_pass_clear(vsvb_context* c, bool jk, int nwfn, int nsp
 
 // nspin_override = 0 turns the J/K launch into a Coulomb-only pass over nwfn
 // general symmetric densities (the exchange accumulators are not touched).
-int vsvb::run_quartets(vsvb_context* c, bool jk, double* e2_dev, int nwfn, const double* dens, double* jacc,
+int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, double* jacc,
                        double* kacc, int nspin_override) {
   hipStream_t st = c->stream;
   const int nspin = nspin_override >= 0 ? nspin_override : (c->nunpd > 0 ? 2 : 1);
@@ -1853,10 +1966,7 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, double* e2_dev, int nwfn, const
   if (c->profile)
     hipLaunchKernelGGL(k_stamp_reduce, dim3(kNQuartetClass), dim3(kStampSlots), 0, st, c->d_stamps.p,
                        c->d_counters.p + kCtrSlots * kCtrStride);
-  if (!jk) {
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, st, c->d_partial.p, (long)poff, 1, e2_dev);
-    HIP_OK(hipGetLastError());
-  }
+  if (!jk) HIP_OK(launch_energy_sum(st, c->d_partial.p, (long)poff, c->enuc, c->d_scal.p));
   return VSVB_OK;
 }
 
@@ -1933,12 +2043,8 @@ int vsvb::check_status(vsvb_context* c, bool for_grad) {
 static int enqueue_energy(vsvb_context* c, const double* coords, const double* coeff) {
   int rc;
   if ((rc = prepare_geometry(c, coords))) return rc;
-  if ((rc = prepare_orbitals(c, coeff, nullptr))) return rc;
-  if ((rc = run_quartets(c, false, c->d_scal.p + 1))) return rc;
-  hipLaunchKernelGGL(k_final_energy, dim3(1), dim3(1), 0, c->stream, c->d_scal.p, c->d_scal.p + 1, c->enuc,
-                     c->d_scal.p + 2);
-  HIP_OK(hipGetLastError());
-  return VSVB_OK;
+  if ((rc = prepare_orbitals(c, coeff, nullptr, 1))) return rc;
+  return run_quartets(c, false);
 }
 
 static int finish_energy(vsvb_context* c, double* energy, double* parts) {
@@ -1977,6 +2083,10 @@ static int energy_impl(vsvb_context* c, const double* coords, const double* coef
 //   F_s = w1 h + F2_s,  dE/dC_s = 2 P_s C_s F_s (1 - R_s S_ao)   (row-major C_s = orbital rows)
 static int gradient_impl(vsvb_context* c, double* grad_dev) {
   hipStream_t st = c->stream;
+  if (c->d_ao_ptr.p) {
+    HIP_OK(launch_orbital_back(st, orb_args(c), nullptr, 1, grad_dev));
+    return VSVB_OK;
+  }
   const int n = c->nbf, ns = c->nsp;
   const size_t nn = (size_t)n * n;
   const int nspin = c->nunpd > 0 ? 2 : 1;
@@ -2013,8 +2123,8 @@ static int enqueue_energy_grad(vsvb_context* c, const double* coords, const doub
                                const double* coeff_dev, double* grad_dev) {
   int rc;
   if ((rc = prepare_geometry(c, coords))) return rc;
-  if ((rc = prepare_orbitals(c, coeff_host, coeff_dev))) return rc;
-  if ((rc = run_quartets(c, true, nullptr))) return rc;
+  if ((rc = prepare_orbitals(c, coeff_host, coeff_dev, 2))) return rc;
+  if ((rc = run_quartets(c, true))) return rc;
   return gradient_impl(c, grad_dev);
 }
 
@@ -2042,6 +2152,8 @@ static int finish_energy_grad(vsvb_context* c, double* energy, double* grad) {
 struct BatchGroup {
   std::vector<int> members;  // indices into vsvb_batch::ctx; members[0] leads
   DevBuf<double> dens, jacc, kacc;
+  DevBuf<OrbArgs> orec;           // the members' orbital records, when they run in one workgroup each
+  std::vector<OrbArgs> h_orec;
 };
 
 // The first run of a batch is enqueued directly and then captured whole
@@ -2306,6 +2418,43 @@ static int batch_plan(vsvb_batch* b) {
   return VSVB_OK;
 }
 
+// Every member's orbital algebra runs in one workgroup: one launch takes them all.
+static bool group_one_launch(const vsvb_batch* b, const BatchGroup& g) {
+  if (g.members.size() < 2) return false;
+  const vsvb_context* lead = b->ctx[g.members[0]];
+  for (int i : g.members) {
+    const vsvb_context* c = b->ctx[i];
+    if (!c->d_ao_ptr.p || c->nbf != lead->nbf || c->nalpha_rows != lead->nalpha_rows || c->ndocc != lead->ndocc ||
+        c->nunpd != lead->nunpd)
+      return false;
+  }
+  return true;
+}
+
+// The members' orbital stage; pass 2: the group's J/K pass follows, and its
+// counters and accumulators are cleared along.
+static int group_orbitals(vsvb_batch* b, BatchGroup& g, int pass) {
+  vsvb_context* lead = b->ctx[g.members[0]];
+  int rc;
+  const int nwfn = (int)g.members.size();
+  if (!group_one_launch(b, g)) {
+    for (int i : g.members)
+      if ((rc = prepare_orbitals(b->ctx[i], nullptr, nullptr, nwfn == 1 ? pass : 0))) return rc;
+    return VSVB_OK;
+  }
+  if (g.h_orec.empty()) {  // constant over the batch's life; written on a direct run, before any capture
+    if (lead->capturing) return fail(VSVB_ERR_DEVICE, "orbital records of a batch group are not on the device");
+    for (int i : g.members) g.h_orec.push_back(orb_args(b->ctx[i]));
+    HIP_OK(g.orec.alloc(g.h_orec.size()));
+    HIP_OK(hipMemcpyAsync(g.orec.p, g.h_orec.data(), g.h_orec.size() * sizeof(OrbArgs), hipMemcpyHostToDevice,
+                          lead->stream));
+  }
+  HIP_OK(launch_orbital_front(lead->stream, g.h_orec[0], g.orec.p, nwfn,
+                              pass_zero(lead, pass, nwfn, g.jacc.p, g.kacc.p)));
+  lead->cleared = pass;
+  return VSVB_OK;
+}
+
 // Geometry and orbital work of one group, and, for a spin-coupled group, its
 // whole pass; with own = true also its own quartet pass and its gradients.
 static int group_front(vsvb_batch* b, BatchGroup& g, bool own) {
@@ -2320,9 +2469,8 @@ static int group_front(vsvb_batch* b, BatchGroup& g, bool own) {
     if ((rc = prepare_orbital_basis(lead, nullptr, nullptr))) return rc;
     return sc_enqueue(lead, true, lead->d_grad.p);
   }
-  for (int i : g.members)
-    if ((rc = prepare_orbitals(b->ctx[i], nullptr, nullptr))) return rc;
   const int nwfn = (int)g.members.size();
+  if ((rc = group_orbitals(b, g, own ? 2 : 0))) return rc;
   if (!own) {
     const int nspin = lead->nunpd > 0 ? 2 : 1;
     HIP_OK(quartet_pass_clear(lead, true, nwfn, nspin, nwfn > 1 ? g.jacc.p : lead->d_J.p,
@@ -2330,8 +2478,8 @@ static int group_front(vsvb_batch* b, BatchGroup& g, bool own) {
     return VSVB_OK;
   }
   if (nwfn > 1) {
-    if ((rc = run_quartets(lead, true, nullptr, nwfn, g.dens.p, g.jacc.p, g.kacc.p))) return rc;
-  } else if ((rc = run_quartets(lead, true, nullptr))) {
+    if ((rc = run_quartets(lead, true, nwfn, g.dens.p, g.jacc.p, g.kacc.p))) return rc;
+  } else if ((rc = run_quartets(lead, true))) {
     return rc;
   }
   return VSVB_OK;
@@ -2340,6 +2488,11 @@ static int group_front(vsvb_batch* b, BatchGroup& g, bool own) {
 static int group_gradients(vsvb_batch* b, BatchGroup& g) {
   vsvb_context* lead = b->ctx[g.members[0]];
   if (lead->npair > 0) return VSVB_OK;
+  if (group_one_launch(b, g)) {
+    for (int i : g.members) b->ctx[i]->enuc = lead->enuc;
+    HIP_OK(launch_orbital_back(lead->stream, g.h_orec[0], g.orec.p, (int)g.members.size(), nullptr));
+    return VSVB_OK;
+  }
   for (int i : g.members) {
     vsvb_context* m = b->ctx[i];
     m->enuc = lead->enuc;
@@ -2458,8 +2611,7 @@ static int tune_leader(vsvb_batch* b, BatchGroup* gs, double (*tuning)[kTuneCols
   vsvb_context* L = b->ctx[gs->members[0]];
   int rc;
   if ((rc = prepare_geometry(L, L->coords.data()))) return rc;
-  for (int i : gs->members)
-    if ((rc = prepare_orbitals(b->ctx[i], nullptr, nullptr))) return rc;
+  if ((rc = group_orbitals(b, *gs, 0))) return rc;
   const int nwfn = (int)gs->members.size();
   const double* dens = nwfn > 1 ? gs->dens.p : L->d_R.p;
   double* jacc = nwfn > 1 ? gs->jacc.p : L->d_J.p;
@@ -3009,8 +3161,8 @@ int vsvb_energy_grad_device(vsvb_context* c, const double* coeff_device, double*
     if ((rc = sc_enqueue(c, true, grad_device))) return rc;
     HIP_OK(hipMemcpyAsync(energy_device, c->d_scal.p + 2, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
   } else {
-    if ((rc = prepare_orbitals(c, nullptr, coeff_device))) return rc;
-    if ((rc = run_quartets(c, true, nullptr))) return rc;
+    if ((rc = prepare_orbitals(c, nullptr, coeff_device, 2))) return rc;
+    if ((rc = run_quartets(c, true))) return rc;
     if ((rc = gradient_impl(c, grad_device))) return rc;
     hipLaunchKernelGGL(k_final_energy, dim3(1), dim3(1), 0, c->stream, c->d_scal.p, c->d_scal.p + 3, c->enuc,
                        energy_device);

@@ -162,6 +162,27 @@ struct SmallLaunch {
   unsigned lds = 0;  // J/K: dynamic LDS, the largest of the classes' exchange staging
 };
 
+// Orbital algebra of one wave function (vsvb_orbital.hip): orbitals up to which
+// it runs in one workgroup, its buffers, and what a quartet pass needs cleared.
+constexpr int kOrbMax = 64;
+constexpr int kOrbMaxBasis = 640;
+struct OrbArgs {
+  const OrbEntry* ent;
+  const int* orb_start;
+  const int *ao_ptr, *ao_orb;  // the orbitals with an entry for each AO
+  const Shell* shells;
+  const double *coeff, *angn, *S, *H, *J, *K;
+  double *Y[2], *V[2];  // per spin: C F, and the m x m matrix of the gradient
+  double *Ct, *Cs, *T, *TH, *Sorb, *Horb, *P, *R, *F, *G, *grad, *partial, *scal;
+  int* status;
+  int nbf, nsp, nsh, totlen, nspin, nalpha, nunpd, ndocc;
+  double dtol;
+};
+struct ZeroArgs {
+  uint32_t* p[4] = {};
+  size_t n[4] = {};  // words
+};
+
 }  // namespace vsvb
 
 struct vsvb_context {
@@ -215,7 +236,7 @@ struct vsvb_context {
   DevBuf<PrimPair> d_pp;
   DevBuf<double> d_pexp, d_pcoef, d_xyz, d_charge, d_boys, d_angn;
   DevBuf<unsigned long long> d_stamps;  // per-class wall-clock slots of the last stage (profiling)
-  DevBuf<int> d_ao_shell, d_orb_start, d_status;
+  DevBuf<int> d_ao_shell, d_orb_start, d_status, d_ao_ptr, d_ao_orb;
   DevBuf<double> d_colk;  // pivot column of the large-matrix inverse
   DevBuf<OrbEntry> d_ent;
   DevBuf<double> d_ndf_d, d_ndf_g;  // NDF gradient scratch: [ndf][nbf] each
@@ -238,6 +259,8 @@ struct vsvb_context {
   int ncu = 0;
   size_t partial_total = 0;
   bool geom_ready = false;
+  int cleared = 0;  // the next quartet pass's counters (1) and accumulators too (2) are already cleared
+  std::vector<int> ao_ptr, ao_orb;
   double enuc = 0.0;
   double last_counters[4] = {0, 0, 0, 0};
   // per-class profiling (events around each class launch when enabled)
@@ -263,11 +286,14 @@ hipError_t launch_reduce(hipStream_t st, const double* partial, long n, int nw, 
 hipError_t launch_gather_grad(vsvb_context* c, const double* gradC, double* grad);
 int prepare_geometry(vsvb_context* c, const double* coords);
 int prepare_orbital_basis(vsvb_context* c, const double* coeff_host, const double* coeff_dev);
-int run_quartets(vsvb_context* c, bool jk, double* e2_dev, int nwfn = 1, const double* dens = nullptr,
+int run_quartets(vsvb_context* c, bool jk, int nwfn = 1, const double* dens = nullptr,
                  double* jacc = nullptr, double* kacc = nullptr, int nspin_override = -1);
 int finish_counters(vsvb_context* c, const unsigned long long* host_counters = nullptr);
 int check_status(vsvb_context* c, bool for_grad);
 
+hipError_t launch_orbital_front(hipStream_t st, const OrbArgs& one, const OrbArgs* recs, int nrec, const ZeroArgs& z);
+hipError_t launch_orbital_back(hipStream_t st, const OrbArgs& one, const OrbArgs* recs, int nrec, double* grad);
+hipError_t launch_energy_sum(hipStream_t st, const double* partial, long n, double enuc, double* scal);
 hipError_t launch_small(const SmallLaunch& s, const QuartetArgs* gs, bool jk, hipStream_t st);
 
 // cooperative kernel for the register-heavy classes (vsvb_eri_coop.hip)

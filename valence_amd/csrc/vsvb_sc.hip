@@ -670,7 +670,7 @@ int vsvb::sc_enqueue(vsvb_context* c, bool want_grad, double* grad_dev) {
   hipLaunchKernelGGL(k_pair_dens, dim3(grid_for(sc.npq * nn)), dim3(256), 0, st, c->d_Cs.p, sc.d_pq.p, sc.npq, nbf,
                      sc.d_pdens.p);
   HIP_OK(hipGetLastError());
-  if ((rc = run_quartets(c, true, nullptr, sc.npq, sc.d_pdens.p, sc.d_pj.p, c->d_K.p, 0))) return rc;
+  if ((rc = run_quartets(c, true, sc.npq, sc.d_pdens.p, sc.d_pj.p, c->d_K.p, 0))) return rc;
   hipLaunchKernelGGL(k_sym_batch, dim3(grid_for(sc.npq * nn)), dim3(256), 0, st, sc.d_pj.p, sc.npq, nbf);
   HIP_OK(hipGetLastError());
   // W^rs = J^rs C^T  ([npq nbf] x nbf times nbf x ns), then (pq|rs) and its exchange ordering
