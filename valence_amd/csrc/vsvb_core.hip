@@ -476,48 +476,125 @@ __global__ void k_shell_screen(const double* __restrict__ Ct, const double* __re
 // ---------------------------------------------------------------------------
 // device: small dense algebra (row-major)
 // ---------------------------------------------------------------------------
-// C[M x N] = alpha * op(A) * op(B) + beta * C;  op(A) is M x K; FP64 matrix cores.
-// One wavefront per 16 x 16 tile of C (the products here are small: many
-// tiles keep the CUs busy), V_MFMA_F64_16X16X4F64 over K in steps of 4; A and
-// B pass through LDS in steps of 16 along K (zero-filled past the edges,
-// transposes applied there).  Lane layout of the instruction (probed on the
-// hardware): A[i][k] is held by lane i + 16k, B[k][j] by lane j + 16k, and
-// D[i][j] by lane j + 16 (i mod 4) in its accumulator register i / 4.
+// C[M x N] = alpha * op(A) * op(B) + beta * C;  op(A) is M x K; FP64 matrix cores
+// (V_MFMA_F64_16X16X4F64, a SIMD is busy with one for 64 cycles).  Lane layout of
+// the instruction (probed on the hardware): A[i][k] is held by lane i + 16k,
+// B[k][j] by lane j + 16k, and D[i][j] by lane j + 16 (i mod 4) in its accumulator
+// register i / 4.
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-__global__ void __launch_bounds__(64) k_gemm(int M, int N, int K, double alpha, const double* __restrict__ A, int lda,
-                                             int ta, const double* __restrict__ B, int ldb, int tb, double beta,
-                                             double* __restrict__ C, int ldc) {
-  __shared__ double As[16][17], Bs[16][17];
-  const int lane = threadIdx.x;
-  const int m0 = blockIdx.y * 16, n0 = blockIdx.x * 16;
+__device__ __forceinline__ void gemm_store(double alpha, double beta, double v, double* c) {
+  *c = alpha * v + (beta == 0.0 ? 0.0 : beta * *c);
+}
+
+// Products with many rows: a workgroup takes 64 x 16 NT elements of C, each of
+// its four wavefronts 16 rows and NT accumulators, so an operand read from LDS
+// feeds NT instructions; the next 16 columns of A and rows of B are on their way
+// while the current ones are multiplied.  Bounded by the matrix cores and the
+// operand loads of the edge tiles: 24576 x 144 x 144 takes 34 us, one
+// wavefront per 16 x 16 tile without that overlap took 285.  NT is 3 or 4,
+// whichever pads N less.
+template <int NT>
+__global__ void __launch_bounds__(256) k_gemm_tile(int M, int N, int K, double alpha, const double* __restrict__ A,
+                                                   int lda, int ta, const double* __restrict__ B, int ldb, int tb,
+                                                   double beta, double* __restrict__ C, int ldc) {
+  constexpr int NC = 16 * NT;
+  __shared__ double As[2][64][17], Bs[2][16][NC + 1];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * NC;
   const int li = lane & 15, lk = lane >> 4;
-  v4d acc = {0.0, 0.0, 0.0, 0.0};
-  for (int k0 = 0; k0 < K; k0 += 16) {
+  double ra[4], rb[NT];
+  auto fetch = [&](int k0) {
 #pragma unroll
-    for (int e = lane; e < 256; e += 64) {
-      const int r = e >> 4, k = e & 15;  // A tile (row r, column k) and B tile (row r, column k)
-      double va = 0.0, vb = 0.0;
-      const int gr = m0 + r, gk = k0 + k;
-      if (gr < M && gk < K) va = ta ? A[(size_t)gk * lda + gr] : A[(size_t)gr * lda + gk];
-      const int bk = k0 + r, bc = n0 + k;
-      if (bk < K && bc < N) vb = tb ? B[(size_t)bc * ldb + bk] : B[(size_t)bk * ldb + bc];
-      As[r][k] = va;
-      Bs[r][k] = vb;
+    for (int x = 0; x < 4; ++x) {
+      const int e = tid + 256 * x, r = m0 + (ta ? e & 63 : e >> 4), k = k0 + (ta ? e >> 6 : e & 15);
+      ra[x] = r < M && k < K ? (ta ? A[(size_t)k * lda + r] : A[(size_t)r * lda + k]) : 0.0;
     }
-    __syncthreads();
 #pragma unroll
-    for (int kk = 0; kk < 16; kk += 4)
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(As[li][kk + lk], Bs[kk + lk][li], acc, 0, 0, 0);
-    __syncthreads();
+    for (int x = 0; x < NT; ++x) {
+      const int e = tid + 256 * x, c = n0 + (tb ? e >> 4 : e % NC), k = k0 + (tb ? e & 15 : e / NC);
+      rb[x] = c < N && k < K ? (tb ? B[(size_t)c * ldb + k] : B[(size_t)k * ldb + c]) : 0.0;
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int e = tid + 256 * x;
+      As[buf][ta ? e & 63 : e >> 4][ta ? e >> 6 : e & 15] = ra[x];
+    }
+#pragma unroll
+    for (int x = 0; x < NT; ++x) {
+      const int e = tid + 256 * x;
+      Bs[buf][tb ? e & 15 : e / NC][tb ? e >> 4 : e % NC] = rb[x];
+    }
+  };
+  v4d acc[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) acc[j] = v4d{0.0, 0.0, 0.0, 0.0};
+  fetch(0);
+  stage(0);
+  for (int k0 = 0, buf = 0; k0 < K; k0 += 16, buf ^= 1) {
+    __syncthreads();  // this step is staged; the other buffer's readers are done
+    if (k0 + 16 < K) fetch(k0 + 16);
+#pragma unroll
+    for (int kk = 0; kk < 16; kk += 4) {
+      const double a = As[buf][16 * wave + li][kk + lk];
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, Bs[buf][kk + lk][16 * j + li], acc[j], 0, 0, 0);
+    }
+    if (k0 + 16 < K) stage(buf ^ 1);
   }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = m0 + lk + 4 * r, col = n0 + li;
-    if (row < M && col < N) {
-      double* c = C + (size_t)row * ldc + col;
-      *c = alpha * acc[r] + (beta == 0.0 ? 0.0 : beta * *c);
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = m0 + 16 * wave + lk + 4 * r, col = n0 + 16 * j + li;
+      if (row < M && col < N) gemm_store(alpha, beta, acc[j][r], C + (size_t)row * ldc + col);
     }
+}
+
+// Few tiles, long K: a workgroup of 16 wavefronts takes one 16 x 16 tile, each
+// wavefront a sixteenth of K with its operands straight from memory, eight steps
+// of loads in flight (nothing is used twice within a wavefront, so LDS would not
+// save a load); the partial tiles are added in LDS in a fixed order.  Bounded by
+// the loads' latency, K / 512 of them one after another: 144 x 144 x 4096 takes
+// 22 us, 285 with one wavefront walking all of K.
+constexpr int kDeepWaves = 16;
+
+__global__ void __launch_bounds__(64 * kDeepWaves)
+    k_gemm_deep(int M, int N, int K, double alpha, const double* __restrict__ A, int lda, int ta,
+                const double* __restrict__ B, int ldb, int tb, double beta, double* __restrict__ C, int ldc) {
+  __shared__ double part[kDeepWaves][256];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int li = lane & 15, lk = lane >> 4;
+  const int row = blockIdx.y * 16 + li, col = blockIdx.x * 16 + li;
+  const int per = ((K + 4 * kDeepWaves - 1) / (4 * kDeepWaves)) * 4;  // a multiple of the instruction's four
+  const int kb = min(K, wave * per), ke = min(K, kb + per);
+  const double* pa = A + (ta ? (size_t)row : (size_t)row * lda);
+  const double* pb = B + (tb ? (size_t)col * ldb : (size_t)col);
+  const size_t sa = ta ? lda : 1, sb = tb ? 1 : ldb;
+  v4d acc = {0.0, 0.0, 0.0, 0.0};
+  for (int k0 = kb; k0 < ke; k0 += 32) {
+    double a[8], b[8];
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      const int k = k0 + 4 * x + lk;
+      a[x] = row < M && k < ke ? pa[(size_t)k * sa] : 0.0;
+      b[x] = col < N && k < ke ? pb[(size_t)k * sb] : 0.0;
+    }
+#pragma unroll
+    for (int x = 0; x < 8; ++x) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[x], b[x], acc, 0, 0, 0);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) part[wave][(lk + 4 * r) * 16 + li] = acc[r];
+  __syncthreads();
+  if (threadIdx.x < 256) {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < kDeepWaves; ++w) s += part[w][threadIdx.x];
+    const int r = blockIdx.y * 16 + (threadIdx.x >> 4), c = blockIdx.x * 16 + (threadIdx.x & 15);
+    if (r < M && c < N) gemm_store(alpha, beta, s, C + (size_t)r * ldc + c);
   }
 }
 
@@ -571,17 +648,36 @@ __global__ void __launch_bounds__(256 * kGemmSlices)
   }
 }
 
-constexpr double kGemmMfmaMin = 8.0e6;  // multiply-adds from which the matrix-core tiles are used
+// From this many multiply-adds the matrix cores take a product, and a long K does
+// so earlier, since the vector tiles walk it in four slices only (1 x 144 x 4096:
+// 71 us there, 22 in k_gemm_deep).  The 64-row tiles need enough
+// workgroups for half of the chip's CUs; below that the 16 x 16 tiles with K split
+// spread the work wider.
+constexpr double kGemmMfmaMin = 8.0e6;
+constexpr int kGemmDeepK = 1024;
+constexpr long kGemmTiles = 128;
 
 hipError_t vsvb::gemm(hipStream_t st, int M, int N, int K, double alpha, const double* A, int lda, bool ta,
                       const double* B, int ldb, bool tb, double beta, double* C, int ldc) {
   if (M <= 0 || N <= 0) return hipSuccess;
-  dim3 g((N + 15) / 16, (M + 15) / 16);
-  if ((double)M * N * K < kGemmMfmaMin)
+  const dim3 g((N + 15) / 16, (M + 15) / 16);
+  const bool large = (double)M * N * K >= kGemmMfmaMin;
+  const int nt = (N + 47) / 48 * 48 < (N + 63) / 64 * 64 ? 3 : 4;
+  const dim3 gt((N + 16 * nt - 1) / (16 * nt), (M + 63) / 64);
+  if (large && (long)gt.x * gt.y >= kGemmTiles) {
+    if (nt == 3)
+      hipLaunchKernelGGL(k_gemm_tile<3>, gt, dim3(256), 0, st, M, N, K, alpha, A, lda, (int)ta, B, ldb, (int)tb, beta,
+                         C, ldc);
+    else
+      hipLaunchKernelGGL(k_gemm_tile<4>, gt, dim3(256), 0, st, M, N, K, alpha, A, lda, (int)ta, B, ldb, (int)tb, beta,
+                         C, ldc);
+  } else if (large || K >= kGemmDeepK) {
+    hipLaunchKernelGGL(k_gemm_deep, g, dim3(64 * kDeepWaves), 0, st, M, N, K, alpha, A, lda, (int)ta, B, ldb, (int)tb,
+                       beta, C, ldc);
+  } else {
     hipLaunchKernelGGL(k_gemm_small, g, dim3(256 * kGemmSlices), 0, st, M, N, K, alpha, A, lda, (int)ta, B, ldb,
                        (int)tb, beta, C, ldc);
-  else
-    hipLaunchKernelGGL(k_gemm, g, dim3(64), 0, st, M, N, K, alpha, A, lda, (int)ta, B, ldb, (int)tb, beta, C, ldc);
+  }
   return hipGetLastError();
 }
 
@@ -689,23 +785,6 @@ __global__ void k_trace_prod(const double* __restrict__ A, int ld, int off, cons
   if (threadIdx.x == 0) out[0] += w * red[0];
 }
 
-// Sum of many partials into out[w] (deterministic order).
-__global__ void k_reduce_partials(const double* __restrict__ partial, long n, int nw, double* __restrict__ out) {
-  __shared__ double red[256];
-  for (int w = 0; w < nw; ++w) {
-    double s = 0.0;
-    for (long i = threadIdx.x; i < n; i += blockDim.x) s += partial[i * nw + w];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-      if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) out[w] = red[0];
-    __syncthreads();
-  }
-}
-
 __global__ void k_fill(double* __restrict__ p, size_t n, double v) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
 }
@@ -755,11 +834,6 @@ hipError_t vsvb::launch_zero(hipStream_t st, void* p, size_t bytes) {
   const size_t n = bytes / sizeof(uint32_t);
   hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)std::min<size_t>(256, (n + 255) / 256 + 1)), dim3(256), 0, st,
                      (uint32_t*)p, n, 0u);
-  return hipGetLastError();
-}
-
-hipError_t vsvb::launch_reduce(hipStream_t st, const double* partial, long n, int nw, double* out) {
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, st, partial, n, nw, out);
   return hipGetLastError();
 }
 

@@ -282,7 +282,6 @@ hipError_t gemm(hipStream_t st, int M, int N, int K, double alpha, const double*
                 const double* B, int ldb, bool tb, double beta, double* C, int ldc);
 hipError_t launch_fill(hipStream_t st, double* p, size_t n, double v);
 hipError_t launch_zero(hipStream_t st, void* p, size_t bytes);  // bytes: a multiple of 4
-hipError_t launch_reduce(hipStream_t st, const double* partial, long n, int nw, double* out);
 hipError_t launch_gather_grad(vsvb_context* c, const double* gradC, double* grad);
 int prepare_geometry(vsvb_context* c, const double* coords);
 int prepare_orbital_basis(vsvb_context* c, const double* coeff_host, const double* coeff_dev);

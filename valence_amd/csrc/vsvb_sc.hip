@@ -405,13 +405,40 @@ __global__ void __launch_bounds__(64) k_pair_regular(const double* __restrict__ 
   }
 }
 
-// scal[0] = sum omega Phi, scal[1] = N = sum omega, scal[4] = sum omega e1 (from the reductions);
-// scal[2] = E, scal[3] = E_el, scal[5] = E1.
-__global__ void k_sc_final(double* __restrict__ scal, double enuc) {
-  const double el = scal[0] / scal[1];
-  scal[3] = el;
+// scal[0] = sum omega Phi, scal[1] = N = sum omega, scal[4] = sum omega e1 over the
+// determinant pairs, in one workgroup (a chain of loads per thread: 50176 pairs 22 us, where
+// a launch of 256 threads per sum took 3 x 49); scal[2] = E,
+// scal[3] = E_el, scal[5] = E1.
+constexpr int kSumThreads = 1024;
+
+__global__ void __launch_bounds__(kSumThreads) k_sc_sums(const double* __restrict__ num, const double* __restrict__ w,
+                                                         const double* __restrict__ e1w, long n, double enuc,
+                                                         double* __restrict__ scal) {
+  __shared__ double red[3][kSumThreads / 64];
+  double s[3] = {0.0, 0.0, 0.0};
+#pragma unroll 4
+  for (long i = threadIdx.x; i < n; i += kSumThreads) {
+    s[0] += num[i];
+    s[1] += w[i];
+    s[2] += e1w[i];
+  }
+  for (int k = 0; k < 3; ++k) {
+    s[k] = wave_sum(s[k]);
+    if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = s[k];
+  }
+  __syncthreads();
+  if (threadIdx.x > 0) return;
+  for (int k = 0; k < 3; ++k) {
+    s[k] = 0.0;
+    for (int v = 0; v < kSumThreads / 64; ++v) s[k] += red[k][v];
+  }
+  const double el = s[0] / s[1];
+  scal[0] = s[0];
+  scal[1] = s[1];
   scal[2] = el + enuc;
-  scal[5] = scal[4] / scal[1];
+  scal[3] = el;
+  scal[4] = s[2];
+  scal[5] = s[2] / s[1];
 }
 
 struct AdjArgs {
@@ -431,54 +458,68 @@ struct AdjArgs {
   double* wv;    // [pairs] omega / N
 };
 
-// Adjoint of one determinant pair: Abar = ((Phi - E_el)/N) omega G^T - G^T Gbar G^T,
-// Gbar[c][r] = (omega/N) (h + J - K_s)[p_r][q_c]; scattered into Shat.
-__global__ void __launch_bounds__(64) k_pair_adjoint(AdjArgs a, long p0) {
+// Adjoint of the determinant pairs: Abar = ((Phi - E_el)/N) omega G^T - G^T Gbar G^T,
+// Gbar[c][r] = (omega/N) (h + J - K_s)[p_r][q_c]; scattered into Shat.  A workgroup
+// takes pairs t, t + gridDim.x, ... below t1 and adds their blocks in LDS (acc) first:
+// all pairs scatter into the same ns^2 numbers, whose atomics bound a workgroup per
+// pair (H12's 4096 pairs, 144 numbers: 135 us; 38 in 512 workgroups).  acc 0
+// (more than fits the LDS): straight into memory.
+__global__ void __launch_bounds__(64) k_pair_adjoint(AdjArgs a, long t1, int acc) {
   extern __shared__ double lds[];
-  const long t = p0 + blockIdx.x;
-  const int S = (int)(t / a.ndet), T = (int)(t % a.ndet);
   const int ns = a.ns, n2 = ns * ns;
   const double N = a.scal[1], el = a.scal[3];
-  const double om = a.w[t];
-  const double f = om / N, g = (a.phi[t] - el) / N * om;
-  if (threadIdx.x == 0) a.wv[t] = f;
-  if (om == 0.0) return;
   const int dmax = a.na > a.nb ? a.na : a.nb;
   double* G = lds;                    // n x n
   double* Gb = lds + dmax * dmax;     // Gbar
   double* M1 = lds + 2 * dmax * dmax; // Gbar G^T
-  for (int spin = 0; spin < 2; ++spin) {
-    const int n = spin == 0 ? a.na : a.nb;
-    if (n == 0) continue;
-    const int* lb = (spin == 0 ? a.alist : a.blist) + (size_t)S * n;
-    const int* lk = (spin == 0 ? a.alist : a.blist) + (size_t)T * n;
-    const double* Gg = (spin == 0 ? a.Ga + (size_t)t * a.na * a.na : a.Gb + (size_t)t * a.nb * a.nb);
-    const double* KX = (spin == 0 ? a.KXa : a.KXb) + (size_t)t * n2;
-    const double* JX = a.JX + (size_t)t * n2;
-    __syncthreads();
-    for (int k = threadIdx.x; k < n * n; k += blockDim.x) {
-      const int c = k / n, r = k % n;
-      const size_t pos = (size_t)lb[r] * ns + lk[c];
-      G[k] = Gg[k];
-      Gb[k] = f * (a.h[pos] + JX[pos] - KX[pos]);
-    }
-    __syncthreads();
-    // M1[i][c] = sum_j Gbar[i][j] G[c][j]
-    for (int k = threadIdx.x; k < n * n; k += blockDim.x) {
-      const int i = k / n, c = k % n;
-      double s = 0.0;
-      for (int j = 0; j < n; ++j) s += Gb[i * n + j] * G[c * n + j];
-      M1[k] = s;
-    }
-    __syncthreads();
-    // Abar[r][c] = g G[c][r] - sum_i G[i][r] M1[i][c]
-    for (int k = threadIdx.x; k < n * n; k += blockDim.x) {
-      const int r = k / n, c = k % n;
-      double s = g * G[c * n + r];
-      for (int i = 0; i < n; ++i) s -= G[i * n + r] * M1[i * n + c];
-      atomicAdd(&a.Shat[(size_t)lb[r] * ns + lk[c]], s);
+  double* sum = lds + 3 * dmax * dmax;
+  for (int k = threadIdx.x; acc && k < n2; k += blockDim.x) sum[k] = 0.0;
+  for (long t = blockIdx.x; t < t1; t += gridDim.x) {
+    const int S = (int)(t / a.ndet), T = (int)(t % a.ndet);
+    const double om = a.w[t];
+    const double f = om / N, g = (a.phi[t] - el) / N * om;
+    if (threadIdx.x == 0) a.wv[t] = f;
+    if (om == 0.0) continue;
+    for (int spin = 0; spin < 2; ++spin) {
+      const int n = spin == 0 ? a.na : a.nb;
+      if (n == 0) continue;
+      const int* lb = (spin == 0 ? a.alist : a.blist) + (size_t)S * n;
+      const int* lk = (spin == 0 ? a.alist : a.blist) + (size_t)T * n;
+      const double* Gg = (spin == 0 ? a.Ga + (size_t)t * a.na * a.na : a.Gb + (size_t)t * a.nb * a.nb);
+      const double* KX = (spin == 0 ? a.KXa : a.KXb) + (size_t)t * n2;
+      const double* JX = a.JX + (size_t)t * n2;
+      __syncthreads();
+      for (int k = threadIdx.x; k < n * n; k += blockDim.x) {
+        const int c = k / n, r = k % n;
+        const size_t pos = (size_t)lb[r] * ns + lk[c];
+        G[k] = Gg[k];
+        Gb[k] = f * (a.h[pos] + JX[pos] - KX[pos]);
+      }
+      __syncthreads();
+      // M1[i][c] = sum_j Gbar[i][j] G[c][j]
+      for (int k = threadIdx.x; k < n * n; k += blockDim.x) {
+        const int i = k / n, c = k % n;
+        double s = 0.0;
+        for (int j = 0; j < n; ++j) s += Gb[i * n + j] * G[c * n + j];
+        M1[k] = s;
+      }
+      __syncthreads();
+      // Abar[r][c] = g G[c][r] - sum_i G[i][r] M1[i][c]
+      for (int k = threadIdx.x; k < n * n; k += blockDim.x) {
+        const int r = k / n, c = k % n;
+        double s = g * G[c * n + r];
+        for (int i = 0; i < n; ++i) s -= G[i * n + r] * M1[i * n + c];
+        const int at = lb[r] * ns + lk[c];
+        if (acc)
+          atomicAdd(&sum[at], s);
+        else
+          atomicAdd(&a.Shat[at], s);
+      }
     }
   }
+  __syncthreads();
+  for (int k = threadIdx.x; acc && k < n2; k += blockDim.x)
+    if (sum[k] != 0.0) atomicAdd(&a.Shat[k], sum[k]);
 }
 
 // Rows of X scaled by wv: Y[t][k] = wv[t] X[t][k].
@@ -522,19 +563,21 @@ __global__ void k_grad_coef(const double* __restrict__ D2, const int* __restrict
   }
 }
 
-// gradC[t][mu] = sum_w sum_q Dh[t][q][w] W[w][mu][q]
-__global__ void k_grad_eri(const double* __restrict__ Dh, const double* __restrict__ W, int npq, int ns, int nbf,
-                           double* __restrict__ gradC) {
-  const size_t tot = (size_t)ns * nbf;
-  for (size_t x = blockIdx.x * (size_t)blockDim.x + threadIdx.x; x < tot; x += (size_t)gridDim.x * blockDim.x) {
-    const int t = (int)(x / nbf), mu = (int)(x % nbf);
-    double v = 0.0;
-    for (int w = 0; w < npq; ++w) {
-      const double* Wm = W + ((size_t)w * nbf + mu) * ns;
-      for (int q = 0; q < ns; ++q) v += Dh[((size_t)t * ns + q) * npq + w] * Wm[q];
-    }
-    gradC[x] = v;
+// gradC[t][mu] = sum_w sum_q Dh[t][q][w] W[w][mu][q], a wavefront per element: a chain
+// of npq ns / 64 loads (H12, 936 products: 8 us; 125 with a thread per element).
+__global__ void __launch_bounds__(256) k_grad_eri(const double* __restrict__ Dh, const double* __restrict__ W, int npq,
+                                                  int ns, int nbf, double* __restrict__ gradC) {
+  const long x = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (x >= (long)ns * nbf) return;  // whole wavefront
+  const int lane = threadIdx.x & 63;
+  const int t = (int)(x / nbf), mu = (int)(x % nbf);
+  double v = 0.0;
+  for (int e = lane; e < npq * ns; e += 64) {
+    const int w = e / ns, q = e - w * ns;
+    v += Dh[((size_t)t * ns + q) * npq + w] * W[((size_t)w * nbf + mu) * ns + q];
   }
+  v = wave_sum(v);
+  if (lane == 0) gradC[x] = v;
 }
 
 // M = X + X^T (n x n)
@@ -704,10 +747,8 @@ int vsvb::sc_enqueue(vsvb_context* c, bool want_grad, double* grad_dev) {
                        sc.npair, sc.nspinc, sc.want_mats ? sc.d_ham.p : nullptr, sc.d_ovl.p);
     HIP_OK(hipGetLastError());
   }
-  HIP_OK(launch_reduce(st, sc.d_num.p, P, 1, c->d_scal.p + 0));
-  HIP_OK(launch_reduce(st, sc.d_w.p, P, 1, c->d_scal.p + 1));
-  HIP_OK(launch_reduce(st, sc.d_e1w.p, P, 1, c->d_scal.p + 4));
-  hipLaunchKernelGGL(k_sc_final, dim3(1), dim3(1), 0, st, c->d_scal.p, c->enuc);
+  hipLaunchKernelGGL(k_sc_sums, dim3(1), dim3(kSumThreads), 0, st, sc.d_num.p, sc.d_w.p, sc.d_e1w.p, P, c->enuc,
+                     c->d_scal.p);
   HIP_OK(hipGetLastError());
   if (!want_grad) return VSVB_OK;
 
@@ -722,12 +763,11 @@ int vsvb::sc_enqueue(vsvb_context* c, bool want_grad, double* grad_dev) {
   HIP_OK(launch_fill(st, sc.d_Shat.p, n2, 0.0));
   AdjArgs aa{c->d_Horb.p, sc.d_JX.p, sc.d_KXa.p, sc.d_KXb.p, sc.d_Ga.p, sc.d_Gb.p, sc.d_w.p, sc.d_phi.p,
              c->d_scal.p, sc.d_alist.p, sc.d_blist.p, sc.ndet, sc.na, sc.nb, ns, sc.d_Shat.p, sc.d_wv.p};
-  const size_t lds_adj = 3 * (size_t)dmax * dmax * sizeof(double);
-  for (long p0 = 0; p0 < P; p0 += chunk) {
-    const unsigned nb = (unsigned)std::min(chunk, P - p0);
-    hipLaunchKernelGGL(k_pair_adjoint, dim3(nb), dim3(64), lds_adj, st, aa, p0);
-    HIP_OK(hipGetLastError());
-  }
+  const size_t lds_blocks = 3 * (size_t)dmax * dmax * sizeof(double), lds_acc = n2 * sizeof(double);
+  const bool acc = lds_blocks + lds_acc <= 65536;
+  hipLaunchKernelGGL(k_pair_adjoint, dim3((unsigned)std::min<long>(P, acc ? 512 : 65536)), dim3(64),
+                     lds_blocks + (acc ? lds_acc : 0), st, aa, P, (int)acc);
+  HIP_OK(hipGetLastError());
   // hhat = sum_t wv_t Gamma^t_t ; D2 = 1/2 Xw^T Xt - 1/2 (exchange-ordered Xwa^T Xa + Xwb^T Xb)
   HIP_OK(gemm(st, 1, n2, (int)P, 1.0, sc.d_wv.p, (int)P, false, sc.d_Xt.p, n2, false, 0.0, sc.d_hhat.p, n2));
   hipLaunchKernelGGL(k_scale_rows, dim3(grid_for(P * n2)), dim3(256), 0, st, sc.d_Xt.p, sc.d_wv.p, P, n2, sc.d_Xw.p);
@@ -742,7 +782,7 @@ int vsvb::sc_enqueue(vsvb_context* c, bool want_grad, double* grad_dev) {
   // four-index term through W^rs, then the overlap and one-electron terms
   hipLaunchKernelGGL(k_grad_coef, dim3(grid_for((size_t)n2 * sc.npq)), dim3(256), 0, st, sc.d_D2.p, sc.d_pq.p,
                      sc.npq, ns, sc.d_Dh.p);
-  hipLaunchKernelGGL(k_grad_eri, dim3(grid_for((size_t)ns * nbf)), dim3(256), 0, st, sc.d_Dh.p, sc.d_W.p, sc.npq, ns,
+  hipLaunchKernelGGL(k_grad_eri, dim3((unsigned)(((size_t)ns * nbf + 3) / 4)), dim3(256), 0, st, sc.d_Dh.p, sc.d_W.p, sc.npq, ns,
                      nbf, c->d_gradC.p);
   HIP_OK(hipGetLastError());
   for (int k = 0; k < 2; ++k) {
