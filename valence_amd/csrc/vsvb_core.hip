@@ -1502,7 +1502,6 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
       h.p.A = A;
       h.p.B = B;
       h.p.npp = shells[A].nprim * shells[B].nprim;
-      h.p.offdiag = M != N;
       h.cls = pair_class_of(shells[A].l, shells[B].l);
       const double* xa = s->coords + 3 * shells[A].atom;
       const double* xb = s->coords + 3 * shells[B].atom;
@@ -1528,6 +1527,8 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   for (auto& h : hp) c->pair_off[h.cls + 1]++;
   for (int cl = 0; cl < kNPairClass; ++cl) c->pair_off[cl + 1] += c->pair_off[cl];
   c->npairs = (int)pairs.size();
+  c->nfun = 0;
+  for (const Pair& P : pairs) c->nfun += ncart(shells[P.A].l) * ncart(shells[P.B].l);
   c->npp = (int)ppsrc.size();
   c->h_shells = shells;
   c->h_pairs = pairs;
@@ -1761,6 +1762,11 @@ static int schedule_pairs(vsvb_context* c) {
     sorted[i] = c->h_pairs[idx[i]];
     skept[i] = kept[idx[i]];
   }
+  for (int cl = 0, f0 = 0; cl < kNPairClass; ++cl) {
+    const int b = c->pair_off[cl], e = c->pair_off[cl + 1];
+    for (int i = b; i < e; ++i) sorted[i].f0 = f0 + i - b;
+    if (e > b) f0 += (e - b) * ncart(c->h_shells[sorted[b].A].l) * ncart(c->h_shells[sorted[b].B].l);
+  }
   c->h_pairs.swap(sorted);
   const int rc = plan_work(c, skept.data());
   if (rc) return rc;
@@ -1908,7 +1914,7 @@ static int prepare_orbitals(vsvb_context* c, const double* coeff_host, const dou
 // Shell-quartet stage.  By default it serves this context's own wave function;
 // a batch group leader passes nwfn > 1 and group-wide density and J/K arrays.
 static QuartetArgs class_args(vsvb_context* c, int bc, int kc, const ClassLaunch& cl, bool jk, int nwfn, int nspin,
-                              const double* dens, double* jacc, double* kacc, double* partial) {
+                              const double* dens, double* jacc, double* kacc, double* partial, double* eri = nullptr) {
   const int q = quartet_class_index(bc, kc);
   QuartetArgs a{};
   const WorkList &B = c->work[bc][cl.lb], &K = c->work[kc][cl.lk];
@@ -1933,6 +1939,10 @@ static QuartetArgs class_args(vsvb_context* c, int bc, int kc, const ClassLaunch
   a.partial = partial;
   a.jacc = jacc;
   a.kacc = kacc;
+  a.eri = eri;
+  a.neri = c->nfun;
+  a.fbra = c->pair_off[bc + 1] - c->pair_off[bc];
+  a.fket = c->pair_off[kc + 1] - c->pair_off[kc];
   a.counters = c->d_counters.p + 4 * q;
   a.stamp = c->profile ? c->d_stamps.p + (size_t)q * 2 * kStampSlots : nullptr;
   a.tile_ctr = c->d_tilectr.p + c->ctr_off[q];
@@ -1973,9 +1983,11 @@ static hipError_t quartet_pass_clear(vsvb_context* c, bool jk, int nwfn, int nsp
 }
 
 // nspin_override = 0 turns the J/K launch into a Coulomb-only pass over nwfn
-// general symmetric densities (the exchange accumulators are not touched).
+// general symmetric densities (the exchange accumulators are not touched).  eri
+// (nfun x nfun, zeroed by the caller): an energy pass stores its integrals there
+// instead of contracting them (QuartetArgs::eri).
 int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, double* jacc,
-                       double* kacc, int nspin_override) {
+                       double* kacc, int nspin_override, double* eri) {
   hipStream_t st = c->stream;
   const int nspin = nspin_override >= 0 ? nspin_override : (c->nunpd > 0 ? 2 : 1);
   if (!dens) dens = c->d_R.p;
@@ -1999,14 +2011,14 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
   // they differ from the last ones (under capture nothing is uploaded; records
   // that differ then take separate launches).
   const int m = jk ? 1 : 0;
-  bool shared = c->small[m].n > 0 && nwfn == 1;
+  bool shared = c->small[m].n > 0 && (nwfn == 1 || eri);
   if (shared) {
     const SmallLaunch& s = c->small[m];
     std::vector<QuartetArgs> rec(s.n);
     for (int k = 0; k < s.n; ++k) {
       const int q = s.q[k], bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
       rec[k] = class_args(c, bc, kc, jk ? c->ljk[q] : c->le[q], jk, nwfn, nspin, dens, jacc, kacc,
-                          c->d_partial.p + offs[q]);
+                          c->d_partial.p + offs[q], eri);
     }
     std::vector<QuartetArgs>& old = c->h_small[m];
     QuartetArgs* dev = c->d_small.p + (size_t)m * kNQuartetClass;
@@ -2030,7 +2042,8 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
     // configuration without any would drop its quartets silently
     if (nb > 0 && nk > 0 && cl.units <= 0)
       return fail(VSVB_ERR_UNSUPPORTED, "quartet class " + std::to_string(q) + " has no launchable work units");
-    const QuartetArgs a = class_args(c, bc, kc, cl, jk, nwfn, nspin, dens, jacc, kacc, c->d_partial.p + offs[q]);
+    const QuartetArgs a = class_args(c, bc, kc, cl, jk, nwfn, nspin, dens, jacc, kacc, c->d_partial.p + offs[q],
+                                     eri);
     HIP_OK(launch_class(c, bc, kc, cl, a, jk));
   }
   if (c->ev0 && c->ev1 && !c->capturing) {
@@ -2040,7 +2053,7 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
   if (c->profile)
     hipLaunchKernelGGL(k_stamp_reduce, dim3(kNQuartetClass), dim3(kStampSlots), 0, st, c->d_stamps.p,
                        c->d_counters.p + kCtrSlots * kCtrStride);
-  if (!jk) HIP_OK(launch_energy_sum(st, c->d_partial.p, (long)poff, c->enuc, c->d_scal.p));
+  if (!jk && !eri) HIP_OK(launch_energy_sum(st, c->d_partial.p, (long)poff, c->enuc, c->d_scal.p));
   return VSVB_OK;
 }
 

@@ -2,7 +2,7 @@
 //
 // Layout in HBM (all FP64 unless noted; one copy per geometry):
 //   Shell      {atom, l, nprim, prim0, ao}                     static per molecule
-//   Pair       {A, B, pp0, npp, cls, offdiag, AB, Q}           one per unordered shell pair
+//   Pair       {A, B, pp0, npp, f0, seg, AB, Q}                one per unordered shell pair
 //   PrimPair   {p, 1/(2p), P, P-A, K}                          one per primitive pair
 // Shell pairs are stored class-major (pair classes ss, ps, pp, ds, dp, dd) and,
 // inside a class, by decreasing primitive-pair count so a wavefront's threads
@@ -74,10 +74,12 @@ struct Shell {
 struct Pair {
   int A, B;        // shells; l(A) >= l(B)
   int pp0, npp;    // primitive pairs
-  int offdiag;     // 1 if A != B
+  int f0;          // the pair's function pair (0, 0) in the list of all pairs' function pairs; (i, j) stands
+                   // (i NB + j) x (pairs of the class) further on
   int seg;         // segment of the pair's primitive list (0 for a whole pair)
   double ABx, ABy, ABz;
   double Q;        // sqrt(max |(ab|ab)|)
+  __host__ __device__ bool offdiag() const { return A != B; }
 };
 
 // 1/sqrt(x) to full FP64 precision: the hardware estimate (relative error

@@ -165,9 +165,18 @@ __device__ __forceinline__ void coop_body(const QuartetArgs& a, const CoopDesc& 
       }
       nq += (P.seg | K.seg) == 0;  // a quartet of segments is counted once
       nprimq += (unsigned long long)P.npp * K.npp;
-      const double deg = (P.offdiag ? 2.0 : 1.0) * (K.offdiag ? 2.0 : 1.0) * ((ib != ik || !a.same) ? 2.0 : 1.0);
+      const double deg = (P.offdiag() ? 2.0 : 1.0) * (K.offdiag() ? 2.0 : 1.0) * ((ib != ik || !a.same) ? 2.0 : 1.0);
       const int ma = a.shells[P.A].ao, mb = a.shells[P.B].ao;
       const int mc = a.shells[K.A].ao, md = a.shells[K.B].ao;
+      if (!kJK && a.eri) {
+        const double h = a.same && ib == ik ? 0.5 : 1.0;
+        double* E = a.eri + (size_t)K.f0 * a.neri + P.f0;
+        for (int idx = lane; idx < NAB * NCD; idx += 64) {
+          const int ab = idx / NCD, cd = idx - ab * NCD;
+          unsafeAtomicAdd(&E[(size_t)(cd * a.fket) * a.neri + ab * a.fbra], h * S[outs[idx]]);
+        }
+        continue;
+      }
       for (int w = 0; w < a.nwfn; ++w) {
         const double* D0 = a.dens + (size_t)w * dstride * nn;
         auto rho = [&](int x, int y) {  // cfac * sum_s D_s[x][y]

@@ -70,6 +70,11 @@ struct QuartetArgs {
   double* partial;      // energy: [parts][gridDim.x * 4][nwfn] per-wave partial sums
   double* jacc;         // J/K mode: Coulomb accumulators [nwfn][nbf][nbf]
   double* kacc;         // J/K mode: exchange accumulators [nwfn][nspin][nbf][nbf]
+  double* eri;          // energy mode: not null = store the integrals instead of contracting them:
+                        // eri[ket function pair][bra function pair], neri in a row, added to, a unit on
+                        // the diagonal of a class paired with itself by half
+  int neri;
+  int fbra, fket;       // distance of a pair's function pairs there (shell pairs of the bra and of the ket class)
   unsigned long long* counters;  // the class's {quartets evaluated, primitive quartets, skipped} in slot 0
   int* tile_ctr;        // J/K and cooperative kernels: work counters, zero before the launch: nstrip per part
   int nstrip;           // J/K strips (bra, or ket when transposed), energy segments of kSegTiles bra tiles: one work
@@ -307,8 +312,20 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
         for (int k = 0; k < NAB * NCD; ++k) v[k] = 0.0;
       }
       if (!__any(act)) continue;  // wave-uniform: nothing to contract
+      if (a.eri) {
+        if (act) {
+          const double h = a.same && ib == ik ? 0.5 : 1.0;
+          double* E = a.eri + (size_t)K.f0 * a.neri + P.f0;
+#pragma unroll
+          for (int kl = 0; kl < NCD; ++kl)
+#pragma unroll
+            for (int ij = 0; ij < NAB; ++ij) 
+              unsafeAtomicAdd(&E[(size_t)(kl * a.fket) * a.neri + (A0 * NB + ij) * a.fbra], h * v[ij * NCD + kl]);
+        }
+        continue;
+      }
       const double deg =
-          act ? (P.offdiag ? 2.0 : 1.0) * (K.offdiag ? 2.0 : 1.0) * ((ib != ik || !a.same) ? 2.0 : 1.0) : 0.0;
+          act ? (P.offdiag() ? 2.0 : 1.0) * (K.offdiag() ? 2.0 : 1.0) * ((ib != ik || !a.same) ? 2.0 : 1.0) : 0.0;
       // inactive lanes read valid blocks and contribute zero
       const int ma = a.shells[P.A].ao + A0, mb = a.shells[P.B].ao;
       const int mc = a.shells[K.A].ao, md = a.shells[K.B].ao;
@@ -499,7 +516,7 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const Plac
         for (int k = 0; k < NAB * NCD; ++k) v[k] = 0.0;
       }
       const bool wact = __any(act);  // wave-uniform
-      const double deg = act ? (P.offdiag ? 2.0 : 1.0) * (K.offdiag ? 2.0 : 1.0) * ((ib != ik || !a.same) ? 2.0 : 1.0)
+      const double deg = act ? (P.offdiag() ? 2.0 : 1.0) * (K.offdiag() ? 2.0 : 1.0) * ((ib != ik || !a.same) ? 2.0 : 1.0)
                              : 0.0;
       // inactive lanes read the block of their (valid) bra pair and contribute zero
       const int ma = a.shells[P.A].ao + A0, mb = a.shells[P.B].ao;
@@ -742,7 +759,7 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const Pla
       }
       const bool wact = __any(act);  // wave-uniform
       // bra and ket classes differ, so every quartet stands for its (cd|ab) image too
-      const double deg = act ? (P.offdiag ? 2.0 : 1.0) * (K.offdiag ? 2.0 : 1.0) * 2.0 : 0.0;
+      const double deg = act ? (P.offdiag() ? 2.0 : 1.0) * (K.offdiag() ? 2.0 : 1.0) * 2.0 : 0.0;
       const int ma = a.shells[P.A].ao + A0, mb = a.shells[P.B].ao;
       const int mc = a.shells[K.A].ao, md = a.shells[K.B].ao;
       const double fj = 0.25 * deg, fk = 0.125 * deg * xfac;

@@ -92,6 +92,12 @@ struct DevBuf {
 };
 
 
+// Function pair (mu, nu) of two shells; same: of one shell, whose functions are
+// listed in both orders.
+struct FnPair {
+  int mu, nu, same;
+};
+
 // Spin-coupled determinant expansion (density_sc / dbra / dket,
 // src/valence.F90:1612-1870): determinant d = isc * 2^npair + mask has the
 // alpha list (pair slots, swapped where mask has the bit; unpaired; docc) and
@@ -107,6 +113,10 @@ struct SpinCoupled {
   DevBuf<int> d_pq;                      // [npq][2] unique orbital pairs (r >= s)
   DevBuf<double> d_cdet;                 // [ndet]
   DevBuf<double> d_pdens, d_pj;          // [npq][nbf][nbf] pair densities / their Coulomb matrices
+  // Integrals stored once for all pair densities (d_M null: contracted on the fly)
+  DevBuf<double> d_M;                    // [nfun][nfun] (ab|cd)
+  DevBuf<FnPair> d_fn;                   // [nfun] the functions of Pair::f0's list
+  DevBuf<double> d_Dp, d_Jp;             // [npq][nfun] packed pair densities / their Coulomb images
   DevBuf<double> d_W;                    // [npq][nbf][nsp]  J^{rs} C^T
   DevBuf<double> d_eri, d_erik;          // [nsp^2][nsp^2]   (pq|rs) and its exchange ordering
   DevBuf<double> d_Ga, d_Gb;             // [npairs][na^2], [npairs][nb^2] inverses
@@ -207,6 +217,7 @@ struct vsvb_context {
                                  // the null stream): the allocation-free entry point
   // sizes
   int natom = 0, nsh = 0, nbf = 0, npairs = 0, npp = 0, nsp = 0, norbs = 0, totlen = 0;
+  int nfun = 0;  // function pairs of all shell pairs (Pair::f0)
   int npair = 0, nunpd = 0, ndocc = 0, ndf = 0, first_ndf = 0;
   int nalpha_rows = 0;  // spatial orbitals with an alpha electron: rows [0, nalpha_rows) of C (nsp, or
                         // nsp - 1 when the last doubly occupied orbital holds only a beta electron)
@@ -286,7 +297,7 @@ hipError_t launch_gather_grad(vsvb_context* c, const double* gradC, double* grad
 int prepare_geometry(vsvb_context* c, const double* coords);
 int prepare_orbital_basis(vsvb_context* c, const double* coeff_host, const double* coeff_dev);
 int run_quartets(vsvb_context* c, bool jk, int nwfn = 1, const double* dens = nullptr,
-                 double* jacc = nullptr, double* kacc = nullptr, int nspin_override = -1);
+                 double* jacc = nullptr, double* kacc = nullptr, int nspin_override = -1, double* eri = nullptr);
 int finish_counters(vsvb_context* c, const unsigned long long* host_counters = nullptr);
 int check_status(vsvb_context* c, bool for_grad);
 

@@ -53,6 +53,79 @@ __global__ void k_pair_dens(const double* __restrict__ Cs, const int* __restrict
   }
 }
 
+// Stored integrals.  All npq pair densities meet the same integrals, so where
+// nfun^2 of them fit (kStoredBytes, and a sixteenth of the free memory, so that
+// many contexts leave room for the next) an energy pass writes each once and a product
+// [npq x nfun] x [nfun x nfun] contracts them; H12's 78 densities took 4.4 ms
+// contracted quartet by quartet, an atomic per density and function pair, and
+// take 0.5 ms this way (0.36 of them the integrals).
+// Below kStoredMin densities the fixed cost (clearing, transposing and reading the
+// matrix, six small launches) is no longer small against what is saved.  The
+// functions of a pair lie a class apart, so that the 64 bra pairs of a wavefront
+// write 64 neighbours (with a pair's functions side by side (pp|ps) took 259 us
+// instead of 53).
+constexpr size_t kStoredBytes = (size_t)1 << 30;
+constexpr int kStoredMin = 10;
+
+struct ClassOffsets {
+  int at[kNPairClass + 1];
+};
+__global__ void k_function_pairs(const Pair* __restrict__ pairs, ClassOffsets off, const Shell* __restrict__ shells,
+                                 FnPair* __restrict__ fn) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= off.at[kNPairClass]) return;
+  int cl = 0;
+  while (t >= off.at[cl + 1]) ++cl;
+  const Pair P = pairs[t];
+  const Shell A = shells[P.A], B = shells[P.B];
+  FnPair* f = fn + P.f0;
+  for (int i = 0; i < ncart(A.l); ++i)
+    for (int j = 0; j < ncart(B.l); ++j, f += off.at[cl + 1] - off.at[cl]) *f = FnPair{A.ao + i, B.ao + j, P.A == P.B};
+}
+
+// Dp[rs][f]: k_pair_dens' element (mu, nu), doubled where the pair stands for (nu, mu) too.
+__global__ void k_pair_dens_packed(const double* __restrict__ Cs, const int* __restrict__ pq, int npq, int nbf,
+                                   const FnPair* __restrict__ fn, int nfun, double* __restrict__ Dp) {
+  const size_t tot = (size_t)npq * nfun;
+  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < tot; t += (size_t)gridDim.x * blockDim.x) {
+    const int w = (int)(t / nfun);
+    const FnPair f = fn[t % nfun];
+    const double* cr = Cs + (size_t)pq[2 * w] * nbf;
+    const double* cs = Cs + (size_t)pq[2 * w + 1] * nbf;
+    Dp[t] = (f.same ? 0.5 : 1.0) * (cr[f.mu] * cs[f.nu] + cs[f.mu] * cr[f.nu]);
+  }
+}
+
+__global__ void k_unpack_coulomb(const double* __restrict__ Jp, const FnPair* __restrict__ fn, int npq, int nfun,
+                                 int nbf, double* __restrict__ J) {
+  const size_t tot = (size_t)npq * nfun, nn = (size_t)nbf * nbf;
+  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < tot; t += (size_t)gridDim.x * blockDim.x) {
+    const FnPair f = fn[t % nfun];
+    double* M = J + t / nfun * nn;
+    M[(size_t)f.mu * nbf + f.nu] = Jp[t];
+    if (!f.same) M[(size_t)f.nu * nbf + f.mu] = Jp[t];
+  }
+}
+
+// M = T + T^T in place, a workgroup per 32 x 32 tile on or below the diagonal and
+// its mirror image, through LDS so that both are read and written along rows.
+__global__ void __launch_bounds__(256) k_sym_tiles(double* __restrict__ M, int n) {
+  __shared__ double lo[32][33], up[32][33];
+  const int bi = blockIdx.y, bj = blockIdx.x, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  if (bj > bi) return;
+  for (int r = ty; r < 32; r += 8) {
+    const int i = bi * 32 + r, j = bj * 32 + tx, it = bj * 32 + r, jt = bi * 32 + tx;
+    lo[r][tx] = i < n && j < n ? M[(size_t)i * n + j] : 0.0;
+    up[r][tx] = it < n && jt < n ? M[(size_t)it * n + jt] : 0.0;
+  }
+  __syncthreads();
+  for (int r = ty; r < 32; r += 8) {
+    const int i = bi * 32 + r, j = bj * 32 + tx, it = bj * 32 + r, jt = bi * 32 + tx;
+    if (i < n && j < n) M[(size_t)i * n + j] = lo[r][tx] + up[tx][r];
+    if (bi != bj && it < n && jt < n) M[(size_t)it * n + jt] = up[r][tx] + lo[tx][r];
+  }
+}
+
 // J = A + A^T for each of nmat n x n accumulators, in place.
 __global__ void k_sym_batch(double* __restrict__ A, int nmat, int n) {
   const size_t nn = (size_t)n * n;
@@ -662,7 +735,17 @@ int vsvb::sc_setup(vsvb_context* c, const vsvb_system* s) {
   HIP_OK(sc.d_blist.alloc(bl.size()));
   HIP_OK(sc.d_cdet.alloc(cd.size()));
   HIP_OK(sc.d_pq.alloc(pq.size()));
-  HIP_OK(sc.d_pdens.alloc(sc.npq * nn));
+  const size_t nf = (size_t)c->nfun;
+  size_t free_bytes = 0, total_bytes = 0;
+  HIP_OK(hipMemGetInfo(&free_bytes, &total_bytes));
+  if (sc.npq >= kStoredMin && nf * nf * sizeof(double) <= std::min(kStoredBytes, free_bytes / 16)) {
+    HIP_OK(sc.d_M.alloc(nf * nf));
+    HIP_OK(sc.d_fn.alloc(nf));
+    HIP_OK(sc.d_Dp.alloc(sc.npq * nf));
+    HIP_OK(sc.d_Jp.alloc(sc.npq * nf));
+  } else {
+    HIP_OK(sc.d_pdens.alloc(sc.npq * nn));
+  }
   HIP_OK(sc.d_pj.alloc(sc.npq * nn));
   HIP_OK(sc.d_W.alloc((size_t)sc.npq * c->nbf * ns));
   HIP_OK(sc.d_eri.alloc(n2 * n2));
@@ -710,12 +793,31 @@ int vsvb::sc_enqueue(vsvb_context* c, bool want_grad, double* grad_dev) {
   const long P = sc.npairs;
   int rc;
   // orbital-pair Coulomb matrices from one pass over the screened shell quartets
-  hipLaunchKernelGGL(k_pair_dens, dim3(grid_for(sc.npq * nn)), dim3(256), 0, st, c->d_Cs.p, sc.d_pq.p, sc.npq, nbf,
-                     sc.d_pdens.p);
-  HIP_OK(hipGetLastError());
-  if ((rc = run_quartets(c, true, sc.npq, sc.d_pdens.p, sc.d_pj.p, c->d_K.p, 0))) return rc;
-  hipLaunchKernelGGL(k_sym_batch, dim3(grid_for(sc.npq * nn)), dim3(256), 0, st, sc.d_pj.p, sc.npq, nbf);
-  HIP_OK(hipGetLastError());
+  if (sc.d_M.p) {
+    const int nf = c->nfun;
+    const unsigned tiles = (unsigned)(nf + 31) / 32;
+    HIP_OK(launch_fill(st, sc.d_M.p, (size_t)nf * nf, 0.0));
+    if ((rc = run_quartets(c, false, 0, nullptr, nullptr, nullptr, 0, sc.d_M.p))) return rc;
+    hipLaunchKernelGGL(k_sym_tiles, dim3(tiles, tiles), dim3(256), 0, st, sc.d_M.p, nf);
+    ClassOffsets off;
+    std::copy(c->pair_off, c->pair_off + kNPairClass + 1, off.at);
+    hipLaunchKernelGGL(k_function_pairs, dim3((c->npairs + 255) / 256), dim3(256), 0, st, c->d_pairs.p, off,
+                       c->d_shells.p, sc.d_fn.p);
+    hipLaunchKernelGGL(k_pair_dens_packed, dim3(grid_for((size_t)sc.npq * nf)), dim3(256), 0, st, c->d_Cs.p, sc.d_pq.p,
+                       sc.npq, nbf, sc.d_fn.p, nf, sc.d_Dp.p);
+    HIP_OK(hipGetLastError());
+    HIP_OK(gemm(st, sc.npq, nf, nf, 1.0, sc.d_Dp.p, nf, false, sc.d_M.p, nf, false, 0.0, sc.d_Jp.p, nf));
+    hipLaunchKernelGGL(k_unpack_coulomb, dim3(grid_for((size_t)sc.npq * nf)), dim3(256), 0, st, sc.d_Jp.p, sc.d_fn.p,
+                       sc.npq, nf, nbf, sc.d_pj.p);
+    HIP_OK(hipGetLastError());
+  } else {
+    hipLaunchKernelGGL(k_pair_dens, dim3(grid_for(sc.npq * nn)), dim3(256), 0, st, c->d_Cs.p, sc.d_pq.p, sc.npq, nbf,
+                       sc.d_pdens.p);
+    HIP_OK(hipGetLastError());
+    if ((rc = run_quartets(c, true, sc.npq, sc.d_pdens.p, sc.d_pj.p, c->d_K.p, 0))) return rc;
+    hipLaunchKernelGGL(k_sym_batch, dim3(grid_for(sc.npq * nn)), dim3(256), 0, st, sc.d_pj.p, sc.npq, nbf);
+    HIP_OK(hipGetLastError());
+  }
   // W^rs = J^rs C^T  ([npq nbf] x nbf times nbf x ns), then (pq|rs) and its exchange ordering
   HIP_OK(gemm_rows(st, (long)sc.npq * nbf, ns, nbf, 1.0, sc.d_pj.p, nbf, c->d_Cs.p, nbf, true, 0.0, sc.d_W.p, ns));
   hipLaunchKernelGGL(k_orb_eri, dim3(grid_for((size_t)sc.npq * n2)), dim3(256), 0, st, c->d_Cs.p, sc.d_W.p,
