@@ -10,8 +10,9 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# from 8e6 multiply-adds and 128 workgroups: 64-row tiles (columns 144, 50, 33, 64, 1100, 130)
-TILES = [(4097, 144, 40), (8200, 50, 33), (8129, 33, 31), (8192, 64, 16), (700, 1100, 17), (3001, 130, 65)]
+# from 8e6 multiply-adds and 128 workgroups: 64-row tiles (columns 144, 50, 33, 64, 1100, 130), 32-row tiles
+TILES = [(4097, 144, 40), (8200, 50, 33), (8129, 33, 31), (8192, 64, 16), (700, 1100, 17), (3001, 130, 65), (32, 8200, 40),
+         (17, 8129, 70), (5, 8300, 200)]
 # K >= 1024, or 8e6 multiply-adds in fewer workgroups: K split over a workgroup's wavefronts
 DEEP = [(1, 144, 4096), (17, 5, 1024), (16, 16, 1025), (3, 2, 1087), (33, 1, 5000), (144, 144, 4096), (500, 130, 129)]
 

@@ -487,27 +487,29 @@ __device__ __forceinline__ void gemm_store(double alpha, double beta, double v, 
   *c = alpha * v + (beta == 0.0 ? 0.0 : beta * *c);
 }
 
-// Products with many rows: a workgroup takes 64 x 16 NT elements of C, each of
-// its four wavefronts 16 rows and NT accumulators, so an operand read from LDS
-// feeds NT instructions; the next 16 columns of A and rows of B are on their way
+// Products with many tiles: a workgroup takes 16 MR x 16 NT elements of C.  MR = 4:
+// each of its four wavefronts 16 rows and NT accumulators, so an operand read from
+// LDS feeds NT instructions; MR = 2 (at most 32 rows): 16 rows and half of the
+// columns each; the next 16 columns of A and rows of B are on their way
 // while the current ones are multiplied.  Bounded by the matrix cores and the
 // operand loads of the edge tiles: 24576 x 144 x 144 takes 34 us, one
 // wavefront per 16 x 16 tile without that overlap took 285.  NT is 3 or 4,
 // whichever pads N less.
-template <int NT>
+template <int MR, int NT>
 __global__ void __launch_bounds__(256) k_gemm_tile(int M, int N, int K, double alpha, const double* __restrict__ A,
                                                    int lda, int ta, const double* __restrict__ B, int ldb, int tb,
                                                    double beta, double* __restrict__ C, int ldc) {
-  constexpr int NC = 16 * NT;
-  __shared__ double As[2][64][17], Bs[2][16][NC + 1];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * NC;
+  constexpr int NC = 16 * NT, RM = 16 * MR, NW = NT * MR / 4;
+  __shared__ double As[2][RM][17], Bs[2][16][NC + 1];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wr = 16 * ((tid >> 6) % MR), wc = 16 * NW * ((tid >> 6) / MR);  // the wavefront's corner of the tile
+  const int m0 = blockIdx.y * RM, n0 = blockIdx.x * NC;
   const int li = lane & 15, lk = lane >> 4;
-  double ra[4], rb[NT];
+  double ra[MR], rb[NT];
   auto fetch = [&](int k0) {
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int e = tid + 256 * x, r = m0 + (ta ? e & 63 : e >> 4), k = k0 + (ta ? e >> 6 : e & 15);
+    for (int x = 0; x < MR; ++x) {
+      const int e = tid + 256 * x, r = m0 + (ta ? e % RM : e >> 4), k = k0 + (ta ? e / RM : e & 15);
       ra[x] = r < M && k < K ? (ta ? A[(size_t)k * lda + r] : A[(size_t)r * lda + k]) : 0.0;
     }
 #pragma unroll
@@ -518,9 +520,9 @@ __global__ void __launch_bounds__(256) k_gemm_tile(int M, int N, int K, double a
   };
   auto stage = [&](int buf) {
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
+    for (int x = 0; x < MR; ++x) {
       const int e = tid + 256 * x;
-      As[buf][ta ? e & 63 : e >> 4][ta ? e >> 6 : e & 15] = ra[x];
+      As[buf][ta ? e % RM : e >> 4][ta ? e / RM : e & 15] = ra[x];
     }
 #pragma unroll
     for (int x = 0; x < NT; ++x) {
@@ -528,9 +530,9 @@ __global__ void __launch_bounds__(256) k_gemm_tile(int M, int N, int K, double a
       Bs[buf][tb ? e & 15 : e / NC][tb ? e >> 4 : e % NC] = rb[x];
     }
   };
-  v4d acc[NT];
+  v4d acc[NW];
 #pragma unroll
-  for (int j = 0; j < NT; ++j) acc[j] = v4d{0.0, 0.0, 0.0, 0.0};
+  for (int j = 0; j < NW; ++j) acc[j] = v4d{0.0, 0.0, 0.0, 0.0};
   fetch(0);
   stage(0);
   for (int k0 = 0, buf = 0; k0 < K; k0 += 16, buf ^= 1) {
@@ -538,18 +540,18 @@ __global__ void __launch_bounds__(256) k_gemm_tile(int M, int N, int K, double a
     if (k0 + 16 < K) fetch(k0 + 16);
 #pragma unroll
     for (int kk = 0; kk < 16; kk += 4) {
-      const double a = As[buf][16 * wave + li][kk + lk];
+      const double a = As[buf][wr + li][kk + lk];
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
-        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, Bs[buf][kk + lk][16 * j + li], acc[j], 0, 0, 0);
+      for (int j = 0; j < NW; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, Bs[buf][kk + lk][wc + 16 * j + li], acc[j], 0, 0, 0);
     }
     if (k0 + 16 < K) stage(buf ^ 1);
   }
 #pragma unroll
-  for (int j = 0; j < NT; ++j)
+  for (int j = 0; j < NW; ++j)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = m0 + 16 * wave + lk + 4 * r, col = n0 + 16 * j + li;
+      const int row = m0 + wr + lk + 4 * r, col = n0 + wc + 16 * j + li;
       if (row < M && col < N) gemm_store(alpha, beta, acc[j][r], C + (size_t)row * ldc + col);
     }
 }
@@ -650,7 +652,7 @@ __global__ void __launch_bounds__(256 * kGemmSlices)
 
 // From this many multiply-adds the matrix cores take a product, and a long K does
 // so earlier, since the vector tiles walk it in four slices only (1 x 144 x 4096:
-// 71 us there, 22 in k_gemm_deep).  The 64-row tiles need enough
+// 71 us there, 22 in k_gemm_deep).  The larger tiles need enough
 // workgroups for half of the chip's CUs; below that the 16 x 16 tiles with K split
 // spread the work wider.
 constexpr double kGemmMfmaMin = 8.0e6;
@@ -662,14 +664,17 @@ hipError_t vsvb::gemm(hipStream_t st, int M, int N, int K, double alpha, const d
   if (M <= 0 || N <= 0) return hipSuccess;
   const dim3 g((N + 15) / 16, (M + 15) / 16);
   const bool large = (double)M * N * K >= kGemmMfmaMin;
-  const int nt = (N + 47) / 48 * 48 < (N + 63) / 64 * 64 ? 3 : 4;
-  const dim3 gt((N + 16 * nt - 1) / (16 * nt), (M + 63) / 64);
+  const int nt = M > 32 && (N + 47) / 48 * 48 < (N + 63) / 64 * 64 ? 3 : 4, mr = M > 32 ? 4 : 2;
+  const dim3 gt((N + 16 * nt - 1) / (16 * nt), (M + 16 * mr - 1) / (16 * mr));
   if (large && (long)gt.x * gt.y >= kGemmTiles) {
-    if (nt == 3)
-      hipLaunchKernelGGL(k_gemm_tile<3>, gt, dim3(256), 0, st, M, N, K, alpha, A, lda, (int)ta, B, ldb, (int)tb, beta,
+    if (mr == 2)
+      hipLaunchKernelGGL((k_gemm_tile<2, 4>), gt, dim3(256), 0, st, M, N, K, alpha, A, lda, (int)ta, B, ldb, (int)tb,
+                         beta, C, ldc);
+    else if (nt == 3)
+      hipLaunchKernelGGL((k_gemm_tile<4, 3>), gt, dim3(256), 0, st, M, N, K, alpha, A, lda, (int)ta, B, ldb, (int)tb, beta,
                          C, ldc);
     else
-      hipLaunchKernelGGL(k_gemm_tile<4>, gt, dim3(256), 0, st, M, N, K, alpha, A, lda, (int)ta, B, ldb, (int)tb, beta,
+      hipLaunchKernelGGL((k_gemm_tile<4, 4>), gt, dim3(256), 0, st, M, N, K, alpha, A, lda, (int)ta, B, ldb, (int)tb, beta,
                          C, ldc);
   } else if (large || K >= kGemmDeepK) {
     hipLaunchKernelGGL(k_gemm_deep, g, dim3(64 * kDeepWaves), 0, st, M, N, K, alpha, A, lda, (int)ta, B, ldb, (int)tb,
@@ -2236,11 +2241,21 @@ static int finish_energy_grad(vsvb_context* c, double* energy, double* grad) {
 // runs one shell-quartet pass whose thread blocks contract each ERI block with
 // every member's density; members alias the leader's geometry buffers and use
 // slices of the group's density / Coulomb / exchange arrays.
+// Members of a group (wave functions on one geometry) from which their J and K come
+// from stored integrals, and most memory for them.  32 wave functions of C8H18 took
+// 46.0 ms quartet by quartet and take 13.9 so: 4.3 for the integrals, 8.2 for passes
+// over the two 4 GB orders of the matrix that do not grow with the members, 1.5 for
+// the members' own algebra; at 8 members the two are about even.  A single C2H6 or
+// C3H8 wave function (0.70 and 1.19 ms) lost 7 and 10 % by it.
+constexpr int kStoredMembers = 8;
+constexpr size_t kStoredGroupBytes = (size_t)16 << 30;
+
 struct BatchGroup {
   std::vector<int> members;  // indices into vsvb_batch::ctx; members[0] leads
   DevBuf<double> dens, jacc, kacc;
   DevBuf<OrbArgs> orec;           // the members' orbital records, when they run in one workgroup each
   std::vector<OrbArgs> h_orec;
+  StoredIntegrals stored;         // of a group of many densities
 };
 
 // The first run of a batch is enqueued directly and then captured whole
@@ -2455,7 +2470,7 @@ static int batch_plan(vsvb_batch* b) {
         for (int gi : ch.groups) {
           BatchGroup& g = b->groups[gi];
           vsvb_context* lead = b->ctx[g.members[0]];
-          if (lead->npair > 0) continue;
+          if (lead->npair > 0 || g.stored.M.p) continue;  // (runs its own pass)
           const int nb = lead->pair_off[bc + 1] - lead->pair_off[bc], nk = lead->pair_off[kc + 1] - lead->pair_off[kc];
           if (nb <= 0 || nk <= 0) continue;
           const ClassLaunch& cl = lead->ljk[q];
@@ -2557,6 +2572,10 @@ static int group_front(vsvb_batch* b, BatchGroup& g, bool own) {
     return sc_enqueue(lead, true, lead->d_grad.p);
   }
   const int nwfn = (int)g.members.size();
+  if (g.stored.M.p) {
+    if ((rc = group_orbitals(b, g, 1))) return rc;
+    return stored_jk(lead, g.stored, nwfn, g.dens.p, g.jacc.p, g.kacc.p);
+  }
   if ((rc = group_orbitals(b, g, own ? 2 : 0))) return rc;
   if (!own) {
     const int nspin = lead->nunpd > 0 ? 2 : 1;
@@ -2821,7 +2840,7 @@ static int tune_batch(vsvb_batch* b) {
   double wmax = 0.0;
   for (auto& g : b->groups) {
     vsvb_context* l = b->ctx[g.members[0]];
-    if (l->npair > 0) continue;
+    if (l->npair > 0 || g.stored.M.p) continue;
     if (g.members.size() == 1) {
       if (!rep[0] && l->nbf == nbf1) rep[0] = &g;
     } else if (g.members.size() > kFewDensities) {
@@ -2840,7 +2859,7 @@ static int tune_batch(vsvb_batch* b) {
   }
   for (auto& g : b->groups) {
     const int k = g.members.size() > kFewDensities ? 1 : 0;
-    if (!rep[k]) continue;
+    if (!rep[k] || g.stored.M.p) continue;
     for (int i : g.members) {
       vsvb_context* c = b->ctx[i];
       if (c->npair > 0) continue;
@@ -3382,7 +3401,12 @@ int vsvb_batch_create(int32_t nwfn, const vsvb_system* const* systems, const vsv
   for (auto& g : bt->groups) {
     vsvb_context* lead = bt->ctx[g.members[0]];
     if (g.members.size() < 2) continue;
-    lead->ndens = (int)g.members.size();  // its work lists are planned with the first geometry
+    if ((int)g.members.size() >= kStoredMembers && lead->npair == 0 && lead->pair_chunk == 0) {
+      const int rc = stored_setup(lead, g.stored, (int)g.members.size(), lead->nunpd > 0 ? 2 : 1, kStoredGroupBytes);
+      if (rc) return rc;
+    }
+    // its work lists are planned with the first geometry
+    lead->ndens = g.stored.M.p ? 1 : (int)g.members.size();
     const size_t nn = (size_t)lead->nbf * lead->nbf;
     const int nspin = lead->nunpd > 0 ? 2 : 1;
     const size_t G = g.members.size();

@@ -98,6 +98,16 @@ struct FnPair {
   int mu, nu, same;
 };
 
+// The two-electron integrals of one geometry (vsvb_stored.hip); M null: not in use.
+struct StoredIntegrals {
+  DevBuf<double> M;   // [nfun][nfun] (ab|cd), rows and columns in the order of Pair::f0
+  DevBuf<FnPair> fn;  // [nfun] the functions of that list
+  DevBuf<int> at;     // [nt] the entry of functions mu >= nu, nt = nbf (nbf + 1) / 2
+  DevBuf<double> N;   // [nt][nt] (ab|cd) by functions
+  DevBuf<double> Dp, Jp;  // [nwfn][nt] Coulomb weights / Coulomb matrices of the densities
+  DevBuf<double> Dt;      // [nbf][nd][xp] densities, fastest index the density
+};
+
 // Spin-coupled determinant expansion (density_sc / dbra / dket,
 // src/valence.F90:1612-1870): determinant d = isc * 2^npair + mask has the
 // alpha list (pair slots, swapped where mask has the bit; unpaired; docc) and
@@ -113,9 +123,7 @@ struct SpinCoupled {
   DevBuf<int> d_pq;                      // [npq][2] unique orbital pairs (r >= s)
   DevBuf<double> d_cdet;                 // [ndet]
   DevBuf<double> d_pdens, d_pj;          // [npq][nbf][nbf] pair densities / their Coulomb matrices
-  // Integrals stored once for all pair densities (d_M null: contracted on the fly)
-  DevBuf<double> d_M;                    // [nfun][nfun] (ab|cd)
-  DevBuf<FnPair> d_fn;                   // [nfun] the functions of Pair::f0's list
+  StoredIntegrals stored;                // contracted with all pair densities (M null: contracted on the fly)
   DevBuf<double> d_Dp, d_Jp;             // [npq][nfun] packed pair densities / their Coulomb images
   DevBuf<double> d_W;                    // [npq][nbf][nsp]  J^{rs} C^T
   DevBuf<double> d_eri, d_erik;          // [nsp^2][nsp^2]   (pq|rs) and its exchange ordering
@@ -296,6 +304,12 @@ hipError_t launch_zero(hipStream_t st, void* p, size_t bytes);  // bytes: a mult
 hipError_t launch_gather_grad(vsvb_context* c, const double* gradC, double* grad);
 int prepare_geometry(vsvb_context* c, const double* coords);
 int prepare_orbital_basis(vsvb_context* c, const double* coeff_host, const double* coeff_dev);
+// Buffers for nwfn wave functions (nspin densities each; 0: the matrix only) if they
+// fit `limit` and a sixteenth of the free memory; otherwise s stays empty.
+int stored_setup(vsvb_context* c, StoredIntegrals& s, int nwfn, int nspin, size_t limit);
+int stored_integrals(vsvb_context* c, StoredIntegrals& s);  // M, fn and at of the current geometry
+// What run_quartets' J/K pass leaves in jacc and kacc, up to the order of the sums.
+int stored_jk(vsvb_context* c, StoredIntegrals& s, int nwfn, const double* dens, double* jacc, double* kacc);
 int run_quartets(vsvb_context* c, bool jk, int nwfn = 1, const double* dens = nullptr,
                  double* jacc = nullptr, double* kacc = nullptr, int nspin_override = -1, double* eri = nullptr);
 int finish_counters(vsvb_context* c, const unsigned long long* host_counters = nullptr);

@@ -54,34 +54,14 @@ __global__ void k_pair_dens(const double* __restrict__ Cs, const int* __restrict
 }
 
 // Stored integrals.  All npq pair densities meet the same integrals, so where
-// nfun^2 of them fit (kStoredBytes, and a sixteenth of the free memory, so that
-// many contexts leave room for the next) an energy pass writes each once and a product
+// nfun^2 of them fit an energy pass writes each once and a product
 // [npq x nfun] x [nfun x nfun] contracts them; H12's 78 densities took 4.4 ms
 // contracted quartet by quartet, an atomic per density and function pair, and
 // take 0.5 ms this way (0.36 of them the integrals).
 // Below kStoredMin densities the fixed cost (clearing, transposing and reading the
-// matrix, six small launches) is no longer small against what is saved.  The
-// functions of a pair lie a class apart, so that the 64 bra pairs of a wavefront
-// write 64 neighbours (with a pair's functions side by side (pp|ps) took 259 us
-// instead of 53).
+// matrix, six small launches) is no longer small against what is saved.
 constexpr size_t kStoredBytes = (size_t)1 << 30;
 constexpr int kStoredMin = 10;
-
-struct ClassOffsets {
-  int at[kNPairClass + 1];
-};
-__global__ void k_function_pairs(const Pair* __restrict__ pairs, ClassOffsets off, const Shell* __restrict__ shells,
-                                 FnPair* __restrict__ fn) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= off.at[kNPairClass]) return;
-  int cl = 0;
-  while (t >= off.at[cl + 1]) ++cl;
-  const Pair P = pairs[t];
-  const Shell A = shells[P.A], B = shells[P.B];
-  FnPair* f = fn + P.f0;
-  for (int i = 0; i < ncart(A.l); ++i)
-    for (int j = 0; j < ncart(B.l); ++j, f += off.at[cl + 1] - off.at[cl]) *f = FnPair{A.ao + i, B.ao + j, P.A == P.B};
-}
 
 // Dp[rs][f]: k_pair_dens' element (mu, nu), doubled where the pair stands for (nu, mu) too.
 __global__ void k_pair_dens_packed(const double* __restrict__ Cs, const int* __restrict__ pq, int npq, int nbf,
@@ -104,25 +84,6 @@ __global__ void k_unpack_coulomb(const double* __restrict__ Jp, const FnPair* __
     double* M = J + t / nfun * nn;
     M[(size_t)f.mu * nbf + f.nu] = Jp[t];
     if (!f.same) M[(size_t)f.nu * nbf + f.mu] = Jp[t];
-  }
-}
-
-// M = T + T^T in place, a workgroup per 32 x 32 tile on or below the diagonal and
-// its mirror image, through LDS so that both are read and written along rows.
-__global__ void __launch_bounds__(256) k_sym_tiles(double* __restrict__ M, int n) {
-  __shared__ double lo[32][33], up[32][33];
-  const int bi = blockIdx.y, bj = blockIdx.x, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  if (bj > bi) return;
-  for (int r = ty; r < 32; r += 8) {
-    const int i = bi * 32 + r, j = bj * 32 + tx, it = bj * 32 + r, jt = bi * 32 + tx;
-    lo[r][tx] = i < n && j < n ? M[(size_t)i * n + j] : 0.0;
-    up[r][tx] = it < n && jt < n ? M[(size_t)it * n + jt] : 0.0;
-  }
-  __syncthreads();
-  for (int r = ty; r < 32; r += 8) {
-    const int i = bi * 32 + r, j = bj * 32 + tx, it = bj * 32 + r, jt = bi * 32 + tx;
-    if (i < n && j < n) M[(size_t)i * n + j] = lo[r][tx] + up[tx][r];
-    if (bi != bj && it < n && jt < n) M[(size_t)it * n + jt] = up[r][tx] + lo[tx][r];
   }
 }
 
@@ -736,11 +697,12 @@ int vsvb::sc_setup(vsvb_context* c, const vsvb_system* s) {
   HIP_OK(sc.d_cdet.alloc(cd.size()));
   HIP_OK(sc.d_pq.alloc(pq.size()));
   const size_t nf = (size_t)c->nfun;
-  size_t free_bytes = 0, total_bytes = 0;
-  HIP_OK(hipMemGetInfo(&free_bytes, &total_bytes));
-  if (sc.npq >= kStoredMin && nf * nf * sizeof(double) <= std::min(kStoredBytes, free_bytes / 16)) {
-    HIP_OK(sc.d_M.alloc(nf * nf));
-    HIP_OK(sc.d_fn.alloc(nf));
+  if (sc.npq >= kStoredMin) {
+    const int rc = stored_setup(c, sc.stored, 0, 0, kStoredBytes);
+    if (rc) return rc;
+  }
+  if (sc.stored.M.p) {
+    c->ndens = 1;  // the quartet pass is an energy pass
     HIP_OK(sc.d_Dp.alloc(sc.npq * nf));
     HIP_OK(sc.d_Jp.alloc(sc.npq * nf));
   } else {
@@ -793,21 +755,14 @@ int vsvb::sc_enqueue(vsvb_context* c, bool want_grad, double* grad_dev) {
   const long P = sc.npairs;
   int rc;
   // orbital-pair Coulomb matrices from one pass over the screened shell quartets
-  if (sc.d_M.p) {
+  if (sc.stored.M.p) {
     const int nf = c->nfun;
-    const unsigned tiles = (unsigned)(nf + 31) / 32;
-    HIP_OK(launch_fill(st, sc.d_M.p, (size_t)nf * nf, 0.0));
-    if ((rc = run_quartets(c, false, 0, nullptr, nullptr, nullptr, 0, sc.d_M.p))) return rc;
-    hipLaunchKernelGGL(k_sym_tiles, dim3(tiles, tiles), dim3(256), 0, st, sc.d_M.p, nf);
-    ClassOffsets off;
-    std::copy(c->pair_off, c->pair_off + kNPairClass + 1, off.at);
-    hipLaunchKernelGGL(k_function_pairs, dim3((c->npairs + 255) / 256), dim3(256), 0, st, c->d_pairs.p, off,
-                       c->d_shells.p, sc.d_fn.p);
+    if ((rc = stored_integrals(c, sc.stored))) return rc;
     hipLaunchKernelGGL(k_pair_dens_packed, dim3(grid_for((size_t)sc.npq * nf)), dim3(256), 0, st, c->d_Cs.p, sc.d_pq.p,
-                       sc.npq, nbf, sc.d_fn.p, nf, sc.d_Dp.p);
+                       sc.npq, nbf, sc.stored.fn.p, nf, sc.d_Dp.p);
     HIP_OK(hipGetLastError());
-    HIP_OK(gemm(st, sc.npq, nf, nf, 1.0, sc.d_Dp.p, nf, false, sc.d_M.p, nf, false, 0.0, sc.d_Jp.p, nf));
-    hipLaunchKernelGGL(k_unpack_coulomb, dim3(grid_for((size_t)sc.npq * nf)), dim3(256), 0, st, sc.d_Jp.p, sc.d_fn.p,
+    HIP_OK(gemm(st, sc.npq, nf, nf, 1.0, sc.d_Dp.p, nf, false, sc.stored.M.p, nf, false, 0.0, sc.d_Jp.p, nf));
+    hipLaunchKernelGGL(k_unpack_coulomb, dim3(grid_for((size_t)sc.npq * nf)), dim3(256), 0, st, sc.d_Jp.p, sc.stored.fn.p,
                        sc.npq, nf, nbf, sc.d_pj.p);
     HIP_OK(hipGetLastError());
   } else {
