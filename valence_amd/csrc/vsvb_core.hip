@@ -1605,7 +1605,6 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   HIP_OK(device_buffer(c, c->d_angn, c->nbf));
   HIP_OK(device_buffer(c, c->d_ao_shell, c->nbf));
   HIP_OK(device_buffer(c, c->d_orb_start, s->norbs + 1));
-  HIP_OK(device_buffer(c, c->d_status, 4));
   HIP_OK(device_buffer(c, c->d_colk, std::max(1, c->nsp)));
   HIP_OK(device_buffer(c, c->d_ent, c->ent.size()));
   HIP_OK(device_buffer(c, c->d_coeff, std::max(1, s->totlen)));
@@ -1630,9 +1629,13 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   HIP_OK(device_buffer(c, c->d_Rfull, nbf2));
   HIP_OK(device_buffer(c, c->d_X, (size_t)c->nsp * c->nbf));
   HIP_OK(device_buffer(c, c->d_Z, (size_t)c->nsp * c->nbf));
-  HIP_OK(device_buffer(c, c->d_grad, std::max(1, s->totlen)));
-  HIP_OK(device_buffer(c, c->d_scal, 16));
-  HIP_OK(device_buffer(c, c->d_counters, kCounterWords));
+  // what a call reads back stands in one block: one copy instead of four, each
+  // some 10 us of a water energy's 220
+  HIP_OK(device_buffer(c, c->d_out, kOutGrad + std::max(1, s->totlen)));
+  c->d_scal.alias(reinterpret_cast<double*>(c->d_out.p), 16);
+  c->d_status.alias(reinterpret_cast<int*>(c->d_out.p + kOutStatus), 4);
+  c->d_counters.alias(c->d_out.p + kOutCounters, kCounterWords);
+  c->d_grad.alias(reinterpret_cast<double*>(c->d_out.p + kOutGrad), std::max(1, s->totlen));
   HIP_OK(device_buffer(c, c->d_stamps, (size_t)2 * kStampSlots * kNQuartetClass));
   // quartet launch geometry (grids sized to the occupancy of each class kernel) and partial buffer
   int ncu = 0;
@@ -2037,9 +2040,36 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
     }
     if (shared) HIP_OK(launch_small(s, dev, jk, st));
   }
+  // Two cooperative classes whose wavefronts all fit the chip at once share a
+  // launch: each runs as long as its longest quartet (water: 2 x 36 us one after the
+  // other, 46 side by side).
+  int pair[2] = {-1, -1};
+  {
+    int k = 0, blocks = 0, fit = 0;
+    for (int q = kNQuartetClass - 1; q >= 0 && k < 2; --q) {
+      const ClassLaunch& cl = jk ? c->ljk[q] : c->le[q];
+      if (!cl.coop || cl.units <= 0) continue;
+      pair[k] = q;
+      blocks += cl.blocks;
+      fit = k == 0 ? coop_occupancy(c->coop_idx[q], jk) : std::min(fit, coop_occupancy(c->coop_idx[q], jk));
+      ++k;
+    }
+    if (k < 2 || blocks > fit * c->ncu) pair[0] = pair[1] = -1;
+  }
+  if (pair[0] >= 0) {
+    QuartetArgs a[2];
+    for (int k = 0; k < 2; ++k) {
+      const int q = pair[k], bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
+      a[k] = class_args(c, bc, kc, jk ? c->ljk[q] : c->le[q], jk, nwfn, nspin, dens, jacc, kacc, c->d_partial.p + offs[q],
+                        eri);
+    }
+    const ClassLaunch *l = jk ? c->ljk : c->le;
+    HIP_OK(launch_coop_pair(c->coop_idx[pair[0]], a[0], l[pair[0]].blocks, c->coop_idx[pair[1]], a[1],
+                            l[pair[1]].blocks, jk, c->device, st));
+  }
   for (int t = 0; t < kNQuartetClass; ++t) {
     const int q = c->class_rev ? kNQuartetClass - 1 - t : t;
-    if (shared && c->in_small[m][q]) continue;
+    if ((shared && c->in_small[m][q]) || q == pair[0] || q == pair[1]) continue;
     const int bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
     const ClassLaunch& cl = jk ? c->ljk[q] : c->le[q];
     const int nb = c->work[bc][0].n, nk = c->work[kc][0].n;
@@ -2067,7 +2097,7 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
 // device.  Class times come from the kernels' wall-clock stamps (profiling on);
 // the stage time from the HIP events of a direct run, or, after a graph replay
 // (whose events were not recorded), from the stamps' overall span.
-int vsvb::finish_counters(vsvb_context* c, const unsigned long long* hcnt) {
+int vsvb::finish_counters(vsvb_context* c, const unsigned long long* hcnt, bool replayed) {
   if (!c->ran_quartets) {  // a batch-group member: its integrals were counted by the leader
     std::memset(c->class_stats, 0, sizeof(c->class_stats));
     std::memset(c->last_counters, 0, sizeof(c->last_counters));
@@ -2075,10 +2105,7 @@ int vsvb::finish_counters(vsvb_context* c, const unsigned long long* hcnt) {
   }
   c->ran_quartets = false;
   unsigned long long h[kCounterWords];
-  if (hcnt)
-    std::memcpy(h, hcnt, sizeof(h));
-  else
-    HIP_OK(hipMemcpy(h, c->d_counters.p, sizeof(h), hipMemcpyDeviceToHost));
+  std::memcpy(h, hcnt, sizeof(h));
   for (int s = 1; s < kCtrSlots; ++s)
     for (int k = 0; k < kCtrStride; ++k) h[k] += h[s * kCtrStride + k];
   const unsigned long long* stamp = h + kCtrSlots * kCtrStride;
@@ -2104,7 +2131,7 @@ int vsvb::finish_counters(vsvb_context* c, const unsigned long long* hcnt) {
     c->class_stats[q][5] = launched ? 1.0 : 0.0;
   }
   double ms = std::nan("");
-  if (!hcnt && c->ev_valid) {
+  if (!replayed && c->ev_valid) {
     float evms = 0.0f;
     HIP_OK(hipEventElapsedTime(&evms, c->ev0, c->ev1));
     ms = evms;
@@ -2118,10 +2145,18 @@ int vsvb::finish_counters(vsvb_context* c, const unsigned long long* hcnt) {
   return VSVB_OK;
 }
 
+int vsvb::fetch_out(vsvb_context* c, bool grad) {
+  const size_t words = kOutGrad + (grad ? (size_t)c->totlen : 0);
+  c->h_out.resize(words);
+  HIP_OK(hipMemcpyAsync(c->h_out.data(), c->d_out.p, words * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                        c->stream));
+  HIP_OK(hipStreamSynchronize(c->stream));
+  return VSVB_OK;
+}
+
 int vsvb::check_status(vsvb_context* c, bool for_grad) {
   int st[4];
-  HIP_OK(hipMemcpyAsync(st, c->d_status.p, sizeof(st), hipMemcpyDeviceToHost, c->stream));
-  HIP_OK(hipStreamSynchronize(c->stream));
+  std::memcpy(st, c->h_out.data() + kOutStatus, sizeof(st));
   if (st[0]) return fail(VSVB_ERR_NUMERIC, "orbital overlap block is not positive definite (linearly dependent orbitals)");
   if (st[2])
     return fail(VSVB_ERR_NUMERIC, "a transition overlap between two determinants of the spin-coupled expansion is "
@@ -2141,10 +2176,10 @@ static int enqueue_energy(vsvb_context* c, const double* coords, const double* c
 
 static int finish_energy(vsvb_context* c, double* energy, double* parts) {
   int rc;
-  double h[3];
-  HIP_OK(hipMemcpyAsync(h, c->d_scal.p, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+  if ((rc = fetch_out(c, false))) return rc;
+  const double* h = reinterpret_cast<const double*>(c->h_out.data());
   if ((rc = check_status(c, false))) return rc;
-  if ((rc = finish_counters(c))) return rc;
+  if ((rc = finish_counters(c, c->h_out.data() + kOutCounters))) return rc;
   if (!std::isfinite(h[2])) return fail(VSVB_ERR_NUMERIC, "non-finite energy");
   if (energy) *energy = h[2];
   if (parts) {
@@ -2222,11 +2257,11 @@ static int enqueue_energy_grad(vsvb_context* c, const double* coords, const doub
 
 static int finish_energy_grad(vsvb_context* c, double* energy, double* grad) {
   int rc;
-  double h[4];
-  HIP_OK(hipMemcpyAsync(h, c->d_scal.p, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-  if (grad) HIP_OK(hipMemcpyAsync(grad, c->d_grad.p, c->totlen * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  if ((rc = fetch_out(c, grad != nullptr))) return rc;
+  const double* h = reinterpret_cast<const double*>(c->h_out.data());
+  if (grad) std::memcpy(grad, h + kOutGrad, c->totlen * sizeof(double));
   if ((rc = check_status(c, true))) return rc;
-  if ((rc = finish_counters(c))) return rc;
+  if ((rc = finish_counters(c, c->h_out.data() + kOutCounters))) return rc;
   const double e = h[0] + h[3] + c->enuc;
   if (!std::isfinite(e)) return fail(VSVB_ERR_NUMERIC, "non-finite energy");
   if (energy) *energy = e;
@@ -2294,6 +2329,13 @@ struct LaneChunk {
   int l0 = 0, l1 = 0;       // its launches glaunch[l0, l1)
 };
 
+struct GatherItem {
+  const unsigned long long* out;  // vsvb_context::d_out
+  double enuc;
+  size_t goff;
+  int len, spin_coupled;
+};
+
 struct vsvb_batch {
   std::vector<vsvb_context*> ctx;
   std::vector<BatchGroup> groups;
@@ -2328,6 +2370,7 @@ struct vsvb_batch {
   hipGraphExec_t exec = nullptr;
   std::vector<size_t> goff;      // offset of each wave function's gradient in d_g
   std::vector<char> ran;         // the wave function ran the quartet stage itself (group leader)
+  DevBuf<GatherItem> d_items;
   DevBuf<double> d_e, d_g;
   DevBuf<int> d_st;
   DevBuf<unsigned long long> d_cnt;
@@ -2673,21 +2716,36 @@ static int batch_launch_stats(vsvb_batch* b) {
 }
 
 // Results of every wave function into the batch's gather arrays.
-static int batch_gather(vsvb_batch* b) {
-  hipStream_t st = b->stream;
+// One wave function's results for the arrays a replay reads back.
+__global__ void k_gather(const GatherItem* __restrict__ items, double* __restrict__ e, double* __restrict__ g,
+                         int* __restrict__ st, unsigned long long* __restrict__ cnt) {
+  const GatherItem x = items[blockIdx.x];
+  const double* scal = reinterpret_cast<const double*>(x.out);
+  const int* status = reinterpret_cast<const int*>(x.out + kOutStatus);
+  if (threadIdx.x == 0) e[blockIdx.x] = x.spin_coupled ? scal[2] : scal[0] + scal[3] + x.enuc;
+  if (threadIdx.x < 4) st[4 * blockIdx.x + threadIdx.x] = status[threadIdx.x];
+  for (int k = threadIdx.x; k < kCnt; k += blockDim.x) cnt[(size_t)kCnt * blockIdx.x + k] = x.out[kOutCounters + k];
+  for (int k = threadIdx.x; k < x.len; k += blockDim.x)
+    g[x.goff + k] = reinterpret_cast<const double*>(x.out + kOutGrad)[k];
+}
+
+// The items of the batch's geometries (the nuclear repulsion is one of their
+// numbers), uploaded before the capture that reads them.
+static int batch_gather_items(vsvb_batch* b) {
+  std::vector<GatherItem> items;
   for (size_t i = 0; i < b->ctx.size(); ++i) {
-    vsvb_context* c = b->ctx[i];
-    if (c->npair > 0) {
-      HIP_OK(hipMemcpyAsync(b->d_e.p + i, c->d_scal.p + 2, sizeof(double), hipMemcpyDeviceToDevice, st));
-    } else {
-      hipLaunchKernelGGL(k_final_energy, dim3(1), dim3(1), 0, st, c->d_scal.p, c->d_scal.p + 3, c->enuc, b->d_e.p + i);
-      HIP_OK(hipGetLastError());
-    }
-    HIP_OK(hipMemcpyAsync(b->d_st.p + 4 * i, c->d_status.p, 4 * sizeof(int), hipMemcpyDeviceToDevice, st));
-    HIP_OK(hipMemcpyAsync(b->d_g.p + b->goff[i], c->d_grad.p, c->totlen * sizeof(double), hipMemcpyDeviceToDevice, st));
-    HIP_OK(hipMemcpyAsync(b->d_cnt.p + kCnt * i, c->d_counters.p, kCnt * sizeof(unsigned long long),
-                          hipMemcpyDeviceToDevice, st));
+    const vsvb_context* c = b->ctx[i];
+    items.push_back(GatherItem{c->d_out.p, c->enuc, b->goff[i], c->totlen, c->npair > 0});
   }
+  HIP_OK(ensure_buffer(b->d_items, items.size()));
+  HIP_OK(hipMemcpy(b->d_items.p, items.data(), items.size() * sizeof(GatherItem), hipMemcpyHostToDevice));
+  return VSVB_OK;
+}
+
+static int batch_gather(vsvb_batch* b) {
+  hipLaunchKernelGGL(k_gather, dim3((unsigned)b->ctx.size()), dim3(256), 0, b->stream, b->d_items.p, b->d_e.p, b->d_g.p,
+                     b->d_st.p, b->d_cnt.p);
+  HIP_OK(hipGetLastError());
   return VSVB_OK;
 }
 
@@ -2880,8 +2938,9 @@ static int tune_batch(vsvb_batch* b) {
 }
 
 static int batch_capture(vsvb_batch* b) {
+  int rc = batch_gather_items(b);
+  if (rc) return rc;
   for (auto* c : b->ctx) c->capturing = true;
-  int rc = VSVB_OK;
   hipError_t e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
   if (e == hipSuccess) {
     rc = batch_enqueue(b);
@@ -2931,7 +2990,7 @@ static int batch_replay(vsvb_batch* b, int32_t want_grad, double* energies, doub
     if (want_grad && grads && grads[i]) std::memcpy(grads[i], b->h_g + b->goff[i], c->totlen * sizeof(double));
     c->ran_quartets = b->ran[i];
     int rc;
-    if ((rc = finish_counters(c, b->h_cnt + kCnt * i))) return rc;
+    if ((rc = finish_counters(c, b->h_cnt + kCnt * i, true))) return rc;
   }
   return VSVB_OK;
 }
@@ -3277,13 +3336,11 @@ int vsvb_energy_grad_device(vsvb_context* c, const double* coeff_device, double*
   HIP_OK(hipEventRecord(c->ev_out, c->stream));
   HIP_OK(hipStreamWaitEvent(caller, c->ev_out, 0));
   // numerical status (singular blocks, masked shells) is known only after the work ran
+  if ((rc = fetch_out(c, false))) return rc;
   if ((rc = check_status(c, true))) return rc;
-  if (c->npair > 0) {
-    int st3 = 0;
-    HIP_OK(hipMemcpy(&st3, c->d_status.p + 3, sizeof(int), hipMemcpyDeviceToHost));
-    if (st3) return fail(VSVB_ERR_UNSUPPORTED, "gradient at a singular spin-coupled transition overlap");
-  }
-  return finish_counters(c);
+  if (c->npair > 0 && reinterpret_cast<const int*>(c->h_out.data() + kOutStatus)[3])
+    return fail(VSVB_ERR_UNSUPPORTED, "gradient at a singular spin-coupled transition overlap");
+  return finish_counters(c, c->h_out.data() + kOutCounters);
 }
 
 int vsvb_debug_buffer(vsvb_context* c, const char* name, double* out, int64_t n) {

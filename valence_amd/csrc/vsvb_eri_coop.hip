@@ -49,7 +49,7 @@ __device__ __forceinline__ double pick3(int d, double x, double y, double z) { r
 
 template <bool kJK>
 __device__ __forceinline__ void coop_body(const QuartetArgs& a, const CoopDesc& d, const int* __restrict__ tab,
-                                          double* S) {
+                                          double* S, unsigned block = 0) {
   const int lane = threadIdx.x;
   const int NA = ncart(d.la), NB = ncart(d.lb), NC = ncart(d.lc), ND = ncart(d.ld);
   const int NAB = NA * NB, NCD = NC * ND;
@@ -309,7 +309,7 @@ __device__ __forceinline__ void coop_body(const QuartetArgs& a, const CoopDesc& 
         if (ww == w) s = esum[ww];
       s = wave_sum(s);
       if (lane == 0)
-        for (int k = 0; k < 4; ++k) a.partial[((size_t)blockIdx.x * 4 + k) * a.nwfn + w] = k == 0 ? s : 0.0;
+        for (int k = 0; k < 4; ++k) a.partial[((size_t)block * 4 + k) * a.nwfn + w] = k == 0 ? s : 0.0;
     }
   }
   stamp_wave(a.stamp, true);
@@ -320,7 +320,18 @@ __device__ __forceinline__ void coop_body(const QuartetArgs& a, const CoopDesc& 
 template <bool kJK>
 __global__ void __launch_bounds__(64) coop_kernel(QuartetArgs a, CoopDesc d, const int* __restrict__ tab) {
   extern __shared__ double S[];
-  coop_body<kJK>(a, d, tab, S);
+  coop_body<kJK>(a, d, tab, S, blockIdx.x);
+}
+
+// Two classes side by side: the first na workgroups take class a, the rest class b.
+template <bool kJK>
+__global__ void __launch_bounds__(64) coop_pair_kernel(QuartetArgs a, CoopDesc da, unsigned na, QuartetArgs b,
+                                                       CoopDesc db, const int* __restrict__ tab) {
+  extern __shared__ double S[];
+  if (blockIdx.x < na)
+    coop_body<kJK>(a, da, tab, S, blockIdx.x);
+  else
+    coop_body<kJK>(b, db, tab, S, blockIdx.x - na);
 }
 
 // J/K mode over several groups (molecules) of a batch in one launch: the
@@ -406,6 +417,21 @@ hipError_t launch_coop(int idx, const QuartetArgs& a, bool jk, int nblocks, int 
     hipLaunchKernelGGL(coop_kernel<true>, dim3(nblocks), dim3(64), lds, st, a, kCoopDesc[idx], t);
   else
     hipLaunchKernelGGL(coop_kernel<false>, dim3(nblocks), dim3(64), lds, st, a, kCoopDesc[idx], t);
+  return hipGetLastError();
+}
+
+hipError_t launch_coop_pair(int ia, const QuartetArgs& a, int na, int ib, const QuartetArgs& b, int nb, bool jk,
+                            int device, hipStream_t st) {
+  const int* t = nullptr;
+  const hipError_t e = coop_tables(device, &t);
+  if (e != hipSuccess) return e;
+  const size_t lds = std::max(coop_lds_bytes(ia, jk), coop_lds_bytes(ib, jk));
+  if (jk)
+    hipLaunchKernelGGL(coop_pair_kernel<true>, dim3(na + nb), dim3(64), lds, st, a, kCoopDesc[ia], (unsigned)na, b,
+                       kCoopDesc[ib], t);
+  else
+    hipLaunchKernelGGL(coop_pair_kernel<false>, dim3(na + nb), dim3(64), lds, st, a, kCoopDesc[ia], (unsigned)na, b,
+                       kCoopDesc[ib], t);
   return hipGetLastError();
 }
 

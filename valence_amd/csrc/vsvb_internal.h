@@ -21,6 +21,7 @@ constexpr size_t kMaxLdsK = 60 * 1024;
 // {evaluated, primitive quartets, skipped, spare}, then per class {earliest
 // start, latest end} stamps.
 constexpr int kCounterWords = kCtrSlots * kCtrStride + 2 * kNQuartetClass;
+constexpr int kOutStatus = 16, kOutCounters = kOutStatus + 2, kOutGrad = kOutCounters + kCounterWords;  // words of d_out
 
 extern thread_local std::string g_last_error;
 int fail(int code, const std::string& msg);
@@ -262,6 +263,8 @@ struct vsvb_context {
   DevBuf<double> d_coeff, d_ndf_scale, d_S, d_H, d_Ct, d_Cs, d_Sorb, d_Horb, d_P, d_R, d_tmp, d_tmp2;
   DevBuf<double> d_partial, d_scal, d_J, d_K, d_F, d_gradC, d_grad, d_Jsym, d_Rfull, d_X, d_Z;
   DevBuf<unsigned long long> d_counters;
+  DevBuf<unsigned long long> d_out;  // d_scal, d_status, d_counters and d_grad, one after the other (kOut...)
+  std::vector<unsigned long long> h_out;
   DevBuf<int> d_tilectr;  // work counters: class q owns [ctr_off[q], ctr_off[q] + ctr_len[q])
   int ctr_off[vsvb::kNQuartetClass] = {0}, ctr_len[vsvb::kNQuartetClass] = {0};
   int ctr_total = 0;
@@ -312,7 +315,8 @@ int stored_integrals(vsvb_context* c, StoredIntegrals& s);  // M, fn and at of t
 int stored_jk(vsvb_context* c, StoredIntegrals& s, int nwfn, const double* dens, double* jacc, double* kacc);
 int run_quartets(vsvb_context* c, bool jk, int nwfn = 1, const double* dens = nullptr,
                  double* jacc = nullptr, double* kacc = nullptr, int nspin_override = -1, double* eri = nullptr);
-int finish_counters(vsvb_context* c, const unsigned long long* host_counters = nullptr);
+int fetch_out(vsvb_context* c, bool grad);  // the call's results into h_out, after everything on its stream
+int finish_counters(vsvb_context* c, const unsigned long long* host_counters, bool replayed = false);
 int check_status(vsvb_context* c, bool for_grad);
 
 hipError_t launch_orbital_front(hipStream_t st, const OrbArgs& one, const OrbArgs* recs, int nrec, const ZeroArgs& z);
@@ -328,6 +332,8 @@ hipError_t coop_prepare(int device);              // step tables resident on the
 hipError_t launch_coop(int idx, const QuartetArgs& a, bool jk, int nblocks, int device, hipStream_t st);
 // J/K mode over ng groups' arguments (device array gs) in one launch; stamp: the
 // launch's wall-clock slots or null
+hipError_t launch_coop_pair(int ia, const QuartetArgs& a, int na, int ib, const QuartetArgs& b, int nb, bool jk,
+                            int device, hipStream_t st);
 hipError_t launch_coop_groups(int idx, const QuartetArgs* gs, int ng, int nblocks, int device,
                               unsigned long long* stamp, hipStream_t st);
 

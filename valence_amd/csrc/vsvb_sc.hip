@@ -893,19 +893,14 @@ int vsvb::sc_matrices(vsvb_context* c, double* ham, double* ovl) {
 
 int vsvb::sc_finish(vsvb_context* c, double* energy, double* parts, double* grad_host) {
   int rc;
-  double h[6];
-  HIP_OK(hipMemcpyAsync(h, c->d_scal.p, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-  if (grad_host)
-    HIP_OK(hipMemcpyAsync(grad_host, c->d_grad.p, c->totlen * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  if ((rc = fetch_out(c, grad_host != nullptr))) return rc;
+  const double* h = reinterpret_cast<const double*>(c->h_out.data());
+  if (grad_host) std::memcpy(grad_host, h + kOutGrad, c->totlen * sizeof(double));
   if ((rc = check_status(c, grad_host != nullptr))) return rc;
-  if (grad_host) {
-    int st3 = 0;
-    HIP_OK(hipMemcpy(&st3, c->d_status.p + 3, sizeof(int), hipMemcpyDeviceToHost));
-    if (st3)
-      return fail(VSVB_ERR_UNSUPPORTED, "gradient at a singular or nearly singular transition overlap of the "
-                                        "spin-coupled expansion (pivot ratio below 1e-9); the energy is exact there");
-  }
-  if ((rc = finish_counters(c))) return rc;
+  if (grad_host && reinterpret_cast<const int*>(c->h_out.data() + kOutStatus)[3])
+    return fail(VSVB_ERR_UNSUPPORTED, "gradient at a singular or nearly singular transition overlap of the "
+                                      "spin-coupled expansion (pivot ratio below 1e-9); the energy is exact there");
+  if ((rc = finish_counters(c, c->h_out.data() + kOutCounters))) return rc;
   if (!std::isfinite(h[2])) return fail(VSVB_ERR_NUMERIC, "non-finite energy");
   if (energy) *energy = h[2];
   if (parts) {
