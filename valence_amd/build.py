@@ -19,7 +19,7 @@ LIB = os.path.join(HERE, "libvsvb_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-SOURCES = ["vsvb_eri_small.hip", "vsvb_core.hip", "vsvb_orbital.hip", "vsvb_stored.hip", "vsvb_sc.hip", "vsvb_eri_coop.hip"] + [f"vsvb_eri_b{b}.hip" for b in range(6)]
+SOURCES = ["vsvb_eri_small.hip", "vsvb_core.hip", "vsvb_pairs.hip", "vsvb_orbital.hip", "vsvb_stored.hip", "vsvb_sc.hip", "vsvb_eri_coop.hip"] + [f"vsvb_eri_b{b}.hip" for b in range(6)]
 ERI_HEADERS = ["vsvb_device.h", "vsvb_eri_kernels.h", "eri_gen.inc", "coop_tables.inc"]
 HOST_HEADERS = ["vsvb_internal.h", "eri_flops.inc", os.path.join("..", "..", "include", "vsvb_hip.h")]
 

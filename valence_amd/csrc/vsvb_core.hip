@@ -123,70 +123,6 @@ static std::vector<double> make_boys_table() {
 // device: geometry preparation
 // ---------------------------------------------------------------------------
 
-__global__ void k_pair_prep(const PPSrc* __restrict__ src, int npp, const Shell* __restrict__ shells,
-                            const double* __restrict__ pexp, const double* __restrict__ pcoef,
-                            const double* __restrict__ xyz, double kfold, PrimPair* __restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= npp) return;
-  const PPSrc s = src[t];
-  const Shell A = shells[s.sA], B = shells[s.sB];
-  const double Ax = xyz[3 * A.atom], Ay = xyz[3 * A.atom + 1], Az = xyz[3 * A.atom + 2];
-  const double Bx = xyz[3 * B.atom], By = xyz[3 * B.atom + 1], Bz = xyz[3 * B.atom + 2];
-  const double a = pexp[s.ia], b = pexp[s.ib], p = a + b, rp = 1.0 / p;
-  const double ABx = Ax - Bx, ABy = Ay - By, ABz = Az - Bz;
-  PrimPair o;
-  o.p = p;
-  o.oo2p = 0.5 * rp;
-  o.Px = (a * Ax + b * Bx) * rp;
-  o.Py = (a * Ay + b * By) * rp;
-  o.Pz = (a * Az + b * Bz) * rp;
-  o.PAx = o.Px - Ax;
-  o.PAy = o.Py - Ay;
-  o.PAz = o.Pz - Az;
-  o.K = pcoef[s.ia] * pcoef[s.ib] * exp(-a * b * rp * (ABx * ABx + ABy * ABy + ABz * ABz)) * rp * kfold;
-  o.pad = 0.0;
-  out[t] = o;
-}
-
-__global__ void k_pair_geom(Pair* __restrict__ pairs, int np, const Shell* __restrict__ shells,
-                            const double* __restrict__ xyz) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= np) return;
-  const Shell A = shells[pairs[t].A], B = shells[pairs[t].B];
-  pairs[t].ABx = xyz[3 * A.atom] - xyz[3 * B.atom];
-  pairs[t].ABy = xyz[3 * A.atom + 1] - xyz[3 * B.atom + 1];
-  pairs[t].ABz = xyz[3 * A.atom + 2] - xyz[3 * B.atom + 2];
-}
-
-// Primitive-pair screening: keep a shell pair's primitive pairs with
-// |K_ab| > kPrimCut (K carries the contraction weights and exp(-ab/(a+b) |AB|^2)),
-// compacted to the front in their original order; the pair's npp becomes the
-// kept count.  A dropped primitive pair changes any ERI by less than
-// kPrimCut * (the largest K) * (a bounded Boys/angular factor).  Measured: at
-// 1e-14 every energy of the oracle fixtures (C8H18, C12H26, H12, LiF8, the
-// reference's inputs) is the same as at 1e-20 to 1e-13 Eh, and the C8H18 J/K
-// pass drops 10% of its primitive quartets' time; 1e-13 starts to move
-// C12H26's energy (7e-12 Eh).  K does not depend on the orbital weights, so the
-// weight gradient stays the exact derivative of the screened energy.
-constexpr double kPrimCut = 1e-14;
-
-__global__ void k_prim_screen(Pair* __restrict__ pairs, int np, const Shell* __restrict__ shells,
-                              PrimPair* __restrict__ pp) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= np) return;
-  Pair P = pairs[t];
-  const int cap = shells[P.A].nprim * shells[P.B].nprim;
-  int k = 0;
-  for (int i = 0; i < cap; ++i) {
-    const PrimPair q = pp[P.pp0 + i];
-    if (fabs(q.K) > kPrimCut) {
-      if (k != i) pp[P.pp0 + k] = q;
-      ++k;
-    }
-  }
-  pairs[t].npp = k;
-}
-
 // Segments of the shell pairs: consecutive parts of a pair's screened primitive
 // list, each a work pair of its own (the contracted integral is the sum over
 // bra segments x ket segments, and the contraction with the densities is linear
@@ -203,209 +139,6 @@ __global__ void k_split(const Pair* __restrict__ pairs, const SegSrc* __restrict
   P.npp = e - b;
   P.seg = s.seg;
   out[t] = P;
-}
-
-// ---------------------------------------------------------------------------
-// device: one-electron integrals (Obara-Saika), one wavefront per shell pair
-// ---------------------------------------------------------------------------
-// cartesian tuples of total order 0..4 in CCA order, cumulative index
-__device__ __forceinline__ constexpr int cart_off(int l) { return l * (l + 1) * (l + 2) / 6; }
-__device__ __forceinline__ constexpr int cart_idx(int lx, int ly, int lz) {
-  return cart_off(lx + ly + lz) + ((ly + lz) * (ly + lz + 1)) / 2 + lz;
-}
-__device__ __forceinline__ void cart_of(int l, int c, int& lx, int& ly, int& lz) {
-  int i = 0;
-  while ((i + 1) * (i + 2) / 2 <= c) ++i;
-  const int j = c - i * (i + 1) / 2;
-  lx = l - i;
-  ly = i - j;
-  lz = j;
-}
-
-// The lanes of the wavefront take the (primitive pair, nuclear centre) items of
-// the pair in turn; the item of centre 0 also adds the primitive pair's overlap
-// and kinetic terms.  Lane sums are reduced across the wavefront at the end.
-template <int LA, int LB>
-__global__ void __launch_bounds__(256) k_one_e(const Pair* __restrict__ pairs, int p0, int np,
-                                               const Shell* __restrict__ shells, const double* __restrict__ pexp,
-                                               const double* __restrict__ pcoef, const double* __restrict__ xyz,
-                                               const double* __restrict__ charge, int natom,
-                                               const double* __restrict__ boys, double* __restrict__ S,
-                                               double* __restrict__ H, int nbf) {
-  constexpr int NA = ncart(LA), NB = ncart(LB), L = LA + LB;
-  constexpr int NE = cart_off(L + 1);        // cartesians of order 0..L
-  constexpr int NBc = cart_off(LB + 1);      // cartesians of order 0..LB
-  const int t = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)));
-  const int lane = threadIdx.x & 63;
-  if (t >= np) return;  // whole wavefront
-  const Pair PR = pairs[p0 + t];
-  const Shell A = shells[PR.A], B = shells[PR.B];
-  const double Ax = xyz[3 * A.atom], Ay = xyz[3 * A.atom + 1], Az = xyz[3 * A.atom + 2];
-  const double Bx = xyz[3 * B.atom], By = xyz[3 * B.atom + 1], Bz = xyz[3 * B.atom + 2];
-  const double AB[3] = {Ax - Bx, Ay - By, Az - Bz};
-  double s[NA * NB], tk[NA * NB], v[NA * NB];
-#pragma unroll
-  for (int k = 0; k < NA * NB; ++k) s[k] = tk[k] = v[k] = 0.0;
-  const int nitem = A.nprim * B.nprim * natom;
-  for (int item = lane; item < nitem; item += 64) {
-    const int ipp = item / natom, c = item - ipp * natom;
-    const int ia = ipp / B.nprim, ib = ipp - ia * B.nprim;
-    {
-      const double a = pexp[A.prim0 + ia], b = pexp[B.prim0 + ib], p = a + b, rp = 1.0 / p;
-      const double mu = a * b * rp;
-      const double cc = pcoef[A.prim0 + ia] * pcoef[B.prim0 + ib];
-      const double Pc[3] = {(a * Ax + b * Bx) * rp, (a * Ay + b * By) * rp, (a * Az + b * Bz) * rp};
-      const double PA[3] = {Pc[0] - Ax, Pc[1] - Ay, Pc[2] - Az};
-      const double PB[3] = {Pc[0] - Bx, Pc[1] - By, Pc[2] - Bz};
-      if (c == 0) {
-      // 1D overlaps, i <= LA, j <= LB + 2
-      double S1[3][LA + 1][LB + 3];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        S1[d][0][0] = sqrt(M_PI * rp) * exp(-mu * AB[d] * AB[d]);
-#pragma unroll
-        for (int i = 0; i <= LA; ++i)
-#pragma unroll
-          for (int j = 0; j <= LB + 2; ++j) {
-            if (i == 0 && j == 0) continue;
-            double val;
-            if (i > 0) {
-              val = PA[d] * S1[d][i - 1][j];
-              if (i > 1) val += (i - 1) * 0.5 * rp * S1[d][i - 2][j];
-              if (j > 0) val += j * 0.5 * rp * S1[d][i - 1][j - 1];
-            } else {
-              val = PB[d] * S1[d][i][j - 1];
-              if (j > 1) val += (j - 1) * 0.5 * rp * S1[d][i][j - 2];
-            }
-            S1[d][i][j] = val;
-          }
-      }
-#pragma unroll
-      for (int ca = 0; ca < NA; ++ca)
-#pragma unroll
-        for (int cb = 0; cb < NB; ++cb) {
-          int ax, ay, az, bx, by, bz;
-          cart_of(LA, ca, ax, ay, az);
-          cart_of(LB, cb, bx, by, bz);
-          const int ai[3] = {ax, ay, az}, bj[3] = {bx, by, bz};
-          double sv[3], tv[3];
-#pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            const int i = ai[d], j = bj[d];
-            sv[d] = S1[d][i][j];
-            const double km = j >= 2 ? S1[d][i][j - 2] : 0.0;
-            tv[d] = -0.5 * (j * (j - 1) * km - 2.0 * b * (2 * j + 1) * sv[d] + 4.0 * b * b * S1[d][i][j + 2]);
-          }
-          s[ca * NB + cb] += cc * sv[0] * sv[1] * sv[2];
-          tk[ca * NB + cb] += cc * (tv[0] * sv[1] * sv[2] + sv[0] * tv[1] * sv[2] + sv[0] * sv[1] * tv[2]);
-        }
-      }
-      // nuclear attraction of centre c: VRR [e|0]^(m), |e| <= L, then HRR to [a|b]
-      const double pre = 2.0 * M_PI * rp * exp(-mu * (AB[0] * AB[0] + AB[1] * AB[1] + AB[2] * AB[2])) * cc;
-      {
-        const double Z = charge[c];
-        if (fabs(Z) <= 1e-12) continue;  // int1e skips |Z| <= 1e-12 (valence.F90:3146)
-        const double PC[3] = {Pc[0] - xyz[3 * c], Pc[1] - xyz[3 * c + 1], Pc[2] - xyz[3 * c + 2]};
-        double F[L + 1];
-        boys_eval<L>(p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]), boys, F);
-        double Vm[L + 1][NE];
-#pragma unroll
-        for (int m = 0; m <= L; ++m) Vm[m][0] = -Z * pre * F[m];
-#pragma unroll
-        for (int l = 1; l <= L; ++l)
-#pragma unroll
-          for (int c2 = 0; c2 < ncart(l); ++c2) {
-            int ex, ey, ez;
-            cart_of(l, c2, ex, ey, ez);
-            const int e[3] = {ex, ey, ez};
-            const int i = ex > 0 ? 0 : (ey > 0 ? 1 : 2);
-            int e1[3] = {ex, ey, ez};
-            e1[i] -= 1;
-            const int i1 = cart_idx(e1[0], e1[1], e1[2]);
-            const int nn = e1[i];
-            int i2 = 0;
-            if (nn > 0) {
-              int e2[3] = {e1[0], e1[1], e1[2]};
-              e2[i] -= 1;
-              i2 = cart_idx(e2[0], e2[1], e2[2]);
-            }
-            const int ie = cart_off(l) + c2;
-#pragma unroll
-            for (int m = 0; m <= L - l; ++m) {
-              double val = PA[i] * Vm[m][i1] - PC[i] * Vm[m + 1][i1];
-              if (nn > 0) val += nn * 0.5 * rp * (Vm[m][i2] - Vm[m + 1][i2]);
-              Vm[m][ie] = val;
-            }
-            (void)e;
-          }
-        // HRR on b: W[e][b] = W[e+1_i][b-1_i] + AB_i W[e][b-1_i]
-        double W[NE][NBc];
-#pragma unroll
-        for (int ie = 0; ie < NE; ++ie) W[ie][0] = Vm[0][ie];
-#pragma unroll
-        for (int lb = 1; lb <= LB; ++lb)
-#pragma unroll
-          for (int cbb = 0; cbb < ncart(lb); ++cbb) {
-            int bx, by, bz;
-            cart_of(lb, cbb, bx, by, bz);
-            const int i = bx > 0 ? 0 : (by > 0 ? 1 : 2);
-            int b1[3] = {bx, by, bz};
-            b1[i] -= 1;
-            const int ib1 = cart_idx(b1[0], b1[1], b1[2]);
-            const int ibb = cart_off(lb) + cbb;
-#pragma unroll
-            for (int le = 0; le <= L - lb; ++le)
-#pragma unroll
-              for (int ce = 0; ce < ncart(le); ++ce) {
-                int ex, ey, ez;
-                cart_of(le, ce, ex, ey, ez);
-                int ep[3] = {ex, ey, ez};
-                ep[i] += 1;
-                const int iep = cart_idx(ep[0], ep[1], ep[2]);
-                const int iee = cart_off(le) + ce;
-                W[iee][ibb] = W[iep][ib1] + AB[i] * W[iee][ib1];
-              }
-          }
-#pragma unroll
-        for (int ca = 0; ca < NA; ++ca)
-#pragma unroll
-          for (int cb = 0; cb < NB; ++cb) v[ca * NB + cb] += W[cart_off(LA) + ca][cart_off(LB) + cb];
-      }
-    }
-  }
-#pragma unroll
-  for (int ca = 0; ca < NA; ++ca)
-#pragma unroll
-    for (int cb = 0; cb < NB; ++cb) {
-      const double sv = vsvb::wave_sum(s[ca * NB + cb]), hv = vsvb::wave_sum(tk[ca * NB + cb] + v[ca * NB + cb]);
-      if (lane == 0) {
-        const int mu = A.ao + ca, nu = B.ao + cb;
-        S[(size_t)mu * nbf + nu] = sv;
-        S[(size_t)nu * nbf + mu] = sv;
-        H[(size_t)mu * nbf + nu] = hv;
-        H[(size_t)nu * nbf + mu] = hv;
-      }
-    }
-}
-
-static hipError_t launch_one_e(int pc, const Pair* pairs, int p0, int np, const Shell* shells, const double* pexp,
-                               const double* pcoef, const double* xyz, const double* charge, int natom,
-                               const double* boys, double* S, double* H, int nbf, hipStream_t st) {
-  if (np <= 0) return hipSuccess;
-  const dim3 g((np + 3) / 4), b(256);  // one wavefront per shell pair
-#define LAUNCH(LA, LB) \
-  hipLaunchKernelGGL((k_one_e<LA, LB>), g, b, 0, st, pairs, p0, np, shells, pexp, pcoef, xyz, charge, natom, boys, S, H, nbf)
-  switch (pc) {
-    case 0: LAUNCH(0, 0); break;
-    case 1: LAUNCH(1, 0); break;
-    case 2: LAUNCH(1, 1); break;
-    case 3: LAUNCH(2, 0); break;
-    case 4: LAUNCH(2, 1); break;
-    case 5: LAUNCH(2, 2); break;
-    default: return hipErrorInvalidValue;
-  }
-#undef LAUNCH
-  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -1046,19 +779,6 @@ static bool straight_allowed(const vsvb_context* c, int q, bool jk, bool tr) {
   return straight_spills()[q * 3 + (jk ? (tr ? 2 : 1) : 0)] <= kMaxSpillPerLane;
 }
 
-static hipError_t launch_schwarz(int pc, Pair* pairs, const PrimPair* pp, const double* boys, int p0, int np,
-                                 hipStream_t st) {
-  switch (pc) {
-    case 0: return launch_schwarz_b0(pairs, pp, boys, p0, np, st);
-    case 1: return launch_schwarz_b1(pairs, pp, boys, p0, np, st);
-    case 2: return launch_schwarz_b2(pairs, pp, boys, p0, np, st);
-    case 3: return launch_schwarz_b3(pairs, pp, boys, p0, np, st);
-    case 4: return launch_schwarz_b4(pairs, pp, boys, p0, np, st);
-    case 5: return launch_schwarz_b5(pairs, pp, boys, p0, np, st);
-  }
-  return hipErrorInvalidValue;
-}
-
 static int quartet_class_index(int bc, int kc) { return bc * (bc + 1) / 2 + kc; }
 
 static int class_parts(int q, bool jk) { return jk ? kPartsJk[q] : kPartsEnergy[q]; }
@@ -1519,14 +1239,11 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
     return x.r2 < y.r2;
   });
   std::vector<Pair> pairs(hp.size());
-  std::vector<PPSrc> ppsrc;
+  c->npp = 0;
   for (size_t i = 0; i < hp.size(); ++i) {
     pairs[i] = hp[i].p;
-    pairs[i].pp0 = (int)ppsrc.size();
-    const Shell& A = shells[pairs[i].A];
-    const Shell& B = shells[pairs[i].B];
-    for (int ia = 0; ia < A.nprim; ++ia)
-      for (int ib = 0; ib < B.nprim; ++ib) ppsrc.push_back(PPSrc{pairs[i].A, pairs[i].B, A.prim0 + ia, B.prim0 + ib});
+    pairs[i].pp0 = c->npp;
+    c->npp += pairs[i].npp;
   }
   for (int cl = 0; cl <= kNPairClass; ++cl) c->pair_off[cl] = 0;
   for (auto& h : hp) c->pair_off[h.cls + 1]++;
@@ -1534,7 +1251,6 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   c->npairs = (int)pairs.size();
   c->nfun = 0;
   for (const Pair& P : pairs) c->nfun += ncart(shells[P.A].l) * ncart(shells[P.B].l);
-  c->npp = (int)ppsrc.size();
   c->h_shells = shells;
   c->h_pairs = pairs;
   c->h_pexp = pexp;
@@ -1595,7 +1311,6 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   const size_t nbf2 = (size_t)c->nbf * c->nbf;
   HIP_OK(device_buffer(c, c->d_shells, c->nsh));
   HIP_OK(device_buffer(c, c->d_pairs, c->npairs));
-  HIP_OK(device_buffer(c, c->d_ppsrc, c->npp));
   HIP_OK(device_buffer(c, c->d_pp, c->npp));
   HIP_OK(device_buffer(c, c->d_pexp, pexp.size()));
   HIP_OK(device_buffer(c, c->d_pcoef, pcoef.size()));
@@ -1710,7 +1425,6 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   static const std::vector<double> boys = make_boys_table();  // the same in every context
   HIP_OK(hipMemcpy(c->d_shells.p, shells.data(), shells.size() * sizeof(Shell), hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(c->d_pairs.p, pairs.data(), pairs.size() * sizeof(Pair), hipMemcpyHostToDevice));
-  HIP_OK(hipMemcpy(c->d_ppsrc.p, ppsrc.data(), ppsrc.size() * sizeof(PPSrc), hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(c->d_pexp.p, pexp.data(), pexp.size() * sizeof(double), hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(c->d_pcoef.p, pcoef.data(), pcoef.size() * sizeof(double), hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(c->d_charge.p, c->charges.data(), c->natom * sizeof(double), hipMemcpyHostToDevice));
@@ -1795,22 +1509,11 @@ int vsvb::prepare_geometry(vsvb_context* c, const double* coords) {
   c->enuc = nuclear_repulsion(c->natom, c->coords.data(), c->charges.data());
   if (!c->capturing)
     HIP_OK(hipMemcpyAsync(c->d_xyz.p, c->coords.data(), 3 * c->natom * sizeof(double), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_pair_geom, dim3((c->npairs + 255) / 256), dim3(256), 0, st, c->d_pairs.p, c->npairs,
-                     c->d_shells.p, c->d_xyz.p);
-  HIP_OK(hipGetLastError());
-  const double kfold = std::sqrt(2.0 * std::pow(M_PI, 2.5));
-  hipLaunchKernelGGL(k_pair_prep, dim3((c->npp + 255) / 256), dim3(256), 0, st, c->d_ppsrc.p, c->npp,
-                     c->d_shells.p, c->d_pexp.p, c->d_pcoef.p, c->d_xyz.p, kfold, c->d_pp.p);
-  HIP_OK(hipGetLastError());
-  hipLaunchKernelGGL(k_prim_screen, dim3((c->npairs + 255) / 256), dim3(256), 0, st, c->d_pairs.p, c->npairs,
-                     c->d_shells.p, c->d_pp.p);
-  HIP_OK(hipGetLastError());
-  for (int pc = 0; pc < kNPairClass; ++pc) {
-    const int p0 = c->pair_off[pc], np = c->pair_off[pc + 1] - p0;
-    HIP_OK(launch_one_e(pc, c->d_pairs.p, p0, np, c->d_shells.p, c->d_pexp.p, c->d_pcoef.p, c->d_xyz.p,
-                        c->d_charge.p, c->natom, c->d_boys.p, c->d_S.p, c->d_H.p, c->nbf, st));
-    HIP_OK(launch_schwarz(pc, c->d_pairs.p, c->d_pp.p, c->d_boys.p, p0, np, st));
-  }
+  PairArgs a{c->d_pairs.p, c->d_shells.p, c->d_pexp.p, c->d_pcoef.p, c->d_xyz.p, c->d_charge.p, c->d_boys.p,
+             c->d_pp.p,    c->d_S.p,      c->d_H.p,    std::sqrt(2.0 * std::pow(M_PI, 2.5)),    c->natom,
+             c->nbf,       {}};
+  std::copy(c->pair_off, c->pair_off + kNPairClass + 1, a.off);
+  HIP_OK(launch_pairs(a, st));
   if (!c->h_seg.empty()) {
     const int ns = (int)c->h_seg.size();
     hipLaunchKernelGGL(k_split, dim3((ns + 255) / 256), dim3(256), 0, st, c->d_pairs.p, c->d_segsrc.p, ns, c->d_split.p);
@@ -3014,7 +2717,6 @@ static bool same_molecule(const vsvb_system* a, const vsvb_system* b) {
 static void share_geometry(vsvb_context* lead, vsvb_context* m) {
   m->d_shells.alias(lead->d_shells.p, lead->d_shells.n);
   m->d_pairs.alias(lead->d_pairs.p, lead->d_pairs.n);
-  m->d_ppsrc.alias(lead->d_ppsrc.p, lead->d_ppsrc.n);
   m->d_pp.alias(lead->d_pp.p, lead->d_pp.n);
   m->d_pexp.alias(lead->d_pexp.p, lead->d_pexp.n);
   m->d_pcoef.alias(lead->d_pcoef.p, lead->d_pcoef.n);

@@ -40,10 +40,4 @@ size_t scratch_b2(int kc, bool jk, bool tr) {
   }
 }
 
-hipError_t launch_schwarz_b2(Pair* pairs, const PrimPair* pp, const double* boys, int p0, int np, hipStream_t st) {
-  if (np <= 0) return hipSuccess;
-  hipLaunchKernelGGL((schwarz_kernel<1, 1>), dim3((np + 3) / 4), dim3(256), 0, st, pairs, pp, boys, p0, np);
-  return hipGetLastError();
-}
-
 }  // namespace vsvb

@@ -46,10 +46,4 @@ size_t scratch_b5(int kc, bool jk, bool tr) {
   }
 }
 
-hipError_t launch_schwarz_b5(Pair* pairs, const PrimPair* pp, const double* boys, int p0, int np, hipStream_t st) {
-  if (np <= 0) return hipSuccess;
-  hipLaunchKernelGGL((schwarz_kernel<2, 2>), dim3((np + 3) / 4), dim3(256), 0, st, pairs, pp, boys, p0, np);
-  return hipGetLastError();
-}
-
 }  // namespace vsvb

@@ -943,33 +943,6 @@ __global__ void __launch_bounds__(256) quartet_jk_groups_kernel(const QuartetArg
   stamp_wave(stamp, true);
 }
 
-// Schwarz bound of every pair of one class, Q = sqrt(max_ab |(ab|ab)|): one
-// wavefront per pair, the lanes split the bra primitive pairs and the partial
-// diagonal integrals are summed across the wave.
-template <int LA, int LB>
-__global__ void __launch_bounds__(256) schwarz_kernel(Pair* pairs, const PrimPair* pp, const double* boys, int p0,
-                                                      int np) {
-  constexpr int NAB = ncart(LA) * ncart(LB);
-  const int lane = threadIdx.x & 63;
-  const int i = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-  if (i >= np) return;
-  const Pair P = pairs[p0 + i];
-  double dsum[NAB];
-#pragma unroll
-  for (int k = 0; k < NAB; ++k) dsum[k] = 0.0;
-  for (int b = lane; b < P.npp; b += 64) {
-    double v[NAB * NAB];
-    eri_block<LA, LB, LA, LB, -1>(pp + P.pp0 + b, 1, pp + P.pp0, P.npp, P.ABx, P.ABy, P.ABz, P.ABx, P.ABy, P.ABz,
-                              boys + kBoysCOff + (size_t)(2 * (LA + LB)) * kBoysCLen, v);
-#pragma unroll
-    for (int k = 0; k < NAB; ++k) dsum[k] += v[k * NAB + k];
-  }
-  double m = 0.0;
-#pragma unroll
-  for (int k = 0; k < NAB; ++k) m = fmax(m, fabs(wave_sum(dsum[k])));
-  if (lane == 0) pairs[p0 + i].Q = sqrt(m);
-}
-
 // Workgroups of `threads` threads that fit a CU at once: 512 registers per lane
 // of a SIMD in blocks of 8, at most 8 wavefronts per SIMD, 160 KB of LDS.  Not
 // hipOccupancyMaxActiveBlocksPerMultiprocessor: the HIP runtime of ROCm 7.2
@@ -1081,11 +1054,5 @@ int occupancy_b4(int kc, bool jk, bool tr, size_t lds);
 size_t scratch_b4(int kc, bool jk, bool tr);
 int occupancy_b5(int kc, bool jk, bool tr, size_t lds);
 size_t scratch_b5(int kc, bool jk, bool tr);
-hipError_t launch_schwarz_b0(Pair*, const PrimPair*, const double*, int, int, hipStream_t);
-hipError_t launch_schwarz_b1(Pair*, const PrimPair*, const double*, int, int, hipStream_t);
-hipError_t launch_schwarz_b2(Pair*, const PrimPair*, const double*, int, int, hipStream_t);
-hipError_t launch_schwarz_b3(Pair*, const PrimPair*, const double*, int, int, hipStream_t);
-hipError_t launch_schwarz_b4(Pair*, const PrimPair*, const double*, int, int, hipStream_t);
-hipError_t launch_schwarz_b5(Pair*, const PrimPair*, const double*, int, int, hipStream_t);
 
 }  // namespace vsvb

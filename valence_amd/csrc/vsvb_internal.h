@@ -33,9 +33,20 @@ int fail(int code, const std::string& msg);
       return ::vsvb::fail(VSVB_ERR_DEVICE, std::string(#expr) + ": " + hipGetErrorString(_e));         \
   } while (0)
 
-struct PPSrc {
-  int sA, sB, ia, ib;  // shell indices of A and B, global primitive indices of A and B
+constexpr double kPrimCut = 1e-14;  // smallest |K| of a kept primitive pair (vsvb_pairs.hip)
+
+// A geometry's shell-pair data (vsvb_pairs.hip): off are the pair classes' ranges.
+struct PairArgs {
+  Pair* pairs;
+  const Shell* shells;
+  const double *pexp, *pcoef, *xyz, *charge, *boys;
+  PrimPair* pp;
+  double *S, *H;
+  double kfold;
+  int natom, nbf;
+  int off[kNPairClass + 1];
 };
+hipError_t launch_pairs(const PairArgs& a, hipStream_t st);
 
 // Segment seg of nseg of shell pair `pair` (index into d_pairs).
 struct SegSrc {
@@ -210,7 +221,6 @@ struct vsvb_context {
   using Shell = vsvb::Shell;
   using Pair = vsvb::Pair;
   using PrimPair = vsvb::PrimPair;
-  using PPSrc = vsvb::PPSrc;
   using OrbEntry = vsvb::OrbEntry;
   int device = 0;
   hipStream_t stream = nullptr;
@@ -252,7 +262,6 @@ struct vsvb_context {
   DevBuf<vsvb::SegSrc> d_segsrc;   // which pair and which part of it each segment is
   DevBuf<Shell> d_shells;
   DevBuf<Pair> d_pairs;
-  DevBuf<PPSrc> d_ppsrc;
   DevBuf<PrimPair> d_pp;
   DevBuf<double> d_pexp, d_pcoef, d_xyz, d_charge, d_boys, d_angn;
   DevBuf<unsigned long long> d_stamps;  // per-class wall-clock slots of the last stage (profiling)
