@@ -1187,7 +1187,7 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   // global shells, per-shell primitive copies, AO map
   std::vector<Shell> shells;
   std::vector<double> pexp, pcoef, angn;
-  std::vector<int> ao_shell, atom_sh0(s->natom + 1);
+  std::vector<int> ao_shell, shell_type, atom_sh0(s->natom + 1);
   int ao = 0;
   for (int a = 0; a < s->natom; ++a) {
     const int t = s->atom_type[a];
@@ -1199,6 +1199,7 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
       sh.l = s->shell_l[ts];
       sh.nprim = s->shell_prim_start[ts + 1] - s->shell_prim_start[ts];
       sh.prim0 = (int)pexp.size();
+      shell_type.push_back(ts);
       sh.ao = ao;
       for (int k = 0; k < sh.nprim; ++k) {
         pexp.push_back(s->prim_exp[s->shell_prim_start[ts] + k]);
@@ -1250,11 +1251,45 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   for (int cl = 0; cl < kNPairClass; ++cl) c->pair_off[cl + 1] += c->pair_off[cl];
   c->npairs = (int)pairs.size();
   c->nfun = 0;
-  for (const Pair& P : pairs) c->nfun += ncart(shells[P.A].l) * ncart(shells[P.B].l);
-  c->h_shells = shells;
+  for (int cl = 0; cl < kNPairClass; ++cl) {
+    c->fun_off[cl] = c->nfun;
+    for (int i = c->pair_off[cl]; i < c->pair_off[cl + 1]; ++i)
+      c->nfun += ncart(shells[pairs[i].A].l) * ncart(shells[pairs[i].B].l);
+  }
   c->h_pairs = pairs;
-  c->h_pexp = pexp;
-  c->h_pcoef = pcoef;
+  // What a schedule needs of every shell pair: its class, its pair of atoms, and the
+  // squared distances up to which its primitive pairs pass the screen, descending
+  // (|K| > kPrimCut solved for the distance, once per pair of shell types).
+  c->pair_cls.resize(pairs.size());
+  c->pair_type.resize(pairs.size());
+  c->prim_reach.resize((size_t)s->nshell_type * s->nshell_type);
+  c->apair_start.assign((size_t)s->natom * (s->natom + 1) / 2 + 1, 0);
+  std::vector<int> atoms(pairs.size());
+  c->most_prims = 0;
+  for (size_t i = 0; i < pairs.size(); ++i) {
+    const Shell &A = shells[pairs[i].A], &B = shells[pairs[i].B];
+    c->pair_cls[i] = hp[i].cls;
+    c->pair_type[i] = shell_type[pairs[i].A] * s->nshell_type + shell_type[pairs[i].B];
+    atoms[i] = std::max(A.atom, B.atom) * (std::max(A.atom, B.atom) + 1) / 2 + std::min(A.atom, B.atom);
+    ++c->apair_start[atoms[i] + 1];
+    c->most_prims = std::max(c->most_prims, pairs[i].npp);
+    std::vector<double>& reach = c->prim_reach[c->pair_type[i]];
+    if (!reach.empty()) continue;
+    for (int ia = 0; ia < A.nprim; ++ia)
+      for (int ib = 0; ib < B.nprim; ++ib) {
+        const double x = pexp[A.prim0 + ia], y = pexp[B.prim0 + ib];
+        const double K0 = std::fabs(pcoef[A.prim0 + ia] * pcoef[B.prim0 + ib]) / (x + y) * kPairFold;
+        const double d2 = std::log(K0 / kPrimCut) * (x + y) / (x * y);
+        reach.push_back(std::isnan(d2) ? 0.0 : d2);
+      }
+    std::sort(reach.begin(), reach.end(), std::greater<double>());
+  }
+  for (size_t k = 1; k < c->apair_start.size(); ++k) c->apair_start[k] += c->apair_start[k - 1];
+  c->apair_ids.resize(pairs.size());
+  {
+    std::vector<int> next(c->apair_start);
+    for (size_t i = 0; i < pairs.size(); ++i) c->apair_ids[next[atoms[i]]++] = (int)i;
+  }
   // orbital entries: map each weight to an AO of the molecule (OBS-local numbering, xm_input)
   c->ent.resize(std::max(1, s->totlen));
   c->orb_start.assign(s->orb_start, s->orb_start + s->norbs + 1);
@@ -1311,6 +1346,8 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   const size_t nbf2 = (size_t)c->nbf * c->nbf;
   HIP_OK(device_buffer(c, c->d_shells, c->nsh));
   HIP_OK(device_buffer(c, c->d_pairs, c->npairs));
+  HIP_OK(device_buffer(c, c->d_psrc, c->npairs));
+  HIP_OK(device_buffer(c, c->d_order, c->npairs));
   HIP_OK(device_buffer(c, c->d_pp, c->npp));
   HIP_OK(device_buffer(c, c->d_pexp, pexp.size()));
   HIP_OK(device_buffer(c, c->d_pcoef, pcoef.size()));
@@ -1424,7 +1461,11 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   // uploads
   static const std::vector<double> boys = make_boys_table();  // the same in every context
   HIP_OK(hipMemcpy(c->d_shells.p, shells.data(), shells.size() * sizeof(Shell), hipMemcpyHostToDevice));
-  HIP_OK(hipMemcpy(c->d_pairs.p, pairs.data(), pairs.size() * sizeof(Pair), hipMemcpyHostToDevice));
+  {
+    std::vector<PairSrc> src;
+    for (const Pair& P : pairs) src.push_back(PairSrc{P.A, P.B, P.pp0});
+    HIP_OK(hipMemcpy(c->d_psrc.p, src.data(), src.size() * sizeof(PairSrc), hipMemcpyHostToDevice));
+  }
   HIP_OK(hipMemcpy(c->d_pexp.p, pexp.data(), pexp.size() * sizeof(double), hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(c->d_pcoef.p, pcoef.data(), pcoef.size() * sizeof(double), hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(c->d_charge.p, c->charges.data(), c->natom * sizeof(double), hipMemcpyHostToDevice));
@@ -1447,52 +1488,38 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
 // is recomputed when the coordinates change.
 static int schedule_pairs(vsvb_context* c) {
   if (c->sched_coords == c->coords) return VSVB_OK;
-  const double kfold = std::sqrt(2.0 * std::pow(M_PI, 2.5));
-  const int np = c->npairs;
-  std::vector<int> kept(np);
-  std::vector<double> r2(np);
-  for (int i = 0; i < np; ++i) {
-    const Pair& P = c->h_pairs[i];
-    const Shell& A = c->h_shells[P.A];
-    const Shell& B = c->h_shells[P.B];
-    const double* xa = c->coords.data() + 3 * A.atom;
-    const double* xb = c->coords.data() + 3 * B.atom;
-    const double d2 = (xa[0] - xb[0]) * (xa[0] - xb[0]) + (xa[1] - xb[1]) * (xa[1] - xb[1]) +
-                      (xa[2] - xb[2]) * (xa[2] - xb[2]);
-    int k = 0;
-    for (int ia = 0; ia < A.nprim; ++ia)
-      for (int ib = 0; ib < B.nprim; ++ib) {
-        const double a = c->h_pexp[A.prim0 + ia], b = c->h_pexp[B.prim0 + ib], p = a + b;
-        const double K = c->h_pcoef[A.prim0 + ia] * c->h_pcoef[B.prim0 + ib] * std::exp(-a * b / p * d2) / p * kfold;
-        if (std::fabs(K) > kPrimCut) ++k;
-      }
-    kept[i] = k;
-    r2[i] = d2;
-  }
-  std::vector<int> idx(np);
-  std::vector<Pair> sorted(np);
-  for (int cl = 0; cl < kNPairClass; ++cl) {
-    const int b = c->pair_off[cl], e = c->pair_off[cl + 1];
-    for (int i = b; i < e; ++i) idx[i] = i;
-    std::stable_sort(idx.begin() + b, idx.begin() + e, [&](int x, int y) {
-      if (kept[x] != kept[y]) return kept[x] > kept[y];
-      return r2[x] < r2[y];
-    });
-  }
-  std::vector<int> skept(np);
-  for (int i = 0; i < np; ++i) {
-    sorted[i] = c->h_pairs[idx[i]];
-    skept[i] = kept[idx[i]];
-  }
-  for (int cl = 0, f0 = 0; cl < kNPairClass; ++cl) {
-    const int b = c->pair_off[cl], e = c->pair_off[cl + 1];
-    for (int i = b; i < e; ++i) sorted[i].f0 = f0 + i - b;
-    if (e > b) f0 += (e - b) * ncart(c->h_shells[sorted[b].A].l) * ncart(c->h_shells[sorted[b].B].l);
-  }
-  c->h_pairs.swap(sorted);
+  const int np = c->npairs, nap = c->natom * (c->natom + 1) / 2;
+  // Shell pairs of one pair of atoms share the distance: the atom pairs are sorted,
+  // and every shell pair goes to the next place of its (class, count) in that order.
+  std::vector<std::pair<double, int>> ap(nap);
+  for (int i = 0, k = 0; i < c->natom; ++i)
+    for (int j = 0; j <= i; ++j, ++k) {
+      const double *xa = c->coords.data() + 3 * i, *xb = c->coords.data() + 3 * j;
+      ap[k] = {(xa[0] - xb[0]) * (xa[0] - xb[0]) + (xa[1] - xb[1]) * (xa[1] - xb[1]) + (xa[2] - xb[2]) * (xa[2] - xb[2]),
+               k};
+    }
+  std::stable_sort(ap.begin(), ap.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
+  const int nk = c->most_prims + 1;
+  std::vector<int> kept(np), start((size_t)kNPairClass * nk + 1, 0), skept(np);
+  auto cell = [&](int i) { return c->pair_cls[i] * nk + (nk - 1 - kept[i]); };  // class, then most primitive pairs first
+  for (const auto& x : ap)
+    for (int e = c->apair_start[x.second]; e < c->apair_start[x.second + 1]; ++e) {
+      const int i = c->apair_ids[e];
+      const std::vector<double>& lim = c->prim_reach[c->pair_type[i]];
+      kept[i] = (int)(std::lower_bound(lim.begin(), lim.end(), x.first, std::greater<double>()) - lim.begin());
+      ++start[cell(i) + 1];
+    }
+  for (size_t k = 1; k < start.size(); ++k) start[k] += start[k - 1];
+  c->h_order.resize(np);
+  for (const auto& x : ap)
+    for (int e = c->apair_start[x.second]; e < c->apair_start[x.second + 1]; ++e) {
+      const int i = c->apair_ids[e], at = start[cell(i)]++;
+      c->h_order[at] = i;
+      skept[at] = kept[i];
+    }
   const int rc = plan_work(c, skept.data());
   if (rc) return rc;
-  HIP_OK(hipMemcpyAsync(c->d_pairs.p, c->h_pairs.data(), np * sizeof(Pair), hipMemcpyHostToDevice, c->stream));
+  HIP_OK(hipMemcpyAsync(c->d_order.p, c->h_order.data(), np * sizeof(int), hipMemcpyHostToDevice, c->stream));
   if (!c->h_seg.empty())
     HIP_OK(hipMemcpyAsync(c->d_segsrc.p, c->h_seg.data(), c->h_seg.size() * sizeof(SegSrc), hipMemcpyHostToDevice,
                           c->stream));
@@ -1509,10 +1536,11 @@ int vsvb::prepare_geometry(vsvb_context* c, const double* coords) {
   c->enuc = nuclear_repulsion(c->natom, c->coords.data(), c->charges.data());
   if (!c->capturing)
     HIP_OK(hipMemcpyAsync(c->d_xyz.p, c->coords.data(), 3 * c->natom * sizeof(double), hipMemcpyHostToDevice, st));
-  PairArgs a{c->d_pairs.p, c->d_shells.p, c->d_pexp.p, c->d_pcoef.p, c->d_xyz.p, c->d_charge.p, c->d_boys.p,
-             c->d_pp.p,    c->d_S.p,      c->d_H.p,    std::sqrt(2.0 * std::pow(M_PI, 2.5)),    c->natom,
-             c->nbf,       {}};
+  PairArgs a{c->d_psrc.p,  c->d_order.p,  c->d_pairs.p, c->d_shells.p, c->d_pexp.p, c->d_pcoef.p, c->d_xyz.p,
+             c->d_charge.p, c->d_boys.p,  c->d_pp.p,    c->d_S.p,      c->d_H.p,    kPairFold,    c->natom,
+             c->nbf,        {},           {}};
   std::copy(c->pair_off, c->pair_off + kNPairClass + 1, a.off);
+  std::copy(c->fun_off, c->fun_off + kNPairClass, a.fun);
   HIP_OK(launch_pairs(a, st));
   if (!c->h_seg.empty()) {
     const int ns = (int)c->h_seg.size();
@@ -2717,6 +2745,8 @@ static bool same_molecule(const vsvb_system* a, const vsvb_system* b) {
 static void share_geometry(vsvb_context* lead, vsvb_context* m) {
   m->d_shells.alias(lead->d_shells.p, lead->d_shells.n);
   m->d_pairs.alias(lead->d_pairs.p, lead->d_pairs.n);
+  m->d_psrc.alias(lead->d_psrc.p, lead->d_psrc.n);
+  m->d_order.alias(lead->d_order.p, lead->d_order.n);
   m->d_pp.alias(lead->d_pp.p, lead->d_pp.n);
   m->d_pexp.alias(lead->d_pexp.p, lead->d_pexp.n);
   m->d_pcoef.alias(lead->d_pcoef.p, lead->d_pcoef.n);

@@ -36,7 +36,13 @@ int fail(int code, const std::string& msg);
 constexpr double kPrimCut = 1e-14;  // smallest |K| of a kept primitive pair (vsvb_pairs.hip)
 
 // A geometry's shell-pair data (vsvb_pairs.hip): off are the pair classes' ranges.
+struct PairSrc {
+  int A, B, pp0;  // shells and first primitive pair
+};
+const double kPairFold = std::sqrt(2.0 * std::pow(M_PI, 2.5));  // factor folded into PrimPair::K
 struct PairArgs {
+  const PairSrc* src;  // shell pairs in their first order
+  const int* order;    // the geometry's order
   Pair* pairs;
   const Shell* shells;
   const double *pexp, *pcoef, *xyz, *charge, *boys;
@@ -45,6 +51,7 @@ struct PairArgs {
   double kfold;
   int natom, nbf;
   int off[kNPairClass + 1];
+  int fun[kNPairClass];  // first entry of a class in the function-pair list (Pair::f0)
 };
 hipError_t launch_pairs(const PairArgs& a, hipStream_t st);
 
@@ -251,9 +258,11 @@ struct vsvb_context {
   // host copies
   std::vector<double> coords, charges, coeff;
   // host copies for the per-geometry pair schedule
-  std::vector<Shell> h_shells;
-  std::vector<Pair> h_pairs;
-  std::vector<double> h_pexp, h_pcoef, sched_coords;
+  std::vector<Pair> h_pairs;  // in their first order
+  std::vector<double> sched_coords;
+  std::vector<int> h_order, pair_cls, pair_type, apair_start, apair_ids;
+  std::vector<std::vector<double>> prim_reach;
+  int most_prims = 0, fun_off[vsvb::kNPairClass] = {0};
   std::vector<vsvb::SegSrc> h_seg;
   std::vector<OrbEntry> ent;
   std::vector<int> orb_start;
@@ -262,6 +271,8 @@ struct vsvb_context {
   DevBuf<vsvb::SegSrc> d_segsrc;   // which pair and which part of it each segment is
   DevBuf<Shell> d_shells;
   DevBuf<Pair> d_pairs;
+  DevBuf<vsvb::PairSrc> d_psrc;
+  DevBuf<int> d_order;
   DevBuf<PrimPair> d_pp;
   DevBuf<double> d_pexp, d_pcoef, d_xyz, d_charge, d_boys, d_angn;
   DevBuf<unsigned long long> d_stamps;  // per-class wall-clock slots of the last stage (profiling)

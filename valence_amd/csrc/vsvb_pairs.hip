@@ -28,7 +28,7 @@ namespace {
 __global__ void __launch_bounds__(256) k_pairs(PairArgs a) {
   const int t = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6))), lane = threadIdx.x & 63;
   if (t >= a.off[kNPairClass]) return;  // whole wavefront
-  const Pair P = a.pairs[t];
+  const PairSrc P = a.src[a.order[t]];
   const Shell A = a.shells[P.A], B = a.shells[P.B];
   const double Ax = a.xyz[3 * A.atom], Ay = a.xyz[3 * A.atom + 1], Az = a.xyz[3 * A.atom + 2];
   const double Bx = a.xyz[3 * B.atom], By = a.xyz[3 * B.atom + 1], Bz = a.xyz[3 * B.atom + 2];
@@ -58,11 +58,9 @@ __global__ void __launch_bounds__(256) k_pairs(PairArgs a) {
     kept += __popcll(m);
   }
   if (lane == 0) {
-    Pair& Q = a.pairs[t];
-    Q.ABx = ABx;
-    Q.ABy = ABy;
-    Q.ABz = ABz;
-    Q.npp = kept;
+    int cl = 0;
+    while (t >= a.off[cl + 1]) ++cl;
+    a.pairs[t] = Pair{P.A, P.B, P.pp0, kept, a.fun[cl] + t - a.off[cl], 0, ABx, ABy, ABz, 0.0};
   }
 }
 
