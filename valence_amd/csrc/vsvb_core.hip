@@ -513,15 +513,17 @@ __global__ void k_trace_prod(const double* __restrict__ A, int ld, int off, cons
                              double w, double* __restrict__ out) {
   __shared__ double red[256];
   double s = 0.0;
-  for (int t = threadIdx.x; t < n * n; t += blockDim.x) s += A[(size_t)(off + t / n) * ld + off + t % n] * B[t];
+  for (int t = blockIdx.x * 256 + threadIdx.x; t < n * n; t += gridDim.x * 256)
+    s += A[(size_t)(off + t / n) * ld + off + t % n] * B[t];
   red[threadIdx.x] = s;
   __syncthreads();
   for (int o = 128; o > 0; o >>= 1) {
     if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[0] += w * red[0];
+  if (threadIdx.x == 0) unsafeAtomicAdd(out, w * red[0]);
 }
+static unsigned trace_blocks(int n) { return (unsigned)std::clamp(n * (long)n / 4096, 1L, 256L); }
 
 __global__ void k_fill(double* __restrict__ p, size_t n, double v) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
@@ -919,32 +921,31 @@ static ClassLaunch straight_launch(vsvb_context* c, int bc, int kc, bool jk, int
 // 0.30 ms on C8H18); the batch tuner still tries every grid.
 constexpr int kDefaultJkPerCu = 4;
 
-// Default J/K orientation of a straight-line class: transposed when its ket
-// strips keep more lanes busy than the bra strips (few bra pairs), or, at equal
-// lane use, when the bra block is the larger one (fewer per-lane atomics); but
-// not into an orientation whose exchange rows no longer fit in LDS (large
-// basis sets) while the other's do, and for large basis sets, at equal lane
-// use, the one with fewer exchange rows.
-constexpr int kLargeBasis = 1024;
+// Default J/K orientation of a straight-line class: the one with the smaller
+// product of its units (strips of 256 pairs, idle lanes included, times the pairs of
+// the other side) and the cost of a unit.  A transposed unit costs `cost` of a
+// normal one, from both orientations' times of every class of C8H18 (210 AOs) and of
+// LiF slabs of 32, 64 and 128 atoms (384, 768, 1536): (ps|ss) 1.7 at every size (1389
+// us against 738, 378 ms against 224); d-heavy bras 0.8 (large bra blocks mean many
+// atomics per lane in a normal unit: (dd|ss) 55 us against 315, 5.3 ms against 10.5);
+// the bras between 0.85 in small bases and 1.3 in large ones, where the larger number
+// of exchange rows of a transposed unit takes LDS from other workgroups ((pp|ps) 231
+// us against 406, but 7.1 ms against 6.3 at 768 AOs and 21 against 7.2 at 1536).  For those
+// bras an orientation whose exchange rows fit in LDS goes before one whose rows do
+// not; d-heavy ones are faster transposed without LDS, too.
+constexpr int kLargeBasis = 300;
 static bool transposed_default(vsvb_context* c, int bc, int kc) {
   if (bc == kc) return false;
   const int nb = c->pair_off[bc + 1] - c->pair_off[bc], nk = c->pair_off[kc + 1] - c->pair_off[kc];
   if (nb <= 0 || nk <= 0) return false;
-  const double ub = (double)nb / (((nb + kStripB - 1) / kStripB) * kStripB);
-  const double uk = (double)nk / (((nk + kStripK - 1) / kStripK) * kStripK);
-  const int nab = ncart(kPairLs[bc][0]) * ncart(kPairLs[bc][1]), ncd = ncart(kPairLs[kc][0]) * ncart(kPairLs[kc][1]);
   // exchange staging: the normal unit holds NC + ND rows of nbf, the transposed one NA + NB
   const size_t row = (size_t)c->nbf * sizeof(double);
-  const int rows_n = ncart(kPairLs[kc][0]) + ncart(kPairLs[kc][1]);
-  const int rows_t = ncart(kPairLs[bc][0]) + ncart(kPairLs[bc][1]);
-  const bool fit_n = row * rows_n <= kMaxLdsK, fit_t = row * rows_t <= kMaxLdsK;
-  if (uk > ub + 0.05) return fit_t || !fit_n;
-  if (ub > uk + 0.05) return false;
-  if (fit_n != fit_t) return fit_t;
-  // large basis: the orientation with fewer exchange rows (LiF128's (ps|ss):
-  // normal 219 ms against transposed 400 ms, as the batch tuner measured it)
-  if (c->nbf >= kLargeBasis && rows_n != rows_t) return rows_t < rows_n;
-  return nab > ncd;
+  const bool fit_n = row * (ncart(kPairLs[kc][0]) + ncart(kPairLs[kc][1])) <= kMaxLdsK;
+  const bool fit_t = row * (ncart(kPairLs[bc][0]) + ncart(kPairLs[bc][1])) <= kMaxLdsK;
+  if (bc < 4 && fit_n != fit_t) return fit_t;
+  const double un = (double)((nb + kStripB - 1) / kStripB) * nk, ut = (double)((nk + kStripK - 1) / kStripK) * nb;
+  const double cost = bc >= 4 ? 0.8 : bc == 1 ? 1.7 : c->nbf < kLargeBasis ? 0.85 : 1.3;
+  return ut * cost < un;
 }
 
 // Cooperative kernel: one unit per (bra pair, ket pair); claim = 0 picks about
@@ -1637,7 +1638,7 @@ static int prepare_orbitals(vsvb_context* c, const double* coeff_host, const dou
     hipLaunchKernelGGL(k_copy_block, dim3((m * m + 255) / 256), dim3(256), 0, st, c->d_Sorb.p, ns, off, m, P);
     HIP_OK(launch_spd_inverse(st, P, m, c->d_status.p, c->d_colk.p, c->grid_inverse_min));
     // E1 += w tr(h_s P_s): closed shell counts both spins (w = 2)
-    hipLaunchKernelGGL(k_trace_prod, dim3(1), dim3(256), 0, st, c->d_Horb.p, ns, off, P, m, nspin == 1 ? 2.0 : 1.0,
+    hipLaunchKernelGGL(k_trace_prod, dim3(trace_blocks(m)), dim3(256), 0, st, c->d_Horb.p, ns, off, P, m, nspin == 1 ? 2.0 : 1.0,
                        c->d_scal.p + 0);
     // R_s = Cs_s^T P_s Cs_s
     const double* Cs = c->d_Cs.p + (size_t)off * n;
@@ -1961,7 +1962,7 @@ static int gradient_impl(vsvb_context* c, double* grad_dev) {
     double* F = c->d_F.p + (size_t)s * nn;
     hipLaunchKernelGGL(k_sym_combine, dim3(gb), dim3(T), 0, st, c->d_K.p + (size_t)s * nn, -1.0, c->d_Jsym.p, cfac,
                        n, F);
-    hipLaunchKernelGGL(k_trace_prod, dim3(1), dim3(256), 0, st, c->d_R.p + (size_t)s * nn, n, 0, F, n, 0.5,
+    hipLaunchKernelGGL(k_trace_prod, dim3(trace_blocks(n)), dim3(256), 0, st, c->d_R.p + (size_t)s * nn, n, 0, F, n, 0.5,
                        c->d_scal.p + 3);
     hipLaunchKernelGGL(k_sym_combine, dim3(gb), dim3(T), 0, st, c->d_H.p, 0.5 * w1, F, 1.0, n, F);
     const double* Ct = c->d_Ct.p + (size_t)off * n;
