@@ -1747,10 +1747,63 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
     offs[q] = poff;
     poff += c->partial_per_class[q];
   }
+  const int m = jk ? 1 : 0;
+  // Two cooperative classes whose wavefronts all fit the chip at once share a
+  // launch: each runs as long as its longest quartet (water: 2 x 36 us one after the
+  // other, 46 side by side).
+  int pair[2] = {-1, -1};
+  struct Join {  // on every return path
+    hipStream_t st = nullptr;
+    hipEvent_t ev = nullptr;
+    ~Join() {
+      if (ev) (void)hipStreamWaitEvent(st, ev, 0);
+    }
+  } join;
+  bool forked = false;
+  {
+    int k = 0, blocks = 0, fit = 0;
+    for (int q = kNQuartetClass - 1; q >= 0 && k < 2; --q) {
+      const ClassLaunch& cl = jk ? c->ljk[q] : c->le[q];
+      if (!cl.coop || cl.units <= 0) continue;
+      pair[k] = q;
+      blocks += cl.blocks;
+      fit = k == 0 ? coop_occupancy(c->coop_idx[q], jk) : std::min(fit, coop_occupancy(c->coop_idx[q], jk));
+      ++k;
+    }
+    if (k < 2 || blocks > fit * c->ncu) pair[0] = pair[1] = -1;
+  }
+  if (pair[0] >= 0) {
+    QuartetArgs a[2];
+    for (int k = 0; k < 2; ++k) {
+      const int q = pair[k], bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
+      a[k] = class_args(c, bc, kc, jk ? c->ljk[q] : c->le[q], jk, nwfn, nspin, dens, jacc, kacc, c->d_partial.p + offs[q],
+                        eri);
+    }
+    // beside the shared launch, on a stream of its own: both are chains on a mostly
+    // idle chip (a water energy 169 us in one stream, 152 so; batches have their own
+    // streams and graphs)
+    if (c->small[m].n > 0 && c->own_stream && !c->capturing) {
+      if (!c->side) {
+        HIP_OK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
+        HIP_OK(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
+        HIP_OK(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+      }
+      HIP_OK(hipEventRecord(c->ev_fork, st));
+      HIP_OK(hipStreamWaitEvent(c->side, c->ev_fork, 0));
+      forked = true;
+    }
+    const ClassLaunch* l = jk ? c->ljk : c->le;
+    HIP_OK(launch_coop_pair(c->coop_idx[pair[0]], a[0], l[pair[0]].blocks, c->coop_idx[pair[1]], a[1],
+                            l[pair[1]].blocks, jk, c->device, forked ? c->side : st));
+    if (forked) {
+      HIP_OK(hipEventRecord(c->ev_join, c->side));
+      join.st = st;
+      join.ev = c->ev_join;
+    }
+  }
   // Small classes share one launch: their argument records go to the device when
   // they differ from the last ones (under capture nothing is uploaded; records
   // that differ then take separate launches).
-  const int m = jk ? 1 : 0;
   bool shared = c->small[m].n > 0 && (nwfn == 1 || eri);
   if (shared) {
     const SmallLaunch& s = c->small[m];
@@ -1772,33 +1825,6 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
     }
     if (shared) HIP_OK(launch_small(s, dev, jk, st));
   }
-  // Two cooperative classes whose wavefronts all fit the chip at once share a
-  // launch: each runs as long as its longest quartet (water: 2 x 36 us one after the
-  // other, 46 side by side).
-  int pair[2] = {-1, -1};
-  {
-    int k = 0, blocks = 0, fit = 0;
-    for (int q = kNQuartetClass - 1; q >= 0 && k < 2; --q) {
-      const ClassLaunch& cl = jk ? c->ljk[q] : c->le[q];
-      if (!cl.coop || cl.units <= 0) continue;
-      pair[k] = q;
-      blocks += cl.blocks;
-      fit = k == 0 ? coop_occupancy(c->coop_idx[q], jk) : std::min(fit, coop_occupancy(c->coop_idx[q], jk));
-      ++k;
-    }
-    if (k < 2 || blocks > fit * c->ncu) pair[0] = pair[1] = -1;
-  }
-  if (pair[0] >= 0) {
-    QuartetArgs a[2];
-    for (int k = 0; k < 2; ++k) {
-      const int q = pair[k], bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
-      a[k] = class_args(c, bc, kc, jk ? c->ljk[q] : c->le[q], jk, nwfn, nspin, dens, jacc, kacc, c->d_partial.p + offs[q],
-                        eri);
-    }
-    const ClassLaunch *l = jk ? c->ljk : c->le;
-    HIP_OK(launch_coop_pair(c->coop_idx[pair[0]], a[0], l[pair[0]].blocks, c->coop_idx[pair[1]], a[1],
-                            l[pair[1]].blocks, jk, c->device, st));
-  }
   for (int t = 0; t < kNQuartetClass; ++t) {
     const int q = c->class_rev ? kNQuartetClass - 1 - t : t;
     if ((shared && c->in_small[m][q]) || q == pair[0] || q == pair[1]) continue;
@@ -1812,6 +1838,10 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
     const QuartetArgs a = class_args(c, bc, kc, cl, jk, nwfn, nspin, dens, jacc, kacc, c->d_partial.p + offs[q],
                                      eri);
     HIP_OK(launch_class(c, bc, kc, cl, a, jk));
+  }
+  if (forked) {
+    join.ev = nullptr;
+    HIP_OK(hipStreamWaitEvent(st, c->ev_join, 0));
   }
   if (c->ev0 && c->ev1 && !c->capturing) {
     HIP_OK(hipEventRecord(c->ev1, st));
@@ -2974,9 +3004,13 @@ int vsvb_context_create(const vsvb_system* sys, const vsvb_options* opt, vsvb_co
 void vsvb_context_destroy(vsvb_context* c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
+  if (c->side) (void)hipStreamSynchronize(c->side);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
+  if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
+  if (c->ev_join) (void)hipEventDestroy(c->ev_join);
+  if (c->side) (void)hipStreamDestroy(c->side);
   if (c->ev_in) (void)hipEventDestroy(c->ev_in);
   if (c->ev_out) (void)hipEventDestroy(c->ev_out);
   hipStream_t st = c->own_stream ? c->stream : nullptr;

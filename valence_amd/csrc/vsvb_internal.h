@@ -234,6 +234,8 @@ struct vsvb_context {
   bool own_stream = true;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   bool ev_valid = false;  // ev0 / ev1 bracket the last quartet pass (a direct run_quartets)
+  hipStream_t side = nullptr;  // cooperative classes beside the shared launch (made at its first use)
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   hipEvent_t ev_in = nullptr, ev_out = nullptr;  // ordering against a caller's stream (device entry)
   double tau = 1e-17;
   int pair_chunk = 0;  // straight-line units: uniform-side pairs per claim (0: from the system size)
