@@ -256,6 +256,16 @@ int vsvb_debug_boys(int32_t L, const double *T, int32_t n, double *out);
  * op(B) K x N (B stored N x K when tb); C is read and overwritten. */
 int vsvb_debug_gemm(int32_t M, int32_t N, int32_t K, int32_t ta, int32_t tb, double alpha, const double *A,
                     const double *B, double beta, double *C);
+/* How the system's quartet classes would be launched at its coordinates by a
+ * context on a device of ncu compute units (diagnostics/tests; planned on the
+ * host, no device needed: without one the kernels' registers and LDS are not
+ * known and count as few).  plan[2][21][8] = per mode (energy, J/K of one wave
+ * function) and class {cooperative kernel 0/1, work list of the bra, of the ket
+ * class (0 = shell pairs, 1 and 2 = segments), work units, workgroups per part,
+ * pairs per claim, transposed units 0/1, shared launch 0/1}.  partial[2] = the
+ * partial sums an energy writes (the larger of these coordinates and the
+ * unscreened primitive lists), and those its context holds. */
+int vsvb_debug_plan(const vsvb_system *sys, const vsvb_options *opt, int32_t ncu, double *plan, int64_t *partial);
 /* Library version string. */
 const char *vsvb_version(void);
 

@@ -858,6 +858,11 @@ static void choose_levels(const vsvb_context* c, int bc, int kc, bool jk, bool t
     }
 }
 
+// Most workgroups (of each part) of a straight-line energy launch.
+static int energy_grid(const vsvb_context* c, int bc, int kc) {
+  return std::min(2048, class_occupancy(bc, kc, false, false, 0) * c->ncu);
+}
+
 static ClassLaunch straight_launch(vsvb_context* c, int bc, int kc, bool jk, int per_cu, bool lds_on, bool tr) {
   ClassLaunch L;
   L.tr = jk && tr && bc != kc;
@@ -866,8 +871,7 @@ static ClassLaunch straight_launch(vsvb_context* c, int bc, int kc, bool jk, int
   L.per_cu = per_cu;
   if (nb <= 0 || nk <= 0) return L;
   if (!jk) {
-    const int occ = class_occupancy(bc, kc, false, false, 0);
-    const int cap = per_cu > 0 ? std::min(per_cu, occ) * c->ncu : std::min(2048, occ * c->ncu);
+    const int cap = energy_grid(c, bc, kc);
     const int nbt = (nb + kTileB - 1) / kTileB;
     // Ket chunks as wide as still leave kEnergyUnitsPerWave units per resident
     // wavefront: large (and sparse) systems claim up to 64 kets at once and
@@ -1046,7 +1050,7 @@ static int plan_work(vsvb_context* c, const int* kept) {
       const ClassLaunch cl = policy_launch(c, q, c->pol[q]);
       if (!cl.overflow && (cl.units > 0 || c->ljk[q].units <= 0)) c->ljk[q] = cl;
     }
-    if (c->d_small.p && c->ndens == 1 && c->coop_idx[q] < 0) {
+    if (c->nlevels > 1 && c->ndens == 1 && c->coop_idx[q] < 0) {
       c->in_small[0][q] = c->le[q].units > 0 && c->le[q].kchunk == 1 && c->le[q].blocks * kPartsEnergy[q] <= kSmallBlocks;
       // the shared J/K launch has the transposed units of classes of different bra and ket
       const ClassLaunch cl = straight_launch(c, bc, kc, true, kDefaultJkPerCu, true, bc != kc);
@@ -1140,7 +1144,7 @@ static OrbArgs orb_args(const vsvb_context* c) {
   return a;
 }
 
-static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_context* c) {
+static int read_options(const vsvb_system* s, const vsvb_options* opt, vsvb_context* c) {
   if (!s) return fail(VSVB_ERR_ARG, "null system");
   if (s->natom < 1 || s->nshell_type < 1) return fail(VSVB_ERR_ARG, "empty molecule or basis");
   c->device = opt ? opt->device : 0;
@@ -1150,15 +1154,21 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   const int gim = opt ? opt->grid_inverse_min : 0;
   if (gim < 0) return fail(VSVB_ERR_ARG, "grid_inverse_min must be 0 (default) or at least 1");
   c->grid_inverse_min = gim > 0 ? gim : kSpdOneBlock + 1;
-  HIP_OK(hipSetDevice(c->device));
-  HIP_OK(hipDeviceGetAttribute(&c->wall_khz, hipDeviceAttributeWallClockRate, c->device));
-  if (!c->arena) {  // the allocation-free entry creates no stream or events: it runs on the null stream
-    if (!c->stream) HIP_OK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-    HIP_OK(hipEventCreate(&c->ev0));
-    HIP_OK(hipEventCreate(&c->ev1));
-    HIP_OK(hipEventCreateWithFlags(&c->ev_in, hipEventDisableTiming));
-    HIP_OK(hipEventCreateWithFlags(&c->ev_out, hipEventDisableTiming));
-  }
+  return VSVB_OK;
+}
+
+// What a context holds of its system on the host: sizes, shells and shell pairs,
+// what a schedule needs of them, orbital entries.
+struct HostBasis {
+  std::vector<Shell> shells;
+  std::vector<double> pexp, pcoef, angn;
+  std::vector<int> ao_shell;
+};
+
+static int describe_system(const vsvb_system* s, const vsvb_options* opt, vsvb_context* c, HostBasis& hb) {
+  std::vector<Shell>& shells = hb.shells;
+  std::vector<double>&pexp = hb.pexp, &pcoef = hb.pcoef, &angn = hb.angn;
+  std::vector<int>& ao_shell = hb.ao_shell;
   c->natom = s->natom;
   c->npair = s->npair;
   c->nunpd = s->nunpd;
@@ -1186,9 +1196,7 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
     norm_prim(s->shell_l[ts], p1 - p0, s->prim_exp + p0, s->prim_coef + p0, con.data() + p0);
   }
   // global shells, per-shell primitive copies, AO map
-  std::vector<Shell> shells;
-  std::vector<double> pexp, pcoef, angn;
-  std::vector<int> ao_shell, shell_type, atom_sh0(s->natom + 1);
+  std::vector<int> shell_type, atom_sh0(s->natom + 1);
   int ao = 0;
   for (int a = 0; a < s->natom; ++a) {
     const int t = s->atom_type[a];
@@ -1343,6 +1351,88 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   c->charges.resize(s->natom);
   for (int a = 0; a < s->natom; ++a) c->charges[a] = s->nuc_charge[s->atom_type[a]];
   c->coeff.assign(s->coeff, s->coeff + s->totlen);
+  return VSVB_OK;
+}
+
+// Work lists and counters of a context of c->ncu CUs; the length of its segment lists.
+static size_t plan_lists(vsvb_context* c) {
+  // work lists: the shell pairs, and for systems of up to kSplitMaxPairs pairs
+  // their segments (counts here for unscreened primitive lists, the most a
+  // geometry can give)
+  size_t seg_cap = 0;
+  for (int pc = 0; pc < kNPairClass; ++pc) {
+    WorkList& W0 = c->work[pc][0];
+    W0.off = c->pair_off[pc];
+    W0.n = W0.cap = c->pair_off[pc + 1] - c->pair_off[pc];
+    for (int l = 1; l < kLevels; ++l) {
+      WorkList& W = c->work[pc][l];
+      W.cap = 0;
+      for (int i = c->pair_off[pc]; i < c->pair_off[pc + 1]; ++i)
+        W.cap += std::max(1, (c->h_pairs[i].npp + kSegLen[l][pc] - 1) / kSegLen[l][pc]);
+      seg_cap += W.cap;
+    }
+  }
+  // work counters: per part one per energy segment of kSegTiles bra tiles and one
+  // per J/K strip (bra strips, or ket strips transposed); one for the cooperative kernel
+  static_assert(kSegTiles * kTileB == kStripB, "an energy segment covers one bra strip");
+  const bool split = c->npairs <= kSplitMaxPairs;
+  c->ctr_total = 0;
+  for (int bc = 0, q = 0; bc < kNPairClass; ++bc)
+    for (int kc = 0; kc <= bc; ++kc, ++q) {
+      int most = 1;
+      for (int l = 0; l < (split ? kLevels : 1); ++l)
+        most = std::max({most, (c->work[bc][l].cap + kStripB - 1) / kStripB, (c->work[kc][l].cap + kStripK - 1) / kStripK});
+      c->ctr_off[q] = c->ctr_total;
+      c->ctr_len[q] = most * std::max(kPartsEnergy[q], kPartsJk[q]);
+      c->ctr_total += c->ctr_len[q];
+      c->coop_idx[q] = coop_class(kPairLs[bc][0], kPairLs[bc][1], kPairLs[kc][0], kPairLs[kc][1]);
+    }
+  return split ? seg_cap : 0;
+}
+
+// Doubles of d_partial: what an energy at any geometry writes, four per workgroup
+// and part of a class.  The longest lists give the largest grids, up to the class's
+// limit (chunks of several kets are fewer units).  Fock tiles leave their shares of
+// E2 there too, at most 20 x 20 per spin; the allocation-free entry, J/K only, has
+// no energy launches.
+static size_t partial_slots(const vsvb_context* c) {
+  size_t slots = 0;
+  for (int bc = 0, q = 0; bc < kNPairClass && !c->arena; ++bc)
+    for (int kc = 0; kc <= bc; ++kc, ++q) {
+      size_t nb = 0, nk = 0;
+      for (int l = 0; l < (c->npairs <= kSplitMaxPairs ? kLevels : 1); ++l) {
+        nb = std::max<size_t>(nb, c->work[bc][l].cap);
+        nk = std::max<size_t>(nk, c->work[kc][l].cap);
+      }
+      if (nb == 0 || nk == 0) continue;
+      const size_t nbt = (nb + kTileB - 1) / kTileB;
+      if (c->coop_idx[q] >= 0)
+        slots += 4 * std::min(nb * nk, (size_t)coop_occupancy(c->coop_idx[q], false) * c->ncu);
+      else
+        slots += 4 * class_parts(q, false) *
+                 std::min(((bc == kc ? kTileB / 2 * nbt * (nbt + 1) : nbt * nk) + 3) / 4, (size_t)energy_grid(c, bc, kc));
+    }
+  return std::max<size_t>(slots, 1024);
+}
+
+static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_context* c) {
+  int rc;
+  if ((rc = read_options(s, opt, c))) return rc;
+  HIP_OK(hipSetDevice(c->device));
+  HIP_OK(hipDeviceGetAttribute(&c->wall_khz, hipDeviceAttributeWallClockRate, c->device));
+  if (!c->arena) {  // the allocation-free entry creates no stream or events: it runs on the null stream
+    if (!c->stream) HIP_OK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+    HIP_OK(hipEventCreate(&c->ev0));
+    HIP_OK(hipEventCreate(&c->ev1));
+    HIP_OK(hipEventCreateWithFlags(&c->ev_in, hipEventDisableTiming));
+    HIP_OK(hipEventCreateWithFlags(&c->ev_out, hipEventDisableTiming));
+  }
+  HostBasis hb;
+  if ((rc = describe_system(s, opt, c, hb))) return rc;
+  const std::vector<Shell>& shells = hb.shells;
+  const std::vector<double>&pexp = hb.pexp, &pcoef = hb.pcoef, &angn = hb.angn;
+  const std::vector<int>& ao_shell = hb.ao_shell;
+  const std::vector<Pair>& pairs = c->h_pairs;
   // device allocations (all of them, here)
   const size_t nbf2 = (size_t)c->nbf * c->nbf;
   HIP_OK(device_buffer(c, c->d_shells, c->nsh));
@@ -1394,54 +1484,14 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
   int ncu = 0;
   HIP_OK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
   c->ncu = ncu;
-  // work lists: the shell pairs, and for systems of up to kSplitMaxPairs pairs
-  // their segments (counts here for unscreened primitive lists, the most a
-  // geometry can give)
-  size_t seg_cap = 0;
-  for (int pc = 0; pc < kNPairClass; ++pc) {
-    WorkList& W0 = c->work[pc][0];
-    W0.off = c->pair_off[pc];
-    W0.n = W0.cap = c->pair_off[pc + 1] - c->pair_off[pc];
-    for (int l = 1; l < kLevels; ++l) {
-      WorkList& W = c->work[pc][l];
-      W.cap = 0;
-      for (int i = c->pair_off[pc]; i < c->pair_off[pc + 1]; ++i)
-        W.cap += std::max(1, (pairs[i].npp + kSegLen[l][pc] - 1) / kSegLen[l][pc]);
-      seg_cap += W.cap;
-    }
-  }
-  // work counters: per part one per energy segment of kSegTiles bra tiles and one
-  // per J/K strip (bra strips, or ket strips transposed); one for the cooperative kernel
-  static_assert(kSegTiles * kTileB == kStripB, "an energy segment covers one bra strip");
-  const bool split = c->npairs <= kSplitMaxPairs;
-  c->ctr_total = 0;
-  for (int bc = 0, q = 0; bc < kNPairClass; ++bc)
-    for (int kc = 0; kc <= bc; ++kc, ++q) {
-      int most = 1;
-      for (int l = 0; l < (split ? kLevels : 1); ++l)
-        most = std::max({most, (c->work[bc][l].cap + kStripB - 1) / kStripB, (c->work[kc][l].cap + kStripK - 1) / kStripK});
-      c->ctr_off[q] = c->ctr_total;
-      c->ctr_len[q] = most * std::max(kPartsEnergy[q], kPartsJk[q]);
-      c->ctr_total += c->ctr_len[q];
-    }
+  const size_t seg_cap = plan_lists(c);
   HIP_OK(device_buffer(c, c->d_tilectr, c->ctr_total));
   HIP_OK(coop_prepare(c->device));
-  // energy partial sums: four slots per workgroup of the largest grid of each class
-  size_t partial_cap = 0;
-  for (int bc = 0, q = 0; bc < kNPairClass; ++bc)
-    for (int kc = 0; kc <= bc; ++kc, ++q) {
-      c->coop_idx[q] = coop_class(kPairLs[bc][0], kPairLs[bc][1], kPairLs[kc][0], kPairLs[kc][1]);
-      const int nb = c->work[bc][0].n, nk = c->work[kc][0].n;
-      if (nb <= 0 || nk <= 0) continue;
-      const size_t blocks = std::min<size_t>(2048, (size_t)class_occupancy(bc, kc, false, false, 0) * ncu);
-      partial_cap += 4 * blocks * class_parts(q, false);
-    }
-  // (also the Fock tiles' shares of E2: at most 20 x 20 per spin)
-  HIP_OK(device_buffer(c, c->d_partial, std::max<size_t>(partial_cap, 512) * 2));
+  HIP_OK(device_buffer(c, c->d_partial, partial_slots(c)));
   // segment lists last: in the allocation-free entry they are left out where
   // the static array has no room for them
   const size_t seg_bytes = seg_cap * (sizeof(Pair) + sizeof(SegSrc)) + 2 * kNQuartetClass * sizeof(QuartetArgs) + 1024;
-  if (split && (!c->arena || c->arena->used + seg_bytes <= c->arena->cap)) {
+  if (seg_cap > 0 && (!c->arena || c->arena->used + seg_bytes <= c->arena->cap)) {
     HIP_OK(device_buffer(c, c->d_split, seg_cap));
     HIP_OK(device_buffer(c, c->d_segsrc, seg_cap));
     HIP_OK(device_buffer(c, c->d_small, 2 * kNQuartetClass));
@@ -1455,10 +1505,7 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
     if (!c->ao_orb.empty())
       HIP_OK(hipMemcpy(c->d_ao_orb.p, c->ao_orb.data(), c->ao_orb.size() * sizeof(int), hipMemcpyHostToDevice));
   }
-  {
-    const int rc = plan_work(c, nullptr);
-    if (rc) return rc;
-  }
+  if ((rc = plan_work(c, nullptr))) return rc;
   // uploads
   static const std::vector<double> boys = make_boys_table();  // the same in every context
   HIP_OK(hipMemcpy(c->d_shells.p, shells.data(), shells.size() * sizeof(Shell), hipMemcpyHostToDevice));
@@ -1487,8 +1534,7 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
 // loops of nearly equal length and Schwarz-skipped quartets cluster.  The
 // order is a schedule only (every unique quartet is still evaluated once); it
 // is recomputed when the coordinates change.
-static int schedule_pairs(vsvb_context* c) {
-  if (c->sched_coords == c->coords) return VSVB_OK;
+static int order_pairs(vsvb_context* c) {
   const int np = c->npairs, nap = c->natom * (c->natom + 1) / 2;
   // Shell pairs of one pair of atoms share the distance: the atom pairs are sorted,
   // and every shell pair goes to the next place of its (class, count) in that order.
@@ -1518,9 +1564,14 @@ static int schedule_pairs(vsvb_context* c) {
       c->h_order[at] = i;
       skept[at] = kept[i];
     }
-  const int rc = plan_work(c, skept.data());
+  return plan_work(c, skept.data());
+}
+
+static int schedule_pairs(vsvb_context* c) {
+  if (c->sched_coords == c->coords) return VSVB_OK;
+  const int rc = order_pairs(c);
   if (rc) return rc;
-  HIP_OK(hipMemcpyAsync(c->d_order.p, c->h_order.data(), np * sizeof(int), hipMemcpyHostToDevice, c->stream));
+  HIP_OK(hipMemcpyAsync(c->d_order.p, c->h_order.data(), c->npairs * sizeof(int), hipMemcpyHostToDevice, c->stream));
   if (!c->h_seg.empty())
     HIP_OK(hipMemcpyAsync(c->d_segsrc.p, c->h_seg.data(), c->h_seg.size() * sizeof(SegSrc), hipMemcpyHostToDevice,
                           c->stream));
@@ -1747,6 +1798,8 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
     offs[q] = poff;
     poff += c->partial_per_class[q];
   }
+  if (!jk && !eri && poff > c->d_partial.n)
+    return fail(VSVB_ERR_UNSUPPORTED, "the energy's partial sums do not fit their buffer");
   const int m = jk ? 1 : 0;
   // Two cooperative classes whose wavefronts all fit the chip at once share a
   // launch: each runs as long as its longest quartet (water: 2 x 36 us one after the
@@ -2981,6 +3034,31 @@ int vsvb_debug_gemm(int32_t M, int32_t N, int32_t K, int32_t ta, int32_t tb, dou
   // row-major storage: op(A) is M x K, so A is stored K x M when transposed
   HIP_OK(gemm(nullptr, M, N, K, alpha, dA.p, ta ? M : K, ta != 0, dB.p, tb ? K : N, tb != 0, beta, dC.p, N));
   HIP_OK(hipMemcpy(C, dC.p, nc * sizeof(double), hipMemcpyDeviceToHost));
+  return VSVB_OK;
+}
+
+int vsvb_debug_plan(const vsvb_system* sys, const vsvb_options* opt, int32_t ncu, double* plan, int64_t* partial) {
+  if (!sys || ncu < 1 || !plan || !partial) return fail(VSVB_ERR_ARG, "invalid plan probe arguments");
+  vsvb_context c;  // host state only
+  c.own_stream = false;
+  HostBasis hb;
+  int rc;
+  if ((rc = read_options(sys, opt, &c))) return rc;
+  if ((rc = describe_system(sys, opt, &c, hb))) return rc;
+  c.ncu = ncu;
+  if (plan_lists(&c) > 0) c.nlevels = kLevels;
+  partial[1] = (int64_t)partial_slots(&c);
+  if ((rc = plan_work(&c, nullptr))) return rc;
+  const size_t unscreened = c.partial_total;
+  if ((rc = order_pairs(&c))) return rc;
+  partial[0] = (int64_t)std::max(unscreened, c.partial_total);
+  for (int m = 0; m < 2; ++m)
+    for (int q = 0; q < kNQuartetClass; ++q) {
+      const ClassLaunch& l = m ? c.ljk[q] : c.le[q];
+      const double row[8] = {(double)l.coop, (double)l.lb, (double)l.lk, (double)l.units, (double)l.blocks,
+                             l.coop ? (double)l.claim : (double)l.kchunk, (double)l.tr, (double)c.in_small[m][q]};
+      std::copy(row, row + 8, plan + (m * kNQuartetClass + q) * 8);
+    }
   return VSVB_OK;
 }
 

@@ -51,7 +51,7 @@ EXPORTS = ["vsvb_context_create", "vsvb_context_destroy", "vsvb_energy", "vsvb_e
            "vsvb_version", "vsvb_batch_uses_graph", "vsvb_batch_tuning", "vsvb_batch_set_graph",
            "vsvb_batch_set_lanes", "vsvb_batch_set_group_launch", "vsvb_batch_launches", "vsvb_debug_gemm",
            "vsvb_spin_matrices", "vsvb_spin_opt", "vsvb_set_spin_coupling", "vsvb_surface",
-           "vsvb_batch_set_coords", "vsvb_surface_batch", "vsvb_energy_grad_static"]
+           "vsvb_batch_set_coords", "vsvb_surface_batch", "vsvb_energy_grad_static", "vsvb_debug_plan"]
 
 _lib = None
 
@@ -100,6 +100,7 @@ def load(path: str = LIB_PATH):
     L.vsvb_batch_set_group_launch.argtypes = [C.c_void_p, C.c_int32]
     L.vsvb_batch_launches.argtypes = [C.c_void_p, _f64p, C.c_int32, C.POINTER(C.c_int32)]
     L.vsvb_energy_grad_static.argtypes = [C.POINTER(CSystem), C.POINTER(COptions), _f64p, _f64p]
+    L.vsvb_debug_plan.argtypes = [C.POINTER(CSystem), C.POINTER(COptions), C.c_int32, _f64p, C.POINTER(C.c_int64)]
     _lib = L
     return L
 
@@ -148,6 +149,17 @@ class _Packed:
                                                 "npair", "nunpd", "ndocc", "ndf", "nspinc", "ntol_d", "ntol_i")},
                           **{k: _ptr(v, _i32p) for k, v in pk.i32.items()},
                           **{k: _ptr(v, _f64p) for k, v in pk.f64.items()})
+
+
+def launch_plan(s: VsvbSystem, ncu: int = 256, pair_chunk: int = 0):
+    """(plan [2, 21, 8], partial sums written, held) of a context of s (vsvb_debug_plan; no device needed)."""
+    plan = np.zeros((2, 21, 8))
+    partial = np.zeros(2, np.int64)
+    pk = _Packed(s)
+    opt = COptions(pair_chunk=pair_chunk)
+    _check(load().vsvb_debug_plan(C.byref(pk.cs), C.byref(opt), ncu, _ptr(plan, _f64p),
+                                  _ptr(partial, C.POINTER(C.c_int64))), "vsvb_debug_plan")
+    return plan, int(partial[0]), int(partial[1])
 
 
 def energy_grad_static(s: VsvbSystem, device: int = 0, want_grad: bool = True):
