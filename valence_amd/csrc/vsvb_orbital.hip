@@ -384,7 +384,8 @@ __device__ void gradient_middle(const OrbArgs& a, double* lds, double* red) {
 }
 
 // Row o of G = dE/dC, 2 (P_s Y_s - V_s T) summed over the spins that hold orbital
-// o, and the gradient of its weights.
+// o, and the gradient of its weights.  Row 0 also writes the zeros of the weights
+// that belong to no occupied orbital.
 __device__ __forceinline__ void gradient_row(const OrbArgs& a, Row r, double* grad, int o, RowScratch& lds) {
   const int tid = r.tid, nt = r.nt, n = a.nbf, ns = a.nsp;
   double* u = lds.w;
@@ -411,6 +412,9 @@ __device__ __forceinline__ void gradient_row(const OrbArgs& a, Row r, double* gr
     const int mu = a.ent[k].tgt;
     grad[k] = a.angn[mu] * a.G[(size_t)o * n + mu];
   }
+  if (o > 0) return;
+  for (int k = tid; k < a.orb_start[0]; k += nt) grad[k] = 0.0;
+  for (int k = a.orb_start[a.nsp] + tid; k < a.totlen; k += nt) grad[k] = 0.0;
 }
 
 template <bool kArray>
