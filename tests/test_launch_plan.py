@@ -26,3 +26,12 @@ def test_partial_sums_of_the_workloads_fit():
     for make in (workloads.config0, workloads.config1, workloads.config2, workloads.config4):
         _, used, held = lib.launch_plan(make())
         assert 0 < used <= held
+
+
+def test_environment_does_not_change_a_plan(monkeypatch):
+    """Plans follow the system alone: no environment variable selects their work lists."""
+    s = workloads.config0()
+    want = lib.launch_plan(s)[0]
+    for value in ("0,0", "1,1", "2,2"):
+        monkeypatch.setenv("VSVB_LV", value)
+        assert (lib.launch_plan(s)[0] == want).all(), value

@@ -831,11 +831,6 @@ constexpr double kTailEnergy = 6.0, kTailJk = 45.0, kTailDensity = 25.0;
 static void choose_levels(const vsvb_context* c, int bc, int kc, bool jk, bool tr, int* lb, int* lk) {
   *lb = *lk = 0;
   if (c->nlevels < 2 || c->pair_chunk > 0) return;  // a forced chunk width: whole pairs
-  if (const char* ev = getenv("VSVB_LV")) {
-    *lb = ev[0] - '0'; *lk = ev[2] - '0';
-    if (bc == kc) *lk = *lb;
-    return;
-  }
   const int q = bc * (bc + 1) / 2 + kc;
   const int nd = jk ? c->ndens : 1;
   const double digest = digestion_flops(q, c->nunpd > 0 ? 2 : 1, jk) * nd;
