@@ -35,3 +35,15 @@ def test_environment_does_not_change_a_plan(monkeypatch):
     for value in ("0,0", "1,1", "2,2"):
         monkeypatch.setenv("VSVB_LV", value)
         assert (lib.launch_plan(s)[0] == want).all(), value
+
+
+@pytest.mark.parametrize("make,shares", [(workloads.config0, True), (workloads.config1, False)])
+def test_forced_chunks_keep_whole_pairs_and_separate_launches(make, shares):
+    """pair_chunk > 0: shell pairs as work lists, a launch per class; by default some
+    classes of these molecules take segments, and water's share a launch."""
+    s = make()
+    default = lib.launch_plan(s)[0]
+    assert default[..., 1:3].any() and (default[..., 7].any() or not shares)
+    for chunk in (1, 2, 64):
+        forced = lib.launch_plan(s, pair_chunk=chunk)[0]
+        assert not forced[..., 1:3].any() and not forced[..., 7].any()

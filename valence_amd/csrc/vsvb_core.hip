@@ -984,7 +984,8 @@ static ClassLaunch policy_launch(vsvb_context* c, int q, const Policy& p) {
 // uncontracted shells.
 constexpr int kSegLen[kLevels][kNPairClass] = {{0, 0, 0, 0, 0, 0}, {9, 6, 3, 3, 1, 1}, {3, 2, 1, 1, 1, 1}};
 // Workgroups up to which a class joins the shared launch of a small system: it
-// runs one workgroup per CU, so a class that fills the chip is faster alone.
+// runs one workgroup per CU, so a class that fills the chip is faster alone.  A
+// forced chunk width keeps every class apart.
 constexpr int kSmallBlocks = 320;
 // Shell pairs up to which a context holds segment lists: above, every class
 // that matters fills the chip with whole pairs.
@@ -1045,7 +1046,7 @@ static int plan_work(vsvb_context* c, const int* kept) {
       const ClassLaunch cl = policy_launch(c, q, c->pol[q]);
       if (!cl.overflow && (cl.units > 0 || c->ljk[q].units <= 0)) c->ljk[q] = cl;
     }
-    if (c->nlevels > 1 && c->ndens == 1 && c->coop_idx[q] < 0) {
+    if (c->nlevels > 1 && c->pair_chunk == 0 && c->ndens == 1 && c->coop_idx[q] < 0) {
       c->in_small[0][q] = c->le[q].units > 0 && c->le[q].kchunk == 1 && c->le[q].blocks * kPartsEnergy[q] <= kSmallBlocks;
       // the shared J/K launch has the transposed units of classes of different bra and ket
       const ClassLaunch cl = straight_launch(c, bc, kc, true, kDefaultJkPerCu, true, bc != kc);
@@ -1798,7 +1799,7 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
   const int m = jk ? 1 : 0;
   // Two cooperative classes whose wavefronts all fit the chip at once share a
   // launch: each runs as long as its longest quartet (water: 2 x 36 us one after the
-  // other, 46 side by side).
+  // other, 46 side by side).  A forced chunk width keeps a launch per class.
   int pair[2] = {-1, -1};
   struct Join {  // on every return path
     hipStream_t st = nullptr;
@@ -1818,7 +1819,7 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
       fit = k == 0 ? coop_occupancy(c->coop_idx[q], jk) : std::min(fit, coop_occupancy(c->coop_idx[q], jk));
       ++k;
     }
-    if (k < 2 || blocks > fit * c->ncu) pair[0] = pair[1] = -1;
+    if (k < 2 || blocks > fit * c->ncu || c->pair_chunk > 0) pair[0] = pair[1] = -1;
   }
   if (pair[0] >= 0) {
     QuartetArgs a[2];
