@@ -18,3 +18,18 @@ def shell_system(ls, natom, nprim=1, norb=2, seed=5):
     atoms = [sorted({k % natom, (k + 1) % natom}) for k in range(norb)]
     orbs = [(a, workloads._rand_orbital(rng, basis, elems, a)) for a in atoms]
     return workloads.assemble(elems, xyz, basis, orbs)
+
+
+def deep_shell_chain(natom, nprim, ls):
+    """A chain of one-primitive shells, 1.6 A apart, behind one atom whose shells have nprim primitives: its
+    pairs' long primitive lists are cut into segments, and the many others fill units of several kets."""
+    rng = np.random.default_rng(11)
+    basis = {"X": (2.0, [(l, np.array([0.9 - 0.2 * l]), np.ones(1)) for l in ls]),
+             "Y": (4.0, [(l, np.sort(np.exp(rng.uniform(np.log(0.2), np.log(500.0), nprim)))[::-1],
+                          rng.uniform(0.1, 1.0, nprim)) for l in ls])}
+    elems = ["Y"] + ["X"] * (natom - 1)
+    xyz = np.zeros((natom, 3))
+    xyz[:, 0] = 1.6 * np.arange(natom)
+    xyz += rng.normal(0.0, 0.05, xyz.shape)
+    orbs = [(a, workloads._rand_orbital(rng, basis, elems, a)) for a in ([0, 1], [2, 3], [60, 61])]
+    return workloads.assemble(elems, xyz, basis, orbs)

@@ -136,6 +136,13 @@ constexpr int kTileB = 64;
 constexpr int kClaimChunk = 16;
 constexpr int kSegTiles = 4;
 
+// Quartets that a screened-out pair of the uniform side leaves unvisited in a tile: the
+// lanes from place lo on that hold a pair's first segment (`first`).  A quartet of
+// segments is counted once, by its first ones.
+__device__ __forceinline__ int first_lanes(unsigned long long first, int lo) {
+  return lo < 64 ? __popcll(first & (~0ull << max(lo, 0))) : 0;
+}
+
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -279,15 +286,14 @@ __device__ __forceinline__ void quartet_energy_body(const QuartetArgs& a, const 
     unsigned long long live = 1;
     if (a.kchunk > 1) {
       const double qmax = wave_max(bra_ok ? P.Q : 0.0);
+      const unsigned long long firsts = __ballot(bra_ok && P.seg == 0);
       const int ikl = k0 + lane;
       bool lv = false;
       if (lane < a.kchunk && ikl < a.nket && (!a.same || ikl <= klast)) {
-        lv = a.ket[ikl].Q * qmax >= a.tau;
-        if (!lv) {  // every bra lane that takes this ket is screened out
-          const int lo = a.same ? max(ikl, tb * kTileB) : tb * kTileB;
-          const int hi = min(a.nbra, tb * kTileB + kTileB);
-          nskip += hi > lo ? hi - lo : 0;
-        }
+        const Pair& K = a.ket[ikl];
+        lv = K.Q * qmax >= a.tau;
+        // every bra lane that takes this ket is screened out
+        if (!lv && K.seg == 0) nskip += first_lanes(firsts, a.same ? ikl - tb * kTileB : 0);
       }
       live = __ballot(lv);
     }
@@ -484,14 +490,14 @@ __device__ __forceinline__ void quartet_jk_body(const QuartetArgs& a, const Plac
       if (lane == 0) s_qmax[wave] = qw;
       __syncthreads();
       const double qmax = fmax(fmax(s_qmax[0], s_qmax[1]), fmax(s_qmax[2], s_qmax[3]));
+      const unsigned long long firsts = __ballot(ib < a.nbra && P.seg == 0);
       const int ikl = k0 + lane;
       bool lv = false;
       if (lane < a.kchunk && ikl < a.nket && (!a.same || ikl <= klast)) {
-        lv = a.ket[ikl].Q * qmax >= a.tau;
-        if (!lv) {  // every bra lane of this wavefront that takes the ket is screened out
-          const int lo = a.same ? max(ikl, tile0) : tile0, hi = min(a.nbra, tile0 + kTileB);
-          nskip += hi > lo ? hi - lo : 0;
-        }
+        const Pair& K = a.ket[ikl];
+        lv = K.Q * qmax >= a.tau;
+        // every bra lane of this wavefront that takes the ket is screened out
+        if (!lv && K.seg == 0) nskip += first_lanes(firsts, a.same ? ikl - tile0 : 0);
       }
       live = __ballot(lv);  // the same in every wavefront of the workgroup
     }
@@ -726,14 +732,13 @@ __device__ __forceinline__ void quartet_jkt_body(const QuartetArgs& a, const Pla
       if (lane == 0) s_qmax[wave] = qw;
       __syncthreads();
       const double qmax = fmax(fmax(s_qmax[0], s_qmax[1]), fmax(s_qmax[2], s_qmax[3]));
+      const unsigned long long firsts = __ballot(kin && K.seg == 0);
       const int ibl = b0 + lane;
       bool lv = false;
       if (lane < a.kchunk && ibl < a.nbra) {
-        lv = a.bra[ibl].Q * qmax >= a.tau;
-        if (!lv) {  // every ket lane of this wavefront is screened out
-          const int hi = min(a.nket, tile0 + kTileB);
-          nskip += hi > tile0 ? hi - tile0 : 0;
-        }
+        const Pair& P = a.bra[ibl];
+        lv = P.Q * qmax >= a.tau;
+        if (!lv && P.seg == 0) nskip += first_lanes(firsts, 0);  // every ket lane of this wavefront is screened out
       }
       live = __ballot(lv);  // the same in every wavefront of the workgroup
     }
