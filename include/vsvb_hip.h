@@ -84,7 +84,11 @@ typedef struct vsvb_context vsvb_context;
 
 /* Creates the device-resident state for one molecule/basis/orbital layout
  * (called where valence_initialize reads the input, src/valence_initialize_module.F90:4-30).
- * All device memory the energy calls need is allocated here. */
+ * All device memory the energy calls need is allocated here.  A spin-coupled
+ * wave function of ten and more orbital pairs (r >= s) also holds the matrix of
+ * its two-electron integrals if that is at most 1 GiB and a sixteenth of the
+ * memory free at creation; otherwise its calls contract them quartet by quartet
+ * (slower; the same energies up to rounding). */
 int vsvb_context_create(const vsvb_system *sys, const vsvb_options *opt, vsvb_context **ctx);
 
 /* Frees everything (valence_finalize, src/valence_finalize_module.F90:3-21). */
@@ -177,6 +181,15 @@ int vsvb_batch_create(int32_t nwfn, const vsvb_system *const *systems, const vsv
 /* energies: [nwfn]; grads: NULL or [nwfn] host pointers of totlen doubles each (NULL entries skipped). */
 int vsvb_batch_run(vsvb_batch *batch, int32_t want_grad, double *energies, double *const *grads);
 void vsvb_batch_destroy(vsvb_batch *batch);
+/* Groups whose J and K come from stored integrals.  A group of eight and more wave
+ * functions on one geometry holds, for the batch's life, two matrices of its
+ * two-electron integrals and its packed densities (8 GB for C8H18's 210 AOs; their
+ * number grows with the fourth power of the AOs) if they are at most 16 GiB and
+ * a sixteenth of the memory free at creation, and no pair_chunk is forced;
+ * otherwise its runs contract the integrals quartet by quartet, as those of
+ * smaller groups do (32 wave functions of C8H18: 46 ms a run instead of 13; the
+ * same results up to rounding).  The matrices are computed anew by every run. */
+int vsvb_batch_stored_groups(vsvb_batch *batch);
 /* 1 when runs replay the captured graph, 0 when they are enqueued directly
  * (before the first run, or after a failed capture: vsvb_last_error says why). */
 int vsvb_batch_uses_graph(vsvb_batch *batch);
@@ -267,6 +280,11 @@ int vsvb_debug_gemm(int32_t M, int32_t N, int32_t K, int32_t ta, int32_t tb, dou
  * partial sums an energy writes (the larger of these coordinates and the
  * unscreened primitive lists), and those its context holds. */
 int vsvb_debug_plan(const vsvb_system *sys, const vsvb_options *opt, int32_t ncu, double *plan, int64_t *partial);
+/* Whether stored two-electron integrals can be set up now for a group of nwfn
+ * wave functions of this system, or (npair > 0) for its orbital-pair densities:
+ * 1, or 0 where they do not fit or their memory is not to be had (diagnostics/
+ * tests; takes the memory and gives it back). */
+int vsvb_debug_stored(const vsvb_system *sys, const vsvb_options *opt, int32_t nwfn);
 /* Library version string. */
 const char *vsvb_version(void);
 

@@ -3058,6 +3058,23 @@ int vsvb_debug_plan(const vsvb_system* sys, const vsvb_options* opt, int32_t ncu
   return VSVB_OK;
 }
 
+int vsvb_debug_stored(const vsvb_system* sys, const vsvb_options* opt, int32_t nwfn) {
+  if (!sys || nwfn < 1) return fail(VSVB_ERR_ARG, "invalid stored-integral probe arguments");
+  vsvb_context c;  // host state only
+  c.own_stream = false;
+  HostBasis hb;
+  StoredIntegrals s;
+  int rc;
+  if ((rc = read_options(sys, opt, &c))) return rc;
+  if ((rc = describe_system(sys, opt, &c, hb))) return rc;
+  (void)hipSetDevice(c.device);
+  if (c.npair > 0)
+    stored_setup(&c, s, 0, 0, kStoredBytes);
+  else
+    stored_setup(&c, s, nwfn, c.nunpd > 0 ? 2 : 1, kStoredGroupBytes);
+  return s.M.p ? 1 : 0;
+}
+
 const char* vsvb_last_error(void) { return g_last_error.c_str(); }
 
 const char* vsvb_version(void) { return "vsvb-mi355x 0.1 (gfx950, FP64 OS/HGP)"; }
@@ -3299,10 +3316,8 @@ int vsvb_batch_create(int32_t nwfn, const vsvb_system* const* systems, const vsv
   for (auto& g : bt->groups) {
     vsvb_context* lead = bt->ctx[g.members[0]];
     if (g.members.size() < 2) continue;
-    if ((int)g.members.size() >= kStoredMembers && lead->npair == 0 && lead->pair_chunk == 0) {
-      const int rc = stored_setup(lead, g.stored, (int)g.members.size(), lead->nunpd > 0 ? 2 : 1, kStoredGroupBytes);
-      if (rc) return rc;
-    }
+    if ((int)g.members.size() >= kStoredMembers && lead->npair == 0 && lead->pair_chunk == 0)
+      stored_setup(lead, g.stored, (int)g.members.size(), lead->nunpd > 0 ? 2 : 1, kStoredGroupBytes);
     // its work lists are planned with the first geometry
     lead->ndens = g.stored.M.p ? 1 : (int)g.members.size();
     const size_t nn = (size_t)lead->nbf * lead->nbf;
@@ -3485,6 +3500,11 @@ int vsvb_batch_tuning(vsvb_batch* b, double* out) {
   if (!b || !out) return fail(VSVB_ERR_ARG, "null argument");
   std::memcpy(out, b->tuning, sizeof(b->tuning));
   return VSVB_OK;
+}
+
+int vsvb_batch_stored_groups(vsvb_batch* b) {
+  if (!b) return fail(VSVB_ERR_ARG, "null batch");
+  return (int)std::count_if(b->groups.begin(), b->groups.end(), [](const BatchGroup& g) { return g.stored.M.p != nullptr; });
 }
 
 int vsvb_batch_uses_graph(vsvb_batch* b) {

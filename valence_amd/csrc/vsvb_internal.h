@@ -105,9 +105,8 @@ struct DevBuf {
     n = count;
     own = false;
   }
-  ~DevBuf() {
-    if (p && own) (void)hipFree(p);
-  }
+  void release() { alias(nullptr, 0); }
+  ~DevBuf() { release(); }
 };
 
 
@@ -330,8 +329,10 @@ hipError_t launch_gather_grad(vsvb_context* c, const double* gradC, double* grad
 int prepare_geometry(vsvb_context* c, const double* coords);
 int prepare_orbital_basis(vsvb_context* c, const double* coeff_host, const double* coeff_dev);
 // Buffers for nwfn wave functions (nspin densities each; 0: the matrix only) if they
-// fit `limit` and a sixteenth of the free memory; otherwise s stays empty.
-int stored_setup(vsvb_context* c, StoredIntegrals& s, int nwfn, int nspin, size_t limit);
+// fit `limit` and a sixteenth of the free memory, and can be allocated; otherwise s
+// stays empty, which is no error.
+constexpr size_t kStoredBytes = (size_t)1 << 30;  // limit of a spin-coupled context
+void stored_setup(vsvb_context* c, StoredIntegrals& s, int nwfn, int nspin, size_t limit);
 int stored_integrals(vsvb_context* c, StoredIntegrals& s);  // M, fn and at of the current geometry
 // What run_quartets' J/K pass leaves in jacc and kacc, up to the order of the sums.
 int stored_jk(vsvb_context* c, StoredIntegrals& s, int nwfn, const double* dens, double* jacc, double* kacc);

@@ -60,7 +60,6 @@ __global__ void k_pair_dens(const double* __restrict__ Cs, const int* __restrict
 // take 0.5 ms this way (0.36 of them the integrals).
 // Below kStoredMin densities the fixed cost (clearing, transposing and reading the
 // matrix, six small launches) is no longer small against what is saved.
-constexpr size_t kStoredBytes = (size_t)1 << 30;
 constexpr int kStoredMin = 10;
 
 // Dp[rs][f]: k_pair_dens' element (mu, nu), doubled where the pair stands for (nu, mu) too.
@@ -697,10 +696,7 @@ int vsvb::sc_setup(vsvb_context* c, const vsvb_system* s) {
   HIP_OK(sc.d_cdet.alloc(cd.size()));
   HIP_OK(sc.d_pq.alloc(pq.size()));
   const size_t nf = (size_t)c->nfun;
-  if (sc.npq >= kStoredMin) {
-    const int rc = stored_setup(c, sc.stored, 0, 0, kStoredBytes);
-    if (rc) return rc;
-  }
+  if (sc.npq >= kStoredMin) stored_setup(c, sc.stored, 0, 0, kStoredBytes);
   if (sc.stored.M.p) {
     c->ndens = 1;  // the quartet pass is an energy pass
     HIP_OK(sc.d_Dp.alloc(sc.npq * nf));

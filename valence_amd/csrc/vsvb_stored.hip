@@ -207,24 +207,33 @@ __global__ void __launch_bounds__(256) k_stored_exchange(const double* __restric
 // Densities padded to what a launch of k_stored_exchange takes at once.
 static int padded(int x) { return x > 16 ? (x + 31) / 32 * 32 : 16; }
 
-int stored_setup(vsvb_context* c, StoredIntegrals& s, int nwfn, int nspin, size_t limit) {
+void stored_setup(vsvb_context* c, StoredIntegrals& s, int nwfn, int nspin, size_t limit) {
   const size_t nf = (size_t)c->nfun, n = (size_t)c->nbf, nt = n * (n + 1) / 2;
   const size_t xp = padded(nwfn * nspin), nd = (n + 15) / 16 * 16;
   const size_t numbers = nf * nf + (nspin > 0 ? nt * nt + 2 * nwfn * nt + n * nd * xp : 0);
   // (many contexts leave room for the next: each takes a sixteenth of what is left)
   size_t free_bytes = 0, total_bytes = 0;
-  HIP_OK(hipMemGetInfo(&free_bytes, &total_bytes));
-  if (numbers * sizeof(double) > std::min(limit, free_bytes / 16)) return VSVB_OK;
-  HIP_OK(s.fn.alloc(nf));
-  HIP_OK(s.at.alloc(nt));
+  hipError_t e = hipMemGetInfo(&free_bytes, &total_bytes);
+  if (e == hipSuccess) limit = std::min(limit, free_bytes / 16);
+  if (numbers * sizeof(double) > limit) return;
+  e = s.fn.alloc(nf);
+  if (e == hipSuccess) e = s.at.alloc(nt);
   if (nspin > 0) {
-    HIP_OK(s.N.alloc(nt * nt));
-    HIP_OK(s.Dp.alloc(nwfn * nt));
-    HIP_OK(s.Jp.alloc(nwfn * nt));
-    HIP_OK(s.Dt.alloc(n * nd * xp));
+    if (e == hipSuccess) e = s.N.alloc(nt * nt);
+    if (e == hipSuccess) e = s.Dp.alloc(nwfn * nt);
+    if (e == hipSuccess) e = s.Jp.alloc(nwfn * nt);
+    if (e == hipSuccess) e = s.Dt.alloc(n * nd * xp);
   }
-  HIP_OK(s.M.alloc(nf * nf));
-  return VSVB_OK;
+  if (e == hipSuccess) e = s.M.alloc(nf * nf);
+  if (e == hipSuccess) return;
+  (void)hipGetLastError();  // the quartet-by-quartet pass runs instead
+  s.M.release();
+  s.N.release();
+  s.Dp.release();
+  s.Jp.release();
+  s.Dt.release();
+  s.at.release();
+  s.fn.release();
 }
 
 int stored_integrals(vsvb_context* c, StoredIntegrals& s) {

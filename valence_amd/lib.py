@@ -51,7 +51,8 @@ EXPORTS = ["vsvb_context_create", "vsvb_context_destroy", "vsvb_energy", "vsvb_e
            "vsvb_version", "vsvb_batch_uses_graph", "vsvb_batch_tuning", "vsvb_batch_set_graph",
            "vsvb_batch_set_lanes", "vsvb_batch_set_group_launch", "vsvb_batch_launches", "vsvb_debug_gemm",
            "vsvb_spin_matrices", "vsvb_spin_opt", "vsvb_set_spin_coupling", "vsvb_surface",
-           "vsvb_batch_set_coords", "vsvb_surface_batch", "vsvb_energy_grad_static", "vsvb_debug_plan"]
+           "vsvb_batch_set_coords", "vsvb_surface_batch", "vsvb_energy_grad_static", "vsvb_debug_plan", "vsvb_debug_stored",
+           "vsvb_batch_stored_groups"]
 
 _lib = None
 
@@ -94,6 +95,7 @@ def load(path: str = LIB_PATH):
     L.vsvb_batch_class_stats.argtypes = [C.c_void_p, _f64p]
     L.vsvb_version.restype = C.c_char_p
     L.vsvb_batch_uses_graph.argtypes = [C.c_void_p]
+    L.vsvb_batch_stored_groups.argtypes = [C.c_void_p]
     L.vsvb_batch_tuning.argtypes = [C.c_void_p, _f64p]
     L.vsvb_batch_set_graph.argtypes = [C.c_void_p, C.c_int32]
     L.vsvb_batch_set_lanes.argtypes = [C.c_void_p, C.c_int32]
@@ -101,6 +103,7 @@ def load(path: str = LIB_PATH):
     L.vsvb_batch_launches.argtypes = [C.c_void_p, _f64p, C.c_int32, C.POINTER(C.c_int32)]
     L.vsvb_energy_grad_static.argtypes = [C.POINTER(CSystem), C.POINTER(COptions), _f64p, _f64p]
     L.vsvb_debug_plan.argtypes = [C.POINTER(CSystem), C.POINTER(COptions), C.c_int32, _f64p, C.POINTER(C.c_int64)]
+    L.vsvb_debug_stored.argtypes = [C.POINTER(CSystem), C.POINTER(COptions), C.c_int32]
     _lib = L
     return L
 
@@ -160,6 +163,15 @@ def launch_plan(s: VsvbSystem, ncu: int = 256, pair_chunk: int = 0):
     _check(load().vsvb_debug_plan(C.byref(pk.cs), C.byref(opt), ncu, _ptr(plan, _f64p),
                                   _ptr(partial, C.POINTER(C.c_int64))), "vsvb_debug_plan")
     return plan, int(partial[0]), int(partial[1])
+
+
+def stored_fits(s: VsvbSystem, nwfn: int = 1, device: int = 0) -> bool:
+    """Whether stored integrals can be set up for nwfn wave functions of s (vsvb_debug_stored)."""
+    pk = _Packed(s)
+    r = load().vsvb_debug_stored(C.byref(pk.cs), C.byref(COptions(device=device)), nwfn)
+    if r < 0:
+        _check(r, "vsvb_debug_stored")
+    return bool(r)
 
 
 def energy_grad_static(s: VsvbSystem, device: int = 0, want_grad: bool = True):
@@ -348,6 +360,13 @@ class Batch:
         if r < 0:
             _check(r, "vsvb_batch_uses_graph")
         return bool(r)
+
+    def stored_groups(self) -> int:
+        """Groups whose J and K come from stored integrals (vsvb_batch_stored_groups)."""
+        r = load().vsvb_batch_stored_groups(self._h)
+        if r < 0:
+            _check(r, "vsvb_batch_stored_groups")
+        return r
 
     def tuning(self) -> np.ndarray:
         """[2, 21, 8] launch choices of the batch tuner (see vsvb_batch_tuning)."""
