@@ -1903,23 +1903,28 @@ int vsvb::run_quartets(vsvb_context* c, bool jk, int nwfn, const double* dens, d
   return VSVB_OK;
 }
 
-// Counters of the last quartet stage.  hcnt: the stage's counters and stamps
-// already gathered to host memory (a batch run), else they are read from the
-// device.  Class times come from the kernels' wall-clock stamps (profiling on);
-// the stage time from the HIP events of a direct run, or, after a graph replay
-// (whose events were not recorded), from the stamps' overall span.
-int vsvb::finish_counters(vsvb_context* c, const unsigned long long* hcnt, bool replayed) {
+// Counters of the last quartet stage.  Class times come from the kernels'
+// wall-clock stamps (profiling on); the stage time from the HIP events of a direct
+// run, or, after a graph replay (whose events were not recorded), from the stamps'
+// overall span.
+int vsvb::finish_counters(vsvb_context* c) {
+  unsigned long long h[kStatWords];
+  const unsigned long long *n = c->h_out.data() + kOutCounters, *stamp = n + kCtrSlots * kCtrStride;
+  std::copy(n, n + kCtrStride, h);
+  for (int s = 1; s < kCtrSlots; ++s)
+    for (int k = 0; k < kCtrStride; ++k) h[k] += n[s * kCtrStride + k];
+  std::copy(stamp, stamp + 2 * kNQuartetClass, h + kCtrStride);
+  return finish_counters(c, h, false);
+}
+
+int vsvb::finish_counters(vsvb_context* c, const unsigned long long* h, bool replayed) {
   if (!c->ran_quartets) {  // a batch-group member: its integrals were counted by the leader
     std::memset(c->class_stats, 0, sizeof(c->class_stats));
     std::memset(c->last_counters, 0, sizeof(c->last_counters));
     return VSVB_OK;
   }
   c->ran_quartets = false;
-  unsigned long long h[kCounterWords];
-  std::memcpy(h, hcnt, sizeof(h));
-  for (int s = 1; s < kCtrSlots; ++s)
-    for (int k = 0; k < kCtrStride; ++k) h[k] += h[s * kCtrStride + k];
-  const unsigned long long* stamp = h + kCtrSlots * kCtrStride;
+  const unsigned long long* stamp = h + kCtrStride;
   const double tick_ms = c->wall_khz > 0 ? 1.0 / c->wall_khz : 0.0;
   const int nspin = c->last_nspin;
   double tot[3] = {0, 0, 0};
@@ -1990,7 +1995,7 @@ static int finish_energy(vsvb_context* c, double* energy, double* parts) {
   if ((rc = fetch_out(c, false))) return rc;
   const double* h = reinterpret_cast<const double*>(c->h_out.data());
   if ((rc = check_status(c, false))) return rc;
-  if ((rc = finish_counters(c, c->h_out.data() + kOutCounters))) return rc;
+  if ((rc = finish_counters(c))) return rc;
   if (!std::isfinite(h[2])) return fail(VSVB_ERR_NUMERIC, "non-finite energy");
   if (energy) *energy = h[2];
   if (parts) {
@@ -2072,7 +2077,7 @@ static int finish_energy_grad(vsvb_context* c, double* energy, double* grad) {
   const double* h = reinterpret_cast<const double*>(c->h_out.data());
   if (grad) std::memcpy(grad, h + kOutGrad, c->totlen * sizeof(double));
   if ((rc = check_status(c, true))) return rc;
-  if ((rc = finish_counters(c, c->h_out.data() + kOutCounters))) return rc;
+  if ((rc = finish_counters(c))) return rc;
   const double e = h[0] + h[3] + c->enuc;
   if (!std::isfinite(e)) return fail(VSVB_ERR_NUMERIC, "non-finite energy");
   if (energy) *energy = e;
@@ -2233,7 +2238,7 @@ static void assign_lanes(vsvb_batch* b, int nl) {
   b->planned = false;
 }
 
-constexpr int kCnt = kCounterWords;  // counters and timing stamps per context
+constexpr int kCnt = kStatWords;  // counters and timing stamps per context
 
 // All device work of one batch run, no host synchronization.  The groups run
 // on the lane streams, which fork from the batch stream at the start and join
@@ -2535,7 +2540,12 @@ __global__ void k_gather(const GatherItem* __restrict__ items, double* __restric
   const int* status = reinterpret_cast<const int*>(x.out + kOutStatus);
   if (threadIdx.x == 0) e[blockIdx.x] = x.spin_coupled ? scal[2] : scal[0] + scal[3] + x.enuc;
   if (threadIdx.x < 4) st[4 * blockIdx.x + threadIdx.x] = status[threadIdx.x];
-  for (int k = threadIdx.x; k < kCnt; k += blockDim.x) cnt[(size_t)kCnt * blockIdx.x + k] = x.out[kOutCounters + k];
+  for (int k = threadIdx.x; k < kCnt; k += blockDim.x) {  // the copies added up, then the stamps
+    const unsigned long long* n = x.out + kOutCounters;
+    unsigned long long s = k < kCtrStride ? 0 : n[kCtrSlots * kCtrStride + k - kCtrStride];
+    for (int m = 0; m < (k < kCtrStride ? kCtrSlots : 0); ++m) s += n[m * kCtrStride + k];
+    cnt[(size_t)kCnt * blockIdx.x + k] = s;
+  }
   for (int k = threadIdx.x; k < x.len; k += blockDim.x)
     g[x.goff + k] = reinterpret_cast<const double*>(x.out + kOutGrad)[k];
 }
@@ -3198,7 +3208,7 @@ int vsvb_energy_grad_device(vsvb_context* c, const double* coeff_device, double*
   if ((rc = check_status(c, true))) return rc;
   if (c->npair > 0 && reinterpret_cast<const int*>(c->h_out.data() + kOutStatus)[3])
     return fail(VSVB_ERR_UNSUPPORTED, "gradient at a singular spin-coupled transition overlap");
-  return finish_counters(c, c->h_out.data() + kOutCounters);
+  return finish_counters(c);
 }
 
 int vsvb_debug_buffer(vsvb_context* c, const char* name, double* out, int64_t n) {

@@ -21,6 +21,7 @@ constexpr size_t kMaxLdsK = 60 * 1024;
 // {evaluated, primitive quartets, skipped, spare}, then per class {earliest
 // start, latest end} stamps.
 constexpr int kCounterWords = kCtrSlots * kCtrStride + 2 * kNQuartetClass;
+constexpr int kStatWords = kCtrStride + 2 * kNQuartetClass;  // the same with the copies added up
 constexpr int kOutStatus = 16, kOutCounters = kOutStatus + 2, kOutGrad = kOutCounters + kCounterWords;  // words of d_out
 
 extern thread_local std::string g_last_error;
@@ -339,7 +340,8 @@ int stored_jk(vsvb_context* c, StoredIntegrals& s, int nwfn, const double* dens,
 int run_quartets(vsvb_context* c, bool jk, int nwfn = 1, const double* dens = nullptr,
                  double* jacc = nullptr, double* kacc = nullptr, int nspin_override = -1, double* eri = nullptr);
 int fetch_out(vsvb_context* c, bool grad);  // the call's results into h_out, after everything on its stream
-int finish_counters(vsvb_context* c, const unsigned long long* host_counters, bool replayed = false);
+int finish_counters(vsvb_context* c, const unsigned long long* stats, bool replayed);  // kStatWords
+int finish_counters(vsvb_context* c);  // of h_out, after a direct call
 int check_status(vsvb_context* c, bool for_grad);
 
 hipError_t launch_orbital_front(hipStream_t st, const OrbArgs& one, const OrbArgs* recs, int nrec, const ZeroArgs& z);

@@ -896,7 +896,7 @@ int vsvb::sc_finish(vsvb_context* c, double* energy, double* parts, double* grad
   if (grad_host && reinterpret_cast<const int*>(c->h_out.data() + kOutStatus)[3])
     return fail(VSVB_ERR_UNSUPPORTED, "gradient at a singular or nearly singular transition overlap of the "
                                       "spin-coupled expansion (pivot ratio below 1e-9); the energy is exact there");
-  if ((rc = finish_counters(c, c->h_out.data() + kOutCounters))) return rc;
+  if ((rc = finish_counters(c))) return rc;
   if (!std::isfinite(h[2])) return fail(VSVB_ERR_NUMERIC, "non-finite energy");
   if (energy) *energy = h[2];
   if (parts) {
