@@ -410,7 +410,6 @@ def gen_class(la, lb, lc, ld, uniform_bra=False, part=None):
 # C8H18, in 36 parts against this kernel: (dd|dp) 0.075 and 0.17 ms in energy
 # mode but 0.18 and 0.18 ms in J/K mode, (dd|dd) 0.05 and 0.08, 0.11 and 0.08 ms,
 # for ten minutes of compilation.
-COOP_DEFAULT = [(2, 2, 2, 1), (2, 2, 2, 2)]
 COOP_CLASSES = [(2, 2, 2, 1), (2, 2, 2, 2)]
 
 
@@ -613,10 +612,8 @@ def write_coop(path: str) -> None:
     lines.append("static const CoopDesc kCoopDesc[kNCoop] = {")
     for d in descs:
         la, lb, lc, ld = d["cls"]
-        dflt = 1 if d["cls"] in COOP_DEFAULT else 0
         lines.append(f"  {{{la}, {lb}, {lc}, {ld}, {d['nT']}, {d['nV']}, {d['nH']}, {d['lds']}, {d['nbase']}, {d['base']}, "
-                     f"{d['nvl']}, {d['voff']}, {d['vsteps']}, {d['targ']}, {d['nhl']}, {d['hoff']}, {d['hsteps']}, {d['out']}, "
-                     f"{dflt}}},")
+                     f"{d['nvl']}, {d['voff']}, {d['vsteps']}, {d['targ']}, {d['nhl']}, {d['hoff']}, {d['hsteps']}, {d['out']}}},")
     lines.append("};")
     text = "\n".join(lines) + "\n"
     if not os.path.exists(path) or open(path).read() != text:

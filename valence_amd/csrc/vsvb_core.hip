@@ -1,14 +1,14 @@
-// VSVB energy path on MI355X: context, device preparation kernels, one-electron
-// integrals, orbital-space algebra, energy and adjoint gradient, C ABI.
+// VSVB energy path on MI355X: context, schedule and launch plans, dense products,
+// energy and adjoint gradient, batches, C ABI.
 //
 // Per call (all on the context's stream, inputs already resident):
-//   geometry  -> primitive-pair data, S_ao / h_ao (Obara-Saika), Schwarz bounds
+//   geometry  -> primitive-pair data, S_ao / h_ao (Obara-Saika), Schwarz bounds (vsvb_pairs.hip)
 //   weights   -> effective orbital weights C (NDF expansion, angn scaling) and the
 //                reference's per-(orbital, shell) weight screen for the ERIs
 //   S = C S_ao C^T, h = C h_ao C^T, P = S^-1 per spin block (closed form of the
 //   first- and second-order cofactors of the spin-orbital overlap), R = C' P C'^T
 //   E1 = sum_s w_s tr(h_s P_s), E2 from the shell-quartet kernels, E = E1 + E2 + E_nuc
-//   gradient: J/K from the same quartets (recomputed, never stored), then
+//   gradient: J/K from the same quartets (computed anew by every call), then
 //   dE/dC_s = 2 P_s C_s F_s (1 - R_s S_ao) with F_s = dE/dR_s.
 #include <hip/hip_runtime.h>
 
@@ -535,8 +535,6 @@ hipError_t vsvb::launch_fill(hipStream_t st, double* p, size_t n, double v) {
   return hipGetLastError();
 }
 
-// Clearing counters, flags and status words is done by a kernel, not a memset,
-// so that the same code can be captured into a HIP graph.
 // Per-class timing slots before a stage: even words (earliest start) ~0, odd
 // words (latest end) 0.  A kernel, not a memset: it may be captured in a graph.
 __global__ void k_stamp_reset(unsigned long long* __restrict__ p, int n) {
@@ -570,6 +568,8 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, size_t n, uint32_t v) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
 }
 
+// Clearing counters, flags and status words is done by a kernel, not a memset,
+// so that the same code can be captured into a HIP graph.
 hipError_t vsvb::launch_zero(hipStream_t st, void* p, size_t bytes) {
   const size_t n = bytes / sizeof(uint32_t);
   hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)std::min<size_t>(256, (n + 255) / 256 + 1)), dim3(256), 0, st,
@@ -739,46 +739,6 @@ static int class_occupancy(int bc, int kc, bool jk, bool tr, size_t lds) {
     case 5: return occupancy_b5(kc, jk, tr, lds);
   }
   return 1;
-}
-
-static size_t class_scratch(int bc, int kc, bool jk, bool tr) {
-  switch (bc) {
-    case 0: return scratch_b0(kc, jk, tr);
-    case 1: return scratch_b1(kc, jk, tr);
-    case 2: return scratch_b2(kc, jk, tr);
-    case 3: return scratch_b3(kc, jk, tr);
-    case 4: return scratch_b4(kc, jk, tr);
-    case 5: return scratch_b5(kc, jk, tr);
-  }
-  return 0;
-}
-
-// A straight-line kernel that spills more than this per lane is not launched
-// where the class has cooperative step tables: the runtime reserves scratch
-// for a spilling dispatch on every hardware queue that runs one, and the
-// batch's group streams run such classes on several queues at once.
-constexpr size_t kMaxSpillPerLane = 2048;
-
-// Spill bytes per lane of every straight-line class kernel: [class][energy, J/K, J/K transposed].
-static const size_t* straight_spills() {
-  static size_t tab[kNQuartetClass][3];
-  static std::once_flag once;
-  std::call_once(once, [] {
-    for (int bc = 0, q = 0; bc < kNPairClass; ++bc)
-      for (int kc = 0; kc <= bc; ++kc, ++q) {
-        tab[q][0] = class_scratch(bc, kc, false, false);
-        tab[q][1] = class_scratch(bc, kc, true, false);
-        tab[q][2] = bc != kc ? class_scratch(bc, kc, true, true) : tab[q][1];
-      }
-  });
-  return &tab[0][0];
-}
-
-// The straight-line kernel of class q may run (mode jk, orientation tr): it
-// spills little, or the class has no cooperative kernel to run instead.
-static bool straight_allowed(const vsvb_context* c, int q, bool jk, bool tr) {
-  if (c->coop_idx[q] < 0) return true;
-  return straight_spills()[q * 3 + (jk ? (tr ? 2 : 1) : 0)] <= kMaxSpillPerLane;
 }
 
 static int quartet_class_index(int bc, int kc) { return bc * (bc + 1) / 2 + kc; }
@@ -975,7 +935,7 @@ static ClassLaunch coop_launch(vsvb_context* c, int q, bool jk, int per_cu, int 
 
 static ClassLaunch policy_launch(vsvb_context* c, int q, const Policy& p) {
   const int bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
-  if (p.coop && c->coop_idx[q] >= 0) return coop_launch(c, q, true, p.per_cu, p.claim);
+  if (c->coop_idx[q] >= 0) return coop_launch(c, q, true, p.per_cu, p.claim);
   return straight_launch(c, bc, kc, true, p.per_cu, p.lds_on, p.tr);
 }
 
@@ -1034,12 +994,10 @@ static int plan_work(vsvb_context* c, const int* kept) {
   }
   for (int q = 0; q < kNQuartetClass; ++q) {
     const int bc = class_bra(q), kc = q - quartet_class_index(bc, 0);
-    const bool coop = coop_default(c->coop_idx[q]);
-    const bool tr = transposed_default(c, bc, kc);
-    const bool coop_e = coop || !straight_allowed(c, q, false, false);
-    const bool coop_jk = coop || !straight_allowed(c, q, true, tr);
-    c->le[q] = coop_e ? coop_launch(c, q, false, 0, 0) : straight_launch(c, bc, kc, false, 0, false, false);
-    c->ljk[q] = coop_jk ? coop_launch(c, q, true, 0, 0) : straight_launch(c, bc, kc, true, kDefaultJkPerCu, true, tr);
+    const bool coop = c->coop_idx[q] >= 0;  // its step tables are all the class has
+    c->le[q] = coop ? coop_launch(c, q, false, 0, 0) : straight_launch(c, bc, kc, false, 0, false, false);
+    c->ljk[q] = coop ? coop_launch(c, q, true, 0, 0)
+                     : straight_launch(c, bc, kc, true, kDefaultJkPerCu, true, transposed_default(c, bc, kc));
     if (c->le[q].overflow || c->ljk[q].overflow)
       return fail(VSVB_ERR_UNSUPPORTED, "shell-pair classes too large for 32-bit work-unit indices");
     if (c->has_pol[q]) {
@@ -1088,11 +1046,11 @@ static hipError_t device_buffer(vsvb_context* c, vsvb::DevBuf<T>& b, size_t coun
   return c->arena ? b.carve(*c->arena, count) : b.alloc(count);
 }
 
-// The orbital algebra of this wave function runs in one workgroup
+// The orbital algebra of this wave function runs along its entry lists
 // (vsvb_orbital.hip): few enough orbitals for its LDS and no more than AOs (its
 // m x m results stand in nsp x nbf arrays), no NDFs, no spin-coupled pairs, and no
 // spin block that is to be inverted grid-wide.
-static bool one_block_orbitals(const vsvb_context* c) {
+static bool entry_list_orbitals(const vsvb_context* c) {
   return c->ndf == 0 && c->npair == 0 && c->nsp <= std::min(kOrbMax, c->nbf) && c->nbf <= kOrbMaxBasis &&
          std::max(c->nalpha_rows, c->ndocc) < c->grid_inverse_min;
 }
@@ -1328,7 +1286,7 @@ static int describe_system(const vsvb_system* s, const vsvb_options* opt, vsvb_c
       c->ent[k] = e;
     }
   }
-  // the orbitals that hold each AO (each once), for the one-workgroup orbital algebra
+  // the orbitals that hold each AO (each once), for the entry-list orbital algebra
   c->ao_ptr.assign(c->nbf + 1, 0);
   if (c->ndf == 0) {
     std::vector<std::vector<int>> of(c->nbf);
@@ -1494,7 +1452,7 @@ static int build_context(const vsvb_system* s, const vsvb_options* opt, vsvb_con
     c->nlevels = kLevels;
   }
   const size_t list_bytes = (c->ao_ptr.size() + c->ao_orb.size()) * sizeof(int) + 1024;
-  if (one_block_orbitals(c) && (!c->arena || c->arena->used + list_bytes <= c->arena->cap)) {
+  if (entry_list_orbitals(c) && (!c->arena || c->arena->used + list_bytes <= c->arena->cap)) {
     HIP_OK(device_buffer(c, c->d_ao_ptr, c->ao_ptr.size()));
     HIP_OK(device_buffer(c, c->d_ao_orb, c->ao_orb.size()));
     HIP_OK(hipMemcpy(c->d_ao_ptr.p, c->ao_ptr.data(), c->ao_ptr.size() * sizeof(int), hipMemcpyHostToDevice));
@@ -1662,8 +1620,8 @@ static ZeroArgs pass_zero(vsvb_context* c, int pass, int nwfn, double* jacc, dou
 }
 
 // Orbital stage of one wave function; pass: the quartet pass that follows (1
-// energy, 2 J/K of this wave function alone, 0 neither), cleared along where the
-// algebra runs in one workgroup.
+// energy, 2 J/K of this wave function alone, 0 neither), cleared along by the
+// entry-list algebra.
 static int prepare_orbitals(vsvb_context* c, const double* coeff_host, const double* coeff_dev, int pass) {
   int rc;
   c->cleared = 0;
@@ -2104,7 +2062,7 @@ constexpr size_t kStoredGroupBytes = (size_t)16 << 30;
 struct BatchGroup {
   std::vector<int> members;  // indices into vsvb_batch::ctx; members[0] leads
   DevBuf<double> dens, jacc, kacc;
-  DevBuf<OrbArgs> orec;           // the members' orbital records, when they run in one workgroup each
+  DevBuf<OrbArgs> orec;           // the members' orbital records, when they have entry lists
   std::vector<OrbArgs> h_orec;
   StoredIntegrals stored;         // of a group of many densities
 };
@@ -2379,7 +2337,7 @@ static int batch_plan(vsvb_batch* b) {
   return VSVB_OK;
 }
 
-// Every member's orbital algebra runs in one workgroup: one launch takes them all.
+// Every member's orbital algebra runs along its entry lists: the group shares its launches.
 static bool group_one_launch(const vsvb_batch* b, const BatchGroup& g) {
   if (g.members.size() < 2) return false;
   const vsvb_context* lead = b->ctx[g.members[0]];
@@ -2531,8 +2489,7 @@ static int batch_launch_stats(vsvb_batch* b) {
   return VSVB_OK;
 }
 
-// Results of every wave function into the batch's gather arrays.
-// One wave function's results for the arrays a replay reads back.
+// Results of every wave function into the arrays a replay reads back, a workgroup each.
 __global__ void k_gather(const GatherItem* __restrict__ items, double* __restrict__ e, double* __restrict__ g,
                          int* __restrict__ st, unsigned long long* __restrict__ cnt) {
   const GatherItem x = items[blockIdx.x];
@@ -2578,8 +2535,8 @@ static int batch_gather(vsvb_batch* b) {
 // most density work -- times every candidate configuration of every class on its
 // own data: the straight-line kernel with 1 or 2 workgroups per CU, with or
 // without the LDS exchange staging, in both orientations (classes with
-// different bra and ket classes), and the cooperative kernel (classes with step
-// tables) with automatic, 1-, 8- or 64-unit claims and 8, 4 or 2 workgroups
+// different bra and ket classes); for classes with step tables the cooperative
+// kernel with automatic, 1-, 8- or 64-unit claims and 8, 4 or 2 workgroups
 // per CU.  Both kernels stay below their occupancy: a class timed alone often
 // ranks 4 or as many straight-line workgroups per CU as fit first, and as many
 // cooperative ones as fit, but in the batch four lane streams run classes side
@@ -2618,39 +2575,39 @@ static int tune_leader(vsvb_batch* b, BatchGroup* gs, double (*tuning)[kTuneCols
       const int q = quartet_class_index(bc, kc);
       if (L->ljk[q].units <= 0 || L->in_small[1][q]) continue;  // (small classes share one launch)
       std::vector<Policy> cand;
+      const bool coop = L->coop_idx[q] >= 0;
       Policy d0;  // the default
-      d0.coop = L->ljk[q].coop;
       d0.tr = L->ljk[q].tr;
-      d0.per_cu = L->ljk[q].coop ? 8 : 2;
+      d0.per_cu = coop ? 8 : 2;
       cand.push_back(d0);
-      const bool st_n = straight_allowed(L, q, true, false), st_t = bc != kc && straight_allowed(L, q, true, true);
-      for (int pc : {1, 2})
-        for (bool lds : {true, false}) {
-          Policy p;
-          p.per_cu = pc;
-          p.lds_on = lds;
-          if (st_n) cand.push_back(p);
-          if (st_t && lds) {
-            p.tr = true;
-            cand.push_back(p);
-          }
-        }
-      if (st_t) {
-        Policy p;
-        p.tr = true;
-        p.lds_on = false;
-        p.per_cu = 2;
-        cand.push_back(p);
-      }
-      if (L->coop_idx[q] >= 0)
+      if (coop) {
         for (int pc : {8, 4, 2})
           for (int cl : {0, 1, 8, 64}) {
             Policy p;
-            p.coop = true;
             p.per_cu = pc;
             p.claim = cl;
             cand.push_back(p);
           }
+      } else {
+        for (int pc : {1, 2})
+          for (bool lds : {true, false}) {
+            Policy p;
+            p.per_cu = pc;
+            p.lds_on = lds;
+            cand.push_back(p);
+            if (bc != kc && lds) {
+              p.tr = true;
+              cand.push_back(p);
+            }
+          }
+        if (bc != kc) {
+          Policy p;
+          p.tr = true;
+          p.lds_on = false;
+          p.per_cu = 2;
+          cand.push_back(p);
+        }
+      }
       double tbest = 1e30, tdef = 0.0;
       for (size_t k = 0; k < cand.size(); ++k) {
         const ClassLaunch cl = policy_launch(L, q, cand[k]);
@@ -2684,7 +2641,7 @@ static int tune_leader(vsvb_batch* b, BatchGroup* gs, double (*tuning)[kTuneCols
         tbest = tdef;
       }
       double* t = tuning[q];
-      t[0] = best[q].coop ? 1 : 0;
+      t[0] = coop ? 1 : 0;
       t[1] = best[q].per_cu;
       t[2] = best[q].lds_on ? 1 : 0;
       t[3] = best[q].claim;

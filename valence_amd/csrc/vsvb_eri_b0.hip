@@ -25,11 +25,4 @@ int occupancy_b0(int kc, bool jk, bool tr, size_t lds) {
   }
 }
 
-size_t scratch_b0(int kc, bool jk, bool tr) {
-  switch (kc) {
-    case 0: return scratch_q<0, 0, 0, 0>(jk, tr);
-    default: return 0;
-  }
-}
-
 }  // namespace vsvb

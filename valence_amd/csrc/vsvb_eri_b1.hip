@@ -28,12 +28,4 @@ int occupancy_b1(int kc, bool jk, bool tr, size_t lds) {
   }
 }
 
-size_t scratch_b1(int kc, bool jk, bool tr) {
-  switch (kc) {
-    case 0: return scratch_q<1, 0, 0, 0>(jk, tr);
-    case 1: return scratch_q<1, 0, 1, 0>(jk, tr);
-    default: return 0;
-  }
-}
-
 }  // namespace vsvb

@@ -31,13 +31,4 @@ int occupancy_b2(int kc, bool jk, bool tr, size_t lds) {
   }
 }
 
-size_t scratch_b2(int kc, bool jk, bool tr) {
-  switch (kc) {
-    case 0: return scratch_q<1, 1, 0, 0>(jk, tr);
-    case 1: return scratch_q<1, 1, 1, 0>(jk, tr);
-    case 2: return scratch_q<1, 1, 1, 1>(jk, tr);
-    default: return 0;
-  }
-}
-
 }  // namespace vsvb

@@ -34,14 +34,4 @@ int occupancy_b3(int kc, bool jk, bool tr, size_t lds) {
   }
 }
 
-size_t scratch_b3(int kc, bool jk, bool tr) {
-  switch (kc) {
-    case 0: return scratch_q<2, 0, 0, 0>(jk, tr);
-    case 1: return scratch_q<2, 0, 1, 0>(jk, tr);
-    case 2: return scratch_q<2, 0, 1, 1>(jk, tr);
-    case 3: return scratch_q<2, 0, 2, 0>(jk, tr);
-    default: return 0;
-  }
-}
-
 }  // namespace vsvb

@@ -37,15 +37,4 @@ int occupancy_b4(int kc, bool jk, bool tr, size_t lds) {
   }
 }
 
-size_t scratch_b4(int kc, bool jk, bool tr) {
-  switch (kc) {
-    case 0: return scratch_q<2, 1, 0, 0>(jk, tr);
-    case 1: return scratch_q<2, 1, 1, 0>(jk, tr);
-    case 2: return scratch_q<2, 1, 1, 1>(jk, tr);
-    case 3: return scratch_q<2, 1, 2, 0>(jk, tr);
-    case 4: return scratch_q<2, 1, 2, 1>(jk, tr);
-    default: return 0;
-  }
-}
-
 }  // namespace vsvb

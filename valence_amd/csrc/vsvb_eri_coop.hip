@@ -1,6 +1,6 @@
 // Cooperative shell-quartet kernel for the classes whose one-lane-per-quartet
-// code does not fit the register file ((dd|pp), (dd|dp), (dd|dd)): one
-// wavefront evaluates one contracted quartet.
+// code does not fit the register file ((dd|dp), (dd|dd); the other d-heavy ones
+// run in parts): one wavefront evaluates one contracted quartet.
 //
 // The same Obara-Saika VRR and Head-Gordon-Pople HRR as the straight-line
 // kernels (csrc/gen_eri.py), executed from step tables: every intermediate
@@ -24,7 +24,6 @@ struct CoopDesc {
   int targ;
   int nhl, hoff, hsteps;
   int out;
-  int dflt;  // used by default (the batch tuner may switch any class with tables)
 };
 
 #include "coop_tables.inc"
@@ -372,8 +371,6 @@ size_t coop_lds_bytes(int idx, bool jk) {
   }
   return n * sizeof(double);
 }
-
-bool coop_default(int idx) { return idx >= 0 && kCoopDesc[idx].dflt != 0; }
 
 int coop_occupancy(int idx, bool jk) {
   struct Table {

@@ -1,18 +1,19 @@
 // Shell-quartet ERI kernels for the VSVB energy path (gfx950, FP64).
 //
-// One thread evaluates one unique AO shell quartet (bra pair >= ket pair) of a
-// fixed angular-momentum class with the generated Obara-Saika / Head-Gordon-
-// Pople code, then contracts the cartesian block on the fly with the AO
-// densities of every wave function that shares the geometry; no ERI is ever
-// stored.  In energy mode a wavefront takes a unit of 64 bra pairs (one per
-// lane) and a chunk of ket pairs, visited one at a time (wave-uniform: the
-// ket's pair and primitive data are scalar loads).  A grid sized to the
-// occupancy takes units from an atomic counter; each wave keeps its own
-// partial sum, so the partials are few (the final sum is over a fixed-size
-// array).  Pairs
-// inside a class are sorted by primitive-pair count, then by centre distance,
-// so a wavefront's lanes run primitive loops of the same length and the
-// Schwarz-skipped quartets gather in the same wavefronts.
+// One thread evaluates one unique AO shell quartet (bra pair >= ket pair), or a
+// quartet of segments of the pairs' primitive lists, of a fixed angular-momentum
+// class with the generated Obara-Saika / Head-Gordon-Pople code, then contracts
+// the cartesian block on the fly with the AO densities of every wave function that
+// shares the geometry, or, where an array for them is given (QuartetArgs::eri),
+// adds it to the stored integrals.  In energy mode a wavefront takes units of 64
+// bra pairs (one per lane) and a chunk of ket pairs, visited one at a time
+// (wave-uniform: the ket's pair and primitive data are scalar loads).  Units go to
+// the wavefronts of a grid sized to the occupancy by a fixed rule, and from work
+// counters where chunks are wide; each wave keeps its own partial sum, so the
+// partials are few (the final sum is over a fixed-size array).  Pairs inside a class
+// are sorted by primitive-pair count, then by centre distance, so a wavefront's
+// lanes run primitive loops of the same length and the Schwarz-skipped quartets
+// gather in the same wavefronts.
 //
 // Density contraction (closed or open shell; RT = Coulomb density, D_s the
 // exchange densities with weight x_s), per unique quartet of degeneracy deg:
@@ -985,13 +986,6 @@ static int occupancy_q(bool jk, bool tr, size_t lds_bytes) {
   return blocks_per_cu(attributes_q<LA, LB, LC, LD>(jk, tr), 256, jk ? lds_bytes : 0);
 }
 
-// Private (scratch) bytes per lane of the straight-line kernel of a class in
-// one mode and orientation: the register spills of its generated code.
-template <int LA, int LB, int LC, int LD>
-static size_t scratch_q(bool jk, bool tr) {
-  return attributes_q<LA, LB, LC, LD>(jk, tr).localSizeBytes;
-}
-
 template <int LA, int LB, int LC, int LD>
 static hipError_t launch_q(const QuartetArgs& a, bool jk, bool tr, int nblocks, size_t lds_bytes, hipStream_t st) {
   if (nblocks <= 0 || a.ntiles <= 0) return hipSuccess;
@@ -1048,16 +1042,10 @@ hipError_t launch_quartet_b5(int kc, const QuartetArgs& a, bool jk, bool tr, int
 hipError_t launch_groups_b5(int kc, const QuartetArgs* gs, int ng, bool tr, int nblocks, size_t lds,
                             unsigned long long* stamp, hipStream_t st);
 int occupancy_b0(int kc, bool jk, bool tr, size_t lds);
-size_t scratch_b0(int kc, bool jk, bool tr);
 int occupancy_b1(int kc, bool jk, bool tr, size_t lds);
-size_t scratch_b1(int kc, bool jk, bool tr);
 int occupancy_b2(int kc, bool jk, bool tr, size_t lds);
-size_t scratch_b2(int kc, bool jk, bool tr);
 int occupancy_b3(int kc, bool jk, bool tr, size_t lds);
-size_t scratch_b3(int kc, bool jk, bool tr);
 int occupancy_b4(int kc, bool jk, bool tr, size_t lds);
-size_t scratch_b4(int kc, bool jk, bool tr);
 int occupancy_b5(int kc, bool jk, bool tr, size_t lds);
-size_t scratch_b5(int kc, bool jk, bool tr);
 
 }  // namespace vsvb

@@ -159,7 +159,6 @@ struct SpinCoupled {
 
 // How one quartet class is launched in J/K mode (the batch tuner's choice).
 struct Policy {
-  bool coop = false;
   int per_cu = 0;
   bool lds_on = true;
   int claim = 0;
@@ -199,8 +198,9 @@ struct SmallLaunch {
   unsigned lds = 0;  // J/K: dynamic LDS, the largest of the classes' exchange staging
 };
 
-// Orbital algebra of one wave function (vsvb_orbital.hip): orbitals up to which
-// it runs in one workgroup, its buffers, and what a quartet pass needs cleared.
+// Orbital algebra of one wave function along its entry lists (vsvb_orbital.hip):
+// most orbitals (two square matrices in LDS) and AOs, its buffers, and what a quartet
+// pass needs cleared.
 constexpr int kOrbMax = 64;
 constexpr int kOrbMaxBasis = 640;
 struct OrbArgs {
@@ -352,7 +352,6 @@ hipError_t launch_small(const SmallLaunch& s, const QuartetArgs* gs, bool jk, hi
 // cooperative kernel for the register-heavy classes (vsvb_eri_coop.hip)
 int coop_class(int la, int lb, int lc, int ld);  // index of the class, or -1
 int coop_occupancy(int idx, bool jk);
-bool coop_default(int idx);
 hipError_t coop_prepare(int device);              // step tables resident on the device
 hipError_t launch_coop(int idx, const QuartetArgs& a, bool jk, int nblocks, int device, hipStream_t st);
 // J/K mode over ng groups' arguments (device array gs) in one launch; stamp: the
