@@ -130,8 +130,8 @@ int vsvb_energy_grad_device(vsvb_context *ctx, const double *coeff_device, doubl
  * library's static 32 MiB device scratch array (one per GPU, held until the
  * process ends); the call allocates and frees nothing, creates no stream or
  * event, and runs on the null stream of opt->device (opt may be NULL).
- * Systems whose buffers exceed the array (C8H18 needs about 11 MiB, C12H26
- * with 310 AOs about 23 MiB) and spin-coupled wave functions (npair > 0) are
+ * Systems whose buffers exceed the array (C8H18 needs about 10 MiB, C12H26
+ * with 310 AOs about 21 MiB) and spin-coupled wave functions (npair > 0) are
  * refused with
  * VSVB_ERR_UNSUPPORTED.  Calls on one GPU share the array: they are
  * serialized by a lock inside the process.  energy: [1]; grad: NULL or
