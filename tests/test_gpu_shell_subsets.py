@@ -1,5 +1,6 @@
 """Bases without some angular momenta, of few and of contracted shells: the energy
-against the oracle to 1e-9 Eh, and the energy of the J/K pass to 1e-10 Eh of it.
+against the oracle to 1e-9 Eh, and the energy of the J/K pass to 1e-10 Eh of it, at three geometries; at
+the widest no primitive pair of two atoms passes the screen.
 Eight d shells, and one of six primitives, have more workgroups of the cooperative
 kernel than any other class.
 """
@@ -26,12 +27,13 @@ def test_energy_matches_oracle(lib, ls, natom, nprim):
     _, used, held = lib.launch_plan(s)
     print(f"l {ls}, {natom} atoms, {nprim} primitives: {used} of {held} partial sums", flush=True)
     assert used <= held
-    ref = oracle.energy(s).energy
     with lib.Context(s) as ctx:
-        for scale in (1.0, 1.5):
-            e = ctx.energy(coords=s.coords * scale)
+        for scale in (1.0, 1.5, 12.0):
+            at = s.copy()
+            at.coords = s.coords * scale
+            ref = oracle.energy(at).energy
+            e = ctx.energy(coords=at.coords)
             eg, g = ctx.energy_grad()
-            print(f"  {e:.12f} J/K {eg:.12f}" + (f" oracle {ref:.12f}" if scale == 1.0 else ""), flush=True)
+            print(f"  x{scale}: {e:.12f} J/K {eg:.12f} oracle {ref:.12f}", flush=True)
+            assert abs(e - ref) <= 1e-9
             assert abs(eg - e) <= 1e-10 and np.all(np.isfinite(g))
-            if scale == 1.0:
-                assert abs(e - ref) <= 1e-9
